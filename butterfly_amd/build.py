@@ -9,6 +9,7 @@ name next to itself (the reference does this in torch_butterfly/__init__.py:8-11
 
     python -m butterfly_amd.build
 """
+import glob
 import os
 import subprocess
 import sys
@@ -67,17 +68,32 @@ def check_kernel_resources(path=RESOURCES):
     return bad, len(gated)
 
 
-def build_hip():
-    cmd = (["hipcc", "-O3", f"--offload-arch={ARCH}", "-std=c++17", "-fPIC", "-shared"] + DEVICE_FLAGS +
-           ["-Rpass-analysis=kernel-resource-usage", "-o", LIB_HIP, os.path.join(CSRC, "butterfly_hip.hip")])
+def _compile_hip(src):
+    """One .hip file to an object beside it; returns (command, exit code, compiler output)."""
+    cmd = (["hipcc", "-O3", f"--offload-arch={ARCH}", "-std=c++17", "-fPIC", "-c"] + DEVICE_FLAGS +
+           ["-Rpass-analysis=kernel-resource-usage", "-o", src[:-len(".hip")] + ".o", src])
     print("+", " ".join(cmd), flush=True)
     r = subprocess.run(cmd, stderr=subprocess.PIPE, text=True)
-    remarks = [l for l in r.stderr.splitlines() if "kernel-resource-usage" in l]
-    other = [l for l in r.stderr.splitlines() if "kernel-resource-usage" not in l]
+    return cmd, r.returncode, r.stderr
+
+
+def build_hip():
+    from concurrent.futures import ThreadPoolExecutor
+    sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
+    with ThreadPoolExecutor(max_workers=min(len(sources), os.cpu_count() or 1, 8)) as pool:
+        results = list(pool.map(_compile_hip, sources))
+    text = "".join(err for _, _, err in results)
+    remarks = [l for l in text.splitlines() if "kernel-resource-usage" in l]
+    other = [l for l in text.splitlines() if "kernel-resource-usage" not in l]
     if other:
         print("\n".join(other), file=sys.stderr, flush=True)
-    if r.returncode != 0:
-        raise subprocess.CalledProcessError(r.returncode, cmd)
+    for cmd, code, _ in results:
+        if code != 0:
+            raise subprocess.CalledProcessError(code, cmd)
+    objects = [src[:-len(".hip")] + ".o" for src in sources]
+    _run(["hipcc", "-shared", f"--offload-arch={ARCH}", "-o", LIB_HIP] + objects)
+    for obj in objects:
+        os.remove(obj)
     with open(RESOURCES, "w") as f:
         f.write("\n".join(remarks) + "\n")
     bad, seen = check_kernel_resources()

@@ -17,10 +17,7 @@
 #include "common.hpp"
 #include "generic.hpp"
 #include "scale.hpp"
-#include "fast.hpp"
-#include "wide.hpp"
-#include "fast4.hpp"
-#include "fast4g.hpp"
+#include "launch.hpp"
 #include "stage.hpp"
 #include "bias.hpp"
 
@@ -98,13 +95,15 @@ Schedule make_schedule(const bf_problem *p, bool base4)
     return sc;
 }
 
-View make_view(const int64_t stride[3], int64_t width, const int *perm = nullptr)
+// tail: width of the last stack where it differs (-1: it does not)
+View make_view(const int64_t stride[3], int64_t width, const int *perm = nullptr, int64_t tail = -1)
 {
     View v;
     v.sb = stride[0];
     v.ss = stride[1];
     v.se = stride[2];
     v.width = width;
+    v.tail = tail < 0 ? width : tail;
     v.perm = perm;
     return v;
 }
@@ -116,6 +115,7 @@ View dense_view(int64_t nstacks, int64_t n)
     v.ss = n;
     v.se = 1;
     v.width = n;
+    v.tail = n;
     v.perm = nullptr;
     return v;
 }
@@ -176,16 +176,11 @@ int num_cu()
     }
     return g_num_cu[device];
 }
-#ifndef BF_FAST_FW_ROWS
-#define BF_FAST_FW_ROWS 4
-#endif
-constexpr int kFastFwRows = BF_FAST_FW_ROWS;  // row groups in flight per forward workgroup
 // Iterations (of kFastFwRows row groups) a forward workgroup must have left before a float pass
 // over two blocks is spread over two workgroups per compute unit (see fw_wg_per_cu).
 #ifndef BF_FAST_FW_PAIR_MIN_ITERS
 #define BF_FAST_FW_PAIR_MIN_ITERS 6
 #endif
-constexpr int kFastFwRowsComplex = 2;       // complex64: half as many (LDS and registers double)
 
 // ---- register-resident multi-pass path (float and complex64, base-2, n <= 2^24) -------------------------
 //
@@ -210,11 +205,6 @@ bool span_ok(const int64_t stride[3], int64_t rows, int64_t width, size_t elem)
 }
 
 constexpr int kMaxPasses = 96;
-// widest span: tiles of 32 consecutive floats (16 consecutive complex64: the same 128 bytes) per
-// setting of the span's bits
-constexpr int kSpanMaxBits = 5;
-constexpr int kSpanMaxBitsComplex = 6;
-constexpr int kSpanMaxStagesComplex = 10;  // stages one complex64 span pass can hold (registers + parked factors)
 constexpr int kMaxLogN = 24;  // the chunk index of the register-resident kernels travels in blockIdx.z
 
 struct Pass {
@@ -247,11 +237,6 @@ int64_t pass_lanes(const bf_problem *p, const Pass &q)
 // not by memory, and two resident workgroups fill each other's gaps (33.3 against 36.2 us at
 // 16384 rows of 1024); each of them loads the whole factor set, so it takes rows to pay off
 // (2048 rows: 10.0 against 8.6 us for one block).  One-block passes run at the memory rate either way.
-// (The 64-register variant of the two-block forward kernel for 512-element rows, decreasing
-// stride first, does not fit its registers -- the build refuses kernels that spill -- so that
-// plan always runs one workgroup per CU.)
-constexpr bool fw_pairable(int L, bool inc) { return !(L == 9 && !inc); }
-
 int fw_wg_per_cu(const bf_problem *p, const Pass &q)
 {
     if (q.wide || q.span || q.NB != 2 || p->dtype != BF_F32 || !fw_pairable(q.L, q.inc)) return 1;
@@ -474,72 +459,6 @@ bool passes_addressable(const bf_problem *p, const PassPlan &pl, bool backward)
     return true;
 }
 
-// paired: the grid holds two workgroups per compute unit (fw_wg_per_cu)
-template <int L, int NB, bool INC>
-void launch_fast_fw_t(bool cplx, bool paired, const FastFwArgs &a, dim3 grid, hipStream_t stream)
-{
-    if constexpr (NB == 1) {
-        if (cplx) {
-            hipLaunchKernelGGL((fast_fw_kernel<float2, FastPlan<L, NB, INC>, kFastFwRowsComplex>), grid, dim3(kFastThreads), 0,
-                               stream, a);
-            return;
-        }
-    } else if constexpr (fw_pairable(L, INC)) {
-        if (paired) {
-            hipLaunchKernelGGL((fast_fw_kernel<float, FastPlan<L, NB, INC>, kFastFwRows, 8>), grid, dim3(kFastThreads), 0,
-                               stream, a);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((fast_fw_kernel<float, FastPlan<L, NB, INC>, kFastFwRows>), grid, dim3(kFastThreads), 0, stream, a);
-}
-
-template <int L, int NB, bool INC>
-void launch_fast_bw_t(bool cplx, bool two_rows, const FastBwArgs &a, dim3 grid, hipStream_t stream)
-{
-    if constexpr (NB == 1) {
-        if (cplx) {
-            hipLaunchKernelGGL((fast_bw_kernel<float2, FastPlan<L, NB, INC>>), grid, dim3(kFastThreads), 0, stream, a);
-            return;
-        }
-        if constexpr (L >= 7) {
-            if (two_rows) {
-                hipLaunchKernelGGL((fast_bw_kernel<float, FastPlan<L, NB, INC>, 2>), grid, dim3(kFastThreads), 0, stream, a);
-                return;
-            }
-        }
-    }
-    hipLaunchKernelGGL((fast_bw_kernel<float, FastPlan<L, NB, INC>>), grid, dim3(kFastThreads), 0, stream, a);
-}
-
-// SpanPlan passes: the LOW kernels on the tiles of a span of q.H high bits.
-template <int H, int MODE>
-bool launch_span_t(bool cplx, bool backward, bool two_rows, const FastFwArgs *fw, const FastBwArgs *bw, dim3 grid,
-                   hipStream_t stream)
-{
-    using P = SpanPlan<H, MODE>;
-    const dim3 block(kFastThreads);
-    // which combinations the host plans: float spans of up to kSpanMaxBits bits, complex64 ones of
-    // up to kSpanMaxBitsComplex bits and kSpanMaxStagesComplex stages
-    constexpr bool for_float = H <= kSpanMaxBits;
-    constexpr bool for_complex = H * (MODE == 2 ? 2 : 1) <= kSpanMaxStagesComplex;
-    if (cplx) {
-        if constexpr (for_complex) {
-            if (!backward) hipLaunchKernelGGL((fast_fw_kernel<float2, P, kFastFwRowsComplex>), grid, block, 0, stream, *fw);
-            else hipLaunchKernelGGL((fast_bw_kernel<float2, P>), grid, block, 0, stream, *bw);
-            return true;
-        }
-        return false;
-    }
-    if constexpr (for_float) {
-        if (!backward) hipLaunchKernelGGL((fast_fw_kernel<float, P, kFastFwRows>), grid, block, 0, stream, *fw);
-        else if (two_rows) hipLaunchKernelGGL((fast_bw_kernel<float, P, 2>), grid, block, 0, stream, *bw);
-        else hipLaunchKernelGGL((fast_bw_kernel<float, P>), grid, block, 0, stream, *bw);
-        return true;
-    }
-    return false;
-}
-
 int launch_span(bool cplx, const Pass &q, bool backward, bool two_rows, const FastFwArgs *fw, const FastBwArgs *bw,
                 dim3 grid, hipStream_t stream)
 {
@@ -549,9 +468,7 @@ int launch_span(bool cplx, const Pass &q, bool backward, bool two_rows, const Fa
     case HH * 3 + 2: ok = launch_span_t<HH, 2>(cplx, backward, two_rows, fw, bw, grid, stream); break;
     bool ok = false;
     switch (q.H * 3 + q.mode) {
-#ifndef BF_DEV_SUBSET
         BF_SPAN_CASES(1) BF_SPAN_CASES(2) BF_SPAN_CASES(3) BF_SPAN_CASES(4) BF_SPAN_CASES(5) BF_SPAN_CASES(6)
-#endif
         default: break;
     }
 #undef BF_SPAN_CASES
@@ -567,19 +484,12 @@ int launch_span(bool cplx, const Pass &q, bool backward, bool two_rows, const Fa
             default: return fail(BF_ERR_UNSUPPORTED, "no fast kernel for this shape");   \
         }                                                                                \
     } while (0)
-// BF_DEV_SUBSET (development builds only): instantiate nothing but the kernels of 1024-element
-// float / complex64 rows, so that a variant of those compiles in a fraction of the time; every
-// other shape answers BF_ERR_UNSUPPORTED.  The shipped library is built without it.
-#ifdef BF_DEV_SUBSET
-#define BF_FAST_SHORT_CASES(FN, ...)
-#else
 #define BF_FAST_SHORT_CASES(FN, ...)                                                     \
     BF_FAST_CASES(FN, 1, __VA_ARGS__) BF_FAST_CASES(FN, 2, __VA_ARGS__)                  \
     BF_FAST_CASES(FN, 3, __VA_ARGS__) BF_FAST_CASES(FN, 4, __VA_ARGS__)                  \
     BF_FAST_CASES(FN, 5, __VA_ARGS__) BF_FAST_CASES(FN, 6, __VA_ARGS__)                  \
     BF_FAST_CASES(FN, 7, __VA_ARGS__) BF_FAST_CASES(FN, 8, __VA_ARGS__)                  \
     BF_FAST_CASES(FN, 9, __VA_ARGS__)
-#endif
 #define BF_FAST_CASES(FN, LL, ...)                              \
     case LL * 4 + 0: FN<LL, 1, false>(__VA_ARGS__); break;      \
     case LL * 4 + 1: FN<LL, 1, true>(__VA_ARGS__); break;       \
@@ -627,19 +537,7 @@ int multipass_forward(const bf_problem *p, const PassPlan &pl, const void *tw, c
                 if (bias_done) *bias_done = true;
             }
             const dim3 grid((unsigned)g.nwg, (unsigned)p->nstacks, 1);
-            const dim3 block(kFastThreads);
-            const bool cplx = p->dtype == BF_C64;
-#ifdef BF_DEV_SUBSET
-            (void)cplx; (void)grid; (void)block; (void)a;
-            return fail(BF_ERR_UNSUPPORTED, "development subset: no whole-block forward kernels");
-#else
-            if (q.L == 12 && q.inc) hipLaunchKernelGGL((wide_fw_kernel<float, 12, true>), grid, block, 0, stream, a);
-            else if (q.L == 12) hipLaunchKernelGGL((wide_fw_kernel<float, 12, false>), grid, block, 0, stream, a);
-            else if (cplx && q.inc) hipLaunchKernelGGL((wide_fw_kernel<float2, 11, true>), grid, block, 0, stream, a);
-            else if (cplx) hipLaunchKernelGGL((wide_fw_kernel<float2, 11, false>), grid, block, 0, stream, a);
-            else if (q.inc) hipLaunchKernelGGL((wide_fw_kernel<float, 11, true>), grid, block, 0, stream, a);
-            else hipLaunchKernelGGL((wide_fw_kernel<float, 11, false>), grid, block, 0, stream, a);
-#endif
+            launch_wide_fw(p->dtype == BF_C64, q.L, q.inc, a, grid, stream);
             BF_HIP_CHECK(hipGetLastError());
         } else {
             const int per_cu = fw_wg_per_cu(p, q);
@@ -676,10 +574,6 @@ int multipass_forward(const bf_problem *p, const PassPlan &pl, const void *tw, c
 
 // ---- base-4 register-resident path (float, even log_n <= 10): one launch per block -----------
 
-constexpr int kFast4FwRows = 4;
-
-constexpr int kFast4GFwRowsComplex = 2;
-
 // base-4 shapes outside fast4.hpp's aligned float kernels
 bool fast4_general(const bf_problem *p) { return p->dtype != BF_F32 || (p->log_n & 1) != 0; }
 
@@ -707,19 +601,9 @@ int fast4_kind(const bf_problem *p, bool base4, bool backward)
 
 bool fast4_ok(const bf_problem *p, bool base4, bool backward) { return fast4_kind(p, base4, backward) != 0; }
 
-template <int L, bool INC>
-void launch_fast4_t(bool backward, const Fast4Args &a, dim3 grid, hipStream_t stream)
-{
-    // row groups per backward iteration: as many as the registers next to the factors allow
-    constexpr int RB = L <= 8 ? 4 : 2;
-    if (backward) hipLaunchKernelGGL((fast4_bw_kernel<L, INC, RB>), grid, dim3(kFastThreads), 0, stream, a);
-    else hipLaunchKernelGGL((fast4_fw_kernel<L, INC, kFast4FwRows>), grid, dim3(kFastThreads), 0, stream, a);
-}
-
 int launch_fast4(int L, bool inc, bool backward, const Fast4Args &a, dim3 grid, hipStream_t stream)
 {
     switch (L * 2 + (inc ? 1 : 0)) {
-#ifndef BF_DEV_SUBSET
         case 2 * 2 + 0: launch_fast4_t<2, false>(backward, a, grid, stream); break;
         case 2 * 2 + 1: launch_fast4_t<2, true>(backward, a, grid, stream); break;
         case 4 * 2 + 0: launch_fast4_t<4, false>(backward, a, grid, stream); break;
@@ -730,21 +614,10 @@ int launch_fast4(int L, bool inc, bool backward, const Fast4Args &a, dim3 grid, 
         case 8 * 2 + 1: launch_fast4_t<8, true>(backward, a, grid, stream); break;
         case 10 * 2 + 0: launch_fast4_t<10, false>(backward, a, grid, stream); break;
         case 10 * 2 + 1: launch_fast4_t<10, true>(backward, a, grid, stream); break;
-#endif
         default: return fail(BF_ERR_UNSUPPORTED, "no base-4 kernel for this shape");
     }
     BF_HIP_CHECK(hipGetLastError());
     return BF_OK;
-}
-
-template <typename T, int L, bool INC>
-void launch_fast4g_t(bool backward, const Fast4GArgs &a, dim3 grid, hipStream_t stream)
-{
-    constexpr int R = sizeof(T) == 4 ? kFast4FwRows : kFast4GFwRowsComplex;
-    // row groups per backward iteration: what the registers next to the factors allow
-    constexpr int RB = sizeof(T) == 4 ? (L <= 7 ? 4 : 2) : (L <= 6 ? 2 : 1);
-    if (backward) hipLaunchKernelGGL((fast4g_bw_kernel<T, L, INC, RB>), grid, dim3(kFastThreads), 0, stream, a);
-    else hipLaunchKernelGGL((fast4g_fw_kernel<T, L, INC, R>), grid, dim3(kFastThreads), 0, stream, a);
 }
 
 // (float L = 10 only runs on the 1024-element chunks of longer rows: whole rows of 1024 take fast4.hpp)
@@ -758,16 +631,12 @@ int launch_fast4g(bool cplx, int L, bool inc, bool backward, const Fast4GArgs &a
     case LL * 2 + 1: launch_fast4g_t<float2, LL, true>(backward, a, grid, stream); break;
     if (cplx) {
         switch (L * 2 + (inc ? 1 : 0)) {
-#ifndef BF_DEV_SUBSET
             BF_C4G(2) BF_C4G(3) BF_C4G(4) BF_C4G(5) BF_C4G(6) BF_C4G(7) BF_C4G(8)
-#endif
             default: return fail(BF_ERR_UNSUPPORTED, "no base-4 kernel for this shape");
         }
     } else {
         switch (L * 2 + (inc ? 1 : 0)) {
-#ifndef BF_DEV_SUBSET
             BF_F4G(3) BF_F4G(5) BF_F4G(7) BF_F4G(9) BF_F4G(10)
-#endif
             default: return fail(BF_ERR_UNSUPPORTED, "no base-4 kernel for this shape");
         }
     }
@@ -1132,7 +1001,7 @@ int check_perms(const bf_problem *p, bool base4, const int *in_perm, const int *
 
 int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, const void *input,
             void *output, void *workspace, size_t workspace_bytes, void *stream_, const void *bias = nullptr,
-            const int *in_perm = nullptr, const int *out_index = nullptr)
+            const int *in_perm = nullptr, const int *out_index = nullptr, int64_t tail = -1)
 {
     int rc = check_problem(p, false);
     if (rc) return rc;
@@ -1151,7 +1020,7 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
         }
     }
     const View in_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
-    const View out_view = make_view(p->output_stride, p->output_size, out_index);
+    const View out_view = make_view(p->output_stride, p->output_size, out_index, tail);
     if (fast4_ok(p, base4, false)) {
         const size_t need = forward_workspace(p, base4);
         if (need > 0 && (!workspace || workspace_bytes < need))
@@ -1195,10 +1064,18 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
 
 // ---- bias gradient ------------------------------------------------------------------------------
 
+// The column sums of the output gradient: `nparts` slices of (S, stride) scalars each, added up by
+// reduce_partials_kernel.  Enough row partitions to fill the GPU, but no fewer than kBiasMinRows
+// rows each: more slices only make the second step longer (1024 slices of two rows each took
+// 206 us at 2048 rows of 512).
+constexpr int64_t kBiasMinRows = 16;
+
 struct BiasGradPlan {
     int64_t cols, nparts, rows_per_part;
     size_t bytes;
 };
+
+int64_t bias_stride(const bf_problem *p) { return (p->output_size + 3) & ~(int64_t)3; }
 
 BiasGradPlan plan_bias_grad(const bf_problem *p)
 {
@@ -1206,31 +1083,42 @@ BiasGradPlan plan_bias_grad(const bf_problem *p)
     if (p->batch <= 0 || p->nstacks <= 0 || p->output_size <= 0) return b;
     b.cols = (p->output_size + kBiasThreads - 1) / kBiasThreads;
     const int64_t want = std::max<int64_t>(1, (int64_t)num_cu() * 8 / (b.cols * p->nstacks));
-    b.nparts = std::min<int64_t>(std::min<int64_t>(want, p->batch), 65535);
+    b.nparts = std::min<int64_t>(want, (p->batch + kBiasMinRows - 1) / kBiasMinRows);
     b.rows_per_part = (p->batch + b.nparts - 1) / b.nparts;
     b.nparts = (p->batch + b.rows_per_part - 1) / b.rows_per_part;
-    b.bytes = align256((size_t)b.nparts * p->nstacks * p->output_size * elem_bytes(p->dtype));
+    b.bytes = align256((size_t)b.nparts * p->nstacks * bias_stride(p) * elem_bytes(p->dtype));
     return b;
 }
 
-template <typename T>
-int launch_bias_grad(const bf_problem *p, const BiasGradPlan &b, const void *grad, void *d_bias, void *workspace,
-                     hipStream_t stream, const int *out_index)
+// What a backward call that also returns the bias gradient carries: the area for the partial
+// column sums, where the result goes, and -- once they have been formed -- the number of slices.
+struct BiasGrad {
+    void *area = nullptr;
+    void *d_bias = nullptr;
+    int64_t nparts = 0;
+    bool formed = false;
+};
+
+// First step of the bias gradient as a kernel of its own, for backward kernels that do not form
+// the column sums on the way.
+int form_bias_sums(const bf_problem *p, const void *grad, const View &g_view, BiasGrad &bg, hipStream_t stream)
 {
+    const BiasGradPlan b = plan_bias_grad(p);
+    bg.formed = true;
+    bg.nparts = b.nparts;
+    if (b.nparts == 0) return BF_OK;
     BiasArgs a = {};
     a.grad = grad;
-    a.view = make_view(p->output_stride, p->output_size, out_index);
-    a.partial = workspace;
-    a.d_bias = d_bias;
+    a.view = g_view;
+    a.partial = bg.area;
+    a.stride = bias_stride(p);
     a.batch = p->batch;
     a.width = p->output_size;
     a.rows_per_part = b.rows_per_part;
     a.nparts = b.nparts;
-    const dim3 grid1((unsigned)b.cols, (unsigned)p->nstacks, (unsigned)b.nparts);
-    hipLaunchKernelGGL((bias_grad_partial_kernel<T>), grid1, dim3(kBiasThreads), 0, stream, a);
-    BF_HIP_CHECK(hipGetLastError());
-    const dim3 grid2((unsigned)b.cols, (unsigned)p->nstacks, 1);
-    hipLaunchKernelGGL((bias_grad_final_kernel<T>), grid2, dim3(kBiasThreads), 0, stream, a);
+    const dim3 grid((unsigned)b.cols, (unsigned)p->nstacks, (unsigned)b.nparts);
+    if (p->dtype == BF_C64) hipLaunchKernelGGL((bias_grad_partial_kernel<float2>), grid, dim3(kBiasThreads), 0, stream, a);
+    else hipLaunchKernelGGL((bias_grad_partial_kernel<float>), grid, dim3(kBiasThreads), 0, stream, a);
     BF_HIP_CHECK(hipGetLastError());
     return BF_OK;
 }
@@ -1377,13 +1265,16 @@ int launch_copy_pad(const bf_problem *p, const void *in, const View &iv, void *o
     return BF_OK;
 }
 
+// bg (may be NULL): bias sums to be added up by the same launch; g_view: the view they were read through
 int launch_reduce(const bf_problem *p, const Schedule &sc, int t0, int t1, int64_t nparts, const void *partial,
-                  int64_t slot, void *d_tw2, void *d_tw4, hipStream_t stream)
+                  int64_t slot, void *d_tw2, void *d_tw4, hipStream_t stream, const BiasGrad *bg = nullptr,
+                  const View *g_view = nullptr)
 {
-    if (p->nstacks == 0 || t1 <= t0) return BF_OK;
+    const bool bias = bg && bg->d_bias && g_view->width > 0;
+    if (p->nstacks == 0 || (t1 <= t0 && !bias)) return BF_OK;
     if (((reinterpret_cast<uintptr_t>(d_tw2) | reinterpret_cast<uintptr_t>(d_tw4)) & 15) != 0)
         return fail(BF_ERR_INVALID, "d_twiddle pointers must be 16-byte aligned");
-    ReduceArgs r;
+    ReduceArgs r = {};
     r.sc = sc;
     r.t0 = t0;
     r.t1 = t1;
@@ -1394,21 +1285,29 @@ int launch_reduce(const bf_problem *p, const Schedule &sc, int t0, int t1, int64
     r.slot = slot;
     r.d_tw2 = static_cast<float *>(d_tw2);
     r.d_tw4 = static_cast<float *>(d_tw4);
-    const dim3 grid((unsigned)((slot * r.elem_floats + 63) / 64), (unsigned)(t1 - t0), (unsigned)p->nstacks);
+    int64_t floats = t1 > t0 ? slot * r.elem_floats : 0;
+    if (bias) {
+        r.bias_partial = static_cast<const float *>(bg->area);
+        r.d_bias = static_cast<float *>(bg->d_bias);
+        r.bias_nparts = (int)bg->nparts;
+        r.bias_stride = bias_stride(p);
+        r.bias_width = g_view->width;
+        r.bias_tail = g_view->tail;
+        floats = std::max(floats, g_view->width * r.elem_floats);
+    }
+    const dim3 grid((unsigned)((floats + 63) / 64), (unsigned)(t1 - t0 + (bias ? 1 : 0)), (unsigned)p->nstacks);
     hipLaunchKernelGGL(reduce_partials_kernel, grid, dim3(256), 0, stream, r);
     BF_HIP_CHECK(hipGetLastError());
     return BF_OK;
 }
 
-// bias_partial / bias_nparts: when given, and when the pass that reads `grad` runs in a kernel
-// that can do it, that kernel also leaves the per-workgroup column sums of grad there
-// (*bias_nparts slices of (S, output_size)); *bias_nparts stays 0 otherwise.
+// bg (may be NULL): the bias gradient is wanted too.  A kernel that can forms the column sums of
+// `grad` while it reads it, otherwise a kernel of its own does; the call's first reduce adds them up.
 int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, const void *input,
              const void *grad, void *d_tw2, void *d_tw4, void *d_input, void *workspace,
-             size_t workspace_bytes, void *stream_, void *bias_partial = nullptr, int64_t *bias_nparts = nullptr,
-             const int *in_perm = nullptr, const int *out_index = nullptr, const void *saved = nullptr)
+             size_t workspace_bytes, void *stream_, BiasGrad *bg = nullptr,
+             const int *in_perm = nullptr, const int *out_index = nullptr, const void *saved = nullptr, int64_t tail = -1)
 {
-    if (bias_nparts) *bias_nparts = 0;
     int rc = check_problem(p, true);
     if (rc) return rc;
     if ((rc = check_perms(p, base4, in_perm, out_index))) return rc;
@@ -1417,9 +1316,10 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     const Schedule sc = make_schedule(p, base4);
     const int64_t n = (int64_t)1 << p->log_n;
     const bool permuted = in_perm || out_index;
+    const View g_view = make_view(p->output_stride, std::min(p->output_size, n), out_index, tail);
     if (p->batch == 0 || p->nstacks == 0) {
-        // no rows: d_input is empty and every d_twiddle entry is an empty sum, whatever the row length
-        return launch_reduce(p, sc, 0, sc.per * sc.nblocks, 0, nullptr, 4 * n, d_tw2, d_tw4, stream);
+        // no rows: d_input is empty and every entry of the other gradients is an empty sum, whatever the row length
+        return launch_reduce(p, sc, 0, sc.per * sc.nblocks, 0, nullptr, 4 * n, d_tw2, d_tw4, stream, bg, &g_view);
     }
     const BwPlan pl = plan_bw(p, base4, saved != nullptr, permuted);
     if (!pl.fits)
@@ -1434,13 +1334,26 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
         return fail(BF_ERR_INVALID, "twiddle and d_twiddle must be 16-byte aligned");
 
     const View x_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
-    const View g_view = make_view(p->output_stride, std::min(p->output_size, n), out_index);
     const View di_view = make_view(p->d_input_stride, p->input_size, in_perm);
     const View dense = dense_view(p->nstacks, n);
     char *ws = static_cast<char *>(workspace);
     const size_t e_bytes = elem_bytes(p->dtype);
 
-    if (pl.nstages == 0) return launch_copy_pad(p, grad, g_view, d_input, di_view, stream);
+    // the reduce of the pass that reads grad, the first one, also finishes the bias gradient
+    auto reduce = [&](int t0, int t1, int64_t nparts) {
+        if (bg && !bg->formed) {
+            const int rc_bias = form_bias_sums(p, grad, g_view, *bg, stream);
+            if (rc_bias) return rc_bias;
+        }
+        BiasGrad *now = bg;
+        bg = nullptr;
+        return launch_reduce(p, sc, t0, t1, nparts, ws + pl.off_partials, pl.slot, d_tw2, d_tw4, stream, now, &g_view);
+    };
+
+    if (pl.nstages == 0) {
+        if (bg && (rc = reduce(0, 0, 0))) return rc;
+        return launch_copy_pad(p, grad, g_view, d_input, di_view, stream);
+    }
 
     if (pl.fast4) {
         const int L = (int)p->log_n;
@@ -1473,8 +1386,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             const bool inc = (p->increasing_stride != 0) != ((k & 1) != 0);
             rc = launch_fast4g(p->dtype == BF_C64, L, inc, true, a, dim3((unsigned)g.nwg, (unsigned)p->nstacks), stream);
             if (rc) return rc;
-            rc = launch_reduce(p, sc, k * per, (k + 1) * per, g.nwg, ws + pl.off_partials, pl.slot, d_tw2, d_tw4,
-                               stream);
+            rc = reduce(k * per, (k + 1) * per, g.nwg);
             if (rc) return rc;
         }
         if (!general && (reinterpret_cast<uintptr_t>(tw4) & 15) != 0)
@@ -1496,8 +1408,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             const bool inc = (p->increasing_stride != 0) != ((k & 1) != 0);
             rc = launch_fast4(L, inc, true, a, dim3((unsigned)g.nwg, (unsigned)p->nstacks), stream);
             if (rc) return rc;
-            rc = launch_reduce(p, sc, k * per, (k + 1) * per, g.nwg, ws + pl.off_partials, pl.slot, d_tw2, d_tw4,
-                               stream);
+            rc = reduce(k * per, (k + 1) * per, g.nwg);
             if (rc) return rc;
         }
         if (p->input_size > n) {
@@ -1534,7 +1445,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                            k == 0 ? d_input : ws + pl.off_gbuf, k == 0 ? dn_view : dense, ws + pl.off_partials, &nparts,
                            stream);
             if (rc) return rc;
-            rc = launch_reduce(p, sc, q.t0, q.t1, nparts, ws + pl.off_partials, pl.slot, d_tw2, d_tw4, stream);
+            rc = reduce(q.t0, q.t1, nparts);
             if (rc) return rc;
         }
         if (p->input_size > n) {
@@ -1589,10 +1500,11 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 a.ngroups = g.ngroups;
                 a.groups_per_wg = g.groups_per_wg;
                 nparts = g.nwg;
-                if (k == P - 1 && bias_partial && bias_nparts && q.L == 10 && p->dtype == BF_F32 && g.nwg <= num_cu()) {
-                    a.bias_partial = bias_partial;
-                    a.bias_width = p->output_size;
-                    *bias_nparts = g.nwg;
+                if (k == P - 1 && bg && q.L == 10 && p->dtype == BF_F32 && g.nwg <= num_cu()) {
+                    a.bias_partial = bg->area;
+                    a.bias_stride = bias_stride(p);
+                    bg->nparts = g.nwg;
+                    bg->formed = true;
                 }
                 const dim3 grid((unsigned)g.nwg, (unsigned)p->nstacks, (unsigned)pass_lanes(p, q));
                 // two row groups in flight once a workgroup has enough of them to fill the pipeline
@@ -1605,7 +1517,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 }
                 BF_HIP_CHECK(hipGetLastError());
             }
-            rc = launch_reduce(p, sc, q.t0, q.t1, nparts, ws + pl.off_partials, pl.slot, d_tw2, d_tw4, stream);
+            rc = reduce(q.t0, q.t1, nparts);
             if (rc) return rc;
         }
         if (p->input_size > n) {
@@ -1658,8 +1570,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 hipLaunchKernelGGL(generic_bw_kernel<float2>, grid, dim3(kGenericThreads), lds, stream, a);
             BF_HIP_CHECK(hipGetLastError());
         }
-        rc = launch_reduce(p, sc, t0, t1, have_rows ? pl.nparts : 0, ws + pl.off_partials, pl.slot, d_tw2, d_tw4,
-                           stream);
+        rc = reduce(t0, t1, have_rows ? pl.nparts : 0);
         if (rc) return rc;
     }
     return BF_OK;
@@ -1776,38 +1687,34 @@ size_t bf_butterfly_bias_grad_workspace_bytes(const bf_problem *p)
     return plan_bias_grad(p).bytes;
 }
 
-// d_bias[s][c] = sum over the batch of grad[b][s][out_index[c]] (out_index NULL: column c)
+// d_bias[s][c] = sum over the batch of grad[b][s][c]
 static int bias_grad(const bf_problem *p, const void *grad, void *d_bias, void *workspace, size_t workspace_bytes,
-                     void *stream, const int *out_index)
+                     void *stream)
 {
     int rc = check_problem(p, false);
     if (rc) return rc;
     if (p->nstacks <= 0 || p->output_size <= 0) return BF_OK;
     if (!d_bias) return fail(BF_ERR_INVALID, "d_bias is NULL");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (p->batch <= 0) {
-        // an empty batch sums to zero: the final kernel over zero partitions writes exactly that
-        BiasArgs a = {};
-        a.d_bias = d_bias;
-        a.width = p->output_size;
-        const dim3 grid((unsigned)((p->output_size + kBiasThreads - 1) / kBiasThreads), (unsigned)p->nstacks, 1);
-        if (p->dtype == BF_C64) hipLaunchKernelGGL((bias_grad_final_kernel<float2>), grid, dim3(kBiasThreads), 0, s, a);
-        else hipLaunchKernelGGL((bias_grad_final_kernel<float>), grid, dim3(kBiasThreads), 0, s, a);
-        BF_HIP_CHECK(hipGetLastError());
-        return BF_OK;
+    BiasGrad bg;
+    bg.area = workspace;
+    bg.d_bias = d_bias;
+    const View g_view = make_view(p->output_stride, p->output_size);
+    if (p->batch > 0) {
+        if (!grad) return fail(BF_ERR_INVALID, "grad is NULL");
+        const size_t need = plan_bias_grad(p).bytes;
+        if (!workspace || workspace_bytes < need)
+            return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+        if ((rc = form_bias_sums(p, grad, g_view, bg, s))) return rc;
     }
-    if (!grad) return fail(BF_ERR_INVALID, "grad is NULL");
-    const BiasGradPlan b = plan_bias_grad(p);
-    if (!workspace || workspace_bytes < b.bytes)
-        return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", b.bytes, workspace_bytes);
-    return p->dtype == BF_C64 ? launch_bias_grad<float2>(p, b, grad, d_bias, workspace, s, out_index)
-                              : launch_bias_grad<float>(p, b, grad, d_bias, workspace, s, out_index);
+    // (over no rows the sums of zero slices: zeros)
+    return launch_reduce(p, make_schedule(p, false), 0, 0, 0, nullptr, 0, nullptr, nullptr, s, &bg, &g_view);
 }
 
 int bf_butterfly_bias_grad(const bf_problem *p, const void *grad, void *d_bias, void *workspace,
                            size_t workspace_bytes, void *stream)
 {
-    return bias_grad(p, grad, d_bias, workspace, workspace_bytes, stream, nullptr);
+    return bias_grad(p, grad, d_bias, workspace, workspace_bytes, stream);
 }
 
 // Bias area behind the backward workspace: room for either the per-workgroup column sums the
@@ -1816,7 +1723,7 @@ int bf_butterfly_bias_grad(const bf_problem *p, const void *grad, void *d_bias, 
 static size_t bias_area_bytes(const bf_problem *p)
 {
     const size_t fused = align256((size_t)num_cu() * std::max<int64_t>(p->nstacks, 1) *
-                                  std::max<int64_t>(p->output_size, 0) * elem_bytes(p->dtype));
+                                  std::max<int64_t>(bias_stride(p), 0) * elem_bytes(p->dtype));
     return std::max(fused, plan_bias_grad(p).bytes);
 }
 
@@ -1837,26 +1744,11 @@ static int bias_backward(const bf_problem *p, const void *twiddle, const void *i
     if (!workspace || workspace_bytes < need)
         return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     if (!d_bias && p->nstacks > 0 && p->output_size > 0) return fail(BF_ERR_INVALID, "d_bias is NULL");
-    char *area = static_cast<char *>(workspace) + main_bytes;
-    int64_t nparts = 0;
-    rc = backward(p, false, twiddle, nullptr, input, grad, d_twiddle, nullptr, d_input, workspace, main_bytes, stream,
-                  area, &nparts, in_perm, out_index, saved);
-    if (rc) return rc;
-    if (p->nstacks <= 0 || p->output_size <= 0) return BF_OK;
-    if (nparts > 0) {
-        // the backward kernel left one slice of column sums per workgroup: add them up in order
-        BiasArgs a = {};
-        a.partial = area;
-        a.d_bias = d_bias;
-        a.width = p->output_size;
-        a.nparts = nparts;
-        const dim3 grid((unsigned)((p->output_size + kBiasThreads - 1) / kBiasThreads), (unsigned)p->nstacks, 1);
-        hipLaunchKernelGGL((bias_grad_final_kernel<float>), grid, dim3(kBiasThreads), 0,
-                           static_cast<hipStream_t>(stream), a);
-        BF_HIP_CHECK(hipGetLastError());
-        return BF_OK;
-    }
-    return bias_grad(p, grad, d_bias, area, bias_area_bytes(p), stream, out_index);
+    BiasGrad bg;
+    bg.area = static_cast<char *>(workspace) + main_bytes;
+    bg.d_bias = d_bias;
+    return backward(p, false, twiddle, nullptr, input, grad, d_twiddle, nullptr, d_input, workspace, main_bytes, stream,
+                    &bg, in_perm, out_index, saved);
 }
 
 int bf_butterfly_multiply_bias_bw(const bf_problem *p, const void *twiddle, const void *input, const void *grad,
@@ -1883,7 +1775,7 @@ int bf_butterfly_multiply_perm_bw(const bf_problem *p, const void *twiddle, cons
         return bias_backward(p, twiddle, input, grad, d_twiddle, d_input, d_bias, workspace, workspace_bytes, stream,
                              in_perm, out_index);
     return backward(p, false, twiddle, nullptr, input, grad, d_twiddle, nullptr, d_input, workspace, workspace_bytes,
-                    stream, nullptr, nullptr, in_perm, out_index);
+                    stream, nullptr, in_perm, out_index);
 }
 
 // Bytes of activations the saving forward leaves for the backward: one dense (B, S, n) plane per
@@ -1977,7 +1869,7 @@ int bf_butterfly_multiply_bw_saved(const bf_problem *p, const void *twiddle, con
         return bias_backward(p, twiddle, input, grad, d_twiddle, d_input, d_bias, workspace, workspace_bytes, stream,
                              in_perm, out_index, saved);
     return backward(p, false, twiddle, nullptr, input, grad, d_twiddle, nullptr, d_input, workspace, workspace_bytes,
-                    stream, nullptr, nullptr, in_perm, out_index, saved);
+                    stream, nullptr, in_perm, out_index, saved);
 }
 
 // One line per launch group of the base-2 schedule, e.g. "low t=0..10 L=10 nb=1 inc=1 chunks=8".
@@ -2105,7 +1997,7 @@ int bf_butterfly_multiply_base4_bw_saved(const bf_problem *p, const void *twiddl
         return fail(BF_ERR_WORKSPACE, "the backward reads %zu bytes of saved activations, %zu given", planes,
                     saved_bytes_given);
     return backward(p, true, twiddle2, twiddle4, input, grad, d_twiddle2, d_twiddle4, d_input, workspace,
-                    workspace_bytes, stream, nullptr, nullptr, nullptr, nullptr, saved);
+                    workspace_bytes, stream, nullptr, nullptr, nullptr, saved);
 }
 
 static int scale_twiddle(bool bw, int dtype, int64_t nstacks, int64_t nblocks, int64_t log_n, int increasing_stride,

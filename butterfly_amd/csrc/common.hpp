@@ -100,6 +100,7 @@ __host__ __device__ __forceinline__ StageInfo stage_info(const Schedule &sc, int
 struct View {
     int64_t sb, ss, se;
     int64_t width;
+    int64_t tail;     // width of the last stack (a layer's outputs need not fill its last stack)
     const int *perm;  // NULL, or n entries: column c of the row as the kernels see it lives in tensor column perm[c]
 };
 
@@ -110,6 +111,13 @@ __device__ __forceinline__ int64_t view_col(const View &v, int64_t col)
 {
     if (v.perm) col = v.perm[col];
     return col < v.width ? col : -1;
+}
+
+// The view as the workgroups of one stack use it.
+__device__ __forceinline__ View stack_view(View v, int stack, int nstacks)
+{
+    if (stack == nstacks - 1) v.width = v.tail;
+    return v;
 }
 
 }  // namespace bf

@@ -763,10 +763,11 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
     const __amdgpu_buffer_rsrc_t out_rs =
         make_rsrc(reinterpret_cast<T *>(a.out) + g0 * SLOTS * a.out_view.sb + stack * a.out_view.ss);
     // thread-constant part of the offsets; the row group adds a wave-uniform part
-    const int64_t in_col = view_col(a.in_view, col), out_col = view_col(a.out_view, col);
+    const View out_view = stack_view(a.out_view, stack, gridDim.y);
+    const int64_t in_col = view_col(a.in_view, col), out_col = view_col(out_view, col);
     const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.in_view.se * EB) : kOob;
     const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.out_view.se * EB) : kOob;
-    const T bias = (a.bias && col < a.out_view.width)
+    const T bias = (a.bias && col < out_view.width)
                        ? reinterpret_cast<const T *>(a.bias)[stack * a.out_view.width + col]
                        : zero_of(T());
 
@@ -893,9 +894,9 @@ struct FastBwArgs {
     int64_t ngroups;
     int64_t groups_per_wg;
     // float kernels on 1024-element rows or chunks only: when set, the column sums of g_out over
-    // this workgroup's rows (a layer's bias gradient) go to (gridDim.x, S, bias_width)
+    // this workgroup's rows (a layer's bias gradient) go to (gridDim.x, S, bias_stride)
     void *bias_partial;
-    int64_t bias_width;
+    int64_t bias_stride;
 };
 
 // Backward kernel, software-pipelined over rows: iteration i runs the forward replay of
@@ -1156,7 +1157,8 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
 
     // --- operand fetch, register flavour: thread t holds its layout-A element
     const __amdgpu_buffer_rsrc_t x_rs = make_rsrc(x_base), g_rs = make_rsrc(g_base);
-    const int64_t x_col = view_col(a.x_view, col), g_col = view_col(a.g_view, col);
+    const View g_view = stack_view(a.g_view, stack, gridDim.y);
+    const int64_t x_col = view_col(a.x_view, col), g_col = view_col(g_view, col);
     const int x_thr = x_col >= 0 ? c.slot * x_row + (int)(x_col * a.x_view.se * EB) : kOob;
     const int g_thr = g_col >= 0 ? c.slot * g_row + (int)(g_col * a.g_view.se * EB) : kOob;
     auto load_x = [&](int grp, bool full = false) {
@@ -1171,7 +1173,7 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
     // group, which lands at the padded word 65 w + l of the slot
     const BufDesc x_desc = make_desc(x_base), g_desc = make_desc(g_base);
     const int slot_d = t >> L, col_d = P::column(chunk, t & (n - 1), a.low_bits);
-    const int64_t x_col_d = view_col(a.x_view, col_d), g_col_d = view_col(a.g_view, col_d);
+    const int64_t x_col_d = view_col(a.x_view, col_d), g_col_d = view_col(g_view, col_d);
     const int x_dma = x_col_d >= 0 ? slot_d * x_row + (int)(x_col_d * a.x_view.se * EB) : kOob;
     const int g_dma = g_col_d >= 0 ? slot_d * g_row + (int)(g_col_d * a.g_view.se * EB) : kOob;
     // (wave-uniform: kept in a scalar register, so the per-row slot offsets are scalar additions)
@@ -1538,8 +1540,8 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
     if constexpr (BIAS_SUM) {
         if (bias_on) {
             const int64_t bcol = P::column(chunk, Q::SB ? c2.eB : c2.eA, a.low_bits);
-            if (bcol < a.bias_width)
-                reinterpret_cast<float *>(a.bias_partial)[((int64_t)blockIdx.x * gridDim.y + stack) * a.bias_width +
+            if (bcol < a.g_view.width)
+                reinterpret_cast<float *>(a.bias_partial)[((int64_t)blockIdx.x * gridDim.y + stack) * a.bias_stride +
                                                           bcol] = lds_bias[t2];
         }
     }

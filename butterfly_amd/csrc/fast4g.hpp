@@ -145,7 +145,8 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_fw_kernel(Fast4GArgs a)
     const __amdgpu_buffer_rsrc_t out_rs =
         make_rsrc(reinterpret_cast<T *>(a.x_out) + g0 * SLOTS * a.xo_view.sb + stack * a.xo_view.ss);
     const int in_row = (int)(a.x_view.sb * EB), out_row = (int)(a.xo_view.sb * EB);
-    const int64_t in_col = view_col(a.x_view, col), out_col = view_col(a.xo_view, col);
+    const int64_t in_col = view_col(a.x_view, col);
+    const int64_t out_col = view_col(stack_view(a.xo_view, stack, gridDim.y), col);
     const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.x_view.se * EB) : kOob;
     const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.xo_view.se * EB) : kOob;
 
@@ -247,7 +248,8 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_bw_kernel(Fast4GArgs a)
     const __amdgpu_buffer_rsrc_t gi_rs =
         make_rsrc(reinterpret_cast<T *>(a.g_in) + g0 * SLOTS * a.gi_view.sb + stack * a.gi_view.ss);
     const int x_row = (int)(a.x_view.sb * EB), g_row = (int)(a.g_view.sb * EB), gi_row = (int)(a.gi_view.sb * EB);
-    const int64_t x_col = view_col(a.x_view, col), g_col = view_col(a.g_view, col), gi_col = view_col(a.gi_view, col);
+    const int64_t x_col = view_col(a.x_view, col), gi_col = view_col(a.gi_view, col);
+    const int64_t g_col = view_col(stack_view(a.g_view, stack, gridDim.y), col);
     const int x_thr = x_col >= 0 ? c.slot * x_row + (int)(x_col * a.x_view.se * EB) : kOob;
     const int g_thr = g_col >= 0 ? c.slot * g_row + (int)(g_col * a.g_view.se * EB) : kOob;
     const int gi_thr = gi_col >= 0 ? c.slot * gi_row + (int)(gi_col * a.gi_view.se * EB) : kOob;

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kGenericThreads) void generic_fw_kernel(GenericFwAr
     T *out = reinterpret_cast<T *>(a.out);
     for (int it = tid; it < (rows << log_n); it += kGenericThreads) {
         const int r = it >> log_n, j = it & (n - 1);
-        const int64_t jc = view_col(a.out_view, j);
+        const int64_t jc = view_col(stack_view(a.out_view, s, gridDim.y), j);
         if (jc >= 0) out[(b0 + r) * a.out_view.sb + s * a.out_view.ss + jc * a.out_view.se] = buf[it];
     }
 }
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kGenericThreads) void generic_bw_kernel(GenericBwAr
     for (int64_t b = blockIdx.x; b < a.batch; b += gridDim.x) {
         for (int j = tid; j < n; j += kGenericThreads) {
             T v = zero_of(T()), gv = zero_of(T());
-            const int64_t xc = view_col(a.x_view, j), gc = view_col(a.g_view, j);
+            const int64_t xc = view_col(a.x_view, j), gc = view_col(stack_view(a.g_view, s, gridDim.y), j);
             if (xc >= 0) v = x_in[b * a.x_view.sb + s * a.x_view.ss + xc * a.x_view.se];
             if (gc >= 0) gv = g_out[b * a.g_view.sb + s * a.g_view.ss + gc * a.g_view.se];
             xs[j] = v;
@@ -263,6 +263,12 @@ struct ReduceArgs {
     int64_t slot;      // scalars reserved per stage in `partial`
     float *d_tw2;
     float *d_tw4;
+    // a layer's bias gradient: one more slice of workgroups (blockIdx.y = t1 - t0) adds up its
+    // partial column sums, (bias_nparts, S, bias_stride) -> (S, bias_width) without its unused tail
+    const float *bias_partial;   // NULL: none
+    float *d_bias;
+    int bias_nparts;
+    int64_t bias_stride, bias_width, bias_tail;   // scalars
 };
 
 // d_twiddle[s][stage][j] = sum over partial slices.  Works on raw floats (a complex sum is
@@ -270,7 +276,7 @@ struct ReduceArgs {
 // of group q (a contiguous sixteenth of them, ascending) for the float4 at j4; the sixteen
 // group sums are then added in ascending q.  The order is fixed by nparts alone, so results
 // are reproducible run to run.
-// grid: (ceil(slot * elem_floats / 64), t1 - t0, S), block 256.
+// grid: (ceil(slot * elem_floats / 64), t1 - t0 (+ 1 with a bias), S), block 256.
 __global__ __launch_bounds__(256) void reduce_partials_kernel(ReduceArgs a)
 {
     __shared__ float4 sm[16][16];
@@ -278,19 +284,22 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(ReduceArgs a)
     const int k = blockIdx.y;
     const int s = blockIdx.z;
     const int nst = a.t1 - a.t0;
-    const StageInfo si = stage_info(a.sc, a.t0 + k);
+    const bool is_bias = k == nst;
+    const StageInfo si = stage_info(a.sc, a.t0 + (is_bias ? 0 : k));
     const int64_t n = (int64_t)1 << a.sc.log_n;
     const int64_t ef = a.elem_floats;
-    const int64_t count = (si.radix4 ? 4 * n : 2 * n) * ef;   // floats in this stage
     const int64_t f = (int64_t)blockIdx.x * 64 + j4 * 4;
     const int64_t slot_f = a.slot * ef;
-    const int64_t wg_stride = a.nstacks * nst * slot_f;
-    const int chunk = (a.nparts + 15) / 16;
+    // floats that exist here, floats between the slices, slices
+    const int64_t count = is_bias ? (s == a.nstacks - 1 ? a.bias_tail : a.bias_width) * ef : (si.radix4 ? 4 * n : 2 * n) * ef;
+    const int64_t wg_stride = a.nstacks * (is_bias ? a.bias_stride * ef : nst * slot_f);
+    const int nparts = is_bias ? a.bias_nparts : a.nparts;
+    const int chunk = (nparts + 15) / 16;
     const int w0 = q * chunk;
-    const int w1 = w0 + chunk < a.nparts ? w0 + chunk : a.nparts;
+    const int w1 = w0 + chunk < nparts ? w0 + chunk : nparts;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     if (f < count) {
-        const float *src = a.partial + ((int64_t)s * nst + k) * slot_f + f;
+        const float *src = is_bias ? a.bias_partial + s * a.bias_stride * ef + f : a.partial + ((int64_t)s * nst + k) * slot_f + f;
 #pragma unroll 8
         for (int w = w0; w < w1; ++w) {
             const float4 v = *reinterpret_cast<const float4 *>(src + (int64_t)w * wg_stride);
@@ -305,6 +314,15 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(ReduceArgs a)
         for (int qq = 1; qq < 16; ++qq) {
             const float4 v = sm[qq][j4];
             t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+        }
+        if (is_bias) {
+            // (any width: neither the columns nor the stacks need start at a multiple of four)
+            float *dst = a.d_bias + s * a.bias_width * ef + f;
+            const float v[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (f + i < count) dst[i] = v[i];
+            return;
         }
         float *dst = si.radix4 ? a.d_tw4 + (s * a.sc.tw4_stack_stride + si.tw_off) * ef
                                : a.d_tw2 + (s * a.sc.tw2_stack_stride + si.tw_off) * ef;

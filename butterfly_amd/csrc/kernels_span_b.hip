@@ -1,0 +1,11 @@
+// Kernels on spans of 4 to 6 high bits (fast.hpp, SpanPlan).
+#include "launch_impl.hpp"
+
+namespace bf {
+
+#define BF_ONE(H, MODE) \
+    template bool launch_span_t<H, MODE>(bool, bool, bool, const FastFwArgs *, const FastBwArgs *, dim3, hipStream_t);
+#define BF_INST(H) BF_ONE(H, 0) BF_ONE(H, 1) BF_ONE(H, 2)
+BF_INST(4) BF_INST(5) BF_INST(6)
+
+}  // namespace bf

@@ -123,15 +123,16 @@ __global__ __launch_bounds__(kFastThreads) void wide_fw_kernel(FastFwArgs a)
     const __amdgpu_buffer_rsrc_t out_rs =
         make_rsrc(reinterpret_cast<T *>(a.out) + r0 * a.out_view.sb + stack * a.out_view.ss);
     const int in_row = (int)(a.in_view.sb * EB), out_row = (int)(a.out_view.sb * EB);
+    const View out_view = stack_view(a.out_view, stack, gridDim.y);
     int in_thr[Q], out_thr[Q], in_dma[Q];
     T bias[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         const int col = (q << 10) | c.eA;
-        bias[q] = (a.bias && col < a.out_view.width)
+        bias[q] = (a.bias && col < out_view.width)
                       ? reinterpret_cast<const T *>(a.bias)[stack * a.out_view.width + col]
                       : zero_of(T());
-        const int64_t in_col = view_col(a.in_view, col), out_col = view_col(a.out_view, col);
+        const int64_t in_col = view_col(a.in_view, col), out_col = view_col(out_view, col);
         in_thr[q] = in_col >= 0 ? (int)(in_col * a.in_view.se * EB) : kOob;
         out_thr[q] = out_col >= 0 ? (int)(out_col * a.out_view.se * EB) : kOob;
         const int64_t in_col_d = view_col(a.in_view, (q << 10) | t);

@@ -643,6 +643,21 @@ def test_bias_folded_into_forward_and_bias_gradient(case):
     assert rel_err(db4.cpu().numpy(), db_ref) < BW_TOL
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.complex64], ids=["f32", "c64"])
+@pytest.mark.parametrize("B, S, width", [(1, 1, 1), (15, 1, 3), (16, 2, 64), (17, 3, 65), (257, 1, 63), (4099, 2, 30),
+                                         (5000, 1, 1001)])
+def test_bias_gradient_partitions(dtype, B, S, width):
+    """Column sums at the edges of the row partitions (16 rows at least) and of the column
+    groups of the adding step (64 floats, four at a time)."""
+    from butterfly_amd import _capi
+    say("bias gradient", dtype, B, S, width)
+    g = randn(np.random.default_rng(B + width), (B, S, width), dtype)
+    db = _capi.bias_grad(dev(g))
+    torch.cuda.synchronize()
+    ref = g.astype(np.complex128).sum(axis=0)
+    assert np.abs(db.cpu().numpy() - ref).max() < 1e-5 * max(1.0, B ** 0.5)
+
+
 def test_bias_operator_autograd():
     """The autograd operator returns the three gradients the separate formulation gives."""
     import butterfly_amd  # noqa: F401
