@@ -11,7 +11,7 @@ import torch
 from torch import nn
 
 from .complex_utils import complex_reshape, real_dtype_to_complex
-from .multiply import butterfly_multiply, butterfly_multiply_bias, butterfly_multiply_perm
+from .multiply import butterfly_layer, butterfly_multiply, butterfly_multiply_bias, butterfly_multiply_perm
 
 _INITS = ("empty", "randn", "ortho", "identity", "fft_no_br", "ifft_no_br")
 
@@ -90,6 +90,8 @@ class Butterfly(nn.Module):
             'ortho', 'identity', 'fft_no_br', 'ifft_no_br', 'empty'.
         nblocks: number of alternating B / B^T blocks.
     """
+
+    _shares_input = True   # all stacks read the same rows
 
     def __init__(self, in_size, out_size, bias=True, complex=False, increasing_stride=True,
                  init="randn", nblocks=1):
@@ -180,7 +182,6 @@ class Butterfly(nn.Module):
             if transpose:
                 in_perm, out_index = out_index, in_perm
         twiddle = self.effective_twiddle()
-        x = self.pre_process(input)
         output_size = self.out_size if self.nstacks == 1 else None
         if subtwiddle:
             log_n = int(math.ceil(math.log2(input.size(-1))))
@@ -201,6 +202,10 @@ class Butterfly(nn.Module):
             inc = not last_inc
         else:
             inc = self.increasing_stride
+        # (out_size of a finished layer may have been lowered: not below its last stack here)
+        if self._shares_input and input.is_cuda and not subtwiddle and self.out_size > (self.nstacks - 1) * self.n:
+            return butterfly_layer(twiddle, input, self.layer_bias(), inc, self.out_size, in_perm, out_index)
+        x = self.pre_process(input)
         if in_perm is not None or out_index is not None:
             cols = output_size if output_size is not None else 1 << twiddle.shape[2]
             bias = None if self.bias is None else self.bias_rows(cols, subtwiddle)
@@ -216,6 +221,15 @@ class Butterfly(nn.Module):
     def effective_twiddle(self):
         """(stacks, nblocks, log_n, n/2, 2, 2) factors the multiply runs with."""
         return self.twiddle
+
+    def layer_bias(self):
+        """The bias of the first out_size columns, or None."""
+        bias = self.bias
+        if bias is None or bias.shape[0] == self.out_size:
+            return bias
+        if bias.shape[0] < self.out_size:
+            raise ValueError("bias is shorter than the output")
+        return bias[:self.out_size]
 
     def bias_rows(self, cols, subtwiddle=False):
         """The bias as the (stacks, cols) tensor that lines up with the multiply's output:
@@ -338,6 +352,8 @@ class ButterflyBmm(Butterfly):
     input: (batch, *, matrix_batch, in_size) -> (batch, *, matrix_batch, out_size).  The
     matrices ride on the stack dimension of one multiply (reference:
     torch_butterfly/butterfly.py:308-397)."""
+
+    _shares_input = False
 
     def __init__(self, in_size, out_size, matrix_batch=1, bias=True, complex=False, increasing_stride=True,
                  init="randn", nblocks=1):

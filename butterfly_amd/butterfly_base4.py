@@ -33,6 +33,9 @@ class ButterflyBase4(Butterfly):
         self.twiddle2._is_structured = True
 
     def forward(self, input):
+        if input.is_cuda and self.out_size > (self.nstacks - 1) * self.n:
+            return torch.ops.torch_butterfly.butterfly_layer_base4(self.twiddle4, self.twiddle2, input, self.layer_bias(),
+                                                                   self.increasing_stride, self.out_size)
         x = self.pre_process(input)
         output_size = self.out_size if self.nstacks == 1 else None
         x = butterfly_multiply_base4(self.twiddle4, self.twiddle2, x, self.increasing_stride,

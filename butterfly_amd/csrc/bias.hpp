@@ -67,4 +67,45 @@ __global__ __launch_bounds__(kBiasThreads) void bias_grad_partial_kernel(BiasArg
         add(add(s0, s1), add(s2, s3));
 }
 
+// ---- input gradient of stacks that share their input ------------------------------------------------
+
+constexpr int kSumStacksPerThread = 4;
+
+struct SumStacksArgs {
+    const void *in;      // (B, S, width) dense floats
+    void *out;           // (B, width) dense
+    int64_t width, nstacks, total;   // total = B * width
+};
+
+// out[b][c] = sum over the stacks of in[b][s][c], ascending.  Bound by the memory it reads; float4
+// accesses where the rows allow them (their width a multiple of four, and every row starts 16-byte
+// aligned then).
+__global__ __launch_bounds__(256) void sum_stacks_kernel(SumStacksArgs a)
+{
+    const float *in = reinterpret_cast<const float *>(a.in);
+    float *out = reinterpret_cast<float *>(a.out);
+    const int64_t step = (int64_t)gridDim.x * 256;
+    const bool wide = (a.width & 3) == 0 && (reinterpret_cast<unsigned long long>(a.out) & 15) == 0;
+    if (wide) {
+        for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; i < a.total; i += step * 4) {
+            const int64_t b = i / a.width;
+            const float *src = in + b * a.nstacks * a.width + (i - b * a.width);
+            float4 t = *reinterpret_cast<const float4 *>(src);
+            for (int64_t s = 1; s < a.nstacks; ++s) {
+                const float4 v = *reinterpret_cast<const float4 *>(src + s * a.width);
+                t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+            }
+            *reinterpret_cast<float4 *>(out + i) = t;
+        }
+        return;
+    }
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.total; i += step) {
+        const int64_t b = i / a.width;
+        const float *src = in + b * a.nstacks * a.width + (i - b * a.width);
+        float t = src[0];
+        for (int64_t s = 1; s < a.nstacks; ++s) t += src[s * a.width];
+        out[i] = t;
+    }
+}
+
 }  // namespace bf

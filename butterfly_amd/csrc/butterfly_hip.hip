@@ -1800,15 +1800,15 @@ size_t bf_butterfly_multiply_saved_bytes(const bf_problem *p)
     return saved_bytes(p);
 }
 
-int bf_butterfly_multiply_fw_saving(const bf_problem *p, const void *twiddle, const void *input, const void *bias,
-                                    const int32_t *in_perm, const int32_t *out_index, void *output, void *saved,
-                                    size_t saved_capacity, void *stream_)
+static int fw_saving(const bf_problem *p, const void *twiddle, const void *input, const void *bias, const int32_t *in_perm,
+                     const int32_t *out_index, void *output, void *saved, size_t saved_capacity, void *stream_,
+                     int64_t tail = -1)
 {
     int rc = check_problem(p, false);
     if (rc) return rc;
     if ((rc = check_perms(p, false, in_perm, out_index))) return rc;
     if ((rc = ensure_attributes())) return rc;
-    const size_t need = saved_bytes(p);
+    const size_t need = saved_bytes_of_plan(p, in_perm || out_index);
     if (need == 0) return fail(BF_ERR_INVALID, "this problem has no activations to save: use bf_butterfly_multiply_fw");
     if (!saved || saved_capacity < need)
         return fail(BF_ERR_WORKSPACE, "room for %zu bytes of saved activations needed, %zu given", need, saved_capacity);
@@ -1822,7 +1822,7 @@ int bf_butterfly_multiply_fw_saving(const bf_problem *p, const void *twiddle, co
     const BwPlan pl = plan_bw(p, false, true, permuted);
     if (mp.npass < 2 || !pl.fast) return fail(BF_ERR_INVALID, "this problem has no activations to save");
     const View in_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
-    const View out_view = make_view(p->output_stride, p->output_size, out_index);
+    const View out_view = make_view(p->output_stride, p->output_size, out_index, tail);
     const View dense = dense_view(p->nstacks, n);
     char *bounds = static_cast<char *>(saved);
     auto boundary = [&](int k) { return bounds + (size_t)(k - 1) * pl.boundary_bytes; };
@@ -1839,6 +1839,18 @@ int bf_butterfly_multiply_fw_saving(const bf_problem *p, const void *twiddle, co
     if (rc || !bias || bias_done) return rc;
     return p->dtype == BF_C64 ? launch_bias_add<float2>(p, bias, output, out_view, stream)
                               : launch_bias_add<float>(p, bias, output, out_view, stream);
+}
+
+int bf_butterfly_multiply_fw_saving(const bf_problem *p, const void *twiddle, const void *input, const void *bias,
+                                    const int32_t *in_perm, const int32_t *out_index, void *output, void *saved,
+                                    size_t saved_capacity, void *stream)
+{
+    const int rc = check_problem(p, false);
+    if (rc) return rc;
+    const size_t need = saved_bytes(p);
+    if (need > 0 && (!saved || saved_capacity < need))
+        return fail(BF_ERR_WORKSPACE, "room for %zu bytes of saved activations needed, %zu given", need, saved_capacity);
+    return fw_saving(p, twiddle, input, bias, in_perm, out_index, output, saved, saved_capacity, stream);
 }
 
 size_t bf_butterfly_multiply_bw_saved_workspace_bytes(const bf_problem *p, int with_bias)
@@ -1941,9 +1953,8 @@ size_t bf_butterfly_multiply_base4_saved_bytes(const bf_problem *p)
     return saved4_bytes(p);
 }
 
-int bf_butterfly_multiply_base4_fw_saving(const bf_problem *p, const void *twiddle4, const void *twiddle2,
-                                          const void *input, void *output, void *saved, size_t saved_capacity,
-                                          void *stream_)
+static int fw4_saving(const bf_problem *p, const void *twiddle4, const void *twiddle2, const void *input, const void *bias,
+                      void *output, void *saved, size_t saved_capacity, void *stream_, int64_t tail = -1)
 {
     int rc = check_problem(p, false);
     if (rc) return rc;
@@ -1960,7 +1971,7 @@ int bf_butterfly_multiply_base4_fw_saving(const bf_problem *p, const void *twidd
     const BwPlan pl = plan_bw(p, true, true);
     const Schedule sc = make_schedule(p, true);
     const View in_view = make_view(p->input_stride, std::min(p->input_size, n), nullptr);
-    const View out_view = make_view(p->output_stride, p->output_size, nullptr);
+    const View out_view = make_view(p->output_stride, p->output_size, nullptr, tail);
     const View dense = dense_view(p->nstacks, n);
     char *planes = static_cast<char *>(saved);
     auto boundary = [&](int k) { return planes + (size_t)(k - 1) * pl.boundary_bytes; };
@@ -1974,7 +1985,16 @@ int bf_butterfly_multiply_base4_fw_saving(const bf_problem *p, const void *twidd
                       : fast4_forward(p, twiddle4, twiddle2, in, out, nullptr, iv, ov, k, k + 1, stream);
         if (rc) return rc;
     }
-    return BF_OK;
+    if (!bias) return BF_OK;
+    return p->dtype == BF_C64 ? launch_bias_add<float2>(p, bias, output, out_view, stream)
+                              : launch_bias_add<float>(p, bias, output, out_view, stream);
+}
+
+int bf_butterfly_multiply_base4_fw_saving(const bf_problem *p, const void *twiddle4, const void *twiddle2,
+                                          const void *input, void *output, void *saved, size_t saved_capacity,
+                                          void *stream)
+{
+    return fw4_saving(p, twiddle4, twiddle2, input, nullptr, output, saved, saved_capacity, stream);
 }
 
 size_t bf_butterfly_multiply_base4_bw_saved_workspace_bytes(const bf_problem *p)
@@ -1998,6 +2018,127 @@ int bf_butterfly_multiply_base4_bw_saved(const bf_problem *p, const void *twiddl
                     saved_bytes_given);
     return backward(p, true, twiddle2, twiddle4, input, grad, d_twiddle2, d_twiddle4, d_input, workspace,
                     workspace_bytes, stream, nullptr, nullptr, nullptr, saved);
+}
+
+// ---- whole layers --------------------------------------------------------------------------------
+
+static int check_layer(const bf_layer *l, bool backward)
+{
+    if (!l) return fail(BF_ERR_INVALID, "layer descriptor is NULL");
+    const bf_problem *p = &l->problem;
+    const int rc = check_problem(p, backward);
+    if (rc) return rc;
+    const int64_t cols = p->nstacks * p->output_size;
+    if (l->total_output > cols || (cols > 0 && l->total_output <= cols - p->output_size))
+        return fail(BF_ERR_INVALID, "total_output must end in the last stack");
+    if (l->base4 && (l->in_perm || l->out_index))
+        return fail(BF_ERR_UNSUPPORTED, "base-4 layers take no column tables");
+    return BF_OK;
+}
+
+// columns of the last stack
+static int64_t layer_tail(const bf_layer *l) { return l->total_output - (l->problem.nstacks - 1) * l->problem.output_size; }
+
+static size_t layer_kept_bytes(const bf_layer *l)
+{
+    return l->base4 ? saved4_bytes(&l->problem) : saved_bytes_of_plan(&l->problem, l->in_perm || l->out_index);
+}
+
+// Backward workspace of a layer: the multiply's own, the partial column sums of the bias gradient,
+// the input gradients of the stacks before they are added up.
+struct LayerBwPlan {
+    bool kept;                 // the kept activations are read
+    size_t off_bias, off_stacks, total;
+};
+
+static LayerBwPlan plan_layer_bw(const bf_layer *l, int with_bias, size_t kept_bytes)
+{
+    const bf_problem *p = &l->problem;
+    LayerBwPlan b = {};
+    // The forward decided what to keep from a plan made with its own strides; this one follows from
+    // those of grad and d_input.  Where it reads no kept activations, or more than there are,
+    // they are recomputed.
+    const size_t reads = kept_bytes > 0 ? layer_kept_bytes(l) : 0;
+    b.kept = reads > 0 && reads <= kept_bytes;
+    b.off_bias = align256(plan_bw(p, l->base4 != 0, b.kept, l->in_perm || l->out_index).total);
+    b.off_stacks = b.off_bias + (with_bias ? align256(bias_area_bytes(p)) : 0);
+    b.total = b.off_stacks;
+    if (l->shared_input && p->nstacks > 1)
+        b.total += align256((size_t)p->batch * p->nstacks * p->input_size * elem_bytes(p->dtype));
+    return b;
+}
+
+size_t bf_layer_kept_bytes(const bf_layer *l)
+{
+    return check_layer(l, true) ? BF_SIZE_INVALID : layer_kept_bytes(l);
+}
+
+size_t bf_layer_fw_workspace_bytes(const bf_layer *l)
+{
+    return check_layer(l, false) ? BF_SIZE_INVALID : forward_workspace(&l->problem, l->base4 != 0);
+}
+
+int bf_layer_fw(const bf_layer *l, const void *input, void *output, void *kept, size_t kept_bytes, void *workspace,
+                size_t workspace_bytes, void *stream)
+{
+    const int rc = check_layer(l, false);
+    if (rc) return rc;
+    const bf_problem *p = &l->problem;
+    const int64_t tail = layer_tail(l);
+    if (kept)
+        return l->base4 ? fw4_saving(p, l->twiddle, l->twiddle2, input, l->bias, output, kept, kept_bytes, stream, tail)
+                        : fw_saving(p, l->twiddle, input, l->bias, l->in_perm, l->out_index, output, kept, kept_bytes,
+                                    stream, tail);
+    return l->base4 ? forward(p, true, l->twiddle2, l->twiddle, input, output, workspace, workspace_bytes, stream, l->bias,
+                              nullptr, nullptr, tail)
+                    : forward(p, false, l->twiddle, nullptr, input, output, workspace, workspace_bytes, stream, l->bias,
+                              l->in_perm, l->out_index, tail);
+}
+
+size_t bf_layer_bw_workspace_bytes(const bf_layer *l, int with_bias, size_t kept_bytes)
+{
+    return check_layer(l, true) ? BF_SIZE_INVALID : plan_layer_bw(l, with_bias, kept_bytes).total;
+}
+
+int bf_layer_bw(const bf_layer *l, const void *input, const void *grad, const void *kept, size_t kept_bytes,
+                void *d_twiddle, void *d_twiddle2, void *d_input, void *d_bias, void *workspace, size_t workspace_bytes,
+                void *stream_)
+{
+    int rc = check_layer(l, true);
+    if (rc) return rc;
+    const bf_problem *p = &l->problem;
+    const LayerBwPlan b = plan_layer_bw(l, d_bias != nullptr, kept ? kept_bytes : 0);
+    if (b.total > 0 && (!workspace || workspace_bytes < b.total))
+        return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", b.total, workspace_bytes);
+    char *ws = static_cast<char *>(workspace);
+    const bool sum = l->shared_input && p->nstacks > 1;
+    bf_problem stacked = *p;
+    void *d_stacks = d_input;
+    if (sum) {
+        stacked.d_input_stride[0] = p->nstacks * p->input_size;
+        stacked.d_input_stride[1] = p->input_size;
+        stacked.d_input_stride[2] = 1;
+        d_stacks = ws + b.off_stacks;
+    }
+    BiasGrad bg;
+    bg.area = ws + b.off_bias;
+    bg.d_bias = d_bias;
+    rc = backward(&stacked, l->base4 != 0, l->base4 ? l->twiddle2 : l->twiddle, l->base4 ? l->twiddle : nullptr, input, grad,
+                  l->base4 ? d_twiddle2 : d_twiddle, l->base4 ? d_twiddle : nullptr, d_stacks, workspace, b.off_bias, stream_,
+                  d_bias ? &bg : nullptr, l->in_perm, l->out_index, b.kept ? kept : nullptr, layer_tail(l));
+    if (rc || !sum || p->batch == 0 || p->input_size == 0) return rc;
+    SumStacksArgs a = {};
+    a.in = d_stacks;
+    a.out = d_input;
+    const int ef = p->dtype == BF_C64 ? 2 : 1;
+    a.width = p->input_size * ef;
+    a.nstacks = p->nstacks;
+    a.total = p->batch * a.width;
+    const int64_t threads = a.total / kSumStacksPerThread + 1;
+    const dim3 grid((unsigned)std::min<int64_t>((threads + 255) / 256, (int64_t)num_cu() * 16));
+    hipLaunchKernelGGL(sum_stacks_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream_), a);
+    BF_HIP_CHECK(hipGetLastError());
+    return BF_OK;
 }
 
 static int scale_twiddle(bool bw, int dtype, int64_t nstacks, int64_t nblocks, int64_t log_n, int increasing_stride,

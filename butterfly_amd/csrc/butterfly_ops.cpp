@@ -14,7 +14,11 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/core/grad_mode.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/library.h>
 
 #include <tuple>
@@ -154,28 +158,6 @@ Tensor dense(const Tensor &t)
     return d;
 }
 
-struct Shapes {
-    int64_t batch, nstacks, nblocks, log_n, n, input_size;
-};
-
-bf_problem make_problem(const Shapes &s, const Tensor &input, bool increasing_stride, int64_t output_size,
-                        const char *who)
-{
-    bf_problem p = {};
-    p.dtype = dtype_code(input, who);
-    p.increasing_stride = increasing_stride;
-    p.batch = s.batch;
-    p.nstacks = s.nstacks;
-    p.log_n = s.log_n;
-    p.nblocks = s.nblocks;
-    p.input_size = s.input_size;
-    p.output_size = output_size;
-    set_strides(p.input_stride, input);
-    return p;
-}
-
-// ---- base-2 -----------------------------------------------------------------------------
-
 // A column table of the *_perm operators: int32, n entries, dense, on the device of `like`.
 // Its entries are the caller's responsibility (each table a permutation of 0..n-1).
 const int32_t *table_ptr(const Tensor &t, Tensor &keep, const Tensor &like, int64_t n, const char *name,
@@ -189,86 +171,429 @@ const int32_t *table_ptr(const Tensor &t, Tensor &keep, const Tensor &like, int6
     return keep.data_ptr<int32_t>();
 }
 
-// Shared body of the forward operators (`bias`, `in_perm`, `out_index` undefined = none).
+// What one call works on, besides the rows.
+struct Operands {
+    Tensor twiddle, twiddle2;      // base 2: twiddle; base 4: twiddle4 and twiddle2
+    Tensor bias;                   // undefined: none
+    Tensor in_perm, out_index;     // undefined: none
+    bool base4 = false;
+    bool increasing_stride = true;
+};
+
+// Shapes and strides of a call.  rows: a 3-d view (batch, nstacks, width) of the caller's input.
+// layer: the stacks share one input (nstacks is then the factors') and out_size counts the columns
+// over all stacks; otherwise it counts those of one stack.
+struct Call {
+    bf_layer desc = {};
+    int64_t n = 0;
+    Tensor twiddle, twiddle2, bias, tables[2];   // dense forms the descriptor points into
+
+    bf_problem &p() { return desc.problem; }
+};
+
+void check_factors(const Operands &o, const Tensor &input, const char *who)
+{
+    const Tensor &twiddle = o.twiddle;
+    CHECK_DEVICE(twiddle); CHECK_DEVICE(input); CHECK_SAME_DEVICE(twiddle, input);
+    CHECK_DIM(twiddle, 6);
+    if (!o.base4) return;
+    const Tensor &twiddle2 = o.twiddle2;
+    CHECK_DEVICE(twiddle2); CHECK_SAME_DEVICE(twiddle2, input);
+    CHECK_DIM(twiddle2, 6);
+    TORCH_CHECK(twiddle2.size(2) <= 1, "twiddle2 must have shape (nstacks, nblocks, log_n % 2, n / 2, 2, 2)");
+}
+
+int64_t log_size(const Operands &o, const char *who)
+{
+    const int64_t log_n = o.base4 ? o.twiddle.size(2) * 2 + o.twiddle2.size(2) : o.twiddle.size(2);
+    TORCH_CHECK(log_n <= 30, who, ": n must be a power of 2");
+    return log_n;
+}
+
+// Checks the factors against the rows and fills everything but the strides of output and d_input.
+void describe(Call &c, const Operands &o, int64_t batch, int64_t nstacks, int64_t input_size, const int64_t (&stride)[3],
+              const Tensor &input, int64_t out_cols, int64_t total, bool shared, const char *who)
+{
+    const int64_t log_n = log_size(o, who), n = (int64_t)1 << log_n, nblocks = o.twiddle.size(1);
+    c.n = n;
+    if (o.base4) {
+        const Tensor &twiddle4 = o.twiddle, &twiddle2 = o.twiddle2;
+        if (log_n / 2 > 0) CHECK_SHAPE(twiddle4, nstacks, nblocks, log_n / 2, n / 4, 4, 4);
+        if (log_n % 2 == 1) CHECK_SHAPE(twiddle2, nstacks, nblocks, 1, n / 2, 2, 2);
+        TORCH_CHECK(twiddle4.scalar_type() == input.scalar_type() && twiddle2.scalar_type() == input.scalar_type(), who,
+                    ": twiddle4, twiddle2 and input must have the same dtype");
+    } else {
+        const Tensor &twiddle = o.twiddle;
+        CHECK_SHAPE(twiddle, nstacks, nblocks, log_n, n / 2, 2, 2);
+        TORCH_CHECK(twiddle.scalar_type() == input.scalar_type(), who, ": twiddle and input must have the same dtype");
+    }
+    bf_problem &p = c.p();
+    p.dtype = dtype_code(input, who);
+    p.increasing_stride = o.increasing_stride;
+    p.batch = batch;
+    p.nstacks = nstacks;
+    p.log_n = log_n;
+    p.nblocks = nblocks;
+    p.input_size = input_size;
+    p.output_size = out_cols;
+    for (int i = 0; i < 3; ++i) {
+        TORCH_CHECK(stride[i] >= 0, "negative strides are not supported");
+        p.input_stride[i] = stride[i];
+    }
+    c.desc.base4 = o.base4;
+    c.desc.shared_input = shared;
+    c.desc.total_output = total;
+    c.twiddle = dense(o.twiddle);
+    c.desc.twiddle = c.twiddle.data_ptr();
+    if (o.base4) {
+        c.twiddle2 = dense(o.twiddle2);
+        c.desc.twiddle2 = c.twiddle2.data_ptr();
+    }
+    if (o.bias.defined()) {
+        const Tensor &bias = o.bias;
+        CHECK_DEVICE(bias); CHECK_SAME_DEVICE(bias, input);
+        TORCH_CHECK(bias.scalar_type() == input.scalar_type(), who, ": bias and input must have the same dtype");
+        c.bias = dense(bias);
+        c.desc.bias = c.bias.data_ptr();
+    }
+    c.desc.in_perm = table_ptr(o.in_perm, c.tables[0], input, n, "in_perm", who);
+    c.desc.out_index = table_ptr(o.out_index, c.tables[1], input, n, "out_index", who);
+    if (c.desc.in_perm || c.desc.out_index) TORCH_CHECK(input_size <= n, who, ": column tables need input_size <= n");
+}
+
+// d_input as backward_call() will lay it out: the forward plans what to keep with the same strides.
+// A multiply's is a slice of an n-wide tensor (what the reference returns), a layer's is dense.
+void set_d_input_strides(Call &c, bool layer)
+{
+    bf_problem &p = c.p();
+    const int64_t width = layer ? p.input_size : std::max(p.input_size, c.n);
+    const int64_t stacks = layer && p.nstacks == 1 ? 1 : p.nstacks;
+    p.d_input_stride[0] = stacks * width;
+    p.d_input_stride[1] = width;
+    p.d_input_stride[2] = 1;
+}
+
+Tensor bytes_like(const Tensor &t, size_t bytes)
+{
+    return at::empty({(int64_t)bytes}, t.options().dtype(at::kByte));
+}
+
 // keep (may be NULL): where the call may leave the intermediate activations that a backward in
 // several passes would otherwise recompute; defined on return when it did.
-Tensor multiply_fw_impl(const Tensor &twiddle, const Tensor &input, const Tensor &bias, bool increasing_stride,
-                        c10::optional<int64_t> output_size, const char *who, const Tensor &in_perm = Tensor(),
-                        const Tensor &out_index = Tensor(), Tensor *keep = nullptr)
+void forward_call(Call &c, const Tensor &x, Tensor &output, Tensor *keep, const char *who)
 {
-    CHECK_DEVICE(twiddle); CHECK_DEVICE(input); CHECK_SAME_DEVICE(twiddle, input);
-    CHECK_DIM(twiddle, 6); CHECK_DIM(input, 3);
-    Shapes s;
-    s.batch = input.size(0);
-    s.nstacks = input.size(1);
-    s.input_size = input.size(2);
-    s.nblocks = twiddle.size(1);
-    s.log_n = twiddle.size(2);
-    TORCH_CHECK(s.log_n <= 30, who, ": n must be a power of 2");
-    s.n = (int64_t)1 << s.log_n;
-    CHECK_SHAPE(twiddle, s.nstacks, s.nblocks, s.log_n, s.n / 2, 2, 2);
-    const int64_t output_size_val = output_size.has_value() ? output_size.value() : s.n;
-    TORCH_CHECK(output_size_val <= s.n, who, ": output_size must be <= n");
-    TORCH_CHECK(output_size_val >= 0, who, ": output_size must be >= 0");
-    TORCH_CHECK(twiddle.scalar_type() == input.scalar_type(), who, ": twiddle and input must have the same dtype");
-    if (input.is_cpu() && !bias.defined() && !in_perm.defined() && !out_index.defined())
-        return host_multiply_fw(twiddle, input, increasing_stride, s.log_n, output_size_val, who);
-    require_device(input, who);
-    Tensor b;
-    if (bias.defined()) {
-        CHECK_DEVICE(bias); CHECK_SAME_DEVICE(bias, input);
-        CHECK_DIM(bias, 2);
-        CHECK_SHAPE(bias, s.nstacks, output_size_val);
-        TORCH_CHECK(bias.scalar_type() == input.scalar_type(), who, ": bias and input must have the same dtype");
-        b = dense(bias);
-    }
-
-    const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    const Tensor tw = dense(twiddle);
-    const Tensor x = input.resolve_conj();
-    Tensor output = at::empty({s.batch, s.nstacks, s.n}, x.options());
-    if (output_size_val < s.n) output = output.slice(2, 0, output_size_val);
-    bf_problem p = make_problem(s, x, increasing_stride, output_size_val, who);
-    set_strides(p.output_stride, output);
-    Tensor keep_in, keep_out;
-    const int32_t *ip = table_ptr(in_perm, keep_in, x, s.n, "in_perm", who);
-    const int32_t *oi = table_ptr(out_index, keep_out, x, s.n, "out_index", who);
-    if (ip || oi) TORCH_CHECK(s.input_size <= s.n, who, ": column tables need input_size <= n");
     if (keep) {
-        // (the backward will make d_input dense over max(input_size, n) columns: same plan)
-        const int64_t dw = std::max(s.input_size, s.n);
-        p.d_input_stride[0] = s.batch > 1 ? s.nstacks * dw : 0;
-        p.d_input_stride[1] = s.nstacks > 1 ? dw : 0;
-        p.d_input_stride[2] = s.input_size > 1 ? 1 : 0;
-        const size_t nsaved = valid_size(bf_butterfly_multiply_saved_bytes(&p));
-        if (nsaved > 0) {
-            *keep = at::empty({(int64_t)nsaved}, x.options().dtype(at::kByte));
-            check_rc(bf_butterfly_multiply_fw_saving(&p, tw.data_ptr(), x.data_ptr(), b.defined() ? b.data_ptr() : nullptr,
-                                                     ip, oi, output.data_ptr(), keep->data_ptr(), nsaved,
-                                                     current_stream()),
+        const size_t kept = valid_size(bf_layer_kept_bytes(&c.desc));
+        if (kept > 0) {
+            *keep = bytes_like(x, kept);
+            check_rc(bf_layer_fw(&c.desc, x.data_ptr(), output.data_ptr(), keep->data_ptr(), kept, nullptr, 0,
+                                 current_stream()),
                      who);
-            return output;
+            return;
         }
     }
-    const size_t ws_bytes = valid_size(bf_butterfly_multiply_fw_workspace_bytes(&p));
-    Tensor ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-    if (ip || oi) {
-        check_rc(bf_butterfly_multiply_perm_fw(&p, tw.data_ptr(), x.data_ptr(), ip, oi,
-                                               b.defined() ? b.data_ptr() : nullptr, output.data_ptr(),
-                                               ws.data_ptr(), ws_bytes, current_stream()),
-                 who);
-        return output;
-    }
-    check_rc(bf_butterfly_multiply_bias_fw(&p, tw.data_ptr(), x.data_ptr(), b.defined() ? b.data_ptr() : nullptr,
-                                           output.data_ptr(), ws.data_ptr(), ws_bytes, current_stream()),
+    const size_t ws_bytes = valid_size(bf_layer_fw_workspace_bytes(&c.desc));
+    Tensor ws;
+    if (ws_bytes > 0) ws = bytes_like(x, ws_bytes);
+    check_rc(bf_layer_fw(&c.desc, x.data_ptr(), output.data_ptr(), nullptr, 0, ws_bytes > 0 ? ws.data_ptr() : nullptr,
+                         ws_bytes, current_stream()),
              who);
+}
+
+struct Gradients {
+    Tensor twiddle, twiddle2, input, bias;
+};
+
+void backward_call(Call &c, const Tensor &x, const Tensor &g, const Tensor &kept, bool with_bias, Gradients &d,
+                   const char *who)
+{
+    const size_t kept_bytes = kept.defined() ? (size_t)kept.numel() : 0;
+    d.twiddle = at::empty_like(c.twiddle);
+    if (c.desc.base4) d.twiddle2 = at::empty_like(c.twiddle2);
+    if (with_bias) d.bias = at::empty({c.desc.total_output}, g.options());
+    const size_t ws_bytes = valid_size(bf_layer_bw_workspace_bytes(&c.desc, with_bias ? 1 : 0, kept_bytes));
+    Tensor ws;
+    if (ws_bytes > 0) ws = bytes_like(x, ws_bytes);
+    check_rc(bf_layer_bw(&c.desc, x.data_ptr(), g.data_ptr(), kept_bytes > 0 ? kept.data_ptr() : nullptr, kept_bytes,
+                         d.twiddle.data_ptr(), c.desc.base4 ? d.twiddle2.data_ptr() : nullptr, d.input.data_ptr(),
+                         with_bias ? d.bias.data_ptr() : nullptr, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
+                         current_stream()),
+             who);
+}
+
+// ---- the multiply operators: input (batch, nstacks, width) ---------------------------------------
+
+// Strides of a 3-d operand, zero where there is nothing to step over.
+void strides_of(int64_t (&dst)[3], const Tensor &t)
+{
+    for (int i = 0; i < 3; ++i) dst[i] = t.size(i) > 1 ? t.stride(i) : 0;
+}
+
+Tensor multiply_fw(const Operands &o, const Tensor &input, c10::optional<int64_t> output_size, Tensor *keep, const char *who)
+{
+    check_factors(o, input, who);
+    CHECK_DIM(input, 3);
+    const int64_t log_n = log_size(o, who), n = (int64_t)1 << log_n;
+    const int64_t batch = input.size(0), nstacks = input.size(1);
+    const int64_t cols = output_size.has_value() ? output_size.value() : n;
+    TORCH_CHECK(cols <= n, who, ": output_size must be <= n");
+    TORCH_CHECK(cols >= 0, who, ": output_size must be >= 0");
+    if (!o.base4 && input.is_cpu() && !o.bias.defined() && !o.in_perm.defined() && !o.out_index.defined()) {
+        const Tensor &twiddle = o.twiddle;
+        CHECK_SHAPE(twiddle, nstacks, o.twiddle.size(1), log_n, n / 2, 2, 2);
+        TORCH_CHECK(twiddle.scalar_type() == input.scalar_type(), who, ": twiddle and input must have the same dtype");
+        return host_multiply_fw(twiddle, input, o.increasing_stride, log_n, cols, who);
+    }
+    require_device(input, who);
+    if (o.bias.defined()) {
+        const Tensor &bias = o.bias;
+        CHECK_DIM(bias, 2);
+        CHECK_SHAPE(bias, nstacks, cols);
+    }
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
+    const Tensor x = input.resolve_conj();
+    int64_t stride[3];
+    strides_of(stride, x);
+    Call c;
+    describe(c, o, batch, nstacks, input.size(2), stride, x, cols, nstacks * cols, false, who);
+    // (a slice of an n-wide tensor when there are fewer columns)
+    Tensor output = cols == n ? at::empty({batch, nstacks, n}, x.options())
+                              : at::empty({batch, nstacks, n}, x.options()).slice(2, 0, cols);
+    strides_of(c.p().output_stride, output);
+    set_d_input_strides(c, false);
+    forward_call(c, x, output, keep, who);
     return output;
+}
+
+// kept: what the forward left in its `keep` (undefined: the backward recomputes what it needs)
+Gradients multiply_bw(const Operands &o, const Tensor &input, const Tensor &grad, const Tensor &kept, bool with_bias,
+                      const char *who)
+{
+    check_factors(o, input, who);
+    CHECK_DEVICE(grad); CHECK_SAME_DEVICE(input, grad);
+    CHECK_DIM(input, 3); CHECK_DIM(grad, 3);
+    const int64_t log_n = log_size(o, who), n = (int64_t)1 << log_n;
+    const int64_t batch = input.size(0), nstacks = input.size(1), input_size = input.size(2), cols = grad.size(2);
+    CHECK_SHAPE(grad, batch, nstacks, cols);
+    TORCH_CHECK(cols <= n, who, ": grad must have at most n columns");
+    TORCH_CHECK(grad.scalar_type() == input.scalar_type(), who, ": grad and input must have the same dtype");
+    Gradients d;
+    if (!o.base4 && input.is_cpu() && !with_bias && !o.in_perm.defined() && !o.out_index.defined()) {
+        const Tensor &twiddle = o.twiddle;
+        CHECK_SHAPE(twiddle, nstacks, o.twiddle.size(1), log_n, n / 2, 2, 2);
+        TORCH_CHECK(twiddle.scalar_type() == input.scalar_type(), who, ": twiddle and input must have the same dtype");
+        std::tie(d.twiddle, d.input) = host_multiply_bw(twiddle, input, grad, o.increasing_stride, log_n, who);
+        return d;
+    }
+    require_device(input, who);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
+    const Tensor x = input.resolve_conj(), g = grad.resolve_conj();
+    int64_t stride[3];
+    strides_of(stride, x);
+    Call c;
+    describe(c, o, batch, nstacks, input_size, stride, x, cols, nstacks * cols, false, who);
+    strides_of(c.p().output_stride, g);
+    set_d_input_strides(c, false);
+    d.input = at::empty({batch, nstacks, std::max(input_size, n)}, x.options());
+    if (input_size < n) d.input = d.input.slice(2, 0, input_size);
+    backward_call(c, x, g, kept, with_bias, d, who);
+    if (with_bias) d.bias = d.bias.view({nstacks, cols});
+    return d;
+}
+
+// ---- whole layers: input (*, width), output (*, out_size) -----------------------------------------
+
+// The rows of a layer's input as a 2-d view or copy.
+Tensor rows_of(const Tensor &input)
+{
+    const Tensor x = input.resolve_conj();
+    return x.dim() == 2 ? x : x.reshape({-1, x.size(-1)});
+}
+
+void describe_layer(Call &c, const Operands &o, const Tensor &x, int64_t out_size, const char *who)
+{
+    const int64_t nstacks = o.twiddle.size(0), n = (int64_t)1 << log_size(o, who);
+    TORCH_CHECK(out_size > (nstacks - 1) * n && out_size <= nstacks * n, who, ": out_size must end in the last stack");
+    if (o.bias.defined()) TORCH_CHECK(o.bias.dim() == 1 && o.bias.size(0) == out_size, who, ": bias must have out_size entries");
+    const int64_t stride[3] = {x.size(0) > 1 ? x.stride(0) : 0, 0, x.size(1) > 1 ? x.stride(1) : 0};
+    describe(c, o, x.size(0), nstacks, x.size(1), stride, x, nstacks == 1 ? out_size : n, out_size, true, who);
+    set_d_input_strides(c, true);
+}
+
+Tensor layer_fw(const Operands &o, const Tensor &input, int64_t out_size, Tensor *keep, const char *who)
+{
+    check_factors(o, input, who);
+    TORCH_CHECK(input.dim() >= 1, who, ": input must have at least one dimension");
+    require_device(input, who);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
+    const Tensor x = rows_of(input);
+    Call c;
+    describe_layer(c, o, x, out_size, who);
+    c10::SmallVector<int64_t, 6> shape(input.sizes().begin(), input.sizes().end());
+    shape.back() = out_size;
+    Tensor output = at::empty(shape, x.options());
+    bf_problem &p = c.p();
+    p.output_stride[0] = out_size;
+    p.output_stride[1] = p.output_size;
+    p.output_stride[2] = 1;
+    forward_call(c, x, output, keep, who);
+    return output;
+}
+
+Gradients layer_bw(const Operands &o, const Tensor &input, const Tensor &grad, const Tensor &kept, bool with_bias,
+                   const char *who)
+{
+    TORCH_CHECK(grad.scalar_type() == input.scalar_type(), who, ": grad and input must have the same dtype");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
+    const Tensor x = rows_of(input), g = rows_of(grad);
+    Call c;
+    describe_layer(c, o, x, g.size(1), who);
+    bf_problem &p = c.p();
+    p.output_stride[0] = g.size(0) > 1 ? g.stride(0) : 0;
+    p.output_stride[2] = g.size(1) > 1 ? g.stride(1) : 0;
+    p.output_stride[1] = p.output_size * p.output_stride[2];
+    Gradients d;
+    d.input = at::empty(input.sizes(), x.options());
+    backward_call(c, x, g, kept, with_bias, d, who);
+    return d;
+}
+
+// ---- autograd ---------------------------------------------------------------------------------------
+//
+// One node for all differentiable operators.  Written against Node itself: the Function wrapper
+// keeps its state in a dictionary of boxed values and prepares for several outputs and in-place
+// ones, which costs more host time than a small multiply takes on the GPU.  Forward-mode
+// derivatives and second derivatives do not exist, as in the reference's Function
+// (csrc/butterfly.cpp:99-118).
+
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+struct MultiplyNode : public torch::autograd::Node {
+    SavedVariable twiddle, twiddle2, input, kept;
+    Tensor in_perm, out_index;
+    bool base4 = false, increasing_stride = true, with_bias = false, layer = false, has_kept = false;
+    const char *who = nullptr;
+
+    // edges: twiddle, twiddle2, input, bias (those that the call does not have lead nowhere)
+    variable_list apply(variable_list &&grads) override
+    {
+        variable_list out(num_outputs());
+        if (!grads[0].defined()) return out;
+        const auto self = getptr();
+        Operands o;
+        o.twiddle = twiddle.unpack(self);
+        if (base4) o.twiddle2 = twiddle2.unpack(self);
+        o.in_perm = in_perm;
+        o.out_index = out_index;
+        o.base4 = base4;
+        o.increasing_stride = increasing_stride;
+        const Tensor x = input.unpack(self), planes = has_kept ? kept.unpack(self) : Tensor();
+        at::AutoDispatchBelowADInplaceOrView below;
+        Gradients d = layer ? layer_bw(o, x, grads[0], planes, with_bias, who)
+                            : multiply_bw(o, x, grads[0], planes, with_bias, who);
+        out[0] = std::move(d.twiddle);
+        out[1] = std::move(d.twiddle2);
+        out[2] = std::move(d.input);
+        out[3] = std::move(d.bias);
+        return out;
+    }
+
+    void release_variables() override
+    {
+        twiddle.reset_data();
+        twiddle2.reset_data();
+        input.reset_data();
+        kept.reset_data();
+    }
+
+    std::string name() const override { return base4 ? "ButterflyMultiplyBase4Backward" : "ButterflyMultiplyBackward"; }
+};
+
+// Runs the forward and, when a gradient will be asked for, hangs the node behind its output.  The
+// forward then runs along the backward's pass plan and keeps the activations between the passes
+// (device tensors whose backward takes several passes: rows beyond 1024, more than two blocks),
+// which the reference's Function leaves to its backward to recompute.
+template <typename F>
+Tensor differentiable(const Operands &o, const Tensor &input, bool layer, const char *who, F &&forward)
+{
+    bool wanted = false;
+    if (at::GradMode::is_enabled()) {
+        for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &input}) wanted = wanted || (t->defined() && t->requires_grad());
+    }
+    if (!wanted) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        return forward(nullptr);
+    }
+    for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &input})
+        TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), who, ": no forward-mode derivative");
+    std::shared_ptr<MultiplyNode> node(new MultiplyNode(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(o.twiddle, o.twiddle2, input, o.bias));
+    Tensor kept, out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        out = forward(input.is_cuda() ? &kept : nullptr);
+    }
+    node->twiddle = SavedVariable(o.twiddle, false);
+    if (o.base4) node->twiddle2 = SavedVariable(o.twiddle2, false);
+    node->input = SavedVariable(input, false);
+    if (kept.defined()) {
+        node->kept = SavedVariable(kept, false);
+        node->has_kept = true;
+    }
+    node->in_perm = o.in_perm;
+    node->out_index = o.out_index;
+    node->base4 = o.base4;
+    node->increasing_stride = o.increasing_stride;
+    node->with_bias = o.bias.defined();
+    node->layer = layer;
+    node->who = who;
+    torch::autograd::set_history(out, node);
+    return out;
+}
+
+// ---- registered operators ------------------------------------------------------------------------------
+
+Tensor opt(const c10::optional<Tensor> &t) { return t.has_value() ? t.value() : Tensor(); }
+
+Operands base2(const Tensor &twiddle, bool increasing_stride, const Tensor &bias = Tensor(),
+               const Tensor &in_perm = Tensor(), const Tensor &out_index = Tensor())
+{
+    Operands o;
+    o.twiddle = twiddle;
+    o.bias = bias;
+    o.in_perm = in_perm;
+    o.out_index = out_index;
+    o.increasing_stride = increasing_stride;
+    return o;
+}
+
+Operands base4(const Tensor &twiddle4, const Tensor &twiddle2, bool increasing_stride, const Tensor &bias = Tensor())
+{
+    Operands o = base2(twiddle4, increasing_stride, bias);
+    o.twiddle2 = twiddle2;
+    o.base4 = true;
+    return o;
 }
 
 Tensor butterfly_multiply_fw(const Tensor twiddle, const Tensor input, bool increasing_stride,
                              c10::optional<int64_t> output_size)
 {
-    return multiply_fw_impl(twiddle, input, Tensor(), increasing_stride, output_size, "butterfly_multiply_fw");
+    return multiply_fw(base2(twiddle, increasing_stride), input, output_size, nullptr, "butterfly_multiply_fw");
+}
+
+std::tuple<Tensor, Tensor> butterfly_multiply_bw(const Tensor twiddle, const Tensor input,
+                                                 const Tensor grad, bool increasing_stride)
+{
+    Gradients d = multiply_bw(base2(twiddle, increasing_stride), input, grad, Tensor(), false, "butterfly_multiply_bw");
+    return {d.twiddle, d.input};
+}
+
+Tensor butterfly_multiply(Tensor twiddle, Tensor input, bool increasing_stride, c10::optional<int64_t> output_size)
+{
+    const char *who = "butterfly_multiply";
+    const Operands o = base2(twiddle, increasing_stride);
+    return differentiable(o, input, false, who, [&](Tensor *keep) { return multiply_fw(o, input, output_size, keep, who); });
 }
 
 // New operators (no counterpart in the reference's op set): the layer bias folded into the
@@ -278,7 +603,103 @@ Tensor butterfly_multiply_bias_fw(const Tensor twiddle, const Tensor input, cons
                                   bool increasing_stride, c10::optional<int64_t> output_size)
 {
     TORCH_CHECK(bias.defined(), "butterfly_multiply_bias_fw: bias is undefined");
-    return multiply_fw_impl(twiddle, input, bias, increasing_stride, output_size, "butterfly_multiply_bias_fw");
+    return multiply_fw(base2(twiddle, increasing_stride, bias), input, output_size, nullptr, "butterfly_multiply_bias_fw");
+}
+
+// (d_twiddle, d_input, d_bias): the backward of butterfly_multiply_bias_fw
+std::tuple<Tensor, Tensor, Tensor> butterfly_multiply_bias_bw(const Tensor twiddle, const Tensor input,
+                                                              const Tensor grad, bool increasing_stride)
+{
+    Gradients d = multiply_bw(base2(twiddle, increasing_stride), input, grad, Tensor(), true, "butterfly_multiply_bias_bw");
+    return {d.twiddle, d.input, d.bias};
+}
+
+Tensor butterfly_multiply_bias(Tensor twiddle, Tensor input, Tensor bias, bool increasing_stride,
+                               c10::optional<int64_t> output_size)
+{
+    const char *who = "butterfly_multiply_bias";
+    TORCH_CHECK(bias.defined(), "butterfly_multiply_bias: bias is undefined");
+    const Operands o = base2(twiddle, increasing_stride, bias);
+    return differentiable(o, input, false, who, [&](Tensor *keep) { return multiply_fw(o, input, output_size, keep, who); });
+}
+
+// New operators: the multiply between two fixed column permutations, folded into the first
+// read and the last write (in front: u[c] = input[in_perm[c]]; behind: output[out_index[c]] =
+// y[c]; bias (nstacks, output_size) indexed by c).  Where the reference chains FixedPermutation
+// and Butterfly modules (torch_butterfly/special.py:17-66), each permutation costs a pass of
+// its own over the activations.  Tables: int32 (n,), undefined = identity.
+Tensor butterfly_multiply_perm_fw(const Tensor twiddle, const Tensor input, c10::optional<Tensor> in_perm,
+                                  c10::optional<Tensor> out_index, c10::optional<Tensor> bias,
+                                  bool increasing_stride, c10::optional<int64_t> output_size)
+{
+    return multiply_fw(base2(twiddle, increasing_stride, opt(bias), opt(in_perm), opt(out_index)), input, output_size,
+                       nullptr, "butterfly_multiply_perm_fw");
+}
+
+// (d_twiddle, d_input, d_bias); d_bias is empty unless with_bias
+std::tuple<Tensor, Tensor, Tensor> butterfly_multiply_perm_bw(const Tensor twiddle, const Tensor input,
+                                                              const Tensor grad, c10::optional<Tensor> in_perm,
+                                                              c10::optional<Tensor> out_index, bool with_bias,
+                                                              bool increasing_stride)
+{
+    Gradients d = multiply_bw(base2(twiddle, increasing_stride, Tensor(), opt(in_perm), opt(out_index)), input, grad,
+                              Tensor(), with_bias, "butterfly_multiply_perm_bw");
+    if (!with_bias) d.bias = at::empty({0}, grad.options());  // the schema has no optional results
+    return {d.twiddle, d.input, d.bias};
+}
+
+Tensor butterfly_multiply_perm(Tensor twiddle, Tensor input, c10::optional<Tensor> in_perm,
+                               c10::optional<Tensor> out_index, c10::optional<Tensor> bias, bool increasing_stride,
+                               c10::optional<int64_t> output_size)
+{
+    const char *who = "butterfly_multiply_perm";
+    const Operands o = base2(twiddle, increasing_stride, opt(bias), opt(in_perm), opt(out_index));
+    return differentiable(o, input, false, who, [&](Tensor *keep) { return multiply_fw(o, input, output_size, keep, who); });
+}
+
+// A whole layer: input (*, width), zero padded or trimmed to n for each of the stacks (the leading
+// dimension of the factors), to the first out_size columns of the stacks' outputs side by side,
+// plus bias (out_size).  in_perm / out_index as above.  What Butterfly.forward does around its
+// multiply (torch_butterfly/butterfly.py:113-169), without the chain of views, slices and pads
+// that autograd would record and replay for it.
+Tensor butterfly_layer(Tensor twiddle, Tensor input, c10::optional<Tensor> bias, c10::optional<Tensor> in_perm,
+                       c10::optional<Tensor> out_index, bool increasing_stride, int64_t out_size)
+{
+    const char *who = "butterfly_layer";
+    const Operands o = base2(twiddle, increasing_stride, opt(bias), opt(in_perm), opt(out_index));
+    return differentiable(o, input, true, who, [&](Tensor *keep) { return layer_fw(o, input, out_size, keep, who); });
+}
+
+Tensor butterfly_layer_base4(Tensor twiddle4, Tensor twiddle2, Tensor input, c10::optional<Tensor> bias,
+                             bool increasing_stride, int64_t out_size)
+{
+    const char *who = "butterfly_layer_base4";
+    const Operands o = base4(twiddle4, twiddle2, increasing_stride, opt(bias));
+    return differentiable(o, input, true, who, [&](Tensor *keep) { return layer_fw(o, input, out_size, keep, who); });
+}
+
+Tensor butterfly_multiply_base4_fw(const Tensor twiddle4, const Tensor twiddle2, const Tensor input,
+                                   bool increasing_stride, c10::optional<int64_t> output_size)
+{
+    return multiply_fw(base4(twiddle4, twiddle2, increasing_stride), input, output_size, nullptr,
+                       "butterfly_multiply_base4_fw");
+}
+
+std::tuple<Tensor, Tensor, Tensor> butterfly_multiply_base4_bw(const Tensor twiddle4, const Tensor twiddle2,
+                                                               const Tensor input, const Tensor grad,
+                                                               bool increasing_stride)
+{
+    Gradients d = multiply_bw(base4(twiddle4, twiddle2, increasing_stride), input, grad, Tensor(), false,
+                              "butterfly_multiply_base4_bw");
+    return {d.twiddle, d.twiddle2, d.input};
+}
+
+Tensor butterfly_multiply_base4(Tensor twiddle4, Tensor twiddle2, Tensor input, bool increasing_stride,
+                                c10::optional<int64_t> output_size)
+{
+    const char *who = "butterfly_multiply_base4";
+    const Operands o = base4(twiddle4, twiddle2, increasing_stride);
+    return differentiable(o, input, false, who, [&](Tensor *keep) { return multiply_fw(o, input, output_size, keep, who); });
 }
 
 // d_bias (nstacks, output_size) = sum of grad (batch, nstacks, output_size) over the batch.
@@ -305,268 +726,6 @@ Tensor butterfly_bias_grad(const Tensor grad)
     check_rc(bf_butterfly_bias_grad(&p, g.data_ptr(), d_bias.data_ptr(), ws.data_ptr(), ws_bytes, current_stream()),
              "butterfly_bias_grad");
     return d_bias;
-}
-
-// Shared body of the backward operators.
-// kept: what the forward left in its `keep` (undefined: the backward recomputes what it needs)
-std::tuple<Tensor, Tensor, Tensor> multiply_bw_impl(const Tensor &twiddle, const Tensor &input, const Tensor &grad,
-                                                    bool increasing_stride, bool with_bias, const char *who,
-                                                    const Tensor &in_perm = Tensor(),
-                                                    const Tensor &out_index = Tensor(), const Tensor &kept = Tensor())
-{
-    CHECK_DEVICE(twiddle); CHECK_DEVICE(input); CHECK_DEVICE(grad);
-    CHECK_SAME_DEVICE(twiddle, input); CHECK_SAME_DEVICE(input, grad);
-    CHECK_DIM(twiddle, 6); CHECK_DIM(input, 3); CHECK_DIM(grad, 3);
-    Shapes s;
-    s.batch = input.size(0);
-    s.nstacks = input.size(1);
-    s.input_size = input.size(2);
-    s.nblocks = twiddle.size(1);
-    s.log_n = twiddle.size(2);
-    TORCH_CHECK(s.log_n <= 30, who, ": n must be a power of 2");
-    s.n = (int64_t)1 << s.log_n;
-    const int64_t output_size = grad.size(2);
-    CHECK_SHAPE(twiddle, s.nstacks, s.nblocks, s.log_n, s.n / 2, 2, 2);
-    CHECK_SHAPE(grad, s.batch, s.nstacks, output_size);
-    TORCH_CHECK(output_size <= s.n, who, ": grad must have at most n columns");
-    TORCH_CHECK(twiddle.scalar_type() == input.scalar_type() && grad.scalar_type() == input.scalar_type(), who,
-                ": twiddle, input and grad must have the same dtype");
-    if (input.is_cpu() && !with_bias && !in_perm.defined() && !out_index.defined()) {
-        auto r = host_multiply_bw(twiddle, input, grad, increasing_stride, s.log_n, who);
-        return std::make_tuple(std::get<0>(r), std::get<1>(r), Tensor());
-    }
-    require_device(input, who);
-
-    const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    const Tensor tw = dense(twiddle);
-    const Tensor x = input.resolve_conj();
-    const Tensor g = grad.resolve_conj();
-    Tensor d_twiddle = at::empty(tw.sizes(), tw.options());
-    Tensor d_input = at::empty({s.batch, s.nstacks, std::max(s.input_size, s.n)}, x.options());
-    if (s.input_size < s.n) d_input = d_input.slice(2, 0, s.input_size);
-    bf_problem p = make_problem(s, x, increasing_stride, output_size, who);
-    set_strides(p.output_stride, g);
-    set_strides(p.d_input_stride, d_input);
-    Tensor d_bias;
-    Tensor keep_in, keep_out;
-    const int32_t *ip = table_ptr(in_perm, keep_in, x, s.n, "in_perm", who);
-    const int32_t *oi = table_ptr(out_index, keep_out, x, s.n, "out_index", who);
-    // The forward decided what to keep from a plan made with its own strides; the backward plans
-    // from the strides of grad and d_input.  Where that plan reads no kept activations, or more
-    // than the forward left, the recomputing call serves the request.
-    bool use_kept = kept.defined();
-    if (use_kept) {
-        const size_t reads = valid_size(bf_butterfly_multiply_saved_bytes(&p));
-        if (reads == 0 || reads > (size_t)kept.numel()) use_kept = false;
-    }
-    if (use_kept) {
-        if (ip || oi) TORCH_CHECK(s.input_size <= s.n, who, ": column tables need input_size <= n");
-        if (with_bias) d_bias = at::empty({s.nstacks, output_size}, g.options());
-        const size_t ws_bytes = valid_size(bf_butterfly_multiply_bw_saved_workspace_bytes(&p, with_bias ? 1 : 0));
-        Tensor ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-        check_rc(bf_butterfly_multiply_bw_saved(&p, tw.data_ptr(), x.data_ptr(), g.data_ptr(), kept.data_ptr(),
-                                                (size_t)kept.numel(), ip, oi,
-                                                d_twiddle.data_ptr(), d_input.data_ptr(),
-                                                with_bias ? d_bias.data_ptr() : nullptr, ws.data_ptr(), ws_bytes,
-                                                current_stream()),
-                 who);
-    } else if (ip || oi) {
-        TORCH_CHECK(s.input_size <= s.n, who, ": column tables need input_size <= n");
-        if (with_bias) d_bias = at::empty({s.nstacks, output_size}, g.options());
-        const size_t ws_bytes = with_bias ? valid_size(bf_butterfly_multiply_bias_bw_workspace_bytes(&p))
-                                          : valid_size(bf_butterfly_multiply_bw_workspace_bytes(&p));
-        Tensor ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-        check_rc(bf_butterfly_multiply_perm_bw(&p, tw.data_ptr(), x.data_ptr(), g.data_ptr(), ip, oi,
-                                               d_twiddle.data_ptr(), d_input.data_ptr(),
-                                               with_bias ? d_bias.data_ptr() : nullptr, ws.data_ptr(), ws_bytes,
-                                               current_stream()),
-                 who);
-    } else if (with_bias) {
-        d_bias = at::empty({s.nstacks, output_size}, g.options());
-        const size_t ws_bytes = valid_size(bf_butterfly_multiply_bias_bw_workspace_bytes(&p));
-        Tensor ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-        check_rc(bf_butterfly_multiply_bias_bw(&p, tw.data_ptr(), x.data_ptr(), g.data_ptr(), d_twiddle.data_ptr(),
-                                               d_input.data_ptr(), d_bias.data_ptr(), ws.data_ptr(), ws_bytes,
-                                               current_stream()),
-                 who);
-    } else {
-        const size_t ws_bytes = valid_size(bf_butterfly_multiply_bw_workspace_bytes(&p));
-        Tensor ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-        check_rc(bf_butterfly_multiply_bw(&p, tw.data_ptr(), x.data_ptr(), g.data_ptr(), d_twiddle.data_ptr(),
-                                          d_input.data_ptr(), ws.data_ptr(), ws_bytes, current_stream()),
-                 who);
-    }
-    return std::make_tuple(d_twiddle, d_input, d_bias);
-}
-
-std::tuple<Tensor, Tensor> butterfly_multiply_bw(const Tensor twiddle, const Tensor input,
-                                                 const Tensor grad, bool increasing_stride)
-{
-    auto r = multiply_bw_impl(twiddle, input, grad, increasing_stride, false, "butterfly_multiply_bw");
-    return std::make_tuple(std::get<0>(r), std::get<1>(r));
-}
-
-// (d_twiddle, d_input, d_bias): the backward of butterfly_multiply_bias_fw
-std::tuple<Tensor, Tensor, Tensor> butterfly_multiply_bias_bw(const Tensor twiddle, const Tensor input,
-                                                              const Tensor grad, bool increasing_stride)
-{
-    return multiply_bw_impl(twiddle, input, grad, increasing_stride, true, "butterfly_multiply_bias_bw");
-}
-
-using torch::autograd::AutogradContext;
-using torch::autograd::variable_list;
-
-class ButterflyMultiply : public torch::autograd::Function<ButterflyMultiply> {
-public:
-    // wants_grad: a gradient will be asked for.  The forward then runs along the backward's pass
-    // plan and keeps the activations between the passes (device tensors whose backward takes
-    // several passes: rows beyond 1024, more than two blocks), which the reference's Function
-    // (csrc/butterfly.cpp:99-118) leaves to its backward to recompute.
-    static Tensor forward(AutogradContext *ctx, Tensor twiddle, Tensor input, bool increasing_stride,
-                          c10::optional<int64_t> output_size, bool wants_grad)
-    {
-        ctx->saved_data["increasing_stride"] = increasing_stride;
-        Tensor kept;
-        Tensor out = multiply_fw_impl(twiddle, input, Tensor(), increasing_stride, output_size, "butterfly_multiply",
-                                      Tensor(), Tensor(), wants_grad && input.is_cuda() ? &kept : nullptr);
-        ctx->saved_data["kept"] = kept.defined();
-        if (kept.defined()) ctx->save_for_backward({twiddle, input, kept});
-        else ctx->save_for_backward({twiddle, input});
-        return out;
-    }
-
-    static variable_list backward(AutogradContext *ctx, variable_list grad_output)
-    {
-        const auto saved = ctx->get_saved_variables();
-        const bool increasing_stride = ctx->saved_data["increasing_stride"].toBool();
-        const Tensor kept = ctx->saved_data["kept"].toBool() ? saved[2] : Tensor();
-        auto result = multiply_bw_impl(saved[0], saved[1], grad_output[0], increasing_stride, false,
-                                       "butterfly_multiply_bw", Tensor(), Tensor(), kept);
-        return {std::get<0>(result), std::get<1>(result), Tensor(), Tensor(), Tensor()};
-    }
-};
-
-bool grad_wanted(std::initializer_list<Tensor> ts)
-{
-    if (!at::GradMode::is_enabled()) return false;
-    for (const Tensor &t : ts)
-        if (t.defined() && t.requires_grad()) return true;
-    return false;
-}
-
-Tensor butterfly_multiply(Tensor twiddle, Tensor input, bool increasing_stride,
-                          c10::optional<int64_t> output_size)
-{
-    return ButterflyMultiply::apply(twiddle, input, increasing_stride, output_size, grad_wanted({twiddle, input}));
-}
-
-class ButterflyMultiplyBias : public torch::autograd::Function<ButterflyMultiplyBias> {
-public:
-    static Tensor forward(AutogradContext *ctx, Tensor twiddle, Tensor input, Tensor bias, bool increasing_stride,
-                          c10::optional<int64_t> output_size, bool wants_grad)
-    {
-        TORCH_CHECK(bias.defined(), "butterfly_multiply_bias: bias is undefined");
-        ctx->saved_data["increasing_stride"] = increasing_stride;
-        Tensor kept;
-        Tensor out = multiply_fw_impl(twiddle, input, bias, increasing_stride, output_size, "butterfly_multiply_bias",
-                                      Tensor(), Tensor(), wants_grad && input.is_cuda() ? &kept : nullptr);
-        ctx->saved_data["kept"] = kept.defined();
-        if (kept.defined()) ctx->save_for_backward({twiddle, input, kept});
-        else ctx->save_for_backward({twiddle, input});
-        return out;
-    }
-
-    static variable_list backward(AutogradContext *ctx, variable_list grad_output)
-    {
-        const auto saved = ctx->get_saved_variables();
-        const bool increasing_stride = ctx->saved_data["increasing_stride"].toBool();
-        const Tensor kept = ctx->saved_data["kept"].toBool() ? saved[2] : Tensor();
-        auto result = multiply_bw_impl(saved[0], saved[1], grad_output[0], increasing_stride, true,
-                                       "butterfly_multiply_bias_bw", Tensor(), Tensor(), kept);
-        return {std::get<0>(result), std::get<1>(result), std::get<2>(result), Tensor(), Tensor(), Tensor()};
-    }
-};
-
-Tensor butterfly_multiply_bias(Tensor twiddle, Tensor input, Tensor bias, bool increasing_stride,
-                               c10::optional<int64_t> output_size)
-{
-    return ButterflyMultiplyBias::apply(twiddle, input, bias, increasing_stride, output_size,
-                                        grad_wanted({twiddle, input, bias}));
-}
-
-// New operators: the multiply between two fixed column permutations, folded into the first
-// read and the last write (in front: u[c] = input[in_perm[c]]; behind: output[out_index[c]] =
-// y[c]; bias (nstacks, output_size) indexed by c).  Where the reference chains FixedPermutation
-// and Butterfly modules (torch_butterfly/special.py:17-66), each permutation costs a pass of
-// its own over the activations.  Tables: int32 (n,), undefined = identity.
-Tensor opt(const c10::optional<Tensor> &t) { return t.has_value() ? t.value() : Tensor(); }
-
-Tensor butterfly_multiply_perm_fw(const Tensor twiddle, const Tensor input, c10::optional<Tensor> in_perm,
-                                  c10::optional<Tensor> out_index, c10::optional<Tensor> bias,
-                                  bool increasing_stride, c10::optional<int64_t> output_size)
-{
-    return multiply_fw_impl(twiddle, input, opt(bias), increasing_stride, output_size, "butterfly_multiply_perm_fw",
-                            opt(in_perm), opt(out_index));
-}
-
-// (d_twiddle, d_input, d_bias); d_bias is undefined unless with_bias
-std::tuple<Tensor, Tensor, Tensor> butterfly_multiply_perm_bw(const Tensor twiddle, const Tensor input,
-                                                              const Tensor grad, c10::optional<Tensor> in_perm,
-                                                              c10::optional<Tensor> out_index, bool with_bias,
-                                                              bool increasing_stride)
-{
-    auto r = multiply_bw_impl(twiddle, input, grad, increasing_stride, with_bias, "butterfly_multiply_perm_bw",
-                              opt(in_perm), opt(out_index));
-    if (!with_bias) std::get<2>(r) = at::empty({0}, grad.options());  // the schema has no optional results
-    return r;
-}
-
-class ButterflyMultiplyPerm : public torch::autograd::Function<ButterflyMultiplyPerm> {
-public:
-    static Tensor forward(AutogradContext *ctx, Tensor twiddle, Tensor input, c10::optional<Tensor> in_perm,
-                          c10::optional<Tensor> out_index, c10::optional<Tensor> bias, bool increasing_stride,
-                          c10::optional<int64_t> output_size, bool wants_grad)
-    {
-        ctx->saved_data["increasing_stride"] = increasing_stride;
-        ctx->saved_data["with_bias"] = bias.has_value();
-        ctx->saved_data["has_in"] = in_perm.has_value();
-        ctx->saved_data["has_out"] = out_index.has_value();
-        Tensor kept;
-        Tensor out = multiply_fw_impl(twiddle, input, opt(bias), increasing_stride, output_size,
-                                      "butterfly_multiply_perm", opt(in_perm), opt(out_index),
-                                      wants_grad && input.is_cuda() ? &kept : nullptr);
-        ctx->saved_data["kept"] = kept.defined();
-        variable_list saved = {twiddle, input};
-        if (in_perm.has_value()) saved.push_back(in_perm.value());
-        if (out_index.has_value()) saved.push_back(out_index.value());
-        if (kept.defined()) saved.push_back(kept);
-        ctx->save_for_backward(saved);
-        return out;
-    }
-
-    static variable_list backward(AutogradContext *ctx, variable_list grad_output)
-    {
-        const auto saved = ctx->get_saved_variables();
-        const bool has_in = ctx->saved_data["has_in"].toBool(), has_out = ctx->saved_data["has_out"].toBool();
-        c10::optional<Tensor> in_perm, out_index;
-        size_t next = 2;
-        if (has_in) in_perm = saved[next++];
-        if (has_out) out_index = saved[next++];
-        const Tensor kept = ctx->saved_data["kept"].toBool() ? saved[next++] : Tensor();
-        const bool with_bias = ctx->saved_data["with_bias"].toBool();
-        auto r = multiply_bw_impl(saved[0], saved[1], grad_output[0], ctx->saved_data["increasing_stride"].toBool(),
-                                  with_bias, "butterfly_multiply_perm_bw", opt(in_perm), opt(out_index), kept);
-        return {std::get<0>(r), std::get<1>(r), Tensor(), Tensor(), with_bias ? std::get<2>(r) : Tensor(), Tensor(),
-                Tensor(), Tensor()};
-    }
-};
-
-Tensor butterfly_multiply_perm(Tensor twiddle, Tensor input, c10::optional<Tensor> in_perm,
-                               c10::optional<Tensor> out_index, c10::optional<Tensor> bias, bool increasing_stride,
-                               c10::optional<int64_t> output_size)
-{
-    return ButterflyMultiplyPerm::apply(twiddle, input, in_perm, out_index, bias, increasing_stride, output_size,
-                                        grad_wanted({twiddle, input, opt(bias)}));
 }
 
 // ---- diagonals folded into the factors ------------------------------------------------------
@@ -645,6 +804,8 @@ std::tuple<Tensor, Tensor, Tensor> butterfly_scale_twiddle_bw(const Tensor twidd
     return {d_tw, d_a, d_b};
 }
 
+using torch::autograd::AutogradContext;
+
 class ButterflyScaleTwiddle : public torch::autograd::Function<ButterflyScaleTwiddle> {
 public:
     static Tensor forward(AutogradContext *ctx, Tensor twiddle, c10::optional<Tensor> in_scale,
@@ -680,164 +841,6 @@ Tensor butterfly_scale_twiddle(Tensor twiddle, c10::optional<Tensor> in_scale, c
     return ButterflyScaleTwiddle::apply(twiddle, in_scale, out_scale, increasing_stride);
 }
 
-// ---- base-4 -----------------------------------------------------------------------------
-
-Shapes base4_shapes(const Tensor &twiddle4, const Tensor &twiddle2, const Tensor &input, const char *who)
-{
-    CHECK_DEVICE(twiddle4); CHECK_DEVICE(twiddle2); CHECK_DEVICE(input);
-    CHECK_SAME_DEVICE(twiddle4, input); CHECK_SAME_DEVICE(twiddle2, input);
-    CHECK_DIM(twiddle4, 6); CHECK_DIM(twiddle2, 6); CHECK_DIM(input, 3);
-    Shapes s;
-    s.batch = input.size(0);
-    s.nstacks = input.size(1);
-    s.input_size = input.size(2);
-    s.nblocks = twiddle4.size(1);
-    s.log_n = twiddle4.size(2) * 2 + twiddle2.size(2);
-    TORCH_CHECK(s.log_n <= 30, who, ": n must be a power of 2");
-    s.n = (int64_t)1 << s.log_n;
-    TORCH_CHECK(twiddle2.size(2) <= 1, "twiddle2 must have shape (nstacks, nblocks, log_n % 2, n / 2, 2, 2)");
-    if (s.log_n / 2 > 0) CHECK_SHAPE(twiddle4, s.nstacks, s.nblocks, s.log_n / 2, s.n / 4, 4, 4);
-    if (s.log_n % 2 == 1) CHECK_SHAPE(twiddle2, s.nstacks, s.nblocks, 1, s.n / 2, 2, 2);
-    require_device(input, who);
-    TORCH_CHECK(twiddle4.scalar_type() == input.scalar_type() && twiddle2.scalar_type() == input.scalar_type(),
-                who, ": twiddle4, twiddle2 and input must have the same dtype");
-    return s;
-}
-
-// keep: when given and the backward of this problem runs in several passes, the forward runs
-// along the backward's plan and leaves the activations between its passes there
-Tensor base4_fw_impl(const Tensor &twiddle4, const Tensor &twiddle2, const Tensor &input, bool increasing_stride,
-                     c10::optional<int64_t> output_size, Tensor *keep)
-{
-    const Shapes s = base4_shapes(twiddle4, twiddle2, input, "butterfly_multiply_base4_fw");
-    const int64_t output_size_val = output_size.has_value() ? output_size.value() : s.n;
-    TORCH_CHECK(output_size_val <= s.n, "butterfly_multiply_base4_fw: output_size must be <= n");
-    TORCH_CHECK(output_size_val >= 0, "butterfly_multiply_base4_fw: output_size must be >= 0");
-    const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    const Tensor tw4 = dense(twiddle4), tw2 = dense(twiddle2);
-    const Tensor x = input.resolve_conj();
-    Tensor output = at::empty({s.batch, s.nstacks, s.n}, x.options());
-    if (output_size_val < s.n) output = output.slice(2, 0, output_size_val);
-    bf_problem p = make_problem(s, x, increasing_stride, output_size_val, "butterfly_multiply_base4_fw");
-    set_strides(p.output_stride, output);
-    if (keep) {
-        // (the backward will make d_input dense over max(input_size, n) columns: same plan)
-        const int64_t dw = std::max(s.input_size, s.n);
-        p.d_input_stride[0] = s.batch > 1 ? s.nstacks * dw : 0;
-        p.d_input_stride[1] = s.nstacks > 1 ? dw : 0;
-        p.d_input_stride[2] = s.input_size > 1 ? 1 : 0;
-        const size_t nsaved = valid_size(bf_butterfly_multiply_base4_saved_bytes(&p));
-        if (nsaved > 0) {
-            *keep = at::empty({(int64_t)nsaved}, x.options().dtype(at::kByte));
-            check_rc(bf_butterfly_multiply_base4_fw_saving(&p, tw4.data_ptr(), tw2.data_ptr(), x.data_ptr(),
-                                                           output.data_ptr(), keep->data_ptr(), nsaved,
-                                                           current_stream()),
-                     "butterfly_multiply_base4");
-            return output;
-        }
-    }
-    const size_t ws_bytes = valid_size(bf_butterfly_multiply_base4_fw_workspace_bytes(&p));
-    Tensor ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-    check_rc(bf_butterfly_multiply_base4_fw(&p, tw4.data_ptr(), tw2.data_ptr(), x.data_ptr(), output.data_ptr(),
-                                            ws.data_ptr(), ws_bytes, current_stream()),
-             "butterfly_multiply_base4_fw");
-    return output;
-}
-
-Tensor butterfly_multiply_base4_fw(const Tensor twiddle4, const Tensor twiddle2, const Tensor input,
-                                   bool increasing_stride, c10::optional<int64_t> output_size)
-{
-    return base4_fw_impl(twiddle4, twiddle2, input, increasing_stride, output_size, nullptr);
-}
-
-// kept: the activations a forward with `keep` left behind (undefined: recompute them)
-std::tuple<Tensor, Tensor, Tensor> base4_bw_impl(const Tensor &twiddle4, const Tensor &twiddle2, const Tensor &input,
-                                                 const Tensor &grad, bool increasing_stride, const Tensor &kept)
-{
-    const Shapes s = base4_shapes(twiddle4, twiddle2, input, "butterfly_multiply_base4_bw");
-    CHECK_DEVICE(grad); CHECK_SAME_DEVICE(input, grad); CHECK_DIM(grad, 3);
-    const int64_t output_size = grad.size(2);
-    CHECK_SHAPE(grad, s.batch, s.nstacks, output_size);
-    TORCH_CHECK(output_size <= s.n, "butterfly_multiply_base4_bw: grad must have at most n columns");
-    TORCH_CHECK(grad.scalar_type() == input.scalar_type(),
-                "butterfly_multiply_base4_bw: grad and input must have the same dtype");
-    const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    const Tensor tw4 = dense(twiddle4), tw2 = dense(twiddle2);
-    const Tensor x = input.resolve_conj();
-    const Tensor g = grad.resolve_conj();
-    Tensor d4 = at::empty(tw4.sizes(), tw4.options());
-    Tensor d2 = at::empty(tw2.sizes(), tw2.options());
-    Tensor d_input = at::empty({s.batch, s.nstacks, std::max(s.input_size, s.n)}, x.options());
-    if (s.input_size < s.n) d_input = d_input.slice(2, 0, s.input_size);
-    bf_problem p = make_problem(s, x, increasing_stride, output_size, "butterfly_multiply_base4_bw");
-    set_strides(p.output_stride, g);
-    set_strides(p.d_input_stride, d_input);
-    // (as in the base-2 backward: the plan of this call decides whether the kept planes serve it)
-    bool use_kept = kept.defined();
-    if (use_kept) {
-        const size_t reads = valid_size(bf_butterfly_multiply_base4_saved_bytes(&p));
-        if (reads == 0 || reads > (size_t)kept.numel()) use_kept = false;
-    }
-    if (use_kept) {
-        const size_t ws_bytes = valid_size(bf_butterfly_multiply_base4_bw_saved_workspace_bytes(&p));
-        Tensor ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-        check_rc(bf_butterfly_multiply_base4_bw_saved(&p, tw4.data_ptr(), tw2.data_ptr(), x.data_ptr(), g.data_ptr(),
-                                                      kept.data_ptr(), (size_t)kept.numel(), d4.data_ptr(), d2.data_ptr(),
-                                                      d_input.data_ptr(),
-                                                      ws.data_ptr(), ws_bytes, current_stream()),
-                 "butterfly_multiply_base4_bw");
-        return std::make_tuple(d4, d2, d_input);
-    }
-    const size_t ws_bytes = valid_size(bf_butterfly_multiply_base4_bw_workspace_bytes(&p));
-    Tensor ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-    check_rc(bf_butterfly_multiply_base4_bw(&p, tw4.data_ptr(), tw2.data_ptr(), x.data_ptr(), g.data_ptr(),
-                                            d4.data_ptr(), d2.data_ptr(), d_input.data_ptr(), ws.data_ptr(),
-                                            ws_bytes, current_stream()),
-             "butterfly_multiply_base4_bw");
-    return std::make_tuple(d4, d2, d_input);
-}
-
-std::tuple<Tensor, Tensor, Tensor> butterfly_multiply_base4_bw(const Tensor twiddle4, const Tensor twiddle2,
-                                                               const Tensor input, const Tensor grad,
-                                                               bool increasing_stride)
-{
-    return base4_bw_impl(twiddle4, twiddle2, input, grad, increasing_stride, Tensor());
-}
-
-class ButterflyMultiplyBase4 : public torch::autograd::Function<ButterflyMultiplyBase4> {
-public:
-    // wants_grad: as in ButterflyMultiply, the forward keeps the activations between the passes of
-    // a backward that runs in several (more than one block, or rows beyond one workgroup's reach)
-    static Tensor forward(AutogradContext *ctx, Tensor twiddle4, Tensor twiddle2, Tensor input,
-                          bool increasing_stride, c10::optional<int64_t> output_size, bool wants_grad)
-    {
-        ctx->saved_data["increasing_stride"] = increasing_stride;
-        Tensor kept;
-        Tensor out = base4_fw_impl(twiddle4, twiddle2, input, increasing_stride, output_size,
-                                   wants_grad ? &kept : nullptr);
-        ctx->saved_data["kept"] = kept.defined();
-        if (kept.defined()) ctx->save_for_backward({twiddle4, twiddle2, input, kept});
-        else ctx->save_for_backward({twiddle4, twiddle2, input});
-        return out;
-    }
-
-    static variable_list backward(AutogradContext *ctx, variable_list grad_output)
-    {
-        const auto saved = ctx->get_saved_variables();
-        const bool increasing_stride = ctx->saved_data["increasing_stride"].toBool();
-        const Tensor kept = ctx->saved_data["kept"].toBool() ? saved[3] : Tensor();
-        auto r = base4_bw_impl(saved[0], saved[1], saved[2], grad_output[0], increasing_stride, kept);
-        return {std::get<0>(r), std::get<1>(r), std::get<2>(r), Tensor(), Tensor(), Tensor()};
-    }
-};
-
-Tensor butterfly_multiply_base4(Tensor twiddle4, Tensor twiddle2, Tensor input, bool increasing_stride,
-                                c10::optional<int64_t> output_size)
-{
-    return ButterflyMultiplyBase4::apply(twiddle4, twiddle2, input, increasing_stride, output_size,
-                                         grad_wanted({twiddle4, twiddle2, input}));
-}
-
 int64_t hip_version() { return bf_hip_version(); }
 
 }  // namespace
@@ -854,6 +857,8 @@ TORCH_LIBRARY(torch_butterfly, m)
     m.def("butterfly_multiply_perm_fw", butterfly_multiply_perm_fw);
     m.def("butterfly_multiply_perm_bw", butterfly_multiply_perm_bw);
     m.def("butterfly_multiply_perm", butterfly_multiply_perm);
+    m.def("butterfly_layer", butterfly_layer);
+    m.def("butterfly_layer_base4", butterfly_layer_base4);
     m.def("butterfly_scale_twiddle_fw", butterfly_scale_twiddle_fw);
     m.def("butterfly_scale_twiddle_bw", butterfly_scale_twiddle_bw);
     m.def("butterfly_scale_twiddle", butterfly_scale_twiddle);

@@ -45,6 +45,17 @@ def butterfly_multiply_bias(twiddle: torch.Tensor, input: torch.Tensor, bias: to
                                                              output_size)
 
 
+def butterfly_layer(twiddle: torch.Tensor, input: torch.Tensor, bias: Optional[torch.Tensor], increasing_stride: bool,
+                    out_size: int, in_perm: Optional[torch.Tensor] = None,
+                    out_index: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """A whole layer on device tensors: input (*, in_size) -> (*, out_size), the stacks of twiddle
+    side by side on one input, bias (out_size) added, column tables as in
+    butterfly_multiply_perm.  One operator (and one autograd node) for what the reference's
+    Butterfly.forward chains (torch_butterfly/butterfly.py:113-169)."""
+    return torch.ops.torch_butterfly.butterfly_layer(twiddle, input, bias, in_perm, out_index, increasing_stride,
+                                                     out_size)
+
+
 def butterfly_multiply_perm(twiddle: torch.Tensor, input: torch.Tensor, in_perm: Optional[torch.Tensor],
                             out_index: Optional[torch.Tensor], bias: Optional[torch.Tensor],
                             increasing_stride: bool, output_size: Optional[int] = None) -> torch.Tensor:

@@ -246,6 +246,37 @@ int bf_butterfly_multiply_base4_bw_saved(const bf_problem *p, const void *twiddl
                                          void *d_twiddle4, void *d_twiddle2, void *d_input,
                                          void *workspace, size_t workspace_bytes, void *stream);
 
+/* A whole layer in one call: nstacks products side by side on one input, of which only the first
+ * total_output columns exist, with bias and column tables.  Everything the calls above do
+ * separately for Butterfly.forward and its backward (torch_butterfly/butterfly.py:113-169 runs
+ * them as a chain of tensor operations: expand, multiply, reshape, slice, add).              */
+typedef struct bf_layer {
+    bf_problem problem;       /* output_size: columns of one stack; output_stride[1]: columns between stacks  */
+    int32_t base4;            /* twiddle = twiddle4 and twiddle2 as for the base-4 calls                      */
+    int32_t shared_input;     /* the stacks read one input (input_stride[1] = 0) and d_input is (B, I), dense:
+                               * the sum over the stacks (d_input_stride[0..2] then only used with one stack) */
+    int64_t total_output;     /* columns that exist, in ((S - 1) * output_size, S * output_size]               */
+    const void *twiddle;
+    const void *twiddle2;
+    const void *bias;         /* total_output entries, or NULL                                                */
+    const int32_t *in_perm;   /* as in bf_butterfly_multiply_perm_fw, or NULL (base 2 only)                   */
+    const int32_t *out_index;
+} bf_layer;
+
+/* Activations the forward call can keep for the backward (as bf_butterfly_multiply_saved_bytes). */
+size_t bf_layer_kept_bytes(const bf_layer *l);
+size_t bf_layer_fw_workspace_bytes(const bf_layer *l);
+/* kept NULL: nothing is kept and the workspace is used; otherwise the other way round. */
+int bf_layer_fw(const bf_layer *l, const void *input, void *output, void *kept, size_t kept_bytes,
+                void *workspace, size_t workspace_bytes, void *stream);
+/* problem.output_stride are the strides of grad.  kept_bytes: size of the area behind `kept` (0 and
+ * NULL: none); where the backward's plan does not fit what was kept, it is recomputed.  d_bias
+ * (total_output entries) may be NULL.                                                            */
+size_t bf_layer_bw_workspace_bytes(const bf_layer *l, int with_bias, size_t kept_bytes);
+int bf_layer_bw(const bf_layer *l, const void *input, const void *grad, const void *kept,
+                size_t kept_bytes, void *d_twiddle, void *d_twiddle2, void *d_input, void *d_bias,
+                void *workspace, size_t workspace_bytes, void *stream);
+
 /* bf_butterfly_multiply_bw for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): same operands and results,
  * but the partial sums and intermediate activations live in a fixed area of
