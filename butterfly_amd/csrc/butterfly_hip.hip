@@ -7,6 +7,7 @@
 #include <hip/hip_version.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -18,6 +19,7 @@
 #include "generic.hpp"
 #include "scale.hpp"
 #include "launch.hpp"
+#include "stream_plan.hpp"
 #include "stage.hpp"
 #include "bias.hpp"
 
@@ -127,7 +129,7 @@ View dense_view(int64_t nstacks, int64_t n)
 
 constexpr int kMaxDevices = 64;
 std::mutex g_device_mutex;
-bool g_attr_done[kMaxDevices];
+std::atomic<bool> g_attr_done[kMaxDevices];
 
 int ensure_attributes()
 {
@@ -136,8 +138,8 @@ int ensure_attributes()
     if (device < 0 || device >= kMaxDevices)
         return fail(BF_ERR_UNSUPPORTED, "device ordinal %d is outside the %d the library keeps state for", device,
                     kMaxDevices);
+    if (g_attr_done[device].load(std::memory_order_acquire)) return BF_OK;
     std::lock_guard<std::mutex> lock(g_device_mutex);
-    if (g_attr_done[device]) return BF_OK;
     const std::pair<const void *, size_t> wanted[] = {
         {reinterpret_cast<const void *>(&generic_fw_kernel<float>), kGenericFwLds},
         {reinterpret_cast<const void *>(&generic_fw_kernel<float2>), kGenericFwLds},
@@ -148,7 +150,7 @@ int ensure_attributes()
         const hipError_t e = hipFuncSetAttribute(w.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)w.second);
         if (e != hipSuccess) return fail(BF_ERR_HIP, "hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     }
-    g_attr_done[device] = true;
+    g_attr_done[device].store(true, std::memory_order_release);
     return BF_OK;
 }
 
@@ -156,7 +158,7 @@ int ensure_attributes()
 // kernels (one workgroup per compute unit), the partial areas and the measured crossovers are
 // sized from it.  Host-only queries on a machine without a device plan for an MI355X (256).
 constexpr int kDefaultNumCU = 256;
-int g_num_cu[kMaxDevices];
+std::atomic<int> g_num_cu[kMaxDevices];
 
 int num_cu()
 {
@@ -165,16 +167,15 @@ int num_cu()
         (void)hipGetLastError();
         return kDefaultNumCU;
     }
-    std::lock_guard<std::mutex> lock(g_device_mutex);
-    if (g_num_cu[device] == 0) {
-        int count = 0;
+    int count = g_num_cu[device].load(std::memory_order_relaxed);
+    if (count == 0) {
         if (hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0) {
             (void)hipGetLastError();
             count = kDefaultNumCU;
         }
-        g_num_cu[device] = count;
+        g_num_cu[device].store(count, std::memory_order_relaxed);
     }
-    return g_num_cu[device];
+    return count;
 }
 // Iterations (of kFastFwRows row groups) a forward workgroup must have left before a float pass
 // over two blocks is spread over two workgroups per compute unit (see fw_wg_per_cu).
@@ -705,6 +706,7 @@ int fast4_forward(const bf_problem *p, const void *tw4, const void *tw2, const v
         return fail(BF_ERR_INVALID, "twiddle4 must be 16-byte aligned");
     for (int k = first; k < last; ++k) {
         Fast4Args a = {};
+        a.nstacks = (int)p->nstacks;
         a.tw4 = static_cast<const float *>(tw4) + (int64_t)k * (L / 2) * (n / 4) * 16;
         a.tw_stack_stride = p->nblocks * (L / 2) * (n / 4) * 16;
         a.x_in = static_cast<const float *>(k == first ? input : scratch);
@@ -911,6 +913,84 @@ int long4_forward(const bf_problem *p, const Schedule &sc, const Plan4Long &pl, 
     return BF_OK;
 }
 
+// ---- factor-streaming forward ---------------------------------------------------------------------
+
+// Rows a workgroup of the streaming kernel takes.
+int64_t stream_rows_per_wg(const bf_problem *p, int waves, int planes)
+{
+    const int nbits = 8 + (waves == 16 ? 4 : waves == 8 ? 3 : 2);
+    return (int64_t)(4 * planes) << (nbits - p->log_n);
+}
+
+// Tiles of one plane up to which the passes of plan4_long are kept: a workgroup reads the factors of
+// the whole schedule by itself (786 KB at 4096 elements and two blocks, 20.9 us on 12 rows), where
+// the chunk pass spreads that over many (19.2 us).
+constexpr int64_t kStreamMinTiles = 16;
+
+struct StreamPick {
+    int waves = 0, planes = 0;   // 0: another path
+};
+
+// Whether the streaming kernel takes this call, and in which size: base-4 rows beyond the reach of
+// the register-resident kernels.  Two planes of rows to a workgroup share each read of the factors
+// (1500 rows of 4096, two blocks: 34 us against 47 with one), unless one plane already leaves no
+// compute unit without work to do (64 rows of 2048: 17.7 us against 23.3).
+StreamPick pick_stream(const bf_problem *p, bool base4)
+{
+    StreamPick k;
+    if (!base4 || p->log_n <= (p->dtype == BF_C64 ? 8 : 10) || p->log_n > kStreamMaxLogN || p->nblocks < 1 ||
+        p->batch <= 0 || p->nstacks <= 0 || p->input_size <= 0 || p->output_size <= 0)
+        return k;
+    // (complex64 rows of 4096 do not fit the registers of sixteen wavefronts)
+    if (p->dtype == BF_C64 && p->log_n == 12) return k;
+    k.waves = p->log_n == 12 ? 16 : 8;
+    const int64_t rows = stream_rows_per_wg(p, k.waves, 1);
+    const int64_t tiles = (p->batch + rows - 1) / rows * p->nstacks;
+    if (tiles <= kStreamMinTiles) k.waves = 0;
+    k.planes = p->dtype == BF_C64 || tiles <= num_cu() ? 1 : 2;
+    return k;
+}
+
+// The first `stages` stages through the streaming kernel.  saves / planes: stage numbers in front of
+// which the activation is also stored, and where.  BF_ERR_UNSUPPORTED when the plan does not fit the kernel: nothing has
+// been launched then.
+int stream_forward(const bf_problem *p, const Schedule &sc, int stages, StreamPick pick, const void *tw2, const void *tw4,
+                   const void *input, void *output, const View &in_view, const View &out_view, const void *bias,
+                   const int *saves, void *const *planes, int nsaves, hipStream_t stream)
+{
+    const int e = (int)elem_bytes(p->dtype);
+    const int64_t n = (int64_t)1 << p->log_n;
+    StreamArgs a = {};
+    if (!plan_stream(sc, stages, e, pick.waves, saves, nsaves, a)) return BF_ERR_UNSUPPORTED;
+    const int64_t rows = stream_rows_per_wg(p, pick.waves, pick.planes);
+    const int64_t dense[3] = {p->nstacks * n, n, 1};
+    // (with room for the rows that the range check masks out)
+    if (!span_ok(p->input_stride, rows, n, e) || !span_ok(p->output_stride, rows, n, e) || !span_ok(dense, rows, n, e))
+        return BF_ERR_UNSUPPORTED;
+    if ((double)sc.tw4_stack_stride * e >= 2147483000.0) return BF_ERR_UNSUPPORTED;
+    a.tw4 = tw4;
+    a.tw4_stack_stride = sc.tw4_stack_stride;
+    a.tw2 = tw2;
+    a.tw2_stack_stride = sc.tw2_stack_stride;
+    a.in = input;
+    a.in_view = in_view;
+    a.out = output;
+    a.out_view = out_view;
+    a.bias = bias;
+    for (int k = 0; k < nsaves; ++k) a.save[k] = planes[k];
+    a.batch = p->batch;
+    auto vec = [&](const View &v, const void *base) {
+        return v.se == 1 && v.width % 4 == 0 && v.tail % 4 == 0 && p->log_n >= 2 && v.sb * e % 16 == 0 &&
+               v.ss * e % 16 == 0 && (reinterpret_cast<uintptr_t>(base) & 15) == 0;
+    };
+    a.in_vec = vec(in_view, input);
+    a.out_vec = vec(out_view, output);
+    const dim3 grid((unsigned)((p->batch + rows - 1) / rows), (unsigned)p->nstacks);
+    if (!launch_stream_fw(p->dtype == BF_C64, pick.waves, pick.planes, a, grid, stream)) return BF_ERR_UNSUPPORTED;
+    BF_HIP_CHECK(hipGetLastError());
+    return BF_OK;
+}
+
 // ---- generic forward ----------------------------------------------------------------------
 
 int launch_generic_fw(const bf_problem *p, const Schedule &sc, int t0, int t1, const void *tw2,
@@ -1021,6 +1101,11 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
     }
     const View in_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
     const View out_view = make_view(p->output_stride, p->output_size, out_index, tail);
+    const StreamPick pick = pick_stream(p, base4);
+    if (pick.waves) {
+        rc = stream_forward(p, sc, sc.per * sc.nblocks, pick, tw2, tw4, input, output, in_view, out_view, bias, nullptr, nullptr, 0, stream);
+        if (rc != BF_ERR_UNSUPPORTED) return rc;
+    }
     if (fast4_ok(p, base4, false)) {
         const size_t need = forward_workspace(p, base4);
         if (need > 0 && (!workspace || workspace_bytes < need))
@@ -1132,7 +1217,9 @@ struct BwPlan {
     int64_t nparts;     // persistent workgroups per stack
     int64_t slot;       // scalars per stage in the partial buffer
     size_t boundary_bytes;  // one (B, S, n) activation plane
-    size_t off_boundaries, off_gbuf, off_partials, total;
+    size_t off_boundaries, off_gbuf, off_partials;
+    size_t total;       // with room for the partial slices of every pass: one reduce for the call
+    size_t least;       // with room for those of one pass at a time: one reduce per pass
     bool fits;
     bool fast;          // register-resident pass plan
     bool fast4;         // base-4 register-resident kernels, one launch per block
@@ -1167,8 +1254,9 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, b
         pl.off_gbuf = off;
         off += p->nblocks > 1 ? pl.boundary_bytes : 0;
         pl.off_partials = off;
-        off += align256((size_t)pl.nparts * p->nstacks * sc.per * pl.slot * e);
-        pl.total = off;
+        const size_t slices = align256((size_t)pl.nparts * p->nstacks * sc.per * pl.slot * e);
+        pl.least = off + slices;
+        pl.total = off + slices * (size_t)p->nblocks;
         return pl;
     }
     const Plan4Long lp = plan4_long(p, base4);
@@ -1178,16 +1266,20 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, b
         pl.nchunks = lp.npass;
         pl.slot = 4 * n;
         pl.boundary_bytes = align256((size_t)p->batch * p->nstacks * row_bytes);
-        int64_t slices = 1;
-        for (int k = 0; k < lp.npass; ++k) slices = std::max(slices, pass4_slices(p, lp.pass[k]));
+        size_t most = 0, all = 0;
+        for (int k = 0; k < lp.npass; ++k) {
+            const size_t bytes = align256((size_t)pass4_slices(p, lp.pass[k]) * p->nstacks * pl.slot * e);
+            most = std::max(most, bytes);
+            all += bytes;
+        }
         size_t off = 0;
         pl.off_boundaries = off;
         off += lp.npass > 1 && !saved_boundaries ? (size_t)(lp.npass - 1) * pl.boundary_bytes : 0;
         pl.off_gbuf = off;
         off += lp.npass > 1 ? pl.boundary_bytes : 0;
         pl.off_partials = off;
-        off += align256((size_t)slices * p->nstacks * pl.slot * e);
-        pl.total = off;
+        pl.least = off + most;
+        pl.total = off + all;
         return pl;
     }
     const PassPlan mp = build_passes(p, base4, false, permuted);
@@ -1199,12 +1291,15 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, b
         pl.nchunks = mp.npass;
         pl.slot = 2 * n;
         pl.boundary_bytes = align256((size_t)p->batch * p->nstacks * row_bytes);
-        int64_t nparts = 1, slices = 1;  // slices: partial (stage, 2n) slices of the pass that needs most
+        int64_t nparts = 1;
+        size_t most = 0, all = 0;
         for (int k = 0; k < mp.npass; ++k) {
             const Pass &q = mp.pass[k];
             const int64_t np = fast_grid(p->batch, q.L, p->nstacks * pass_lanes(p, q), 1, 1, row_cap(p, true), true).nwg;
             nparts = std::max(nparts, np);
-            slices = std::max(slices, np * (q.t1 - q.t0));
+            const size_t bytes = align256((size_t)(np * (q.t1 - q.t0)) * p->nstacks * pl.slot * e);
+            most = std::max(most, bytes);
+            all += bytes;
         }
         pl.nparts = nparts;
         size_t off = 0;
@@ -1213,8 +1308,8 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, b
         pl.off_gbuf = off;
         off += mp.npass > 1 ? pl.boundary_bytes : 0;
         pl.off_partials = off;
-        off += align256((size_t)slices * p->nstacks * pl.slot * e);
-        pl.total = off;
+        pl.least = off + most;
+        pl.total = off + all;
         return pl;
     }
     pl.fits = 2 * row_bytes <= kGenericBwLds;
@@ -1232,7 +1327,7 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, b
     off += pl.nchunks > 1 ? pl.boundary_bytes : 0;
     pl.off_partials = off;
     off += align256((size_t)pl.nparts * p->nstacks * pl.chunk * pl.slot * e);
-    pl.total = off;
+    pl.least = pl.total = off;
     return pl;
 }
 
@@ -1266,26 +1361,28 @@ int launch_copy_pad(const bf_problem *p, const void *in, const View &iv, void *o
 }
 
 // bg (may be NULL): bias sums to be added up by the same launch; g_view: the view they were read through
-int launch_reduce(const bf_problem *p, const Schedule &sc, int t0, int t1, int64_t nparts, const void *partial,
+int launch_reduce(const bf_problem *p, const Schedule &sc, const ReduceSegment *segs, int nsegs, const void *partial,
                   int64_t slot, void *d_tw2, void *d_tw4, hipStream_t stream, const BiasGrad *bg = nullptr,
                   const View *g_view = nullptr)
 {
     const bool bias = bg && bg->d_bias && g_view->width > 0;
-    if (p->nstacks == 0 || (t1 <= t0 && !bias)) return BF_OK;
+    ReduceArgs r = {};
+    for (int k = 0; k < nsegs; ++k) {
+        if (segs[k].t1 <= segs[k].t0) continue;
+        r.seg[r.nsegs++] = segs[k];
+        r.nstages += segs[k].t1 - segs[k].t0;
+    }
+    if (p->nstacks == 0 || (r.nstages == 0 && !bias)) return BF_OK;
     if (((reinterpret_cast<uintptr_t>(d_tw2) | reinterpret_cast<uintptr_t>(d_tw4)) & 15) != 0)
         return fail(BF_ERR_INVALID, "d_twiddle pointers must be 16-byte aligned");
-    ReduceArgs r = {};
     r.sc = sc;
-    r.t0 = t0;
-    r.t1 = t1;
-    r.nparts = (int)nparts;
     r.elem_floats = p->dtype == BF_C64 ? 2 : 1;
     r.nstacks = p->nstacks;
     r.partial = static_cast<const float *>(partial);
     r.slot = slot;
     r.d_tw2 = static_cast<float *>(d_tw2);
     r.d_tw4 = static_cast<float *>(d_tw4);
-    int64_t floats = t1 > t0 ? slot * r.elem_floats : 0;
+    int64_t floats = r.nstages > 0 ? slot * r.elem_floats : 0;
     if (bias) {
         r.bias_partial = static_cast<const float *>(bg->area);
         r.d_bias = static_cast<float *>(bg->d_bias);
@@ -1295,7 +1392,7 @@ int launch_reduce(const bf_problem *p, const Schedule &sc, int t0, int t1, int64
         r.bias_tail = g_view->tail;
         floats = std::max(floats, g_view->width * r.elem_floats);
     }
-    const dim3 grid((unsigned)((floats + 63) / 64), (unsigned)(t1 - t0 + (bias ? 1 : 0)), (unsigned)p->nstacks);
+    const dim3 grid((unsigned)((floats + 63) / 64), (unsigned)(r.nstages + (bias ? 1 : 0)), (unsigned)p->nstacks);
     hipLaunchKernelGGL(reduce_partials_kernel, grid, dim3(256), 0, stream, r);
     BF_HIP_CHECK(hipGetLastError());
     return BF_OK;
@@ -1319,14 +1416,15 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     const View g_view = make_view(p->output_stride, std::min(p->output_size, n), out_index, tail);
     if (p->batch == 0 || p->nstacks == 0) {
         // no rows: d_input is empty and every entry of the other gradients is an empty sum, whatever the row length
-        return launch_reduce(p, sc, 0, sc.per * sc.nblocks, 0, nullptr, 4 * n, d_tw2, d_tw4, stream, bg, &g_view);
+        const ReduceSegment none = {0, sc.per * sc.nblocks, 0, 0};
+        return launch_reduce(p, sc, &none, 1, nullptr, 4 * n, d_tw2, d_tw4, stream, bg, &g_view);
     }
     const BwPlan pl = plan_bw(p, base4, saved != nullptr, permuted);
     if (!pl.fits)
         return fail(BF_ERR_UNSUPPORTED, "n = %lld does not fit in LDS for the backward pass", (long long)n);
     if (saved && !(pl.fast || pl.fast4 || pl.long4)) return fail(BF_ERR_INVALID, "this problem has no saved activations");
     const char *saved_planes = static_cast<const char *>(saved);
-    if (pl.total > 0 && (!workspace || workspace_bytes < pl.total))
+    if (pl.least > 0 && (!workspace || workspace_bytes < pl.least))
         return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", pl.total, workspace_bytes);
     if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
         return fail(BF_ERR_WORKSPACE, "workspace must be 16-byte aligned");
@@ -1339,15 +1437,30 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     char *ws = static_cast<char *>(workspace);
     const size_t e_bytes = elem_bytes(p->dtype);
 
-    // the reduce of the pass that reads grad, the first one, also finishes the bias gradient
-    auto reduce = [&](int t0, int t1, int64_t nparts) {
+    // Partial slices: every pass leaves its own behind the previous one's, for one reduce at the end
+    // of the call; where the workspace has no room for that, each pass is reduced before the next.
+    // A reduce also finishes the bias gradient, whose sums the first pass has formed by then.
+    const bool one_reduce = workspace_bytes >= pl.total && pl.total > pl.least;
+    ReduceSegment segs[kReduceSegments];
+    int nsegs = 0;
+    size_t used = 0;   // bytes of the partial area
+    auto partials = [&] { return ws + pl.off_partials + used; };
+    auto finish = [&] {
         if (bg && !bg->formed) {
             const int rc_bias = form_bias_sums(p, grad, g_view, *bg, stream);
             if (rc_bias) return rc_bias;
         }
         BiasGrad *now = bg;
         bg = nullptr;
-        return launch_reduce(p, sc, t0, t1, nparts, ws + pl.off_partials, pl.slot, d_tw2, d_tw4, stream, now, &g_view);
+        const int n_now = nsegs;
+        nsegs = 0;
+        return launch_reduce(p, sc, segs, n_now, ws + pl.off_partials, pl.slot, d_tw2, d_tw4, stream, now, &g_view);
+    };
+    auto reduce = [&](int t0, int t1, int64_t nparts) {
+        segs[nsegs++] = ReduceSegment{t0, t1, (int)nparts, (int64_t)(used / 4)};
+        if (!one_reduce) return finish();
+        used += align256((size_t)nparts * p->nstacks * (t1 - t0) * pl.slot * e_bytes);
+        return nsegs == kReduceSegments ? finish() : BF_OK;
     };
 
     if (pl.nstages == 0) {
@@ -1380,7 +1493,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             a.g_view = k == P - 1 ? g_view : dense;
             a.g_in = k == 0 ? d_input : ws + pl.off_gbuf;
             a.gi_view = k == 0 ? dn_view : dense;
-            a.partial = ws + pl.off_partials;
+            a.partial = partials();
             a.ngroups = g.ngroups;
             a.groups_per_wg = g.groups_per_wg;
             const bool inc = (p->increasing_stride != 0) != ((k & 1) != 0);
@@ -1393,6 +1506,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             return fail(BF_ERR_INVALID, "twiddle4 must be 16-byte aligned");
         for (int k = P - 1; k >= 0 && !general; --k) {
             Fast4Args a = {};
+            a.nstacks = (int)p->nstacks;
             a.tw4 = static_cast<const float *>(tw4) + (int64_t)k * per * (n / 4) * 16;
             a.tw_stack_stride = sc.tw4_stack_stride;
             a.x_in = static_cast<const float *>(k == 0 ? input : boundary(k));
@@ -1401,7 +1515,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             a.g_view = k == P - 1 ? g_view : dense;
             a.g_in = static_cast<float *>(k == 0 ? d_input : ws + pl.off_gbuf);
             a.gi_view = k == 0 ? dn_view : dense;
-            a.partial = reinterpret_cast<float *>(ws + pl.off_partials);
+            a.partial = reinterpret_cast<float *>(partials());
             a.batch = p->batch;
             a.ngroups = g.ngroups;
             a.groups_per_wg = g.groups_per_wg;
@@ -1411,6 +1525,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             rc = reduce(k * per, (k + 1) * per, g.nwg);
             if (rc) return rc;
         }
+        if (nsegs > 0 && (rc = finish())) return rc;
         if (p->input_size > n) {
             View tail = di_view;
             tail.width = p->input_size - n;
@@ -1431,7 +1546,23 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                          : ws + pl.off_boundaries + (size_t)(k - 1) * pl.boundary_bytes;
         };
         // forward replay: boundary k = activation entering pass k (k >= 1), unless the forward kept them
-        for (int k = 0; k + 1 < P && !saved; ++k) {
+        bool replayed = saved != nullptr;
+        const StreamPick pick = pick_stream(p, true);
+        if (!replayed && P > 1 && pick.waves && P - 2 <= kStreamMaxSaves) {
+            int saves[kStreamMaxSaves];
+            void *planes[kStreamMaxSaves];
+            for (int k = 1; k + 1 < P; ++k) {
+                saves[k - 1] = lp.pass[k].t0;
+                planes[k - 1] = const_cast<char *>(boundary(k));
+            }
+            bf_problem replay = *p;
+            for (int i = 0; i < 3; ++i) replay.output_stride[i] = i == 0 ? p->nstacks * n : i == 1 ? n : 1;
+            rc = stream_forward(&replay, sc, lp.pass[P - 1].t0, pick, tw2, tw4, input, const_cast<char *>(boundary(P - 1)),
+                                x_view, dense, nullptr, saves, planes, P - 2, stream);
+            if (rc != BF_OK && rc != BF_ERR_UNSUPPORTED) return rc;
+            replayed = rc == BF_OK;
+        }
+        for (int k = 0; k + 1 < P && !replayed; ++k) {
             rc = long4_forward(p, sc, lp, tw2, tw4, k == 0 ? input : boundary(k), const_cast<char *>(boundary(k + 1)),
                                nullptr, k == 0 ? x_view : dense, dense, k, k + 1, stream);
             if (rc) return rc;
@@ -1442,12 +1573,13 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             int64_t nparts = 0;
             rc = run_pass4(p, sc, q, true, tw2, tw4, k == 0 ? input : boundary(k), k == 0 ? x_view : dense, nullptr,
                            dense, k == P - 1 ? grad : ws + pl.off_gbuf, k == P - 1 ? g_view : dense,
-                           k == 0 ? d_input : ws + pl.off_gbuf, k == 0 ? dn_view : dense, ws + pl.off_partials, &nparts,
+                           k == 0 ? d_input : ws + pl.off_gbuf, k == 0 ? dn_view : dense, partials(), &nparts,
                            stream);
             if (rc) return rc;
             rc = reduce(q.t0, q.t1, nparts);
             if (rc) return rc;
         }
+        if (nsegs > 0 && (rc = finish())) return rc;
         if (p->input_size > n) {
             View tail = di_view;
             tail.width = p->input_size - n;
@@ -1495,7 +1627,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 a.g_view = gv;
                 a.g_in = gin;
                 a.gi_view = giv;
-                a.partial = ws + pl.off_partials;
+                a.partial = partials();
                 a.batch = p->batch;
                 a.ngroups = g.ngroups;
                 a.groups_per_wg = g.groups_per_wg;
@@ -1520,6 +1652,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             rc = reduce(q.t0, q.t1, nparts);
             if (rc) return rc;
         }
+        if (nsegs > 0 && (rc = finish())) return rc;
         if (p->input_size > n) {
             // input wider than n: those columns get a zero gradient
             View tail = di_view;
@@ -1625,11 +1758,11 @@ int bf_butterfly_multiply_bw_noalloc(const bf_problem *p, const void *twiddle, c
     if (!pl.fits)
         return fail(BF_ERR_UNSUPPORTED, "n = %lld does not fit in LDS for the backward pass",
                     (long long)((int64_t)1 << p->log_n));
-    if (pl.total > kScratchBytes)
+    if (pl.least > kScratchBytes)
         return fail(BF_ERR_WORKSPACE,
                     "this problem needs %zu bytes of scratch, the built-in area holds %zu: use "
                     "bf_butterfly_multiply_bw with a workspace of the caller's",
-                    pl.total, kScratchBytes);
+                    pl.least, kScratchBytes);
     void *area = nullptr;
     if ((rc = scratch_of_current_device(&area))) return rc;
     // every partial slice and boundary activation in the area is written by this call's own
@@ -1708,7 +1841,7 @@ static int bias_grad(const bf_problem *p, const void *grad, void *d_bias, void *
         if ((rc = form_bias_sums(p, grad, g_view, bg, s))) return rc;
     }
     // (over no rows the sums of zero slices: zeros)
-    return launch_reduce(p, make_schedule(p, false), 0, 0, 0, nullptr, 0, nullptr, nullptr, s, &bg, &g_view);
+    return launch_reduce(p, make_schedule(p, false), nullptr, 0, nullptr, 0, nullptr, nullptr, s, &bg, &g_view);
 }
 
 int bf_butterfly_bias_grad(const bf_problem *p, const void *grad, void *d_bias, void *workspace,
@@ -1977,6 +2110,18 @@ static int fw4_saving(const bf_problem *p, const void *twiddle4, const void *twi
     auto boundary = [&](int k) { return planes + (size_t)(k - 1) * pl.boundary_bytes; };
     const int P = pl.nchunks;
     const Plan4Long lp = pl.long4 ? plan4_long(p, true) : Plan4Long();
+    const StreamPick pick = pick_stream(p, true);
+    if (pick.waves && P - 1 <= kStreamMaxSaves) {
+        int saves[kStreamMaxSaves];
+        void *at[kStreamMaxSaves];
+        for (int k = 1; k < P; ++k) {
+            saves[k - 1] = pl.long4 ? lp.pass[k].t0 : k * sc.per;
+            at[k - 1] = boundary(k);
+        }
+        const int rc_stream = stream_forward(p, sc, sc.per * sc.nblocks, pick, twiddle2, twiddle4, input, output, in_view,
+                                             out_view, bias, saves, at, P - 1, stream);
+        if (rc_stream != BF_ERR_UNSUPPORTED) return rc_stream;
+    }
     for (int k = 0; k < P; ++k) {
         const void *in = k == 0 ? input : boundary(k);
         void *out = k == P - 1 ? output : boundary(k + 1);

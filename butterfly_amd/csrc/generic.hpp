@@ -253,17 +253,26 @@ __global__ __launch_bounds__(kGenericThreads) void generic_bw_kernel(GenericBwAr
     }
 }
 
+// The partial slices one pass has left: (nparts, S, t1 - t0, slot) scalars.
+struct ReduceSegment {
+    int t0, t1;
+    int nparts;          // number of per-workgroup partial slices
+    int64_t offset;      // floats from the start of the partial area
+};
+constexpr int kReduceSegments = 8;
+
 struct ReduceArgs {
     Schedule sc;
-    int t0, t1;
-    int nparts;        // number of per-workgroup partial slices
+    ReduceSegment seg[kReduceSegments];
+    int nsegs;
+    int nstages;       // over all segments
     int elem_floats;   // 1 for float, 2 for complex64
     int64_t nstacks;
     const float *partial;
     int64_t slot;      // scalars reserved per stage in `partial`
     float *d_tw2;
     float *d_tw4;
-    // a layer's bias gradient: one more slice of workgroups (blockIdx.y = t1 - t0) adds up its
+    // a layer's bias gradient: one more slice of workgroups (blockIdx.y = nstages) adds up its
     // partial column sums, (bias_nparts, S, bias_stride) -> (S, bias_width) without its unused tail
     const float *bias_partial;   // NULL: none
     float *d_bias;
@@ -276,16 +285,27 @@ struct ReduceArgs {
 // of group q (a contiguous sixteenth of them, ascending) for the float4 at j4; the sixteen
 // group sums are then added in ascending q.  The order is fixed by nparts alone, so results
 // are reproducible run to run.
-// grid: (ceil(slot * elem_floats / 64), t1 - t0 (+ 1 with a bias), S), block 256.
+// One launch finishes all passes of a backward call: a launch of its own for each pass costs more
+// than the sums (four launches of 5.8 us against one of 8 at 1500 rows of 2048, base 4).
+// grid: (ceil(slot * elem_floats / 64), nstages (+ 1 with a bias), S), block 256.
 __global__ __launch_bounds__(256) void reduce_partials_kernel(ReduceArgs a)
 {
     __shared__ float4 sm[16][16];
     const int j4 = threadIdx.x & 15, q = threadIdx.x >> 4;
     const int k = blockIdx.y;
     const int s = blockIdx.z;
-    const int nst = a.t1 - a.t0;
-    const bool is_bias = k == nst;
-    const StageInfo si = stage_info(a.sc, a.t0 + (is_bias ? 0 : k));
+    const bool is_bias = k == a.nstages;
+    ReduceSegment seg = a.seg[0];
+    int first = 0;   // stages of the segments in front
+    for (int i = 1; i < a.nsegs; ++i) {
+        const int here = first + (a.seg[i - 1].t1 - a.seg[i - 1].t0);
+        if (k < here) break;
+        first = here;
+        seg = a.seg[i];
+    }
+    const int ks = is_bias ? 0 : k - first;   // stage within its segment
+    const int nst = seg.t1 - seg.t0;
+    const StageInfo si = stage_info(a.sc, seg.t0 + ks);
     const int64_t n = (int64_t)1 << a.sc.log_n;
     const int64_t ef = a.elem_floats;
     const int64_t f = (int64_t)blockIdx.x * 64 + j4 * 4;
@@ -293,13 +313,13 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(ReduceArgs a)
     // floats that exist here, floats between the slices, slices
     const int64_t count = is_bias ? (s == a.nstacks - 1 ? a.bias_tail : a.bias_width) * ef : (si.radix4 ? 4 * n : 2 * n) * ef;
     const int64_t wg_stride = a.nstacks * (is_bias ? a.bias_stride * ef : nst * slot_f);
-    const int nparts = is_bias ? a.bias_nparts : a.nparts;
+    const int nparts = is_bias ? a.bias_nparts : seg.nparts;
     const int chunk = (nparts + 15) / 16;
     const int w0 = q * chunk;
     const int w1 = w0 + chunk < nparts ? w0 + chunk : nparts;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     if (f < count) {
-        const float *src = is_bias ? a.bias_partial + s * a.bias_stride * ef + f : a.partial + ((int64_t)s * nst + k) * slot_f + f;
+        const float *src = is_bias ? a.bias_partial + s * a.bias_stride * ef + f : a.partial + seg.offset + ((int64_t)s * nst + ks) * slot_f + f;
 #pragma unroll 8
         for (int w = w0; w < w1; ++w) {
             const float4 v = *reinterpret_cast<const float4 *>(src + (int64_t)w * wg_stride);

@@ -6,6 +6,7 @@
 #include "wide.hpp"
 #include "fast4.hpp"
 #include "fast4g.hpp"
+#include "stream.hpp"
 
 namespace bf {
 
@@ -40,6 +41,9 @@ void launch_fast4_t(bool backward, const Fast4Args &a, dim3 grid, hipStream_t st
 
 template <typename T, int L, bool INC>
 void launch_fast4g_t(bool backward, const Fast4GArgs &a, dim3 grid, hipStream_t stream);
+
+// waves, planes: W and RB of stream_fw_kernel; false where there is no such kernel
+bool launch_stream_fw(bool cplx, int waves, int planes, const StreamArgs &a, dim3 grid, hipStream_t stream);
 
 void launch_wide_fw(bool cplx, int L, bool inc, const FastFwArgs &a, dim3 grid, hipStream_t stream);
 

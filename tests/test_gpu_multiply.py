@@ -658,6 +658,43 @@ def test_bias_gradient_partitions(dtype, B, S, width):
     assert np.abs(db.cpu().numpy() - ref).max() < 1e-5 * max(1.0, B ** 0.5)
 
 
+@pytest.mark.parametrize("case", [
+    # (dtype, B, S, L, nb, I, O, inc): tiles of 4 and 8 rows (one and two planes), rows missing from the
+    # last one, rows narrower than n read and written four at a time or one by one
+    (np.float32, 1, 1, 11, 1, None, None, True), (np.float32, 9, 3, 11, 2, 2001, 1999, False),
+    (np.float32, 2049, 2, 11, 1, 1024, None, False), (np.float32, 2063, 1, 11, 3, None, 1030, True),
+    (np.float32, 3, 1, 12, 3, 4095, None, False), (np.float32, 4, 2, 12, 1, None, 4092, True),
+    (np.float32, 1027, 1, 12, 2, None, None, True), (np.float32, 1031, 1, 12, 1, 4000, 17, False),
+    (np.complex64, 17, 2, 9, 2, 500, None, True), (np.complex64, 9, 1, 10, 3, None, 1022, False),
+    (np.complex64, 5, 1, 11, 2, 2048, 2047, True), (np.complex64, 1030, 1, 11, 1, None, None, False)],
+    ids=lambda c: f"{np.dtype(c[0]).name}-B{c[1]}-S{c[2]}-L{c[3]}-nb{c[4]}-I{c[5]}-O{c[6]}-inc{int(c[7])}")
+def test_base4_long_rows_streaming(case):
+    """The single-launch base-4 forward against the oracle, alone and leaving the activations of
+    the backward's passes behind (whose gradients must match too)."""
+    from butterfly_amd import _capi
+    dtype, B, S, L, nb, I, O, inc = case
+    say("base4 long", case)
+    rng = np.random.default_rng(4100 + L * 7 + nb + B)
+    n = 1 << L
+    tw4 = (randn(rng, (S, nb, L // 2, n // 4, 4, 4), dtype) / 2).astype(dtype)
+    tw2 = (randn(rng, (S, nb, L % 2, n // 2, 2, 2), dtype) / np.sqrt(2)).astype(dtype)
+    x = randn(rng, (B, S, n if I is None else I), dtype)
+    g = randn(rng, (B, S, n if O is None else O), dtype)
+    y = _capi.multiply_base4_fw(dev(tw4), dev(tw2), dev(x), inc, O)
+    torch.cuda.synchronize()
+    assert rel_err(y.cpu().numpy(), oracle.butterfly_base4_fw(tw4, tw2, x, inc, O)) < FW_TOL
+    if B <= 64:
+        d4_ref, d2_ref, dx_ref = oracle.butterfly_base4_bw(tw4, tw2, x, g, inc)
+        leaves = [dev(t).requires_grad_() for t in (tw4, tw2, x)]
+        out = torch.ops.torch_butterfly.butterfly_multiply_base4(*leaves, inc, O)
+        wanted = [t for t in leaves if t.numel() > 0]
+        grads = torch.autograd.grad(out, wanted, dev(g))
+        torch.cuda.synchronize()
+        assert rel_err(out.detach().cpu().numpy(), y.cpu().numpy()) < FW_TOL
+        for got, ref in zip(grads, [r for r in (d4_ref, d2_ref, dx_ref) if r.size > 0]):
+            assert rel_err(got.cpu().numpy(), ref) < BW_TOL
+
+
 def test_bias_operator_autograd():
     """The autograd operator returns the three gradients the separate formulation gives."""
     import butterfly_amd  # noqa: F401
