@@ -214,6 +214,7 @@ struct Pass {
     int L, NB;      // LOW: FastPlan<L, NB, inc> on chunks of 2^L elements
     bool inc;
     bool span;      // SPAN: SpanPlan<H, mode> on tiles, H adjacent bits from `lb` up (L = 10, NB = 1)
+    bool edge;      // EDGE: EdgePlan<inc> on tiles, bits 0..5, at a column table (L = 10, NB = 1)
     int H, lb;
     int mode;       // 0: one sweep up, 1: one sweep down, 2: up then down
 };
@@ -265,8 +266,13 @@ int64_t wide_min_rows(const bf_problem *p)
     return p->nblocks == 1 ? 0 : 4096;
 }
 
-// permuted: the call reads or writes its rows through column tables (see the low width below)
-PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false, bool permuted = false)
+// Column tables of a call.
+enum { kTableIn = 1, kTableOut = 2, kTablesAny = 4 };
+
+int tables_of(const int *in_perm, const int *out_index) { return (in_perm ? kTableIn : 0) | (out_index ? kTableOut : 0); }
+
+// tables: the call reads or writes its rows through column tables (see EDGE and the low width below)
+PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false, int tables = 0)
 {
     PassPlan pl;
     const int L = (int)p->log_n;
@@ -276,6 +282,11 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
     const int NS = L * (int)p->nblocks;
     // complex64 needs twice the registers per stage: one block per LOW pass
     const int max_nb = p->dtype == BF_C64 ? 1 : 2;
+    // complex64 rows of 2048 and 4096 with tables: each where a pass over bits 0..5 reads (ascending)
+    // or writes (descending) the rows, so that it can run on the tiles made for that
+    const bool last_inc = (p->increasing_stride != 0) != (((p->nblocks - 1) & 1) != 0);
+    const bool edges = tables && p->dtype == BF_C64 && (L == 11 || L == 12) &&
+                       (!(tables & kTableIn) || p->increasing_stride != 0) && (!(tables & kTableOut) || !last_inc);
     if (L <= 10) {
         for (int k = 0; k < p->nblocks; k += max_nb) {
             if (pl.npass == kMaxPasses) return pl;
@@ -287,7 +298,7 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
             q.L = L;
             q.inc = (p->increasing_stride != 0) != ((k & 1) != 0);
         }
-    } else if (L <= 12 && forward_only && (p->dtype == BF_F32 || L == 11) &&
+    } else if (L <= 12 && forward_only && !edges && (p->dtype == BF_F32 || L == 11) &&
                p->batch * p->nstacks >= wide_min_rows(p)) {
         for (int k = 0; k < p->nblocks; ++k) {
             if (pl.npass == kMaxPasses) return pl;
@@ -312,10 +323,10 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
         const int nspans = (L - 10 + span_max - 1) / span_max;
         // (rows up to 2^16 only: shorter chunks mean more rows per workgroup, and beyond that the
         // rows a workgroup must reach with 32-bit offsets run out)
-        // Not through column tables either: a gather or scatter touches one element per 128-byte
-        // line and short chunk, where chunks of 1024 still find several (measured on the bit
-        // reversal of special.fft: 1.30 ms against 0.92 ms per step).
-        const int low = cplx && L <= 16 && !permuted ? std::max(6, L - span_max * nspans) : 10;
+        // Not through column tables either, where no EDGE pass fits: a gather or scatter touches one
+        // element per 128-byte line and short chunk, where chunks of 1024 still find several (measured
+        // on the bit reversal of special.fft(4096): 1.30 ms against 0.92 ms per step; with EDGE 0.59).
+        const int low = cplx && L <= 16 && (!tables || edges) ? std::max(6, L - span_max * nspans) : 10;
         pl.low = low;
         const int hbits = L - low;
         int group_lb[16], group_bits[16], ngroups = 0;
@@ -360,6 +371,10 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
                 if ((u - t) != low && (u - t) != 2 * low) return pl;
                 q.NB = (u - t) / low;
                 q.inc = stage_bit(p, t) == 0;
+                if (edges && q.NB == 1 && ((q.inc && t == 0 && (tables & kTableIn)) || (!q.inc && u == NS && (tables & kTableOut)))) {
+                    q.edge = true;
+                    q.L = 10;
+                }
             }
             t = u;
         }
@@ -564,6 +579,9 @@ int multipass_forward(const bf_problem *p, const PassPlan &pl, const void *tw, c
                 a.low_bits = q.lb;
                 const int rc = launch_span(p->dtype == BF_C64, q, false, false, &a, nullptr, grid, stream);
                 if (rc) return rc;
+            } else if (q.edge) {
+                a.low_bits = (int)p->log_n;
+                launch_edge(q.inc, &a, nullptr, grid, stream);
             } else {
                 BF_FAST_DISPATCH(launch_fast_fw_t, q, p->dtype == BF_C64, per_cu == 2, a, grid, stream);
             }
@@ -1031,8 +1049,14 @@ int launch_generic_fw(const bf_problem *p, const Schedule &sc, int t0, int t1, c
 }
 
 // Workspace of the forward call: one dense activation when the pass plan has several passes.
-size_t forward_workspace(const bf_problem *p, bool base4)
+size_t forward_workspace(const bf_problem *p, bool base4, int tables)
 {
+    if (tables == kTablesAny) {
+        // (the query that does not say: room for any)
+        size_t most = 0;
+        for (int t = 0; t < kTablesAny; ++t) most = std::max(most, forward_workspace(p, base4, t));
+        return most;
+    }
     if (fast4_ok(p, base4, false)) {
         const int64_t n4 = (int64_t)1 << p->log_n;
         return p->nblocks > 1 ? align256((size_t)p->batch * p->nstacks * n4 * elem_bytes(p->dtype)) : 0;
@@ -1040,7 +1064,7 @@ size_t forward_workspace(const bf_problem *p, bool base4)
     const Plan4Long lp = plan4_long(p, base4);
     if (lp.ok)
         return lp.npass > 1 ? align256(((size_t)p->batch * p->nstacks << p->log_n) * elem_bytes(p->dtype)) : 0;
-    const PassPlan mp = build_passes(p, base4, true);
+    const PassPlan mp = build_passes(p, base4, true, tables);
     if (!mp.ok || mp.npass <= 1 || !passes_addressable(p, mp, false)) return 0;
     const int64_t n = (int64_t)1 << p->log_n;
     return align256((size_t)p->batch * p->nstacks * n * elem_bytes(p->dtype));
@@ -1107,7 +1131,7 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
         if (rc != BF_ERR_UNSUPPORTED) return rc;
     }
     if (fast4_ok(p, base4, false)) {
-        const size_t need = forward_workspace(p, base4);
+        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index));
         if (need > 0 && (!workspace || workspace_bytes < need))
             return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         rc = fast4_forward(p, tw4, tw2, input, output, workspace, in_view, out_view, 0, (int)p->nblocks, stream);
@@ -1117,7 +1141,7 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
     }
     const Plan4Long lp = plan4_long(p, base4);
     if (lp.ok) {
-        const size_t need = forward_workspace(p, base4);
+        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index));
         if (need > 0 && (!workspace || workspace_bytes < need))
             return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         rc = long4_forward(p, sc, lp, tw2, tw4, input, output, workspace, in_view, out_view, 0, lp.npass, stream);
@@ -1125,9 +1149,10 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
         return p->dtype == BF_C64 ? launch_bias_add<float2>(p, bias, output, out_view, stream)
                                   : launch_bias_add<float>(p, bias, output, out_view, stream);
     }
-    const PassPlan mp = build_passes(p, base4, true, in_perm || out_index);
+    const int tables = tables_of(in_perm, out_index);
+    const PassPlan mp = build_passes(p, base4, true, tables);
     if (mp.ok && passes_addressable(p, mp, false)) {
-        const size_t need = forward_workspace(p, base4);
+        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index));
         if (need > 0 && (!workspace || workspace_bytes < need))
             return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
@@ -1228,7 +1253,7 @@ struct BwPlan {
 
 // saved_boundaries: the activations entering every pass after the first come from the caller
 // (left behind by the forward call that saves them) instead of being recomputed into the workspace.
-BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, bool permuted = false)
+BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, int tables = 0)
 {
     BwPlan pl = {};
     const int64_t n = (int64_t)1 << p->log_n;
@@ -1282,7 +1307,7 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, b
         pl.total = off + all;
         return pl;
     }
-    const PassPlan mp = build_passes(p, base4, false, permuted);
+    const PassPlan mp = build_passes(p, base4, false, tables);
     if (mp.ok && passes_addressable(p, mp, true)) {
         // boundaries: the activation entering every pass after the first; one gradient plane
         // that the passes update in place; partial slices sized for the widest pass.
@@ -1412,14 +1437,14 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const Schedule sc = make_schedule(p, base4);
     const int64_t n = (int64_t)1 << p->log_n;
-    const bool permuted = in_perm || out_index;
+    const int tables = tables_of(in_perm, out_index);
     const View g_view = make_view(p->output_stride, std::min(p->output_size, n), out_index, tail);
     if (p->batch == 0 || p->nstacks == 0) {
         // no rows: d_input is empty and every entry of the other gradients is an empty sum, whatever the row length
         const ReduceSegment none = {0, sc.per * sc.nblocks, 0, 0};
         return launch_reduce(p, sc, &none, 1, nullptr, 4 * n, d_tw2, d_tw4, stream, bg, &g_view);
     }
-    const BwPlan pl = plan_bw(p, base4, saved != nullptr, permuted);
+    const BwPlan pl = plan_bw(p, base4, saved != nullptr, tables);
     if (!pl.fits)
         return fail(BF_ERR_UNSUPPORTED, "n = %lld does not fit in LDS for the backward pass", (long long)n);
     if (saved && !(pl.fast || pl.fast4 || pl.long4)) return fail(BF_ERR_INVALID, "this problem has no saved activations");
@@ -1593,7 +1618,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     }
 
     if (pl.fast) {
-        const PassPlan mp = build_passes(p, base4, false, permuted);
+        const PassPlan mp = build_passes(p, base4, false, tables);
         const int P = mp.npass;
         char *bounds = saved ? const_cast<char *>(static_cast<const char *>(saved)) : ws + pl.off_boundaries;
         auto boundary = [&](int k) { return bounds + (size_t)(k - 1) * pl.boundary_bytes; };
@@ -1644,6 +1669,9 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                     a.low_bits = q.lb;
                     rc = launch_span(p->dtype == BF_C64, q, true, g.groups_per_wg >= 16, nullptr, &a, grid, stream);
                     if (rc) return rc;
+                } else if (q.edge) {
+                    a.low_bits = (int)p->log_n;
+                    launch_edge(q.inc, nullptr, &a, grid, stream);
                 } else {
                     BF_FAST_DISPATCH(launch_fast_bw_t, q, p->dtype == BF_C64, g.groups_per_wg >= 16, a, grid, stream);
                 }
@@ -1742,7 +1770,9 @@ int scratch_of_current_device(void **ptr)
 // Workspace of a base-2 backward call whatever its column tables: the plan may differ with them.
 size_t bw_workspace_total(const bf_problem *p, bool saved_boundaries)
 {
-    return std::max(plan_bw(p, false, saved_boundaries, false).total, plan_bw(p, false, saved_boundaries, true).total);
+    size_t most = 0;
+    for (int t = 0; t < kTablesAny; ++t) most = std::max(most, plan_bw(p, false, saved_boundaries, t).total);
+    return most;
 }
 
 }  // namespace
@@ -1779,7 +1809,7 @@ const char *bf_last_error(void) { return g_last_error.c_str(); }
 size_t bf_butterfly_multiply_fw_workspace_bytes(const bf_problem *p)
 {
     if (check_problem(p, false)) return BF_SIZE_INVALID;
-    return forward_workspace(p, false);
+    return forward_workspace(p, false, kTablesAny);
 }
 
 int bf_butterfly_multiply_fw(const bf_problem *p, const void *twiddle, const void *input,
@@ -1805,7 +1835,7 @@ int bf_butterfly_multiply_bw(const bf_problem *p, const void *twiddle, const voi
 size_t bf_butterfly_multiply_base4_fw_workspace_bytes(const bf_problem *p)
 {
     if (check_problem(p, false)) return BF_SIZE_INVALID;
-    return forward_workspace(p, true);
+    return forward_workspace(p, true, 0);
 }
 
 int bf_butterfly_multiply_bias_fw(const bf_problem *p, const void *twiddle, const void *input, const void *bias,
@@ -1872,7 +1902,7 @@ static int bias_backward(const bf_problem *p, const void *twiddle, const void *i
 {
     int rc = check_problem(p, true);
     if (rc) return rc;
-    const size_t main_bytes = align256(plan_bw(p, false, saved != nullptr, in_perm || out_index).total);
+    const size_t main_bytes = align256(plan_bw(p, false, saved != nullptr, tables_of(in_perm, out_index)).total);
     const size_t need = main_bytes + bias_area_bytes(p);
     if (!workspace || workspace_bytes < need)
         return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
@@ -1914,9 +1944,9 @@ int bf_butterfly_multiply_perm_bw(const bf_problem *p, const void *twiddle, cons
 // Bytes of activations the saving forward leaves for the backward: one dense (B, S, n) plane per
 // pass of the backward plan after the first; 0 when the backward is a single pass (or runs on
 // kernels that do not use such planes).
-static size_t saved_bytes_of_plan(const bf_problem *p, bool permuted)
+static size_t saved_bytes_of_plan(const bf_problem *p, int tables)
 {
-    const BwPlan pl = plan_bw(p, false, true, permuted);
+    const BwPlan pl = plan_bw(p, false, true, tables);
     if (!pl.fits || !pl.fast || pl.nchunks <= 1) return 0;
     return (size_t)(pl.nchunks - 1) * pl.boundary_bytes;
 }
@@ -1924,7 +1954,9 @@ static size_t saved_bytes_of_plan(const bf_problem *p, bool permuted)
 // room for the saved activations of a call with or without column tables (the plans may differ)
 static size_t saved_bytes(const bf_problem *p)
 {
-    return std::max(saved_bytes_of_plan(p, false), saved_bytes_of_plan(p, true));
+    size_t most = 0;
+    for (int t = 0; t < kTablesAny; ++t) most = std::max(most, saved_bytes_of_plan(p, t));
+    return most;
 }
 
 size_t bf_butterfly_multiply_saved_bytes(const bf_problem *p)
@@ -1941,7 +1973,7 @@ static int fw_saving(const bf_problem *p, const void *twiddle, const void *input
     if (rc) return rc;
     if ((rc = check_perms(p, false, in_perm, out_index))) return rc;
     if ((rc = ensure_attributes())) return rc;
-    const size_t need = saved_bytes_of_plan(p, in_perm || out_index);
+    const size_t need = saved_bytes_of_plan(p, tables_of(in_perm, out_index));
     if (need == 0) return fail(BF_ERR_INVALID, "this problem has no activations to save: use bf_butterfly_multiply_fw");
     if (!saved || saved_capacity < need)
         return fail(BF_ERR_WORKSPACE, "room for %zu bytes of saved activations needed, %zu given", need, saved_capacity);
@@ -1950,9 +1982,9 @@ static int fw_saving(const bf_problem *p, const void *twiddle, const void *input
         return fail(BF_ERR_INVALID, "twiddle and the saved area must be 16-byte aligned");
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const int64_t n = (int64_t)1 << p->log_n;
-    const bool permuted = in_perm || out_index;
-    const PassPlan mp = build_passes(p, false, false, permuted);
-    const BwPlan pl = plan_bw(p, false, true, permuted);
+    const int tables = tables_of(in_perm, out_index);
+    const PassPlan mp = build_passes(p, false, false, tables);
+    const BwPlan pl = plan_bw(p, false, true, tables);
     if (mp.npass < 2 || !pl.fast) return fail(BF_ERR_INVALID, "this problem has no activations to save");
     const View in_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
     const View out_view = make_view(p->output_stride, p->output_size, out_index, tail);
@@ -2005,7 +2037,7 @@ int bf_butterfly_multiply_bw_saved(const bf_problem *p, const void *twiddle, con
     // The planes this call reads follow from its own plan (strides of grad and d_input, column
     // tables): the caller's area must hold them.  A plan of a single pass reads none and runs as
     // the plain call does (its workspace is the same either way).
-    const size_t planes = saved_bytes_of_plan(p, in_perm || out_index);
+    const size_t planes = saved_bytes_of_plan(p, tables_of(in_perm, out_index));
     if (planes == 0) saved = nullptr;
     else if (saved_bytes_given < planes)
         return fail(BF_ERR_WORKSPACE, "the backward reads %zu bytes of saved activations, %zu given", planes,
@@ -2186,7 +2218,7 @@ static int64_t layer_tail(const bf_layer *l) { return l->total_output - (l->prob
 
 static size_t layer_kept_bytes(const bf_layer *l)
 {
-    return l->base4 ? saved4_bytes(&l->problem) : saved_bytes_of_plan(&l->problem, l->in_perm || l->out_index);
+    return l->base4 ? saved4_bytes(&l->problem) : saved_bytes_of_plan(&l->problem, tables_of(l->in_perm, l->out_index));
 }
 
 // Backward workspace of a layer: the multiply's own, the partial column sums of the bias gradient,
@@ -2205,7 +2237,7 @@ static LayerBwPlan plan_layer_bw(const bf_layer *l, int with_bias, size_t kept_b
     // they are recomputed.
     const size_t reads = kept_bytes > 0 ? layer_kept_bytes(l) : 0;
     b.kept = reads > 0 && reads <= kept_bytes;
-    b.off_bias = align256(plan_bw(p, l->base4 != 0, b.kept, l->in_perm || l->out_index).total);
+    b.off_bias = align256(plan_bw(p, l->base4 != 0, b.kept, tables_of(l->in_perm, l->out_index)).total);
     b.off_stacks = b.off_bias + (with_bias ? align256(bias_area_bytes(p)) : 0);
     b.total = b.off_stacks;
     if (l->shared_input && p->nstacks > 1)
@@ -2220,7 +2252,7 @@ size_t bf_layer_kept_bytes(const bf_layer *l)
 
 size_t bf_layer_fw_workspace_bytes(const bf_layer *l)
 {
-    return check_layer(l, false) ? BF_SIZE_INVALID : forward_workspace(&l->problem, l->base4 != 0);
+    return check_layer(l, false) ? BF_SIZE_INVALID : forward_workspace(&l->problem, l->base4 != 0, tables_of(l->in_perm, l->out_index));
 }
 
 int bf_layer_fw(const bf_layer *l, const void *input, void *output, void *kept, size_t kept_bytes, void *workspace,

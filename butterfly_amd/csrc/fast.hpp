@@ -82,8 +82,11 @@ struct PlanOps {
     static constexpr int fw_transposes_total(int start = 0)
     {
         int c = fw_transposes_before(D::NS, start);
-        return c + (layout(D::NS - 1) != 0 ? 1 : 0);
+        return c + (layout(D::NS - 1) != D::OUT_LAYOUT ? 1 : 0);
     }
+    // Layout in which rows are read (and their gradients written) / written (and read) where they
+    // travel through registers, and in which the d_twiddle sums leave.
+    static constexpr int IN_LAYOUT = 0, OUT_LAYOUT = 0, SUM_LAYOUT = 0;
 };
 
 // NB whole blocks of a row (or 1024-element chunk of a row) of 2^L elements.
@@ -140,6 +143,45 @@ struct SpanPlan : PlanOps<SpanPlan<H, MODE>> {
     {
         const int col = column(tile, e, lb);
         const int pb = lb + s_bit - (10 - H);
+        return ((col >> (pb + 1)) << pb) | (col & ((1 << pb) - 1));
+    }
+};
+
+// The stages on bits 0..5 of a row of 2048 or 4096 complex64 elements whose far side is reached
+// through a column table: INC, the first pass, rows in through in_perm; otherwise the last pass, rows out
+// through out_index.  Chunks of 64 (or 1024) adjacent columns would touch one element of every
+// 128-byte line when the table is the bit reversal of an FFT, so the tile takes all 64 settings of
+// the bits 0..5 and all 16 of the top four bits, highest first: behind a bit reversal those are runs
+// of 16 adjacent elements.  Layout A puts the top bits on the lanes and serves the table's side,
+// layout B the bits 0..5 (64 adjacent elements a wavefront) and serves the stages and the other side.
+// For other tables this tile is as good as any.  (lb: log2 of the row length.)
+// special.fft(4096) at 8192 rows: the pass took 206 us forward and 446 backward on chunks of 1024.
+template <bool INC>
+struct EdgePlan : PlanOps<EdgePlan<INC>> {
+    static constexpr int LOG = 10;
+    static constexpr int NS = 6;
+    static constexpr int NSWAP = 4;
+    static constexpr int SLOTS = 1;
+    static constexpr int IN_LAYOUT = INC ? 0 : 1, OUT_LAYOUT = INC ? 1 : 0, SUM_LAYOUT = 1;
+    // column bits 0..3 are the tile's bits 6..9, bits 4 and 5 its bits 4 and 5
+    static constexpr int bit(int s)
+    {
+        const int c = INC ? s : 5 - s;
+        return c < 4 ? 6 + c : c;
+    }
+    static constexpr int layout(int) { return 1; }
+    static constexpr int layout_before(int s, int start = 0) { return s == 0 ? start : 1; }
+    static constexpr int fw_transposes_before(int s, int start = 0) { return s > 0 && start == 0 ? 1 : 0; }
+    static constexpr int fw_transposes_total(int start = 0) { return (start == 0 ? 1 : 0) + (OUT_LAYOUT == 0 ? 1 : 0); }
+    __device__ static __forceinline__ int column(int tile, int e, int lb)
+    {
+        const int top = ((e & 1) << 3) | ((e & 2) << 1) | ((e & 4) >> 1) | ((e & 8) >> 3);
+        return ((e >> 6) & 15) | (e & 48) | (tile << 6) | (top << (lb - 4));
+    }
+    __device__ static __forceinline__ int64_t pair_base(int) { return 0; }
+    __device__ static __forceinline__ int pair_index(int tile, int e, int s_bit, int lb)
+    {
+        const int col = column(tile, e, lb), pb = s_bit >= 6 ? s_bit - 6 : s_bit;
         return ((col >> (pb + 1)) << pb) | (col & ((1 << pb) - 1));
     }
 };
@@ -699,7 +741,7 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
     // float rows are fetched straight into LDS, up to two iterations (2 R row groups) ahead, and
     // the walk starts in the layout of its first stage; complex64 rows arrive in registers, layout A
     constexpr bool DIRECT = sizeof(T) == 4;
-    constexpr int SF = DIRECT ? P::layout(0) : 0;
+    constexpr int SF = DIRECT ? P::layout(0) : P::IN_LAYOUT;
     constexpr int TT = P::fw_transposes_total(SF);  // barriers per iteration
     __shared__ __align__(16) T lds[TT > 0 ? 2 * R * kFastRowWords : 1];
     // Row slots in LDS: four sets of R, an iteration's requests starting at its top, two
@@ -715,7 +757,9 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
     const int stack = blockIdx.y;
     const int chunk = blockIdx.z;
     const FastCoords c = fast_coords<L>(t);
-    const int col = P::column(chunk, c.eA, a.low_bits);  // column of this thread's element in the full row
+    // columns of the thread's element in the full row, as it is read and as it is written
+    const int col_in = P::column(chunk, P::IN_LAYOUT ? c.eB : c.eA, a.low_bits);
+    const int col = P::IN_LAYOUT == P::OUT_LAYOUT ? col_in : P::column(chunk, P::OUT_LAYOUT ? c.eB : c.eA, a.low_bits);
 
     const int64_t g0 = (int64_t)blockIdx.x * a.groups_per_wg;
     const int64_t g1 = g0 + a.groups_per_wg < a.ngroups ? g0 + a.groups_per_wg : a.ngroups;
@@ -764,7 +808,7 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
         make_rsrc(reinterpret_cast<T *>(a.out) + g0 * SLOTS * a.out_view.sb + stack * a.out_view.ss);
     // thread-constant part of the offsets; the row group adds a wave-uniform part
     const View out_view = stack_view(a.out_view, stack, gridDim.y);
-    const int64_t in_col = view_col(a.in_view, col), out_col = view_col(out_view, col);
+    const int64_t in_col = view_col(a.in_view, col_in), out_col = view_col(out_view, col);
     const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.in_view.se * EB) : kOob;
     const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.out_view.se * EB) : kOob;
     const T bias = (a.bias && col < out_view.width)
@@ -853,10 +897,10 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
 #pragma unroll
             for (int r = 0; r < R; ++r) v[r] = fw_product<K>(v[r], ta[s], tb[s], c.bperm_addr);
         });
-        if constexpr (P::layout(NS - 1) != 0) {
+        if constexpr (P::layout(NS - 1) != P::OUT_LAYOUT) {
             constexpr int nth = P::fw_transposes_before(NS, SF);
             T *buf = lds + ((nth + flip) & 1) * R * kFastRowWords;
-            transpose_rows<T, R, DIRECT, YOUNGER>(buf, c.fB, c.fA, v);
+            transpose_rows<T, R, DIRECT, YOUNGER>(buf, P::OUT_LAYOUT ? c.fA : c.fB, P::OUT_LAYOUT ? c.fB : c.fA, v);
             if constexpr (DIRECT)
                 fetch_phase(grel + 2 * R, ((grel / R) + 2) & (SETS - 1), std::integral_constant<int, nth + 1>{}, full);
         }
@@ -911,8 +955,8 @@ struct FastBwArgs {
 template <typename P, bool DIRECT>
 struct BwPipe {
     static constexpr int NS = P::NS;
-    static constexpr int SF = DIRECT ? P::layout(0) : 0;       // layout the forward walk starts in
-    static constexpr int SB = DIRECT ? P::layout(NS - 1) : 0;  // layout the reverse walk starts in
+    static constexpr int SF = DIRECT ? P::layout(0) : P::IN_LAYOUT;        // layout the forward walk starts in
+    static constexpr int SB = DIRECT ? P::layout(NS - 1) : P::OUT_LAYOUT;  // layout the reverse walk starts in
     // phase in which forward stage s / reverse stage s runs = layout changes up to and
     // including the one in front of it
     static constexpr int fphase(int s)
@@ -930,14 +974,15 @@ struct BwPipe {
         return c;
     }
     static constexpr int nF = fphase(NS - 1);
-    static constexpr int nB = bphase(0) + (P::layout(0) != 0 ? 1 : 0);  // + closing transpose back to A
+    static constexpr int nB = bphase(0) + (P::layout(0) != P::IN_LAYOUT ? 1 : 0);  // + closing transpose of the gradient
     // layout of each walk during phase k
     static constexpr int flay(int k) { return SF ^ (k & 1); }
     static constexpr int blay(int k) { return SB ^ (k & 1); }
     // When the reverse walk ends in layout B and the forward walk has no transpose left to
     // share a barrier with, the closing transpose of the reverse walk is carried into the
     // next iteration and rides on that iteration's first barrier.
-    static constexpr bool DEFER = P::layout(0) != 0 && nF < nB && nB >= 2;
+    static constexpr bool DEFER = P::layout(0) != P::IN_LAYOUT && nF < nB && nB >= 2;
+    static_assert(!DEFER || P::IN_LAYOUT == 0, "a carried transpose goes from layout B to layout A");
     static constexpr int K = DEFER ? nB - 1 : (nF > nB ? nF : nB);  // phases 0..K; phase k >= 1 opens with transposes #k
     static constexpr int f_count(int k)
     {
@@ -1107,7 +1152,9 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
     const int stack = blockIdx.y;
     const int chunk = blockIdx.z;
     const FastCoords c = fast_coords<L>(t);
-    const int col = P::column(chunk, c.eA, a.low_bits);  // column of this thread's element in the full row
+    // columns of the thread's element in the full row, as x is read and as the output gradient is
+    const int col = P::column(chunk, P::IN_LAYOUT ? c.eB : c.eA, a.low_bits);
+    const int col_out = P::IN_LAYOUT == P::OUT_LAYOUT ? col : P::column(chunk, P::OUT_LAYOUT ? c.eB : c.eA, a.low_bits);
 
     T ta[NS], tb[NS], tc[NS], acc_self[NS], acc_cross[NS];
     auto load_all_factors = [&] {
@@ -1158,7 +1205,7 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
     // --- operand fetch, register flavour: thread t holds its layout-A element
     const __amdgpu_buffer_rsrc_t x_rs = make_rsrc(x_base), g_rs = make_rsrc(g_base);
     const View g_view = stack_view(a.g_view, stack, gridDim.y);
-    const int64_t x_col = view_col(a.x_view, col), g_col = view_col(g_view, col);
+    const int64_t x_col = view_col(a.x_view, col), g_col = view_col(g_view, col_out);
     const int x_thr = x_col >= 0 ? c.slot * x_row + (int)(x_col * a.x_view.se * EB) : kOob;
     const int g_thr = g_col >= 0 ? c.slot * g_row + (int)(g_col * a.g_view.se * EB) : kOob;
     auto load_x = [&](int grp, bool full = false) {
@@ -1565,9 +1612,10 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
         constexpr Late late = [] {
             Late l{};
             for (int s = 0; s < NS; ++s)
-                if (P::layout(s) != 0) l.s[l.n++] = s;
+                if (P::layout(s) != P::SUM_LAYOUT) l.s[l.n++] = s;
             return l;
         }();
+        static_assert(late.n == 0 || P::SUM_LAYOUT == 0, "sums move from layout B to layout A");
         if constexpr (late.n > 0) {
             T *stage = TB_LDS ? lds_tb : lds;
             constexpr int room = (TB_LDS ? NS * kFastThreads : 4 * R * kFastRowWords) / (2 * kFastRowWords);
@@ -1591,7 +1639,7 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
         static_for<0, NS>([&](auto S) {
             constexpr int s = S;
             constexpr int bit = P::bit(s);
-            const int e = c2.eA;
+            const int e = P::SUM_LAYOUT ? c2.eB : c2.eA;
             const int r = (e >> bit) & 1;
             const int i = P::pair_index(chunk, e, bit, a.low_bits);
             T *d = part + (int64_t)s * a.partial_slot + i * 4;

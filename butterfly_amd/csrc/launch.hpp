@@ -36,6 +36,9 @@ template <int H, int MODE>
 bool launch_span_t(bool cplx, bool backward, bool two_rows, const FastFwArgs *fw, const FastBwArgs *bw, dim3 grid,
                    hipStream_t stream);
 
+// EdgePlan passes (complex64)
+void launch_edge(bool inc, const FastFwArgs *fw, const FastBwArgs *bw, dim3 grid, hipStream_t stream);
+
 template <int L, bool INC>
 void launch_fast4_t(bool backward, const Fast4Args &a, dim3 grid, hipStream_t stream);
 

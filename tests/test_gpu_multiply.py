@@ -803,6 +803,19 @@ def test_permutations_folded_into_first_read_and_last_write(case):
     assert torch.equal(plain, same)
 
 
+@pytest.mark.parametrize("case", [
+    # complex64 rows of 2048 and 4096: a table on the ascending first pass, on the descending last
+    # one, on both (two and four passes), on neither of them (three blocks), padded, trimmed, stacks
+    (np.complex64, 5, 1, 11, 1, None, None, True, "i", True), (np.complex64, 300, 2, 11, 1, 2000, None, True, "i", False),
+    (np.complex64, 67, 1, 12, 1, 4095, 4001, True, "i", True), (np.complex64, 1, 1, 12, 1, None, None, False, "o", False),
+    (np.complex64, 70, 1, 12, 1, None, 4095, False, "o", True), (np.complex64, 33, 1, 11, 1, 1030, 2000, False, "o", False),
+    (np.complex64, 21, 1, 12, 2, None, None, True, "io", False), (np.complex64, 21, 1, 11, 2, 2000, 2001, True, "io", True),
+    (np.complex64, 9, 2, 12, 2, None, None, True, "i", False), (np.complex64, 9, 1, 12, 3, None, None, True, "i", False)],
+    ids=lambda c: f"B{c[1]}-S{c[2]}-L{c[3]}-nb{c[4]}-I{c[5]}-O{c[6]}-inc{int(c[7])}-{c[8]}-bias{int(c[9])}")
+def test_permutations_on_the_tiles_made_for_them(case):
+    test_permutations_folded_into_first_read_and_last_write(case)
+
+
 def test_perm_operator_autograd_and_checks():
     """The autograd operator equals gather -> multiply -> + bias -> gather under autograd."""
     import butterfly_amd  # noqa: F401
