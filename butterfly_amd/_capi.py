@@ -30,7 +30,7 @@ SYMBOLS = [
     "bf_butterfly_multiply_bw_saved_workspace_bytes", "bf_butterfly_multiply_bw_saved",
     "bf_butterfly_multiply_base4_saved_bytes", "bf_butterfly_multiply_base4_fw_saving",
     "bf_butterfly_multiply_base4_bw_saved_workspace_bytes", "bf_butterfly_multiply_base4_bw_saved",
-    "bf_layer_kept_bytes", "bf_layer_fw_workspace_bytes", "bf_layer_fw", "bf_layer_bw_workspace_bytes", "bf_layer_bw",
+    "bf_layer_takes_real", "bf_layer_kept_bytes", "bf_layer_fw_workspace_bytes", "bf_layer_fw", "bf_layer_bw_workspace_bytes", "bf_layer_bw",
 ]
 
 NOALLOC_SCRATCH_BYTES = 48 << 20

@@ -10,7 +10,7 @@ import numbers
 import torch
 from torch import nn
 
-from .complex_utils import complex_reshape, real_dtype_to_complex
+from .complex_utils import complex_reshape, real2complex, real_dtype_to_complex
 from .multiply import butterfly_layer, butterfly_multiply, butterfly_multiply_bias, butterfly_multiply_perm
 
 _INITS = ("empty", "randn", "ortho", "identity", "fft_no_br", "ifft_no_br")
@@ -154,7 +154,7 @@ class Butterfly(nn.Module):
                     tw[:, 1:] = torch.eye(2, dtype=tw.dtype)
 
     def forward(self, input, transpose=False, conjugate=False, subtwiddle=False, in_perm=None, out_index=None,
-                in_scale=None, out_scale=None):
+                in_scale=None, out_scale=None, real_input=False, real_output=False):
         """input (batch, *, in_size) -> (batch, *, out_size).
 
         transpose / conjugate apply the transposed / conjugated matrix; subtwiddle uses only
@@ -168,7 +168,10 @@ class Butterfly(nn.Module):
         in_scale / out_scale (vectors of in_size / out_size entries): a diagonal matrix directly
         in front of / behind the layer (between the layer and the permutation of in_perm /
         out_index, if there is one).  They are multiplied into the first / last factor, an
-        n-sized operation that autograd differentiates, instead of into the activations."""
+        n-sized operation that autograd differentiates, instead of into the activations.
+
+        real_input / real_output (complex layers): the layer takes real numbers / returns the real
+        part of its output, as between Real2Complex and Complex2Real modules."""
         if in_scale is not None or out_scale is not None:
             if subtwiddle or transpose:
                 raise ValueError("in_scale / out_scale cannot be combined with subtwiddle or transpose")
@@ -193,8 +196,18 @@ class Butterfly(nn.Module):
             output_size = None
         if conjugate and self.complex:
             twiddle = twiddle.conj()
+        # (out_size of a finished layer may have been lowered: not below its last stack here)
+        native = self._shares_input and input.is_cuda and not subtwiddle and self.out_size > (self.nstacks - 1) * self.n
         if in_scale is not None or out_scale is not None:
-            twiddle = scale_twiddle(twiddle, self.increasing_stride, in_scale, out_scale)
+            if native and twiddle.dtype in (torch.float32, torch.complex64):
+                for v in (in_scale, out_scale):
+                    if v is not None and v.is_complex() and not twiddle.is_complex():
+                        raise ValueError("a complex diagonal cannot be folded into real factors")
+                in_scale, out_scale = (v if v is None or v.dtype == twiddle.dtype else v.to(twiddle.dtype)
+                                       for v in (in_scale, out_scale))
+            else:
+                twiddle = scale_twiddle(twiddle, self.increasing_stride, in_scale, out_scale)
+                in_scale = out_scale = None
         if transpose:
             # (prod of stages)^T: transpose every 2x2 and reverse the stage and block order
             twiddle = twiddle.transpose(-1, -2).flip([1, 2])
@@ -202,9 +215,11 @@ class Butterfly(nn.Module):
             inc = not last_inc
         else:
             inc = self.increasing_stride
-        # (out_size of a finished layer may have been lowered: not below its last stack here)
-        if self._shares_input and input.is_cuda and not subtwiddle and self.out_size > (self.nstacks - 1) * self.n:
-            return butterfly_layer(twiddle, input, self.layer_bias(), inc, self.out_size, in_perm, out_index)
+        if native:
+            return butterfly_layer(twiddle, input, self.layer_bias(), inc, self.out_size, in_perm, out_index, in_scale,
+                                   out_scale, real_input, real_output)
+        if real_input:
+            input = real2complex(input)
         x = self.pre_process(input)
         if in_perm is not None or out_index is not None:
             cols = output_size if output_size is not None else 1 << twiddle.shape[2]
@@ -216,7 +231,8 @@ class Butterfly(nn.Module):
             # the kernel that writes the output adds the bias, laid out as (stacks, columns)
             cols = output_size if output_size is not None else 1 << twiddle.shape[2]
             x = butterfly_multiply_bias(twiddle, x, self.bias_rows(cols, subtwiddle), inc, output_size)
-        return self.post_process(input, x, out_size=x.size(-1) if subtwiddle else None, add_bias=False)
+        x = self.post_process(input, x, out_size=x.size(-1) if subtwiddle else None, add_bias=False)
+        return x.real if real_output else x
 
     def effective_twiddle(self):
         """(stacks, nblocks, log_n, n/2, 2, 2) factors the multiply runs with."""

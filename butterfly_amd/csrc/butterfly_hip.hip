@@ -269,6 +269,10 @@ int64_t wide_min_rows(const bf_problem *p)
 // Column tables of a call.
 enum { kTableIn = 1, kTableOut = 2, kTablesAny = 4 };
 
+// Sides of a complex64 call whose rows are real numbers (the input gradient like the input, the
+// output's gradient like the output).  With `tables` in the planning functions.
+enum { kRealIn = 8, kRealOut = 16 };
+
 int tables_of(const int *in_perm, const int *out_index) { return (in_perm ? kTableIn : 0) | (out_index ? kTableOut : 0); }
 
 // tables: the call reads or writes its rows through column tables (see EDGE and the low width below)
@@ -285,7 +289,7 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
     // complex64 rows of 2048 and 4096 with tables: each where a pass over bits 0..5 reads (ascending)
     // or writes (descending) the rows, so that it can run on the tiles made for that
     const bool last_inc = (p->increasing_stride != 0) != (((p->nblocks - 1) & 1) != 0);
-    const bool edges = tables && p->dtype == BF_C64 && (L == 11 || L == 12) &&
+    const bool edges = (tables & (kTableIn | kTableOut)) && p->dtype == BF_C64 && (L == 11 || L == 12) &&
                        (!(tables & kTableIn) || p->increasing_stride != 0) && (!(tables & kTableOut) || !last_inc);
     if (L <= 10) {
         for (int k = 0; k < p->nblocks; k += max_nb) {
@@ -298,7 +302,7 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
             q.L = L;
             q.inc = (p->increasing_stride != 0) != ((k & 1) != 0);
         }
-    } else if (L <= 12 && forward_only && !edges && (p->dtype == BF_F32 || L == 11) &&
+    } else if (L <= 12 && forward_only && !edges && !(tables & (kRealIn | kRealOut)) && (p->dtype == BF_F32 || L == 11) &&
                p->batch * p->nstacks >= wide_min_rows(p)) {
         for (int k = 0; k < p->nblocks; ++k) {
             if (pl.npass == kMaxPasses) return pl;
@@ -326,7 +330,7 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
         // Not through column tables either, where no EDGE pass fits: a gather or scatter touches one
         // element per 128-byte line and short chunk, where chunks of 1024 still find several (measured
         // on the bit reversal of special.fft(4096): 1.30 ms against 0.92 ms per step; with EDGE 0.59).
-        const int low = cplx && L <= 16 && (!tables || edges) ? std::max(6, L - span_max * nspans) : 10;
+        const int low = cplx && L <= 16 && (!(tables & (kTableIn | kTableOut)) || edges) ? std::max(6, L - span_max * nspans) : 10;
         pl.low = low;
         const int hbits = L - low;
         int group_lb[16], group_bits[16], ngroups = 0;
@@ -520,10 +524,10 @@ void fill_stage_table(int *dst, int cap, const Pass &q)
 // Forward through the pass plan.  `scratch` holds one dense (B, S, n) activation when there
 // is more than one pass (passes run in place on it).
 // `bias` (may be NULL) is added by the last pass when that pass runs in a kernel that can do
-// it; *bias_done says whether it was.
+// it; *bias_done says whether it was.  real: kRealIn / kRealOut, for the first / last of these passes.
 int multipass_forward(const bf_problem *p, const PassPlan &pl, const void *tw, const void *input, void *output,
                       void *scratch, const View &in_view, const View &out_view, int first, int last,
-                      hipStream_t stream, const void *bias = nullptr, bool *bias_done = nullptr)
+                      hipStream_t stream, const void *bias = nullptr, bool *bias_done = nullptr, int real = 0)
 {
     if (bias_done) *bias_done = false;
     const int64_t n = (int64_t)1 << p->log_n;
@@ -574,6 +578,8 @@ int multipass_forward(const bf_problem *p, const PassPlan &pl, const void *tw, c
                 a.bias = bias;
                 if (bias_done) *bias_done = true;
             }
+            a.in_real = k == first && (real & kRealIn);
+            a.out_real = k == last - 1 && (real & kRealOut);
             const dim3 grid((unsigned)g.nwg, (unsigned)p->nstacks, (unsigned)pass_lanes(p, q));
             if (q.span) {
                 a.low_bits = q.lb;
@@ -1105,7 +1111,7 @@ int check_perms(const bf_problem *p, bool base4, const int *in_perm, const int *
 
 int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, const void *input,
             void *output, void *workspace, size_t workspace_bytes, void *stream_, const void *bias = nullptr,
-            const int *in_perm = nullptr, const int *out_index = nullptr, int64_t tail = -1)
+            const int *in_perm = nullptr, const int *out_index = nullptr, int64_t tail = -1, int real = 0)
 {
     int rc = check_problem(p, false);
     if (rc) return rc;
@@ -1131,7 +1137,7 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
         if (rc != BF_ERR_UNSUPPORTED) return rc;
     }
     if (fast4_ok(p, base4, false)) {
-        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index));
+        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index) | real);
         if (need > 0 && (!workspace || workspace_bytes < need))
             return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         rc = fast4_forward(p, tw4, tw2, input, output, workspace, in_view, out_view, 0, (int)p->nblocks, stream);
@@ -1141,7 +1147,7 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
     }
     const Plan4Long lp = plan4_long(p, base4);
     if (lp.ok) {
-        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index));
+        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index) | real);
         if (need > 0 && (!workspace || workspace_bytes < need))
             return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         rc = long4_forward(p, sc, lp, tw2, tw4, input, output, workspace, in_view, out_view, 0, lp.npass, stream);
@@ -1149,10 +1155,9 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
         return p->dtype == BF_C64 ? launch_bias_add<float2>(p, bias, output, out_view, stream)
                                   : launch_bias_add<float>(p, bias, output, out_view, stream);
     }
-    const int tables = tables_of(in_perm, out_index);
-    const PassPlan mp = build_passes(p, base4, true, tables);
+    const PassPlan mp = build_passes(p, base4, true, tables_of(in_perm, out_index) | real);
     if (mp.ok && passes_addressable(p, mp, false)) {
-        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index));
+        const size_t need = forward_workspace(p, base4, tables_of(in_perm, out_index) | real);
         if (need > 0 && (!workspace || workspace_bytes < need))
             return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
@@ -1161,11 +1166,12 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
             return fail(BF_ERR_INVALID, "twiddle must be 16-byte aligned");
         bool bias_done = false;
         rc = multipass_forward(p, mp, tw2, input, output, workspace, in_view, out_view, 0, mp.npass, stream, bias,
-                               &bias_done);
+                               &bias_done, real);
         if (rc || !bias || bias_done) return rc;
         return p->dtype == BF_C64 ? launch_bias_add<float2>(p, bias, output, out_view, stream)
                                   : launch_bias_add<float>(p, bias, output, out_view, stream);
     }
+    if (real) return fail(BF_ERR_UNSUPPORTED, "rows of real numbers: not in the LDS fallback kernels");
     rc = launch_generic_fw(p, sc, 0, sc.per * sc.nblocks, tw2, tw4, input, in_view, output, out_view, stream);
     if (rc || !bias) return rc;
     return p->dtype == BF_C64 ? launch_bias_add<float2>(p, bias, output, out_view, stream)
@@ -1428,7 +1434,8 @@ int launch_reduce(const bf_problem *p, const Schedule &sc, const ReduceSegment *
 int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, const void *input,
              const void *grad, void *d_tw2, void *d_tw4, void *d_input, void *workspace,
              size_t workspace_bytes, void *stream_, BiasGrad *bg = nullptr,
-             const int *in_perm = nullptr, const int *out_index = nullptr, const void *saved = nullptr, int64_t tail = -1)
+             const int *in_perm = nullptr, const int *out_index = nullptr, const void *saved = nullptr, int64_t tail = -1,
+             int real = 0)
 {
     int rc = check_problem(p, true);
     if (rc) return rc;
@@ -1461,6 +1468,8 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     const View dense = dense_view(p->nstacks, n);
     char *ws = static_cast<char *>(workspace);
     const size_t e_bytes = elem_bytes(p->dtype);
+    if (real && (!pl.fast || p->input_size > n || (bg && (real & kRealOut))))
+        return fail(BF_ERR_UNSUPPORTED, "rows of real numbers: register-resident kernels and inputs up to n only");
 
     // Partial slices: every pass leaves its own behind the previous one's, for one reduce at the end
     // of the call; where the workspace has no room for that, each pass is reduced before the next.
@@ -1625,7 +1634,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
         // forward replay: boundary k = activation entering pass k (k >= 1)
         for (int k = 0; k + 1 < P && !saved; ++k) {
             rc = multipass_forward(p, mp, tw2, k == 0 ? input : boundary(k), boundary(k + 1), nullptr,
-                                   k == 0 ? x_view : dense, dense, k, k + 1, stream);
+                                   k == 0 ? x_view : dense, dense, k, k + 1, stream, nullptr, nullptr, k == 0 ? real & kRealIn : 0);
             if (rc) return rc;
         }
         const View dn_view = make_view(p->d_input_stride, std::min(p->input_size, n), in_perm);
@@ -1657,6 +1666,8 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 a.ngroups = g.ngroups;
                 a.groups_per_wg = g.groups_per_wg;
                 nparts = g.nwg;
+                a.x_real = k == 0 && (real & kRealIn);
+                a.g_real = k == P - 1 && (real & kRealOut);
                 if (k == P - 1 && bg && q.L == 10 && p->dtype == BF_F32 && g.nwg <= num_cu()) {
                     a.bias_partial = bg->area;
                     a.bias_stride = bias_stride(p);
@@ -1967,7 +1978,7 @@ size_t bf_butterfly_multiply_saved_bytes(const bf_problem *p)
 
 static int fw_saving(const bf_problem *p, const void *twiddle, const void *input, const void *bias, const int32_t *in_perm,
                      const int32_t *out_index, void *output, void *saved, size_t saved_capacity, void *stream_,
-                     int64_t tail = -1)
+                     int64_t tail = -1, int real = 0)
 {
     int rc = check_problem(p, false);
     if (rc) return rc;
@@ -1995,12 +2006,13 @@ static int fw_saving(const bf_problem *p, const void *twiddle, const void *input
     // the passes of the backward plan, each into its own plane: plane k = activation entering pass k
     for (int k = 0; k + 1 < P; ++k) {
         rc = multipass_forward(p, mp, twiddle, k == 0 ? input : boundary(k), boundary(k + 1), nullptr,
-                               k == 0 ? in_view : dense, dense, k, k + 1, stream);
+                               k == 0 ? in_view : dense, dense, k, k + 1, stream, nullptr, nullptr,
+                               k == 0 ? real & kRealIn : 0);
         if (rc) return rc;
     }
     bool bias_done = false;
     rc = multipass_forward(p, mp, twiddle, boundary(P - 1), output, nullptr, dense, out_view, P - 1, P, stream, bias,
-                           &bias_done);
+                           &bias_done, real & kRealOut);
     if (rc || !bias || bias_done) return rc;
     return p->dtype == BF_C64 ? launch_bias_add<float2>(p, bias, output, out_view, stream)
                               : launch_bias_add<float>(p, bias, output, out_view, stream);
@@ -2210,7 +2222,25 @@ static int check_layer(const bf_layer *l, bool backward)
         return fail(BF_ERR_INVALID, "total_output must end in the last stack");
     if (l->base4 && (l->in_perm || l->out_index))
         return fail(BF_ERR_UNSUPPORTED, "base-4 layers take no column tables");
+    if ((l->real_input || l->real_output) && (l->base4 || p->dtype != BF_C64 || (l->real_output && l->bias)))
+        return fail(BF_ERR_UNSUPPORTED, "rows of real numbers: complex64 base-2 layers only, real outputs without bias");
     return BF_OK;
+}
+
+static int layer_flags(const bf_layer *l)
+{
+    return tables_of(l->in_perm, l->out_index) | (l->real_input ? kRealIn : 0) | (l->real_output ? kRealOut : 0);
+}
+static int layer_real(const bf_layer *l) { return layer_flags(l) & (kRealIn | kRealOut); }
+
+int bf_layer_takes_real(const bf_layer *l)
+{
+    if (check_layer(l, true)) return 0;
+    const bf_problem *p = &l->problem;
+    if (p->batch == 0 || p->nstacks == 0) return 1;
+    const PassPlan mp = build_passes(p, false, true, layer_flags(l));
+    return mp.ok && passes_addressable(p, mp, false) && p->input_size <= (int64_t)1 << p->log_n &&
+           plan_bw(p, false, false, layer_flags(l)).fast;
 }
 
 // columns of the last stack
@@ -2252,7 +2282,7 @@ size_t bf_layer_kept_bytes(const bf_layer *l)
 
 size_t bf_layer_fw_workspace_bytes(const bf_layer *l)
 {
-    return check_layer(l, false) ? BF_SIZE_INVALID : forward_workspace(&l->problem, l->base4 != 0, tables_of(l->in_perm, l->out_index));
+    return check_layer(l, false) ? BF_SIZE_INVALID : forward_workspace(&l->problem, l->base4 != 0, layer_flags(l));
 }
 
 int bf_layer_fw(const bf_layer *l, const void *input, void *output, void *kept, size_t kept_bytes, void *workspace,
@@ -2265,11 +2295,11 @@ int bf_layer_fw(const bf_layer *l, const void *input, void *output, void *kept, 
     if (kept)
         return l->base4 ? fw4_saving(p, l->twiddle, l->twiddle2, input, l->bias, output, kept, kept_bytes, stream, tail)
                         : fw_saving(p, l->twiddle, input, l->bias, l->in_perm, l->out_index, output, kept, kept_bytes,
-                                    stream, tail);
+                                    stream, tail, layer_real(l));
     return l->base4 ? forward(p, true, l->twiddle2, l->twiddle, input, output, workspace, workspace_bytes, stream, l->bias,
                               nullptr, nullptr, tail)
                     : forward(p, false, l->twiddle, nullptr, input, output, workspace, workspace_bytes, stream, l->bias,
-                              l->in_perm, l->out_index, tail);
+                              l->in_perm, l->out_index, tail, layer_real(l));
 }
 
 size_t bf_layer_bw_workspace_bytes(const bf_layer *l, int with_bias, size_t kept_bytes)
@@ -2302,12 +2332,12 @@ int bf_layer_bw(const bf_layer *l, const void *input, const void *grad, const vo
     bg.d_bias = d_bias;
     rc = backward(&stacked, l->base4 != 0, l->base4 ? l->twiddle2 : l->twiddle, l->base4 ? l->twiddle : nullptr, input, grad,
                   l->base4 ? d_twiddle2 : d_twiddle, l->base4 ? d_twiddle : nullptr, d_stacks, workspace, b.off_bias, stream_,
-                  d_bias ? &bg : nullptr, l->in_perm, l->out_index, b.kept ? kept : nullptr, layer_tail(l));
+                  d_bias ? &bg : nullptr, l->in_perm, l->out_index, b.kept ? kept : nullptr, layer_tail(l), layer_real(l));
     if (rc || !sum || p->batch == 0 || p->input_size == 0) return rc;
     SumStacksArgs a = {};
     a.in = d_stacks;
     a.out = d_input;
-    const int ef = p->dtype == BF_C64 ? 2 : 1;
+    const int ef = p->dtype == BF_C64 && !l->real_input ? 2 : 1;
     a.width = p->input_size * ef;
     a.nstacks = p->nstacks;
     a.total = p->batch * a.width;

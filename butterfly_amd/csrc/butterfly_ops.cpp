@@ -176,9 +176,16 @@ struct Operands {
     Tensor twiddle, twiddle2;      // base 2: twiddle; base 4: twiddle4 and twiddle2
     Tensor bias;                   // undefined: none
     Tensor in_perm, out_index;     // undefined: none
+    Tensor in_scale, out_scale;    // layers, base 2: diagonals folded into the factors; undefined: none
     bool base4 = false;
     bool increasing_stride = true;
+    bool real_input = false;       // layers, complex64: the input is real / only the output's real part is wanted
+    bool real_output = false;
 };
+
+void scale_factors(const Tensor &twiddle, const Operands &o, Tensor &scaled, const char *who);
+void scale_factors_bw(const Tensor &twiddle, const Operands &o, const Tensor &grad, Tensor &d_twiddle, Tensor &d_in,
+                      Tensor &d_out, const char *who);
 
 // Shapes and strides of a call.  rows: a 3-d view (batch, nstacks, width) of the caller's input.
 // layer: the stacks share one input (nstacks is then the factors') and out_size counts the columns
@@ -225,10 +232,16 @@ void describe(Call &c, const Operands &o, int64_t batch, int64_t nstacks, int64_
     } else {
         const Tensor &twiddle = o.twiddle;
         CHECK_SHAPE(twiddle, nstacks, nblocks, log_n, n / 2, 2, 2);
-        TORCH_CHECK(twiddle.scalar_type() == input.scalar_type(), who, ": twiddle and input must have the same dtype");
+        if (o.real_input) {
+            TORCH_CHECK(twiddle.scalar_type() == at::kComplexFloat && input.scalar_type() == at::kFloat, who,
+                        ": a real input needs complex64 twiddle and float32 input");
+        } else {
+            TORCH_CHECK(twiddle.scalar_type() == input.scalar_type(), who, ": twiddle and input must have the same dtype");
+        }
+        TORCH_CHECK(!o.real_output || twiddle.is_complex(), who, ": a real output needs complex64 twiddle");
     }
     bf_problem &p = c.p();
-    p.dtype = dtype_code(input, who);
+    p.dtype = dtype_code(o.twiddle, who);
     p.increasing_stride = o.increasing_stride;
     p.batch = batch;
     p.nstacks = nstacks;
@@ -242,6 +255,8 @@ void describe(Call &c, const Operands &o, int64_t batch, int64_t nstacks, int64_
     }
     c.desc.base4 = o.base4;
     c.desc.shared_input = shared;
+    c.desc.real_input = o.real_input;
+    c.desc.real_output = o.real_output;
     c.desc.total_output = total;
     c.twiddle = dense(o.twiddle);
     c.desc.twiddle = c.twiddle.data_ptr();
@@ -252,7 +267,7 @@ void describe(Call &c, const Operands &o, int64_t batch, int64_t nstacks, int64_
     if (o.bias.defined()) {
         const Tensor &bias = o.bias;
         CHECK_DEVICE(bias); CHECK_SAME_DEVICE(bias, input);
-        TORCH_CHECK(bias.scalar_type() == input.scalar_type(), who, ": bias and input must have the same dtype");
+        TORCH_CHECK(bias.scalar_type() == o.twiddle.scalar_type(), who, ": bias and input must have the same dtype");
         c.bias = dense(bias);
         c.desc.bias = c.bias.data_ptr();
     }
@@ -301,7 +316,7 @@ void forward_call(Call &c, const Tensor &x, Tensor &output, Tensor *keep, const 
 }
 
 struct Gradients {
-    Tensor twiddle, twiddle2, input, bias;
+    Tensor twiddle, twiddle2, input, bias, in_scale, out_scale;
 };
 
 void backward_call(Call &c, const Tensor &x, const Tensor &g, const Tensor &kept, bool with_bias, Gradients &d,
@@ -310,7 +325,7 @@ void backward_call(Call &c, const Tensor &x, const Tensor &g, const Tensor &kept
     const size_t kept_bytes = kept.defined() ? (size_t)kept.numel() : 0;
     d.twiddle = at::empty_like(c.twiddle);
     if (c.desc.base4) d.twiddle2 = at::empty_like(c.twiddle2);
-    if (with_bias) d.bias = at::empty({c.desc.total_output}, g.options());
+    if (with_bias) d.bias = at::empty({c.desc.total_output}, c.twiddle.options());
     const size_t ws_bytes = valid_size(bf_layer_bw_workspace_bytes(&c.desc, with_bias ? 1 : 0, kept_bytes));
     Tensor ws;
     if (ws_bytes > 0) ws = bytes_like(x, ws_bytes);
@@ -420,41 +435,85 @@ void describe_layer(Call &c, const Operands &o, const Tensor &x, int64_t out_siz
     set_d_input_strides(c, true);
 }
 
-Tensor layer_fw(const Operands &o, const Tensor &input, int64_t out_size, Tensor *keep, const char *who)
+// The rows of real numbers in a form the kernels take: as they are, or (schedules that only the
+// fallback kernels run, a bias in front of a real output) as complex ones.
+bool takes_real(Call &c, const Operands &o)
 {
+    return (!o.real_input && !o.real_output) || bf_layer_takes_real(&c.desc) != 0;
+}
+Tensor as_complex(const Tensor &t) { return t.to(at::kComplexFloat); }
+
+Tensor layer_fw(const Operands &o_, const Tensor &input, int64_t out_size, Tensor *keep, Tensor *scaled, const char *who)
+{
+    Operands o = o_;
     check_factors(o, input, who);
     TORCH_CHECK(input.dim() >= 1, who, ": input must have at least one dimension");
     require_device(input, who);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    const Tensor x = rows_of(input);
-    Call c;
-    describe_layer(c, o, x, out_size, who);
+    if (o.in_scale.defined() || o.out_scale.defined()) {
+        Tensor with;
+        scale_factors(o.twiddle, o, with, who);
+        o.twiddle = with;
+        if (scaled) *scaled = with;
+    }
+    Tensor x = rows_of(input);
     c10::SmallVector<int64_t, 6> shape(input.sizes().begin(), input.sizes().end());
     shape.back() = out_size;
-    Tensor output = at::empty(shape, x.options());
-    bf_problem &p = c.p();
-    p.output_stride[0] = out_size;
-    p.output_stride[1] = p.output_size;
-    p.output_stride[2] = 1;
-    forward_call(c, x, output, keep, who);
-    return output;
+    auto run = [&](Tensor &output) {
+        Call c;
+        describe_layer(c, o, x, out_size, who);
+        bf_problem &p = c.p();
+        p.output_stride[0] = out_size;
+        p.output_stride[1] = p.output_size;
+        p.output_stride[2] = 1;
+        if (!takes_real(c, o)) return false;
+        output = at::empty(shape, o.real_output ? x.options().dtype(at::kFloat) : o.twiddle.options());
+        forward_call(c, x, output, keep, who);
+        return true;
+    };
+    Tensor output;
+    if (run(output)) return output;
+    const bool real_output = o.real_output;
+    if (o.real_input) x = as_complex(x);
+    o.real_input = o.real_output = false;
+    run(output);
+    return real_output ? at::real(output).contiguous() : output;
 }
 
-Gradients layer_bw(const Operands &o, const Tensor &input, const Tensor &grad, const Tensor &kept, bool with_bias,
-                   const char *who)
+Gradients layer_bw(const Operands &o_, const Tensor &input, const Tensor &grad, const Tensor &kept, const Tensor &scaled,
+                   bool with_bias, const char *who)
 {
-    TORCH_CHECK(grad.scalar_type() == input.scalar_type(), who, ": grad and input must have the same dtype");
+    Operands o = o_;
+    TORCH_CHECK(o.real_output ? grad.scalar_type() == at::kFloat : grad.scalar_type() == o.twiddle.scalar_type(), who,
+                ": grad and output must have the same dtype");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    const Tensor x = rows_of(input), g = rows_of(grad);
-    Call c;
-    describe_layer(c, o, x, g.size(1), who);
-    bf_problem &p = c.p();
-    p.output_stride[0] = g.size(0) > 1 ? g.stride(0) : 0;
-    p.output_stride[2] = g.size(1) > 1 ? g.stride(1) : 0;
-    p.output_stride[1] = p.output_size * p.output_stride[2];
+    if (scaled.defined()) o.twiddle = scaled;
+    Tensor x = rows_of(input), g = rows_of(grad);
     Gradients d;
-    d.input = at::empty(input.sizes(), x.options());
-    backward_call(c, x, g, kept, with_bias, d, who);
+    auto run = [&] {
+        Call c;
+        describe_layer(c, o, x, g.size(1), who);
+        bf_problem &p = c.p();
+        p.output_stride[0] = g.size(0) > 1 ? g.stride(0) : 0;
+        p.output_stride[2] = g.size(1) > 1 ? g.stride(1) : 0;
+        p.output_stride[1] = p.output_size * p.output_stride[2];
+        if (!takes_real(c, o) || (with_bias && o.real_output)) return false;
+        d.input = at::empty(input.sizes(), x.options());
+        backward_call(c, x, g, kept, with_bias, d, who);
+        return true;
+    };
+    if (!run()) {
+        const bool real_input = o.real_input;
+        if (o.real_input) x = as_complex(x);
+        if (o.real_output) g = as_complex(g);
+        o.real_input = o.real_output = false;
+        run();
+        if (real_input) d.input = at::real(d.input).contiguous();
+    }
+    if (scaled.defined()) {
+        const Tensor d_scaled = d.twiddle;
+        scale_factors_bw(o_.twiddle, o_, d_scaled, d.twiddle, d.in_scale, d.out_scale, who);
+    }
     return d;
 }
 
@@ -470,12 +529,13 @@ using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
 struct MultiplyNode : public torch::autograd::Node {
-    SavedVariable twiddle, twiddle2, input, kept;
+    SavedVariable twiddle, twiddle2, input, kept, in_scale, out_scale, scaled;
     Tensor in_perm, out_index;
     bool base4 = false, increasing_stride = true, with_bias = false, layer = false, has_kept = false;
+    bool real_input = false, real_output = false, has_scaled = false;
     const char *who = nullptr;
 
-    // edges: twiddle, twiddle2, input, bias (those that the call does not have lead nowhere)
+    // edges: twiddle, twiddle2, input, bias, in_scale, out_scale (those that the call does not have lead nowhere)
     variable_list apply(variable_list &&grads) override
     {
         variable_list out(num_outputs());
@@ -488,14 +548,24 @@ struct MultiplyNode : public torch::autograd::Node {
         o.out_index = out_index;
         o.base4 = base4;
         o.increasing_stride = increasing_stride;
+        o.real_input = real_input;
+        o.real_output = real_output;
         const Tensor x = input.unpack(self), planes = has_kept ? kept.unpack(self) : Tensor();
+        Tensor with;
+        if (has_scaled) {
+            o.in_scale = in_scale.unpack(self);
+            o.out_scale = out_scale.unpack(self);
+            with = scaled.unpack(self);
+        }
         at::AutoDispatchBelowADInplaceOrView below;
-        Gradients d = layer ? layer_bw(o, x, grads[0], planes, with_bias, who)
+        Gradients d = layer ? layer_bw(o, x, grads[0], planes, with, with_bias, who)
                             : multiply_bw(o, x, grads[0], planes, with_bias, who);
         out[0] = std::move(d.twiddle);
         out[1] = std::move(d.twiddle2);
         out[2] = std::move(d.input);
         out[3] = std::move(d.bias);
+        out[4] = std::move(d.in_scale);
+        out[5] = std::move(d.out_scale);
         return out;
     }
 
@@ -505,6 +575,9 @@ struct MultiplyNode : public torch::autograd::Node {
         twiddle2.reset_data();
         input.reset_data();
         kept.reset_data();
+        in_scale.reset_data();
+        out_scale.reset_data();
+        scaled.reset_data();
     }
 
     std::string name() const override { return base4 ? "ButterflyMultiplyBase4Backward" : "ButterflyMultiplyBackward"; }
@@ -519,20 +592,21 @@ Tensor differentiable(const Operands &o, const Tensor &input, bool layer, const 
 {
     bool wanted = false;
     if (at::GradMode::is_enabled()) {
-        for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &input}) wanted = wanted || (t->defined() && t->requires_grad());
+        for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &o.in_scale, &o.out_scale, &input})
+            wanted = wanted || (t->defined() && t->requires_grad());
     }
     if (!wanted) {
         at::AutoDispatchBelowADInplaceOrView below;
-        return forward(nullptr);
+        return forward(nullptr, nullptr);
     }
-    for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &input})
+    for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &o.in_scale, &o.out_scale, &input})
         TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), who, ": no forward-mode derivative");
     std::shared_ptr<MultiplyNode> node(new MultiplyNode(), torch::autograd::deleteNode);
-    node->set_next_edges(torch::autograd::collect_next_edges(o.twiddle, o.twiddle2, input, o.bias));
-    Tensor kept, out;
+    node->set_next_edges(torch::autograd::collect_next_edges(o.twiddle, o.twiddle2, input, o.bias, o.in_scale, o.out_scale));
+    Tensor kept, scaled, out;
     {
         at::AutoDispatchBelowADInplaceOrView below;
-        out = forward(input.is_cuda() ? &kept : nullptr);
+        out = forward(input.is_cuda() ? &kept : nullptr, &scaled);
     }
     node->twiddle = SavedVariable(o.twiddle, false);
     if (o.base4) node->twiddle2 = SavedVariable(o.twiddle2, false);
@@ -541,6 +615,14 @@ Tensor differentiable(const Operands &o, const Tensor &input, bool layer, const 
         node->kept = SavedVariable(kept, false);
         node->has_kept = true;
     }
+    if (scaled.defined()) {
+        node->in_scale = SavedVariable(o.in_scale, false);
+        node->out_scale = SavedVariable(o.out_scale, false);
+        node->scaled = SavedVariable(scaled, false);
+        node->has_scaled = true;
+    }
+    node->real_input = o.real_input;
+    node->real_output = o.real_output;
     node->in_perm = o.in_perm;
     node->out_index = o.out_index;
     node->base4 = o.base4;
@@ -593,7 +675,7 @@ Tensor butterfly_multiply(Tensor twiddle, Tensor input, bool increasing_stride, 
 {
     const char *who = "butterfly_multiply";
     const Operands o = base2(twiddle, increasing_stride);
-    return differentiable(o, input, false, who, [&](Tensor *keep) { return multiply_fw(o, input, output_size, keep, who); });
+    return differentiable(o, input, false, who, [&](Tensor *keep, Tensor *) { return multiply_fw(o, input, output_size, keep, who); });
 }
 
 // New operators (no counterpart in the reference's op set): the layer bias folded into the
@@ -620,7 +702,7 @@ Tensor butterfly_multiply_bias(Tensor twiddle, Tensor input, Tensor bias, bool i
     const char *who = "butterfly_multiply_bias";
     TORCH_CHECK(bias.defined(), "butterfly_multiply_bias: bias is undefined");
     const Operands o = base2(twiddle, increasing_stride, bias);
-    return differentiable(o, input, false, who, [&](Tensor *keep) { return multiply_fw(o, input, output_size, keep, who); });
+    return differentiable(o, input, false, who, [&](Tensor *keep, Tensor *) { return multiply_fw(o, input, output_size, keep, who); });
 }
 
 // New operators: the multiply between two fixed column permutations, folded into the first
@@ -654,7 +736,7 @@ Tensor butterfly_multiply_perm(Tensor twiddle, Tensor input, c10::optional<Tenso
 {
     const char *who = "butterfly_multiply_perm";
     const Operands o = base2(twiddle, increasing_stride, opt(bias), opt(in_perm), opt(out_index));
-    return differentiable(o, input, false, who, [&](Tensor *keep) { return multiply_fw(o, input, output_size, keep, who); });
+    return differentiable(o, input, false, who, [&](Tensor *keep, Tensor *) { return multiply_fw(o, input, output_size, keep, who); });
 }
 
 // A whole layer: input (*, width), zero padded or trimmed to n for each of the stacks (the leading
@@ -662,12 +744,22 @@ Tensor butterfly_multiply_perm(Tensor twiddle, Tensor input, c10::optional<Tenso
 // plus bias (out_size).  in_perm / out_index as above.  What Butterfly.forward does around its
 // multiply (torch_butterfly/butterfly.py:113-169), without the chain of views, slices and pads
 // that autograd would record and replay for it.
+// in_scale (up to n entries) / out_scale (up to nstacks * n): diagonals directly in front of /
+// behind the factors, multiplied into the first / last of them.  real_input / real_output, complex
+// factors: the input is real, only the real part of the output is returned.
 Tensor butterfly_layer(Tensor twiddle, Tensor input, c10::optional<Tensor> bias, c10::optional<Tensor> in_perm,
-                       c10::optional<Tensor> out_index, bool increasing_stride, int64_t out_size)
+                       c10::optional<Tensor> out_index, c10::optional<Tensor> in_scale, c10::optional<Tensor> out_scale,
+                       bool increasing_stride, int64_t out_size, bool real_input, bool real_output)
 {
     const char *who = "butterfly_layer";
-    const Operands o = base2(twiddle, increasing_stride, opt(bias), opt(in_perm), opt(out_index));
-    return differentiable(o, input, true, who, [&](Tensor *keep) { return layer_fw(o, input, out_size, keep, who); });
+    Operands o = base2(twiddle, increasing_stride, opt(bias), opt(in_perm), opt(out_index));
+    o.in_scale = opt(in_scale);
+    o.out_scale = opt(out_scale);
+    o.real_input = real_input;
+    o.real_output = real_output;
+    return differentiable(o, input, true, who, [&](Tensor *keep, Tensor *scaled) {
+        return layer_fw(o, input, out_size, keep, scaled, who);
+    });
 }
 
 Tensor butterfly_layer_base4(Tensor twiddle4, Tensor twiddle2, Tensor input, c10::optional<Tensor> bias,
@@ -675,7 +767,9 @@ Tensor butterfly_layer_base4(Tensor twiddle4, Tensor twiddle2, Tensor input, c10
 {
     const char *who = "butterfly_layer_base4";
     const Operands o = base4(twiddle4, twiddle2, increasing_stride, opt(bias));
-    return differentiable(o, input, true, who, [&](Tensor *keep) { return layer_fw(o, input, out_size, keep, who); });
+    return differentiable(o, input, true, who, [&](Tensor *keep, Tensor *) {
+        return layer_fw(o, input, out_size, keep, nullptr, who);
+    });
 }
 
 Tensor butterfly_multiply_base4_fw(const Tensor twiddle4, const Tensor twiddle2, const Tensor input,
@@ -699,7 +793,7 @@ Tensor butterfly_multiply_base4(Tensor twiddle4, Tensor twiddle2, Tensor input, 
 {
     const char *who = "butterfly_multiply_base4";
     const Operands o = base4(twiddle4, twiddle2, increasing_stride);
-    return differentiable(o, input, false, who, [&](Tensor *keep) { return multiply_fw(o, input, output_size, keep, who); });
+    return differentiable(o, input, false, who, [&](Tensor *keep, Tensor *) { return multiply_fw(o, input, output_size, keep, who); });
 }
 
 // d_bias (nstacks, output_size) = sum of grad (batch, nstacks, output_size) over the batch.
@@ -805,6 +899,24 @@ std::tuple<Tensor, Tensor, Tensor> butterfly_scale_twiddle_bw(const Tensor twidd
 }
 
 using torch::autograd::AutogradContext;
+
+void scale_factors(const Tensor &twiddle, const Operands &o, Tensor &scaled, const char *)
+{
+    scaled = butterfly_scale_twiddle_fw(twiddle, o.in_scale.defined() ? c10::optional<Tensor>(o.in_scale) : c10::nullopt,
+                                        o.out_scale.defined() ? c10::optional<Tensor>(o.out_scale) : c10::nullopt,
+                                        o.increasing_stride);
+}
+
+void scale_factors_bw(const Tensor &twiddle, const Operands &o, const Tensor &grad, Tensor &d_twiddle, Tensor &d_in,
+                      Tensor &d_out, const char *)
+{
+    auto r = butterfly_scale_twiddle_bw(twiddle, o.in_scale.defined() ? c10::optional<Tensor>(o.in_scale) : c10::nullopt,
+                                        o.out_scale.defined() ? c10::optional<Tensor>(o.out_scale) : c10::nullopt, grad,
+                                        o.increasing_stride);
+    d_twiddle = std::get<0>(r);
+    if (o.in_scale.defined()) d_in = std::get<1>(r);
+    if (o.out_scale.defined()) d_out = std::get<2>(r);
+}
 
 class ButterflyScaleTwiddle : public torch::autograd::Function<ButterflyScaleTwiddle> {
 public:

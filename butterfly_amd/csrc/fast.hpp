@@ -450,6 +450,25 @@ __device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, int voff, in
     __builtin_amdgcn_raw_buffer_store_b64(raw, r, voff, soff, 0);
 }
 
+// The same for rows that may hold real numbers only (wave-uniform `real`; complex64).
+template <typename T>
+__device__ __forceinline__ T buf_load_any(__amdgpu_buffer_rsrc_t r, int voff, int soff, bool real)
+{
+    if constexpr (sizeof(T) == 8) {
+        if (real) return make_float2(buf_load<float>(r, voff, soff), 0.0f);
+    }
+    return buf_load<T>(r, voff, soff);
+}
+__device__ __forceinline__ void buf_store_any(__amdgpu_buffer_rsrc_t r, int voff, int soff, float v, bool)
+{
+    buf_store(r, voff, soff, v);
+}
+__device__ __forceinline__ void buf_store_any(__amdgpu_buffer_rsrc_t r, int voff, int soff, float2 v, bool real)
+{
+    if (real) buf_store(r, voff, soff, v.x);
+    else buf_store(r, voff, soff, v);
+}
+
 // ---- rows fetched straight into LDS -----------------------------------------------------------
 // A buffer load with the LDS modifier writes the dword each lane fetches to LDS at
 // M0 + 4 * lane: no register holds the row while it is in flight, and the thread that later
@@ -520,6 +539,7 @@ struct FastFwArgs {
     int64_t groups_per_wg;
     const void *bias;          // NULL, or (S, out_view.width) dense: added to every output row
     int low_bits;              // SpanPlan passes: position of the lowest high bit of the span
+    int in_real, out_real;     // complex64: the rows read are real numbers / only real parts are written
 };
 
 // (lets the float-only branch of load_factors compile for complex64, where it is never taken)
@@ -732,7 +752,10 @@ constexpr int fw_operations_behind_awaited_rows()
 // WAVES: wavefronts per SIMD the kernel is compiled for.  8 keeps it within 64 registers, so that
 // two workgroups fit a compute unit (see TWO_SETS for the LDS side); the host asks for that where
 // two resident workgroups pay off.
-template <typename T, typename P, int R, int WAVES = 4>
+// REAL: a complex64 kernel whose rows may be real numbers on either far side (in_real, out_real).  A
+// kernel of its own: the choice in the row loop keeps the compiler from overlapping its loads with the
+// stages (special.fft(4096) at 8192 rows, 696 us a step against 594).
+template <typename T, typename P, int R, int WAVES = 4, bool REAL = false>
 __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs a)
 {
     constexpr int L = P::LOG;
@@ -766,8 +789,13 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
     const int ng = (int)(g1 - g0);
     const int64_t row_end = g1 * SLOTS < a.batch ? g1 * SLOTS : a.batch;
     const int rows_valid = (int)(row_end - g0 * SLOTS);
-    const T *in_base = reinterpret_cast<const T *>(a.in) + g0 * SLOTS * a.in_view.sb + stack * a.in_view.ss;
-    const int in_row = (int)(a.in_view.sb * EB), out_row = (int)(a.out_view.sb * EB);
+    // complex64 rows may be real on the far side: half the bytes, nothing to convert them
+    static_assert(!REAL || EB == 8, "complex64 only");
+    const bool in_real = REAL && a.in_real, out_real = REAL && a.out_real;
+    const int in_eb = in_real ? EB / 2 : EB, out_eb = out_real ? EB / 2 : EB;
+    const char *in_base = reinterpret_cast<const char *>(a.in) +
+                          (g0 * SLOTS * a.in_view.sb + stack * a.in_view.ss) * in_eb;
+    const int in_row = (int)(a.in_view.sb * in_eb), out_row = (int)(a.out_view.sb * out_eb);
 
     // LDS flavour: lane l of wavefront w fetches element 64 w + l of each row group, which lands
     // at the padded word 65 w + l of the group's slot; `set` alternates between iterations
@@ -805,12 +833,12 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
 
     const __amdgpu_buffer_rsrc_t in_rs = make_rsrc(in_base);
     const __amdgpu_buffer_rsrc_t out_rs =
-        make_rsrc(reinterpret_cast<T *>(a.out) + g0 * SLOTS * a.out_view.sb + stack * a.out_view.ss);
+        make_rsrc(reinterpret_cast<char *>(a.out) + (g0 * SLOTS * a.out_view.sb + stack * a.out_view.ss) * out_eb);
     // thread-constant part of the offsets; the row group adds a wave-uniform part
     const View out_view = stack_view(a.out_view, stack, gridDim.y);
     const int64_t in_col = view_col(a.in_view, col_in), out_col = view_col(out_view, col);
-    const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.in_view.se * EB) : kOob;
-    const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.out_view.se * EB) : kOob;
+    const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.in_view.se * in_eb) : kOob;
+    const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.out_view.se * out_eb) : kOob;
     const T bias = (a.bias && col < out_view.width)
                        ? reinterpret_cast<const T *>(a.bias)[stack * a.out_view.width + col]
                        : zero_of(T());
@@ -819,7 +847,7 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const bool ok = (grel + r) * SLOTS + c.slot < rows_valid;
-            v[r] = buf_load<T>(in_rs, ok ? in_thr : kOob, (grel + r) * SLOTS * in_row);
+            v[r] = buf_load_any<T>(in_rs, ok ? in_thr : kOob, (grel + r) * SLOTS * in_row, in_real);
         }
     };
     // The requests of an iteration are spread over its phases (phase 0: the top, phase p: behind
@@ -908,7 +936,7 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const bool ok = full || (grel + r) * SLOTS + c.slot < rows_valid;
-            buf_store(out_rs, ok ? out_thr : kOob, (grel + r) * SLOTS * out_row, add(v[r], bias));
+            buf_store_any(out_rs, ok ? out_thr : kOob, (grel + r) * SLOTS * out_row, add(v[r], bias), out_real);
         }
     };
     int grel = 0;
@@ -941,6 +969,7 @@ struct FastBwArgs {
     // this workgroup's rows (a layer's bias gradient) go to (gridDim.x, S, bias_stride)
     void *bias_partial;
     int64_t bias_stride;
+    int x_real, g_real;        // complex64: x (and its gradient) / the output gradient are real numbers
 };
 
 // Backward kernel, software-pipelined over rows: iteration i runs the forward replay of
@@ -1116,7 +1145,8 @@ __device__ __forceinline__ void get_rows(const T *base, int idx, T (&v)[R])
 // R: row groups in flight per walk.  Two are possible where one block of float factors
 // leaves half of the registers free; each barrier and each LDS round trip then serves two
 // rows, and every thread runs four independent dependency chains instead of two.
-template <typename T, typename P, int R = 1>
+// REAL: as for fast_fw_kernel (x_real, g_real).
+template <typename T, typename P, int R = 1, bool REAL = false>
 __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
 {
     constexpr int L = P::LOG;
@@ -1188,33 +1218,36 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
     const int ng = (int)(g1 - g0);
     const int64_t row_end = g1 * SLOTS < a.batch ? g1 * SLOTS : a.batch;
     const int rows_valid = (int)(row_end - g0 * SLOTS);
-    const T *x_base = reinterpret_cast<const T *>(a.x_in) + g0 * SLOTS * a.x_view.sb + stack * a.x_view.ss;
-    const T *g_base = reinterpret_cast<const T *>(a.g_out) + g0 * SLOTS * a.g_view.sb + stack * a.g_view.ss;
+    static_assert(!REAL || EB == 8, "complex64 only");
+    const bool x_real = REAL && a.x_real, g_real = REAL && a.g_real;
+    const int x_eb = x_real ? EB / 2 : EB, g_eb = g_real ? EB / 2 : EB;
+    const char *x_base = reinterpret_cast<const char *>(a.x_in) + (g0 * SLOTS * a.x_view.sb + stack * a.x_view.ss) * x_eb;
+    const char *g_base = reinterpret_cast<const char *>(a.g_out) + (g0 * SLOTS * a.g_view.sb + stack * a.g_view.ss) * g_eb;
     const __amdgpu_buffer_rsrc_t gi_rs =
-        make_rsrc(reinterpret_cast<T *>(a.g_in) + g0 * SLOTS * a.gi_view.sb + stack * a.gi_view.ss);
-    const int x_row = (int)(a.x_view.sb * EB), g_row = (int)(a.g_view.sb * EB), gi_row = (int)(a.gi_view.sb * EB);
+        make_rsrc(reinterpret_cast<char *>(a.g_in) + (g0 * SLOTS * a.gi_view.sb + stack * a.gi_view.ss) * x_eb);
+    const int x_row = (int)(a.x_view.sb * x_eb), g_row = (int)(a.g_view.sb * g_eb), gi_row = (int)(a.gi_view.sb * x_eb);
     const int64_t gi_col = view_col(a.gi_view, col);
-    const int gi_thr = gi_col >= 0 ? c.slot * gi_row + (int)(gi_col * a.gi_view.se * EB) : kOob;
+    const int gi_thr = gi_col >= 0 ? c.slot * gi_row + (int)(gi_col * a.gi_view.se * x_eb) : kOob;
     auto group_ok = [&](int grp) { return grp >= 0 && grp * SLOTS + c.slot < rows_valid; };
     // (`full`: the caller knows that the group exists for every row slot of the workgroup)
     auto store_grad = [&](int grp, T gval, bool full = false) {
-        if (full) buf_store(gi_rs, gi_thr, grp * SLOTS * gi_row, gval);
-        else buf_store(gi_rs, group_ok(grp) ? gi_thr : kOob, (grp < 0 ? 0 : grp) * SLOTS * gi_row, gval);
+        if (full) buf_store_any(gi_rs, gi_thr, grp * SLOTS * gi_row, gval, x_real);
+        else buf_store_any(gi_rs, group_ok(grp) ? gi_thr : kOob, (grp < 0 ? 0 : grp) * SLOTS * gi_row, gval, x_real);
     };
 
     // --- operand fetch, register flavour: thread t holds its layout-A element
     const __amdgpu_buffer_rsrc_t x_rs = make_rsrc(x_base), g_rs = make_rsrc(g_base);
     const View g_view = stack_view(a.g_view, stack, gridDim.y);
     const int64_t x_col = view_col(a.x_view, col), g_col = view_col(g_view, col_out);
-    const int x_thr = x_col >= 0 ? c.slot * x_row + (int)(x_col * a.x_view.se * EB) : kOob;
-    const int g_thr = g_col >= 0 ? c.slot * g_row + (int)(g_col * a.g_view.se * EB) : kOob;
+    const int x_thr = x_col >= 0 ? c.slot * x_row + (int)(x_col * a.x_view.se * x_eb) : kOob;
+    const int g_thr = g_col >= 0 ? c.slot * g_row + (int)(g_col * a.g_view.se * g_eb) : kOob;
     auto load_x = [&](int grp, bool full = false) {
-        if (full) return buf_load<T>(x_rs, x_thr, grp * SLOTS * x_row);
-        return buf_load<T>(x_rs, group_ok(grp) ? x_thr : kOob, (grp < 0 ? 0 : grp) * SLOTS * x_row);
+        if (full) return buf_load_any<T>(x_rs, x_thr, grp * SLOTS * x_row, x_real);
+        return buf_load_any<T>(x_rs, group_ok(grp) ? x_thr : kOob, (grp < 0 ? 0 : grp) * SLOTS * x_row, x_real);
     };
     auto load_g = [&](int grp, bool full = false) {
-        if (full) return buf_load<T>(g_rs, g_thr, grp * SLOTS * g_row);
-        return buf_load<T>(g_rs, group_ok(grp) ? g_thr : kOob, (grp < 0 ? 0 : grp) * SLOTS * g_row);
+        if (full) return buf_load_any<T>(g_rs, g_thr, grp * SLOTS * g_row, g_real);
+        return buf_load_any<T>(g_rs, group_ok(grp) ? g_thr : kOob, (grp < 0 ? 0 : grp) * SLOTS * g_row, g_real);
     };
     // --- operand fetch, LDS flavour: lane l of wavefront w fetches element 64 w + l of the row
     // group, which lands at the padded word 65 w + l of the slot

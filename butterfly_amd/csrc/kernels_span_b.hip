@@ -11,10 +11,21 @@ BF_INST(4) BF_INST(5) BF_INST(6)
 void launch_edge(bool inc, const FastFwArgs *fw, const FastBwArgs *bw, dim3 grid, hipStream_t stream)
 {
     const dim3 block(kFastThreads);
-    if (fw && inc) hipLaunchKernelGGL((fast_fw_kernel<float2, EdgePlan<true>, kFastFwRowsComplex>), grid, block, 0, stream, *fw);
-    else if (fw) hipLaunchKernelGGL((fast_fw_kernel<float2, EdgePlan<false>, kFastFwRowsComplex>), grid, block, 0, stream, *fw);
-    else if (inc) hipLaunchKernelGGL((fast_bw_kernel<float2, EdgePlan<true>>), grid, block, 0, stream, *bw);
-    else hipLaunchKernelGGL((fast_bw_kernel<float2, EdgePlan<false>>), grid, block, 0, stream, *bw);
+#define BF_EDGE(INC)                                                                                              \
+    do {                                                                                                         \
+        using P = EdgePlan<INC>;                                                                                 \
+        if (fw && (fw->in_real || fw->out_real))                                                                 \
+            hipLaunchKernelGGL((fast_fw_kernel<float2, P, kFastFwRowsComplex, 4, true>), grid, block, 0, stream, *fw);  \
+        else if (fw)                                                                                             \
+            hipLaunchKernelGGL((fast_fw_kernel<float2, P, kFastFwRowsComplex>), grid, block, 0, stream, *fw);    \
+        else if (bw->x_real || bw->g_real)                                                                       \
+            hipLaunchKernelGGL((fast_bw_kernel<float2, P, 1, true>), grid, block, 0, stream, *bw);               \
+        else                                                                                                     \
+            hipLaunchKernelGGL((fast_bw_kernel<float2, P>), grid, block, 0, stream, *bw);                        \
+    } while (0)
+    if (inc) BF_EDGE(true);
+    else BF_EDGE(false);
+#undef BF_EDGE
 }
 
 }  // namespace bf

@@ -10,6 +10,11 @@ template <int L, int NB, bool INC>
 void launch_fast_fw_t(bool cplx, bool paired, const FastFwArgs &a, dim3 grid, hipStream_t stream)
 {
     if constexpr (NB == 1) {
+        if (cplx && (a.in_real || a.out_real)) {
+            hipLaunchKernelGGL((fast_fw_kernel<float2, FastPlan<L, NB, INC>, kFastFwRowsComplex, 4, true>), grid,
+                               dim3(kFastThreads), 0, stream, a);
+            return;
+        }
         if (cplx) {
             hipLaunchKernelGGL((fast_fw_kernel<float2, FastPlan<L, NB, INC>, kFastFwRowsComplex>), grid, dim3(kFastThreads), 0,
                                stream, a);
@@ -29,6 +34,10 @@ template <int L, int NB, bool INC>
 void launch_fast_bw_t(bool cplx, bool two_rows, const FastBwArgs &a, dim3 grid, hipStream_t stream)
 {
     if constexpr (NB == 1) {
+        if (cplx && (a.x_real || a.g_real)) {
+            hipLaunchKernelGGL((fast_bw_kernel<float2, FastPlan<L, NB, INC>, 1, true>), grid, dim3(kFastThreads), 0, stream, a);
+            return;
+        }
         if (cplx) {
             hipLaunchKernelGGL((fast_bw_kernel<float2, FastPlan<L, NB, INC>>), grid, dim3(kFastThreads), 0, stream, a);
             return;
@@ -56,6 +65,17 @@ bool launch_span_t(bool cplx, bool backward, bool two_rows, const FastFwArgs *fw
     constexpr bool for_complex = H * (MODE == 2 ? 2 : 1) <= kSpanMaxStagesComplex;
     if (cplx) {
         if constexpr (for_complex) {
+            // (a span of both sweeps stands in the middle of a schedule: its rows are the workspace's)
+            if constexpr (MODE != 2) {
+                if (!backward && (fw->in_real || fw->out_real)) {
+                    hipLaunchKernelGGL((fast_fw_kernel<float2, P, kFastFwRowsComplex, 4, true>), grid, block, 0, stream, *fw);
+                    return true;
+                }
+                if (backward && (bw->x_real || bw->g_real)) {
+                    hipLaunchKernelGGL((fast_bw_kernel<float2, P, 1, true>), grid, block, 0, stream, *bw);
+                    return true;
+                }
+            }
             if (!backward) hipLaunchKernelGGL((fast_fw_kernel<float2, P, kFastFwRowsComplex>), grid, block, 0, stream, *fw);
             else hipLaunchKernelGGL((fast_bw_kernel<float2, P>), grid, block, 0, stream, *bw);
             return true;

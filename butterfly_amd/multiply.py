@@ -47,13 +47,17 @@ def butterfly_multiply_bias(twiddle: torch.Tensor, input: torch.Tensor, bias: to
 
 def butterfly_layer(twiddle: torch.Tensor, input: torch.Tensor, bias: Optional[torch.Tensor], increasing_stride: bool,
                     out_size: int, in_perm: Optional[torch.Tensor] = None,
-                    out_index: Optional[torch.Tensor] = None) -> torch.Tensor:
+                    out_index: Optional[torch.Tensor] = None, in_scale: Optional[torch.Tensor] = None,
+                    out_scale: Optional[torch.Tensor] = None, real_input: bool = False,
+                    real_output: bool = False) -> torch.Tensor:
     """A whole layer on device tensors: input (*, in_size) -> (*, out_size), the stacks of twiddle
     side by side on one input, bias (out_size) added, column tables as in
-    butterfly_multiply_perm.  One operator (and one autograd node) for what the reference's
+    butterfly_multiply_perm, diagonals in_scale / out_scale directly in front of / behind the
+    factors multiplied into the first / last of them.  real_input / real_output: complex factors
+    between real numbers (the real part of the output).  One operator (and one autograd node) for what the reference's
     Butterfly.forward chains (torch_butterfly/butterfly.py:113-169)."""
-    return torch.ops.torch_butterfly.butterfly_layer(twiddle, input, bias, in_perm, out_index, increasing_stride,
-                                                     out_size)
+    return torch.ops.torch_butterfly.butterfly_layer(twiddle, input, bias, in_perm, out_index, in_scale, out_scale,
+                                                     increasing_stride, out_size, real_input, real_output)
 
 
 def butterfly_multiply_perm(twiddle: torch.Tensor, input: torch.Tensor, in_perm: Optional[torch.Tensor],

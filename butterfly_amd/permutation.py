@@ -5,7 +5,8 @@ import numpy as np
 import torch
 from torch import nn
 
-from .complex_utils import index_last_dim
+from .complex_utils import Complex2Real, Real2Complex, index_last_dim
+from .diagonal import Diagonal
 
 
 def bitreversal_permutation(n, pytorch_format=False):
@@ -69,65 +70,87 @@ class FixedPermutation(nn.Module):
 class FusedSequential(nn.Sequential):
     """nn.Sequential (same children, indexing and state) whose forward folds what stands
     directly around a Butterfly into that layer's own call: a FixedPermutation in front of or
-    behind it becomes part of the kernels' first read / last write, and a Diagonal between that
+    behind it becomes part of the kernels' first read / last write, a Diagonal between that
     permutation and the layer (or alone next to the layer) is multiplied into the layer's first /
-    last factor, so neither costs a pass of its own over the activations.  The accepted
-    patterns are [FixedPermutation] [Diagonal] Butterfly [Diagonal] [FixedPermutation]; any
+    last factor, and Real2Complex in front / Complex2Real behind a complex layer become the way it
+    reads / writes its rows, so none costs a pass of its own over the activations.  The accepted
+    patterns are [FixedPermutation] [Real2Complex] [Diagonal] Butterfly [Diagonal]
+    [FixedPermutation] [Complex2Real], with a permutation and a conversion in either order; any
     other sequence of children runs one after the other as usual."""
 
     def forward(self, input):
         from .butterfly import Butterfly, ButterflyBmm  # (butterfly.py does not import this module)
-        from .diagonal import Diagonal
-        mods = list(self)
-
-        def is_layer(m):
-            return isinstance(m, Butterfly) and not isinstance(m, ButterflyBmm)
-
-        def is_perm(m, size):
-            return isinstance(m, FixedPermutation) and m.permutation.dim() == 1 and m.permutation.numel() == size
-
-        def is_scale(m, size, layer):
-            return (isinstance(m, Diagonal) and m.diagonal.dim() == 1 and m.diagonal.numel() == size
-                    and (layer.complex or not m.diagonal.is_complex()))
-
-        i = 0
-        while i < len(mods):
-            # the layer that a permutation and / or a diagonal at position i would lead to
+        mods = list(self._modules.values())
+        if not input.is_cuda:
+            for m in mods:
+                input = m(input)
+            return input
+        i, count = 0, len(mods)
+        while i < count:
+            # the layer that a permutation, a conversion and a diagonal at position i would lead to
+            front = scale_in = to_complex = None
             j = i
-            while j < len(mods) and j - i < 2 and isinstance(mods[j], (FixedPermutation, Diagonal)):
+            while j < count and scale_in is None:
+                m = mods[j]
+                if isinstance(m, FixedPermutation) and front is None:
+                    front = m
+                elif isinstance(m, Real2Complex) and to_complex is None:
+                    to_complex = m
+                elif isinstance(m, Diagonal):
+                    scale_in = m
+                else:
+                    break
                 j += 1
-            layer = mods[j] if j < len(mods) and is_layer(mods[j]) else None
-            front = scale_in = None
-            if layer is not None and input.is_cuda and input.is_complex() == layer.complex:
-                lead = mods[i:j]
-                if len(lead) == 2 and is_perm(lead[0], layer.in_size) and is_scale(lead[1], layer.in_size, layer):
-                    front, scale_in = lead
-                elif len(lead) == 1 and is_perm(lead[0], layer.in_size):
-                    front = lead[0]
-                elif len(lead) == 1 and is_scale(lead[0], layer.in_size, layer):
-                    scale_in = lead[0]
-                elif lead:
-                    layer = None
-            else:
-                layer = None if j > i else layer
-            if layer is None or not input.is_cuda or input.is_complex() != layer.complex:
+            layer = mods[j] if j < count else None
+            if not (isinstance(layer, Butterfly) and not isinstance(layer, ButterflyBmm)
+                    and self._fits(layer, input, front, to_complex, scale_in)):
                 input = mods[i](input)
                 i += 1
                 continue
             i = j + 1
-            back = scale_out = None
-            if i < len(mods) and layer.bias is None and is_scale(mods[i], layer.out_size, layer):
+            back = scale_out = to_real = None
+            plain = layer.bias is None
+            if i < count and plain and isinstance(mods[i], Diagonal) and self._scales(mods[i], layer.out_size, layer):
                 scale_out = mods[i]
                 i += 1
-            if i < len(mods) and layer.nstacks == 1 and is_perm(mods[i], layer.out_size):
-                back = mods[i]
+            while i < count:
+                m = mods[i]
+                if (isinstance(m, FixedPermutation) and back is None and layer.nstacks == 1
+                        and self._permutes(m, layer.out_size)):
+                    back = m
+                elif isinstance(m, Complex2Real) and to_real is None and layer.complex and plain:
+                    to_real = m
+                else:
+                    break
                 i += 1
             n = 1 << layer.log_n
             input = layer(input, in_perm=None if front is None else front.column_table(n, False),
                           out_index=None if back is None else back.column_table(n, True),
                           in_scale=None if scale_in is None else scale_in.diagonal,
-                          out_scale=None if scale_out is None else scale_out.diagonal)
+                          out_scale=None if scale_out is None else scale_out.diagonal,
+                          real_input=to_complex is not None, real_output=to_real is not None)
         return input
+
+    @staticmethod
+    def _permutes(m, size):
+        return m.permutation.dim() == 1 and m.permutation.numel() == size
+
+    @staticmethod
+    def _scales(m, size, layer):
+        d = m.diagonal
+        return d.dim() == 1 and d.numel() == size and (layer.complex or not d.is_complex())
+
+    def _fits(self, layer, input, front, to_complex, scale_in):
+        """Whether the modules found in front of the layer can be folded into its call on `input`."""
+        if to_complex is not None:
+            # (the layer's float32 rows are read as they are; other real types are converted first)
+            if not layer.complex or input.dtype != torch.float32:
+                return False
+        elif input.is_complex() != layer.complex:
+            return False
+        if front is not None and not self._permutes(front, layer.in_size):
+            return False
+        return scale_in is None or self._scales(scale_in, layer.in_size, layer)
 
 
 def wavelet_permutation(n, pytorch_format=False):

@@ -255,6 +255,8 @@ typedef struct bf_layer {
     int32_t base4;            /* twiddle = twiddle4 and twiddle2 as for the base-4 calls                      */
     int32_t shared_input;     /* the stacks read one input (input_stride[1] = 0) and d_input is (B, I), dense:
                                * the sum over the stacks (d_input_stride[0..2] then only used with one stack) */
+    int32_t real_input;       /* complex64, base 2: input and d_input are real numbers (a complex layer behind */
+    int32_t real_output;      /* Real2Complex) / output and grad are (one in front of Complex2Real; no bias)   */
     int64_t total_output;     /* columns that exist, in ((S - 1) * output_size, S * output_size]               */
     const void *twiddle;
     const void *twiddle2;
@@ -262,6 +264,10 @@ typedef struct bf_layer {
     const int32_t *in_perm;   /* as in bf_butterfly_multiply_perm_fw, or NULL (base 2 only)                   */
     const int32_t *out_index;
 } bf_layer;
+
+/* 1 when both calls can run with the layer's real_input / real_output as they stand (strides of the
+ * real sides in floats), 0 when the caller has to convert. */
+int bf_layer_takes_real(const bf_layer *l);
 
 /* Activations the forward call can keep for the backward (as bf_butterfly_multiply_saved_bytes). */
 size_t bf_layer_kept_bytes(const bf_layer *l);

@@ -354,3 +354,35 @@ def test_fused_sequential_folds_diagonals():
         layer(torch.randn(2, 64, device="cuda"), out_scale=torch.ones(64, device="cuda"))
     with pytest.raises(ValueError):
         layer(torch.randn(2, 64, device="cuda"), transpose=True, in_scale=torch.ones(64, device="cuda"))
+
+
+@pytest.mark.parametrize("make, n, lead", [
+    ("circulant", 2, (5,)), ("circulant", 64, (37,)), ("circulant", 100, (4, 9)),
+    ("circulant", 700, (33,)), ("circulant", 1024, (2100,)), ("circulant", 1500, (301,)), ("circulant", 5000, (3,)),
+    ("dct2", 32, (7,)), ("dct3", 256, (65,)), ("dct4", 2048, (21,)), ("dct2", 4096, (19,)), ("dst2", 1024, (2, 40)),
+    ("bias", 500, (17,))], ids=lambda v: str(v))
+def test_real_numbers_around_complex_layers(make, n, lead):
+    """Real2Complex / Complex2Real folded into the layer's reads and writes (every kind of pass
+    that can stand there, and the layers that have to convert after all) against the same
+    modules one after the other, gradients included."""
+    import butterfly_amd
+    from butterfly_amd import special
+    from butterfly_amd.complex_utils import Complex2Real, Real2Complex
+    from butterfly_amd.permutation import FusedSequential
+    torch.manual_seed(n)
+    if make == "circulant":
+        fused = special.circulant(torch.randn(n) / n ** 0.5).cuda()
+    elif make == "bias":
+        fused = FusedSequential(Real2Complex(), butterfly_amd.Butterfly(n, 700, complex=True, nblocks=2), Complex2Real()).cuda()
+    else:
+        fused = (special.dct if make[:3] == "dct" else special.dst)(n, type=int(make[3]), normalized=True).cuda()
+    plain = torch.nn.Sequential(*fused)
+    x = torch.randn(*lead, n, device="cuda", requires_grad=True)
+    with torch.no_grad():
+        y0 = fused(x)
+    y, z = fused(x), plain(x)
+    assert y.dtype == torch.float32 and y.shape == z.shape and torch.equal(y, y0)
+    g = torch.randn_like(z)
+    wanted = [x, *fused.parameters()]
+    for a, b in [(y, z)] + list(zip(torch.autograd.grad(y, wanted, g), torch.autograd.grad(z, wanted, g))):
+        assert (a - b).norm().item() <= 1e-5 * b.norm().item()
