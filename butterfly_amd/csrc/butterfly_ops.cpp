@@ -459,15 +459,30 @@ Tensor layer_fw(const Operands &o_, const Tensor &input, int64_t out_size, Tenso
     Tensor x = rows_of(input);
     c10::SmallVector<int64_t, 6> shape(input.sizes().begin(), input.sizes().end());
     shape.back() = out_size;
+    // Rows of several stacks start at multiples of 128 bytes: the stacks are written by different
+    // workgroups, and in rows that start anywhere each of their ends would share its cache line with
+    // another one's (7282 rows of 45 stacks of 64 complex64, 2821 columns: 77 us against 68).
+    const int64_t line = 128 / (o.real_output ? 4 : (int64_t)o.twiddle.element_size());
+    const int64_t pitch = o.twiddle.size(0) > 1 ? (out_size + line - 1) / line * line : out_size;
     auto run = [&](Tensor &output) {
         Call c;
         describe_layer(c, o, x, out_size, who);
         bf_problem &p = c.p();
-        p.output_stride[0] = out_size;
+        p.output_stride[0] = pitch;
         p.output_stride[1] = p.output_size;
         p.output_stride[2] = 1;
         if (!takes_real(c, o)) return false;
-        output = at::empty(shape, o.real_output ? x.options().dtype(at::kFloat) : o.twiddle.options());
+        const auto options = o.real_output ? x.options().dtype(at::kFloat) : o.twiddle.options();
+        if (pitch == out_size) {
+            output = at::empty(shape, options);
+        } else {
+            c10::SmallVector<int64_t, 6> stride(shape.size(), 1);
+            for (int64_t d = (int64_t)shape.size() - 2, step = pitch; d >= 0; --d) {
+                stride[d] = step;
+                step *= std::max<int64_t>(shape[d], 1);
+            }
+            output = at::empty_strided(shape, stride, options);
+        }
         forward_call(c, x, output, keep, who);
         return true;
     };
