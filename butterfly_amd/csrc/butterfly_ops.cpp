@@ -461,9 +461,12 @@ Tensor layer_fw(const Operands &o_, const Tensor &input, int64_t out_size, Tenso
     shape.back() = out_size;
     // Rows of several stacks start at multiples of 128 bytes: the stacks are written by different
     // workgroups, and in rows that start anywhere each of their ends would share its cache line with
-    // another one's (7282 rows of 45 stacks of 64 complex64, 2821 columns: 77 us against 68).
+    // another one's (7282 rows of 45 stacks of 64 complex64, 2821 columns: 77 us against 64).
+    // Only where the last stack is cut short: whole stacks fill a contiguous tensor.
     const int64_t line = 128 / (o.real_output ? 4 : (int64_t)o.twiddle.element_size());
-    const int64_t pitch = o.twiddle.size(0) > 1 ? (out_size + line - 1) / line * line : out_size;
+    const int64_t nstacks = o.twiddle.size(0);
+    const bool cut = nstacks > 1 && out_size < (nstacks << log_size(o, who));
+    const int64_t pitch = cut ? (out_size + line - 1) / line * line : out_size;
     auto run = [&](Tensor &output) {
         Call c;
         describe_layer(c, o, x, out_size, who);
@@ -555,6 +558,8 @@ struct MultiplyNode : public torch::autograd::Node {
     {
         variable_list out(num_outputs());
         if (!grads[0].defined()) return out;
+        // (against another thread's release_variables or pass over the same graph)
+        std::lock_guard<std::mutex> lock(mutex_);
         const auto self = getptr();
         Operands o;
         o.twiddle = twiddle.unpack(self);
@@ -586,6 +591,7 @@ struct MultiplyNode : public torch::autograd::Node {
 
     void release_variables() override
     {
+        std::lock_guard<std::mutex> lock(mutex_);
         twiddle.reset_data();
         twiddle2.reset_data();
         input.reset_data();
@@ -605,6 +611,9 @@ struct MultiplyNode : public torch::autograd::Node {
 template <typename F>
 Tensor differentiable(const Operands &o, const Tensor &input, bool layer, const char *who, F &&forward)
 {
+    // (a tangent would be dropped silently, with gradients asked for or not)
+    for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &o.in_scale, &o.out_scale, &input})
+        TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), who, ": no forward-mode derivative");
     bool wanted = false;
     if (at::GradMode::is_enabled()) {
         for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &o.in_scale, &o.out_scale, &input})
@@ -614,8 +623,6 @@ Tensor differentiable(const Operands &o, const Tensor &input, bool layer, const 
         at::AutoDispatchBelowADInplaceOrView below;
         return forward(nullptr, nullptr);
     }
-    for (const Tensor *t : {&o.twiddle, &o.twiddle2, &o.bias, &o.in_scale, &o.out_scale, &input})
-        TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), who, ": no forward-mode derivative");
     std::shared_ptr<MultiplyNode> node(new MultiplyNode(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(o.twiddle, o.twiddle2, input, o.bias, o.in_scale, o.out_scale));
     Tensor kept, scaled, out;

@@ -9,6 +9,8 @@ import pytest
 import scipy.linalg
 import torch
 
+from conftest import rel_err
+
 pytestmark = pytest.mark.gpu
 
 
@@ -326,3 +328,21 @@ def test_random_layer_configurations_match_the_host_path(chunk):
                 assert a.shape == b.shape
                 if b.numel():
                     assert (a.cpu() - b).abs().max().item() <= 2e-4 * max(1.0, b.abs().max().item())
+
+
+@pytest.mark.parametrize("n, out_size, contiguous", [(4, 12, True), (16, 80, True), (32, 96, True), (32, 32, True),
+                                                     (32, 17, True), (32, 65, False)])
+def test_whole_stacks_fill_a_contiguous_tensor(n, out_size, contiguous):
+    """Rows are only spaced out where the last stack is cut short (its output was a slice of whole
+    stacks before layers became one operator): any other output can be viewed flat."""
+    import butterfly_amd
+    say("layer output", n, out_size)
+    layer = butterfly_amd.Butterfly(n, out_size).cuda()
+    x = torch.randn(3, 5, n, device="cuda")
+    y = layer(x)
+    assert y.shape == (3, 5, out_size)
+    assert y.is_contiguous() == contiguous
+    assert y.view(-1, out_size).shape == (15, out_size)
+    host = butterfly_amd.Butterfly(n, out_size)
+    host.load_state_dict(layer.state_dict())
+    assert rel_err(y.detach().cpu().numpy(), host(x.cpu()).detach().numpy()) < 1e-5

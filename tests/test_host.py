@@ -769,3 +769,18 @@ def test_permuted_multiply_of_size_one_on_the_host():
     y = butterfly_multiply_perm(tw, x, table, table, bias, True, None)
     assert y.shape == (4, 3, 1) and torch.allclose(y, x + bias)
     assert torch.allclose(butterfly_multiply_perm(tw, x, None, None, None, False, 1), x)
+
+
+@pytest.mark.parametrize("with_grad", [False, True])
+def test_forward_mode_is_refused(with_grad):
+    """A tangent is refused, with gradients recorded or not, instead of being dropped."""
+    import torch.autograd.forward_ad as forward_ad
+
+    import butterfly_amd
+    twiddle, x = torch.randn(1, 1, 3, 4, 2, 2), torch.randn(2, 1, 8)
+    with forward_ad.dual_level(), torch.set_grad_enabled(with_grad):
+        dual = forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises(RuntimeError):
+            butterfly_amd.butterfly_multiply(twiddle, dual, True)
+        with pytest.raises(RuntimeError):
+            butterfly_amd.butterfly_multiply(forward_ad.make_dual(twiddle, twiddle), x, True)
