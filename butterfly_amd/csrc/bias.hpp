@@ -20,7 +20,7 @@ struct BiasArgs {
     const void *grad;      // gradient: (B, S, width) through `view`
     void *partial;         // (nparts, S, stride)
     int64_t stride;        // width rounded up: every slice starts at a multiple of 16 bytes
-    View view;
+    StackView view;
     int64_t batch;
     int64_t width;         // columns that exist (output_size)
     int64_t rows_per_part;
@@ -34,7 +34,7 @@ __global__ __launch_bounds__(kBiasThreads) void bias_add_kernel(BiasArgs a)
     const int64_t col = (int64_t)blockIdx.x * kBiasThreads + threadIdx.x;
     const int stack = blockIdx.y;
     if (col >= a.width) return;
-    const int64_t vc = view_col(stack_view(a.view, stack, gridDim.y), col);
+    const int64_t vc = view_col(stack_view(a.view, stack), col);
     if (vc < 0) return;
     const T b = reinterpret_cast<const T *>(a.bias)[stack * a.width + col];
     T *out = reinterpret_cast<T *>(a.out) + stack * a.view.ss + vc * a.view.se;
@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kBiasThreads) void bias_grad_partial_kernel(BiasArg
     const int64_t col = (int64_t)blockIdx.x * kBiasThreads + threadIdx.x;
     const int stack = blockIdx.y;
     if (col >= a.width) return;
-    const int64_t vc = view_col(stack_view(a.view, stack, gridDim.y), col);
+    const int64_t vc = view_col(stack_view(a.view, stack), col);
     const T *g = reinterpret_cast<const T *>(a.grad) + stack * a.view.ss + (vc < 0 ? 0 : vc) * a.view.se;
     const int64_t r0 = (int64_t)blockIdx.z * a.rows_per_part;
     const int64_t r1 = vc < 0 ? r0 : (r0 + a.rows_per_part < a.batch ? r0 + a.rows_per_part : a.batch);

@@ -97,27 +97,30 @@ Schedule make_schedule(const bf_problem *p, bool base4)
     return sc;
 }
 
-// tail: width of the last stack where it differs (-1: it does not)
-View make_view(const int64_t stride[3], int64_t width, const int *perm = nullptr, int64_t tail = -1)
+// tail: width of the last of nstacks stacks where it differs (-1: it does not)
+StackView make_view(const int64_t stride[3], int64_t width, const int *perm = nullptr, int64_t tail = -1,
+                    int64_t nstacks = 0)
 {
-    View v;
+    StackView v;
     v.sb = stride[0];
     v.ss = stride[1];
     v.se = stride[2];
     v.width = width;
-    v.tail = tail < 0 ? width : tail;
+    v.last = tail < 0 || tail == width ? -1 : (int)(nstacks - 1);
+    v.cut = v.last < 0 ? 0 : (int)(width - tail);
     v.perm = perm;
     return v;
 }
 
-View dense_view(int64_t nstacks, int64_t n)
+StackView dense_view(int64_t nstacks, int64_t n)
 {
-    View v;
+    StackView v;
     v.sb = nstacks * n;
     v.ss = n;
     v.se = 1;
     v.width = n;
-    v.tail = n;
+    v.last = -1;
+    v.cut = 0;
     v.perm = nullptr;
     return v;
 }
@@ -526,18 +529,18 @@ void fill_stage_table(int *dst, int cap, const Pass &q)
 // `bias` (may be NULL) is added by the last pass when that pass runs in a kernel that can do
 // it; *bias_done says whether it was.  real: kRealIn / kRealOut, for the first / last of these passes.
 int multipass_forward(const bf_problem *p, const PassPlan &pl, const void *tw, const void *input, void *output,
-                      void *scratch, const View &in_view, const View &out_view, int first, int last,
+                      void *scratch, const StackView &in_view, const StackView &out_view, int first, int last,
                       hipStream_t stream, const void *bias = nullptr, bool *bias_done = nullptr, int real = 0)
 {
     if (bias_done) *bias_done = false;
     const int64_t n = (int64_t)1 << p->log_n;
-    const View dense = dense_view(p->nstacks, n);
+    const StackView dense = dense_view(p->nstacks, n);
     for (int k = first; k < last; ++k) {
         const Pass &q = pl.pass[k];
         const void *src = k == first ? input : scratch;
         void *dst = k == last - 1 ? output : scratch;
-        const View sv = k == first ? in_view : dense;
-        const View dv = k == last - 1 ? out_view : dense;
+        const StackView sv = k == first ? in_view : dense;
+        const StackView dv = k == last - 1 ? out_view : dense;
         if (q.wide) {
             const FastGrid g = wide_grid(p->batch, p->nstacks);
             FastFwArgs a = {};
@@ -704,11 +707,11 @@ int fast4_fw_wg_per_cu(const bf_problem *p)
 
 // forward of blocks [first, last) through the base-4 kernels; `scratch` as in multipass_forward
 int fast4_forward(const bf_problem *p, const void *tw4, const void *tw2, const void *input, void *output,
-                  void *scratch, const View &in_view, const View &out_view, int first, int last, hipStream_t stream)
+                  void *scratch, const StackView &in_view, const StackView &out_view, int first, int last, hipStream_t stream)
 {
     const int64_t n = (int64_t)1 << p->log_n;
     const int L = (int)p->log_n;
-    const View dense = dense_view(p->nstacks, n);
+    const StackView dense = dense_view(p->nstacks, n);
     const FastGrid g = fast_grid(p->batch, L, p->nstacks, fast4_fw_rows(p), fast4_fw_wg_per_cu(p));
     if (fast4_general(p)) {
         for (int k = first; k < last; ++k) {
@@ -730,7 +733,6 @@ int fast4_forward(const bf_problem *p, const void *tw4, const void *tw2, const v
         return fail(BF_ERR_INVALID, "twiddle4 must be 16-byte aligned");
     for (int k = first; k < last; ++k) {
         Fast4Args a = {};
-        a.nstacks = (int)p->nstacks;
         a.tw4 = static_cast<const float *>(tw4) + (int64_t)k * (L / 2) * (n / 4) * 16;
         a.tw_stack_stride = p->nblocks * (L / 2) * (n / 4) * 16;
         a.x_in = static_cast<const float *>(k == first ? input : scratch);
@@ -851,8 +853,8 @@ int64_t pass4_slices(const bf_problem *p, const Pass4 &q)
 // One pass forward (backward == false: x_in -> x_out) or backward (x_in, g_out -> g_in and the
 // pass's partial slices; *nparts receives their number per stage).
 int run_pass4(const bf_problem *p, const Schedule &sc, const Pass4 &q, bool backward, const void *tw2, const void *tw4,
-              const void *x_in, const View &x_view, void *x_out, const View &xo_view, const void *g_out,
-              const View &g_view, void *g_in, const View &gi_view, void *partial, int64_t *nparts, hipStream_t stream)
+              const void *x_in, const StackView &x_view, void *x_out, const StackView &xo_view, const void *g_out,
+              const StackView &g_view, void *g_in, const StackView &gi_view, void *partial, int64_t *nparts, hipStream_t stream)
 {
     const int64_t n = (int64_t)1 << p->log_n;
     const int L = (int)p->log_n;
@@ -922,11 +924,11 @@ int run_pass4(const bf_problem *p, const Schedule &sc, const Pass4 &q, bool back
 
 // passes [first, last) forward; `scratch` holds the activation between passes (in place)
 int long4_forward(const bf_problem *p, const Schedule &sc, const Plan4Long &pl, const void *tw2, const void *tw4,
-                  const void *input, void *output, void *scratch, const View &in_view, const View &out_view,
+                  const void *input, void *output, void *scratch, const StackView &in_view, const StackView &out_view,
                   int first, int last, hipStream_t stream)
 {
     const int64_t n = (int64_t)1 << p->log_n;
-    const View dense = dense_view(p->nstacks, n);
+    const StackView dense = dense_view(p->nstacks, n);
     for (int k = first; k < last; ++k) {
         const int rc = run_pass4(p, sc, pl.pass[k], false, tw2, tw4, k == first ? input : scratch,
                                  k == first ? in_view : dense, k == last - 1 ? output : scratch,
@@ -979,7 +981,7 @@ StreamPick pick_stream(const bf_problem *p, bool base4)
 // which the activation is also stored, and where.  BF_ERR_UNSUPPORTED when the plan does not fit the kernel: nothing has
 // been launched then.
 int stream_forward(const bf_problem *p, const Schedule &sc, int stages, StreamPick pick, const void *tw2, const void *tw4,
-                   const void *input, void *output, const View &in_view, const View &out_view, const void *bias,
+                   const void *input, void *output, const StackView &in_view, const StackView &out_view, const void *bias,
                    const int *saves, void *const *planes, int nsaves, hipStream_t stream)
 {
     const int e = (int)elem_bytes(p->dtype);
@@ -1003,8 +1005,8 @@ int stream_forward(const bf_problem *p, const Schedule &sc, int stages, StreamPi
     a.bias = bias;
     for (int k = 0; k < nsaves; ++k) a.save[k] = planes[k];
     a.batch = p->batch;
-    auto vec = [&](const View &v, const void *base) {
-        return v.se == 1 && v.width % 4 == 0 && v.tail % 4 == 0 && p->log_n >= 2 && v.sb * e % 16 == 0 &&
+    auto vec = [&](const StackView &v, const void *base) {
+        return v.se == 1 && v.width % 4 == 0 && v.cut % 4 == 0 && p->log_n >= 2 && v.sb * e % 16 == 0 &&
                v.ss * e % 16 == 0 && (reinterpret_cast<uintptr_t>(base) & 15) == 0;
     };
     a.in_vec = vec(in_view, input);
@@ -1018,8 +1020,8 @@ int stream_forward(const bf_problem *p, const Schedule &sc, int stages, StreamPi
 // ---- generic forward ----------------------------------------------------------------------
 
 int launch_generic_fw(const bf_problem *p, const Schedule &sc, int t0, int t1, const void *tw2,
-                      const void *tw4, const void *in, const View &in_view, void *out,
-                      const View &out_view, hipStream_t stream)
+                      const void *tw4, const void *in, const StackView &in_view, void *out,
+                      const StackView &out_view, hipStream_t stream)
 {
     const int64_t n = (int64_t)1 << p->log_n;
     const size_t row_bytes = (size_t)n * elem_bytes(p->dtype);
@@ -1078,7 +1080,7 @@ size_t forward_workspace(const bf_problem *p, bool base4, int tables)
 
 // output += bias over all rows, for schedules whose last pass could not add it itself
 template <typename T>
-int launch_bias_add(const bf_problem *p, const void *bias, void *output, const View &out_view, hipStream_t stream)
+int launch_bias_add(const bf_problem *p, const void *bias, void *output, const StackView &out_view, hipStream_t stream)
 {
     if (p->batch <= 0 || p->nstacks <= 0 || p->output_size <= 0) return BF_OK;
     BiasArgs a = {};
@@ -1129,8 +1131,8 @@ int forward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, c
             if (base4 && (p->log_n & 1) && !tw2) return fail(BF_ERR_INVALID, "twiddle2 is NULL");
         }
     }
-    const View in_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
-    const View out_view = make_view(p->output_stride, p->output_size, out_index, tail);
+    const StackView in_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
+    const StackView out_view = make_view(p->output_stride, p->output_size, out_index, tail, p->nstacks);
     const StreamPick pick = pick_stream(p, base4);
     if (pick.waves) {
         rc = stream_forward(p, sc, sc.per * sc.nblocks, pick, tw2, tw4, input, output, in_view, out_view, bias, nullptr, nullptr, 0, stream);
@@ -1217,7 +1219,7 @@ struct BiasGrad {
 
 // First step of the bias gradient as a kernel of its own, for backward kernels that do not form
 // the column sums on the way.
-int form_bias_sums(const bf_problem *p, const void *grad, const View &g_view, BiasGrad &bg, hipStream_t stream)
+int form_bias_sums(const bf_problem *p, const void *grad, const StackView &g_view, BiasGrad &bg, hipStream_t stream)
 {
     const BiasGradPlan b = plan_bias_grad(p);
     bg.formed = true;
@@ -1363,7 +1365,7 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, i
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void copy_pad_kernel(const T *in, View iv, T *out, View ov, int64_t batch)
+__global__ __launch_bounds__(256) void copy_pad_kernel(const T *in, StackView iv, T *out, StackView ov, int64_t batch)
 {
     const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int s = blockIdx.y;
@@ -1375,7 +1377,7 @@ __global__ __launch_bounds__(256) void copy_pad_kernel(const T *in, View iv, T *
     }
 }
 
-int launch_copy_pad(const bf_problem *p, const void *in, const View &iv, void *out, const View &ov,
+int launch_copy_pad(const bf_problem *p, const void *in, const StackView &iv, void *out, const StackView &ov,
                     hipStream_t stream)
 {
     if (p->batch == 0 || p->nstacks == 0 || ov.width == 0) return BF_OK;
@@ -1394,7 +1396,7 @@ int launch_copy_pad(const bf_problem *p, const void *in, const View &iv, void *o
 // bg (may be NULL): bias sums to be added up by the same launch; g_view: the view they were read through
 int launch_reduce(const bf_problem *p, const Schedule &sc, const ReduceSegment *segs, int nsegs, const void *partial,
                   int64_t slot, void *d_tw2, void *d_tw4, hipStream_t stream, const BiasGrad *bg = nullptr,
-                  const View *g_view = nullptr)
+                  const StackView *g_view = nullptr)
 {
     const bool bias = bg && bg->d_bias && g_view->width > 0;
     ReduceArgs r = {};
@@ -1420,7 +1422,7 @@ int launch_reduce(const bf_problem *p, const Schedule &sc, const ReduceSegment *
         r.bias_nparts = (int)bg->nparts;
         r.bias_stride = bias_stride(p);
         r.bias_width = g_view->width;
-        r.bias_tail = g_view->tail;
+        r.bias_tail = g_view->width - g_view->cut;
         floats = std::max(floats, g_view->width * r.elem_floats);
     }
     const dim3 grid((unsigned)((floats + 63) / 64), (unsigned)(r.nstages + (bias ? 1 : 0)), (unsigned)p->nstacks);
@@ -1445,7 +1447,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     const Schedule sc = make_schedule(p, base4);
     const int64_t n = (int64_t)1 << p->log_n;
     const int tables = tables_of(in_perm, out_index);
-    const View g_view = make_view(p->output_stride, std::min(p->output_size, n), out_index, tail);
+    const StackView g_view = make_view(p->output_stride, std::min(p->output_size, n), out_index, tail, p->nstacks);
     if (p->batch == 0 || p->nstacks == 0) {
         // no rows: d_input is empty and every entry of the other gradients is an empty sum, whatever the row length
         const ReduceSegment none = {0, sc.per * sc.nblocks, 0, 0};
@@ -1463,9 +1465,9 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     if (!base4 && ((reinterpret_cast<uintptr_t>(tw2) | reinterpret_cast<uintptr_t>(d_tw2)) & 15) != 0)
         return fail(BF_ERR_INVALID, "twiddle and d_twiddle must be 16-byte aligned");
 
-    const View x_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
-    const View di_view = make_view(p->d_input_stride, p->input_size, in_perm);
-    const View dense = dense_view(p->nstacks, n);
+    const StackView x_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
+    const StackView di_view = make_view(p->d_input_stride, p->input_size, in_perm);
+    const StackView dense = dense_view(p->nstacks, n);
     char *ws = static_cast<char *>(workspace);
     const size_t e_bytes = elem_bytes(p->dtype);
     if (real && (!pl.fast || p->input_size > n || (bg && (real & kRealOut))))
@@ -1517,7 +1519,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                                k == 0 ? x_view : dense, dense, k, k + 1, stream);
             if (rc) return rc;
         }
-        const View dn_view = make_view(p->d_input_stride, std::min(p->input_size, n), in_perm);
+        const StackView dn_view = make_view(p->d_input_stride, std::min(p->input_size, n), in_perm);
         const FastGrid g = fast_grid(p->batch, L, p->nstacks, 1, 1);
         for (int k = P - 1; k >= 0 && general; --k) {
             Fast4GArgs a = fast4g_block_args(p, tw4, tw2, k);
@@ -1540,7 +1542,6 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             return fail(BF_ERR_INVALID, "twiddle4 must be 16-byte aligned");
         for (int k = P - 1; k >= 0 && !general; --k) {
             Fast4Args a = {};
-            a.nstacks = (int)p->nstacks;
             a.tw4 = static_cast<const float *>(tw4) + (int64_t)k * per * (n / 4) * 16;
             a.tw_stack_stride = sc.tw4_stack_stride;
             a.x_in = static_cast<const float *>(k == 0 ? input : boundary(k));
@@ -1561,9 +1562,9 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
         }
         if (nsegs > 0 && (rc = finish())) return rc;
         if (p->input_size > n) {
-            View tail = di_view;
+            StackView tail = di_view;
             tail.width = p->input_size - n;
-            View none = tail;
+            StackView none = tail;
             none.width = 0;
             char *base = static_cast<char *>(d_input) + (size_t)n * p->d_input_stride[2] * e_bytes;
             rc = launch_copy_pad(p, base, none, base, tail, stream);
@@ -1601,7 +1602,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                                nullptr, k == 0 ? x_view : dense, dense, k, k + 1, stream);
             if (rc) return rc;
         }
-        const View dn_view = make_view(p->d_input_stride, std::min(p->input_size, n), in_perm);
+        const StackView dn_view = make_view(p->d_input_stride, std::min(p->input_size, n), in_perm);
         for (int k = P - 1; k >= 0; --k) {
             const Pass4 &q = lp.pass[k];
             int64_t nparts = 0;
@@ -1615,9 +1616,9 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
         }
         if (nsegs > 0 && (rc = finish())) return rc;
         if (p->input_size > n) {
-            View tail = di_view;
+            StackView tail = di_view;
             tail.width = p->input_size - n;
-            View none = tail;
+            StackView none = tail;
             none.width = 0;
             char *base = static_cast<char *>(d_input) + (size_t)n * p->d_input_stride[2] * e_bytes;
             rc = launch_copy_pad(p, base, none, base, tail, stream);
@@ -1637,15 +1638,15 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                                    k == 0 ? x_view : dense, dense, k, k + 1, stream, nullptr, nullptr, k == 0 ? real & kRealIn : 0);
             if (rc) return rc;
         }
-        const View dn_view = make_view(p->d_input_stride, std::min(p->input_size, n), in_perm);
+        const StackView dn_view = make_view(p->d_input_stride, std::min(p->input_size, n), in_perm);
         for (int k = P - 1; k >= 0; --k) {
             const Pass &q = mp.pass[k];
             const void *xin = k == 0 ? input : boundary(k);
-            const View xv = k == 0 ? x_view : dense;
+            const StackView xv = k == 0 ? x_view : dense;
             const void *gout = k == P - 1 ? grad : ws + pl.off_gbuf;
-            const View gv = k == P - 1 ? g_view : dense;
+            const StackView gv = k == P - 1 ? g_view : dense;
             void *gin = k == 0 ? d_input : ws + pl.off_gbuf;
-            const View giv = k == 0 ? dn_view : dense;
+            const StackView giv = k == 0 ? dn_view : dense;
             int64_t nparts = 0;
             {
                 const FastGrid g = fast_grid(p->batch, q.L, p->nstacks * pass_lanes(p, q), 1, 1, row_cap(p, true), true);
@@ -1694,9 +1695,9 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
         if (nsegs > 0 && (rc = finish())) return rc;
         if (p->input_size > n) {
             // input wider than n: those columns get a zero gradient
-            View tail = di_view;
+            StackView tail = di_view;
             tail.width = p->input_size - n;
-            View none = tail;
+            StackView none = tail;
             none.width = 0;
             char *base = static_cast<char *>(d_input) + (size_t)n * p->d_input_stride[2] * e_bytes;
             rc = launch_copy_pad(p, base, none, base, tail, stream);
@@ -1873,7 +1874,7 @@ static int bias_grad(const bf_problem *p, const void *grad, void *d_bias, void *
     BiasGrad bg;
     bg.area = workspace;
     bg.d_bias = d_bias;
-    const View g_view = make_view(p->output_stride, p->output_size);
+    const StackView g_view = make_view(p->output_stride, p->output_size);
     if (p->batch > 0) {
         if (!grad) return fail(BF_ERR_INVALID, "grad is NULL");
         const size_t need = plan_bias_grad(p).bytes;
@@ -1997,9 +1998,9 @@ static int fw_saving(const bf_problem *p, const void *twiddle, const void *input
     const PassPlan mp = build_passes(p, false, false, tables);
     const BwPlan pl = plan_bw(p, false, true, tables);
     if (mp.npass < 2 || !pl.fast) return fail(BF_ERR_INVALID, "this problem has no activations to save");
-    const View in_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
-    const View out_view = make_view(p->output_stride, p->output_size, out_index, tail);
-    const View dense = dense_view(p->nstacks, n);
+    const StackView in_view = make_view(p->input_stride, std::min(p->input_size, n), in_perm);
+    const StackView out_view = make_view(p->output_stride, p->output_size, out_index, tail, p->nstacks);
+    const StackView dense = dense_view(p->nstacks, n);
     char *bounds = static_cast<char *>(saved);
     auto boundary = [&](int k) { return bounds + (size_t)(k - 1) * pl.boundary_bytes; };
     const int P = mp.npass;
@@ -2147,9 +2148,9 @@ static int fw4_saving(const bf_problem *p, const void *twiddle4, const void *twi
     const int64_t n = (int64_t)1 << p->log_n;
     const BwPlan pl = plan_bw(p, true, true);
     const Schedule sc = make_schedule(p, true);
-    const View in_view = make_view(p->input_stride, std::min(p->input_size, n), nullptr);
-    const View out_view = make_view(p->output_stride, p->output_size, nullptr, tail);
-    const View dense = dense_view(p->nstacks, n);
+    const StackView in_view = make_view(p->input_stride, std::min(p->input_size, n), nullptr);
+    const StackView out_view = make_view(p->output_stride, p->output_size, nullptr, tail, p->nstacks);
+    const StackView dense = dense_view(p->nstacks, n);
     char *planes = static_cast<char *>(saved);
     auto boundary = [&](int k) { return planes + (size_t)(k - 1) * pl.boundary_bytes; };
     const int P = pl.nchunks;
@@ -2169,7 +2170,7 @@ static int fw4_saving(const bf_problem *p, const void *twiddle4, const void *twi
     for (int k = 0; k < P; ++k) {
         const void *in = k == 0 ? input : boundary(k);
         void *out = k == P - 1 ? output : boundary(k + 1);
-        const View &iv = k == 0 ? in_view : dense, &ov = k == P - 1 ? out_view : dense;
+        const StackView &iv = k == 0 ? in_view : dense, &ov = k == P - 1 ? out_view : dense;
         rc = pl.long4 ? long4_forward(p, sc, lp, twiddle2, twiddle4, in, out, nullptr, iv, ov, k, k + 1, stream)
                       : fast4_forward(p, twiddle4, twiddle2, in, out, nullptr, iv, ov, k, k + 1, stream);
         if (rc) return rc;

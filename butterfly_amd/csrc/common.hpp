@@ -100,7 +100,6 @@ __host__ __device__ __forceinline__ StageInfo stage_info(const Schedule &sc, int
 struct View {
     int64_t sb, ss, se;
     int64_t width;
-    int64_t tail;     // width of the last stack (a layer's outputs need not fill its last stack)
     const int *perm;  // NULL, or n entries: column c of the row as the kernels see it lives in tensor column perm[c]
 };
 
@@ -113,11 +112,22 @@ __device__ __forceinline__ int64_t view_col(const View &v, int64_t col)
     return col < v.width ? col : -1;
 }
 
+// The far side of a layer's outputs, which need not fill its last stack.  The one stack that differs and
+// its missing columns travel in eight bytes of the one view that needs them: read through gridDim, or with a
+// tail in every view, they sat behind the second 128 bytes of the kernel arguments, a cache line of
+// its own that each workgroup waited for in front of its first row (fast4_fw_kernel of 16384 rows of 4
+// stacks of 256: 23.6 against 23.3 us).
+struct StackView : View {
+    int last;   // the stack that is cut short, -1: none
+    int cut;    // columns it lacks
+};
+
 // The view as the workgroups of one stack use it.
-__device__ __forceinline__ View stack_view(View v, int stack, int nstacks)
+__device__ __forceinline__ View stack_view(const StackView &v, int stack)
 {
-    if (stack == nstacks - 1) v.width = v.tail;
-    return v;
+    View w = v;
+    if (stack == v.last) w.width -= v.cut;
+    return w;
 }
 
 }  // namespace bf

@@ -533,7 +533,7 @@ struct FastFwArgs {
     const void *in;
     View in_view;
     void *out;
-    View out_view;
+    StackView out_view;
     int64_t batch;
     int64_t ngroups;           // ceil(batch / SLOTS)
     int64_t groups_per_wg;
@@ -835,7 +835,7 @@ __global__ __launch_bounds__(kFastThreads, WAVES) void fast_fw_kernel(FastFwArgs
     const __amdgpu_buffer_rsrc_t out_rs =
         make_rsrc(reinterpret_cast<char *>(a.out) + (g0 * SLOTS * a.out_view.sb + stack * a.out_view.ss) * out_eb);
     // thread-constant part of the offsets; the row group adds a wave-uniform part
-    const View out_view = stack_view(a.out_view, stack, gridDim.y);
+    const View out_view = stack_view(a.out_view, stack);
     const int64_t in_col = view_col(a.in_view, col_in), out_col = view_col(out_view, col);
     const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.in_view.se * in_eb) : kOob;
     const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.out_view.se * out_eb) : kOob;
@@ -958,7 +958,7 @@ struct FastBwArgs {
     const void *x_in;
     View x_view;
     const void *g_out;
-    View g_view;
+    StackView g_view;
     void *g_in;
     View gi_view;
     void *partial;             // (gridDim.x, S, NS, partial_slot)
@@ -1237,7 +1237,7 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
 
     // --- operand fetch, register flavour: thread t holds its layout-A element
     const __amdgpu_buffer_rsrc_t x_rs = make_rsrc(x_base), g_rs = make_rsrc(g_base);
-    const View g_view = stack_view(a.g_view, stack, gridDim.y);
+    const View g_view = stack_view(a.g_view, stack);
     const int64_t x_col = view_col(a.x_view, col), g_col = view_col(g_view, col_out);
     const int x_thr = x_col >= 0 ? c.slot * x_row + (int)(x_col * a.x_view.se * x_eb) : kOob;
     const int g_thr = g_col >= 0 ? c.slot * g_row + (int)(g_col * a.g_view.se * g_eb) : kOob;

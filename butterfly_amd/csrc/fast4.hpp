@@ -125,14 +125,13 @@ struct Fast4Args {
     const float *x_in;
     View x_view;
     float *x_out;              // forward output
-    View xo_view;
+    StackView xo_view;
     const float *g_out;        // backward
-    View g_view;
+    StackView g_view;
     float *g_in;
     View gi_view;
     float *partial;            // (gridDim.x, S, L/2, 4 n)
     int64_t batch;
-    int nstacks;
     int64_t ngroups;
     int64_t groups_per_wg;
 };
@@ -199,7 +198,7 @@ __global__ __launch_bounds__(kFastThreads) void fast4_fw_kernel(Fast4Args a)
     const __amdgpu_buffer_rsrc_t out_rs = make_rsrc(a.x_out + g0 * SLOTS * a.xo_view.sb + stack * a.xo_view.ss);
     const int in_row = (int)(a.x_view.sb * 4), out_row = (int)(a.xo_view.sb * 4);
     const int64_t in_col = view_col(a.x_view, c.eA);
-    const int64_t out_col = view_col(stack_view(a.xo_view, stack, a.nstacks), c.eA);
+    const int64_t out_col = view_col(stack_view(a.xo_view, stack), c.eA);
     const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.x_view.se * 4) : kOob;
     const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.xo_view.se * 4) : kOob;
 
@@ -291,7 +290,7 @@ __global__ __launch_bounds__(kFastThreads) void fast4_bw_kernel(Fast4Args a)
     const __amdgpu_buffer_rsrc_t gi_rs = make_rsrc(a.g_in + g0 * SLOTS * a.gi_view.sb + stack * a.gi_view.ss);
     const int x_row = (int)(a.x_view.sb * 4), g_row = (int)(a.g_view.sb * 4), gi_row = (int)(a.gi_view.sb * 4);
     const int64_t x_col = view_col(a.x_view, c.eA), gi_col = view_col(a.gi_view, c.eA);
-    const int64_t g_col = view_col(stack_view(a.g_view, stack, a.nstacks), c.eA);
+    const int64_t g_col = view_col(stack_view(a.g_view, stack), c.eA);
     const int x_thr = x_col >= 0 ? c.slot * x_row + (int)(x_col * a.x_view.se * 4) : kOob;
     const int g_thr = g_col >= 0 ? c.slot * g_row + (int)(g_col * a.g_view.se * 4) : kOob;
     const int gi_thr = gi_col >= 0 ? c.slot * gi_row + (int)(gi_col * a.gi_view.se * 4) : kOob;

@@ -59,9 +59,9 @@ struct Fast4GArgs {
     const void *x_in;
     View x_view;
     void *x_out;               // forward output
-    View xo_view;
+    StackView xo_view;
     const void *g_out;         // backward
-    View g_view;
+    StackView g_view;
     void *g_in;
     View gi_view;
     void *partial;             // (gridDim.x, S, NS, 4 n) scalars
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_fw_kernel(Fast4GArgs a)
         make_rsrc(reinterpret_cast<T *>(a.x_out) + g0 * SLOTS * a.xo_view.sb + stack * a.xo_view.ss);
     const int in_row = (int)(a.x_view.sb * EB), out_row = (int)(a.xo_view.sb * EB);
     const int64_t in_col = view_col(a.x_view, col);
-    const int64_t out_col = view_col(stack_view(a.xo_view, stack, gridDim.y), col);
+    const int64_t out_col = view_col(stack_view(a.xo_view, stack), col);
     const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.x_view.se * EB) : kOob;
     const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.xo_view.se * EB) : kOob;
 
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_bw_kernel(Fast4GArgs a)
         make_rsrc(reinterpret_cast<T *>(a.g_in) + g0 * SLOTS * a.gi_view.sb + stack * a.gi_view.ss);
     const int x_row = (int)(a.x_view.sb * EB), g_row = (int)(a.g_view.sb * EB), gi_row = (int)(a.gi_view.sb * EB);
     const int64_t x_col = view_col(a.x_view, col), gi_col = view_col(a.gi_view, col);
-    const int64_t g_col = view_col(stack_view(a.g_view, stack, gridDim.y), col);
+    const int64_t g_col = view_col(stack_view(a.g_view, stack), col);
     const int x_thr = x_col >= 0 ? c.slot * x_row + (int)(x_col * a.x_view.se * EB) : kOob;
     const int g_thr = g_col >= 0 ? c.slot * g_row + (int)(g_col * a.g_view.se * EB) : kOob;
     const int gi_thr = gi_col >= 0 ? c.slot * gi_row + (int)(gi_col * a.gi_view.se * EB) : kOob;

@@ -20,7 +20,7 @@ struct GenericFwArgs {
     const void *in;
     View in_view;
     void *out;
-    View out_view;
+    StackView out_view;
 };
 
 // One 2x2 stage on R rows held in LDS at buf[r * n + j].
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kGenericThreads) void generic_fw_kernel(GenericFwAr
     T *out = reinterpret_cast<T *>(a.out);
     for (int it = tid; it < (rows << log_n); it += kGenericThreads) {
         const int r = it >> log_n, j = it & (n - 1);
-        const int64_t jc = view_col(stack_view(a.out_view, s, gridDim.y), j);
+        const int64_t jc = view_col(stack_view(a.out_view, s), j);
         if (jc >= 0) out[(b0 + r) * a.out_view.sb + s * a.out_view.ss + jc * a.out_view.se] = buf[it];
     }
 }
@@ -123,7 +123,7 @@ struct GenericBwArgs {
     const void *x_in;      // input of stage t0
     View x_view;
     const void *g_out;     // gradient w.r.t. the output of stage t1 - 1
-    View g_view;
+    StackView g_view;
     void *g_in;            // gradient w.r.t. the input of stage t0
     View gi_view;          // columns in [n, width) are zero-filled
     void *partial;         // (gridDim.x, S, t1 - t0, slot) per-workgroup d_twiddle sums
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kGenericThreads) void generic_bw_kernel(GenericBwAr
     for (int64_t b = blockIdx.x; b < a.batch; b += gridDim.x) {
         for (int j = tid; j < n; j += kGenericThreads) {
             T v = zero_of(T()), gv = zero_of(T());
-            const int64_t xc = view_col(a.x_view, j), gc = view_col(stack_view(a.g_view, s, gridDim.y), j);
+            const int64_t xc = view_col(a.x_view, j), gc = view_col(stack_view(a.g_view, s), j);
             if (xc >= 0) v = x_in[b * a.x_view.sb + s * a.x_view.ss + xc * a.x_view.se];
             if (gc >= 0) gv = g_out[b * a.g_view.sb + s * a.g_view.ss + gc * a.g_view.se];
             xs[j] = v;

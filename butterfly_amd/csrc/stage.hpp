@@ -26,9 +26,9 @@ struct StageArgs {
     const void *x_in;
     View x_view;
     void *x_out;               // forward
-    View xo_view;
+    StackView xo_view;
     const void *g_out;         // backward
-    View g_view;
+    StackView g_view;
     void *g_in;
     View gi_view;
     void *partial;             // (gridDim.x, S, slot) scalars
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kStageThreads) void stage_fw_kernel(StageArgs a)
     stage_columns<RADIX>(q, a.log_stride, col);
 #pragma unroll
     for (int c = 0; c < RADIX; ++c) {
-        const int64_t ic = view_col(a.x_view, col[c]), oc = view_col(stack_view(a.xo_view, stack, gridDim.y), col[c]);
+        const int64_t ic = view_col(a.x_view, col[c]), oc = view_col(stack_view(a.xo_view, stack), col[c]);
         in_off[c] = ic >= 0 ? ic * a.x_view.se : -1;
         out_off[c] = oc >= 0 ? oc * a.xo_view.se : -1;
     }
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kStageThreads) void stage_bw_kernel(StageArgs a)
     stage_columns<RADIX>(q, a.log_stride, col);
 #pragma unroll
     for (int c = 0; c < RADIX; ++c) {
-        const int64_t xc = view_col(a.x_view, col[c]), gc = view_col(stack_view(a.g_view, stack, gridDim.y), col[c]), ic = view_col(a.gi_view, col[c]);
+        const int64_t xc = view_col(a.x_view, col[c]), gc = view_col(stack_view(a.g_view, stack), col[c]), ic = view_col(a.gi_view, col[c]);
         x_off[c] = xc >= 0 ? xc * a.x_view.se : -1;
         g_off[c] = gc >= 0 ? gc * a.g_view.se : -1;
         gi_off[c] = ic >= 0 ? ic * a.gi_view.se : -1;

@@ -66,7 +66,7 @@ struct StreamArgs {
     const void *in;
     View in_view;
     void *out;
-    View out_view;
+    StackView out_view;
     const void *bias;         // NULL, or the columns of all stacks side by side
     void *save[kStreamMaxSaves];   // dense (B, S, n) planes
     int64_t batch;
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(W * 64, W == 16 ? 4 : 2) void stream_fw_kernel(Stre
     const int hi_rows = 1 << (NBITS - L);              // row groups (of four) in a plane
     const int64_t row0 = (int64_t)blockIdx.x * (4 * RB * hi_rows);
     const int rows_valid = (int)(a.batch - row0 < 4 * RB * hi_rows ? a.batch - row0 : 4 * RB * hi_rows);
-    const View in_view = a.in_view, out_view = stack_view(a.out_view, stack, gridDim.y);
+    const View in_view = a.in_view, out_view = stack_view(a.out_view, stack);
     const T *in = reinterpret_cast<const T *>(a.in) + row0 * in_view.sb + stack * in_view.ss;
     T *out = reinterpret_cast<T *>(a.out) + row0 * out_view.sb + stack * out_view.ss;
     const __amdgpu_buffer_rsrc_t in_rs = make_rsrc(in), out_rs = make_rsrc(out);

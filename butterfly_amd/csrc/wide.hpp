@@ -123,7 +123,7 @@ __global__ __launch_bounds__(kFastThreads) void wide_fw_kernel(FastFwArgs a)
     const __amdgpu_buffer_rsrc_t out_rs =
         make_rsrc(reinterpret_cast<T *>(a.out) + r0 * a.out_view.sb + stack * a.out_view.ss);
     const int in_row = (int)(a.in_view.sb * EB), out_row = (int)(a.out_view.sb * EB);
-    const View out_view = stack_view(a.out_view, stack, gridDim.y);
+    const View out_view = stack_view(a.out_view, stack);
     int in_thr[Q], out_thr[Q], in_dma[Q];
     T bias[Q];
 #pragma unroll
