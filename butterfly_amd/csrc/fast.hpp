@@ -965,8 +965,8 @@ struct FastBwArgs {
     int64_t batch;
     int64_t ngroups;
     int64_t groups_per_wg;
-    // float kernels on 1024-element rows or chunks only: when set, the column sums of g_out over
-    // this workgroup's rows (a layer's bias gradient) go to (gridDim.x, S, bias_stride)
+    // float kernels only: when set, the column sums of g_out over this workgroup's rows (a layer's
+    // bias gradient) go to (gridDim.x, S, bias_stride)
     void *bias_partial;
     int64_t bias_stride;
     int x_real, g_real;        // complex64: x (and its gradient) / the output gradient are real numbers
@@ -1177,7 +1177,7 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
     __shared__ T lds_ta[NTA > 0 ? NTA * kFastThreads : 1];
     // row slots: 4 sets of R for x, then 4 sets of R for the output gradient
     __shared__ float lds_rows[DIRECT ? 8 * R * kFastRowWords : 1];
-    __shared__ float lds_bias[(DIRECT && SLOTS == 1) ? kFastThreads : 1];
+    __shared__ float lds_bias[DIRECT ? kFastThreads : 1];
     const int t = threadIdx.x;
     const int stack = blockIdx.y;
     const int chunk = blockIdx.z;
@@ -1268,7 +1268,7 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
     // Column sum of the output gradient (see FastBwArgs::bias_partial): the thread adds the
     // element it reads at the top of every reverse sweep, into a private LDS word (a register
     // held across the row loop is one too many for the two-block schedules).
-    constexpr bool BIAS_SUM = DIRECT && SLOTS == 1;
+    constexpr bool BIAS_SUM = DIRECT;
     const bool bias_on = BIAS_SUM && a.bias_partial != nullptr;
     if constexpr (BIAS_SUM) lds_bias[t] = 0.0f;
     auto fetch_x = [&](int j, bool full = false) {
@@ -1617,7 +1617,7 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
 #pragma unroll
         for (int r = 0; r < R; ++r) store_grad(R * flush_it + r, done[r]);
     }
-    if constexpr (BIAS_SUM) {
+    if constexpr (BIAS_SUM && SLOTS == 1) {
         if (bias_on) {
             const int64_t bcol = P::column(chunk, Q::SB ? c2.eB : c2.eA, a.low_bits);
             if (bcol < a.g_view.width)
@@ -1682,6 +1682,21 @@ __global__ __launch_bounds__(kFastThreads) void fast_bw_kernel(FastBwArgs a)
         // (the factor slots in LDS are dead by now and serve as the staging area)
         __shared__ T red_own[TB_LDS ? 1 : 2 * 1024];
         T *red = TB_LDS ? lds_tb : red_own;
+        if constexpr (BIAS_SUM) {
+            // the slots' column sums, in ascending order too
+            if (bias_on) {
+                __syncthreads();
+                red[c2.slot * n + (Q::SB ? c2.eB : c2.eA)] = lds_bias[t2];
+                __syncthreads();
+                if (t2 < n && t2 < a.g_view.width) {
+                    T sum = red[t2];
+#pragma unroll 4
+                    for (int sl = 1; sl < SLOTS; ++sl) sum = add(sum, red[sl * n + t2]);
+                    reinterpret_cast<float *>(a.bias_partial)[((int64_t)blockIdx.x * gridDim.y + stack) * a.bias_stride +
+                                                              t2] = sum;
+                }
+            }
+        }
         static_for<0, NS>([&](auto S) {
             constexpr int s = S;
             constexpr int bit = P::bit(s);

@@ -643,6 +643,18 @@ def test_bias_folded_into_forward_and_bias_gradient(case):
     assert rel_err(db4.cpu().numpy(), db_ref) < BW_TOL
 
 
+@pytest.mark.parametrize("case", [
+    # several rows a workgroup (512 down to one), rows missing from the last group, columns missing, one
+    # and two row groups in flight, rows that start their sweep in either layout
+    (np.float32, 1, 1, 1, 1, None, None, True), (np.float32, 1025, 2, 3, 2, None, 5, False),
+    (np.float32, 37, 3, 5, 1, 20, 31, True), (np.float32, 4099, 1, 6, 2, None, None, False),
+    (np.float32, 33001, 1, 7, 1, None, 101, True), (np.float32, 301, 4, 8, 2, 200, 130, True),
+    (np.float32, 8301, 1, 9, 1, 400, 500, False), (np.float32, 511, 2, 9, 2, None, None, True)],
+    ids=lambda c: f"B{c[1]}-S{c[2]}-L{c[3]}-nb{c[4]}-I{c[5]}-O{c[6]}-inc{int(c[7])}")
+def test_bias_gradient_formed_on_short_rows(case):
+    test_bias_folded_into_forward_and_bias_gradient(case)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.complex64], ids=["f32", "c64"])
 @pytest.mark.parametrize("B, S, width", [(1, 1, 1), (15, 1, 3), (16, 2, 64), (17, 3, 65), (257, 1, 63), (4099, 2, 30),
                                          (5000, 1, 1001)])
