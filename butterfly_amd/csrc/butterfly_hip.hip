@@ -850,11 +850,34 @@ int64_t pass4_slices(const bf_problem *p, const Pass4 &q)
     return stage_grid(p, stage_info(make_schedule(p, true), q.t0).radix4 ? 4 : 2).nparts;
 }
 
+int64_t bias_stride(const bf_problem *p) { return (p->output_size + 3) & ~(int64_t)3; }
+
+// What a backward call that also returns the bias gradient carries: the area for the partial
+// column sums, where the result goes, and -- once they have been formed -- the number of slices.
+struct BiasGrad {
+    void *area = nullptr;
+    void *d_bias = nullptr;
+    int64_t nparts = 0;
+    bool formed = false;
+};
+
+// Has the backward kernel that reads the output gradient form the column sums (float kernels).
+template <typename Args>
+void form_bias_sums_in(Args &a, const bf_problem *p, int64_t nwg, BiasGrad *bg)
+{
+    if (!bg || p->dtype != BF_F32 || nwg > num_cu()) return;
+    a.bias_partial = static_cast<decltype(a.bias_partial)>(bg->area);
+    a.bias_stride = bias_stride(p);
+    bg->nparts = nwg;
+    bg->formed = true;
+}
+
 // One pass forward (backward == false: x_in -> x_out) or backward (x_in, g_out -> g_in and the
 // pass's partial slices; *nparts receives their number per stage).
 int run_pass4(const bf_problem *p, const Schedule &sc, const Pass4 &q, bool backward, const void *tw2, const void *tw4,
               const void *x_in, const StackView &x_view, void *x_out, const StackView &xo_view, const void *g_out,
-              const StackView &g_view, void *g_in, const StackView &gi_view, void *partial, int64_t *nparts, hipStream_t stream)
+              const StackView &g_view, void *g_in, const StackView &gi_view, void *partial, int64_t *nparts, hipStream_t stream,
+              BiasGrad *bg = nullptr)
 {
     const int64_t n = (int64_t)1 << p->log_n;
     const int L = (int)p->log_n;
@@ -882,6 +905,7 @@ int run_pass4(const bf_problem *p, const Schedule &sc, const Pass4 &q, bool back
         a.ngroups = g.ngroups;
         a.groups_per_wg = g.groups_per_wg;
         if (nparts) *nparts = g.nwg;
+        form_bias_sums_in(a, p, g.nwg, bg);
         return launch_fast4g(cplx, q.LC, q.inc, backward, a,
                              dim3((unsigned)g.nwg, (unsigned)p->nstacks, (unsigned)(n >> q.LC)), stream);
     }
@@ -1193,8 +1217,6 @@ struct BiasGradPlan {
     size_t bytes;
 };
 
-int64_t bias_stride(const bf_problem *p) { return (p->output_size + 3) & ~(int64_t)3; }
-
 BiasGradPlan plan_bias_grad(const bf_problem *p)
 {
     BiasGradPlan b = {};
@@ -1207,15 +1229,6 @@ BiasGradPlan plan_bias_grad(const bf_problem *p)
     b.bytes = align256((size_t)b.nparts * p->nstacks * bias_stride(p) * elem_bytes(p->dtype));
     return b;
 }
-
-// What a backward call that also returns the bias gradient carries: the area for the partial
-// column sums, where the result goes, and -- once they have been formed -- the number of slices.
-struct BiasGrad {
-    void *area = nullptr;
-    void *d_bias = nullptr;
-    int64_t nparts = 0;
-    bool formed = false;
-};
 
 // First step of the bias gradient as a kernel of its own, for backward kernels that do not form
 // the column sums on the way.
@@ -1532,6 +1545,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             a.partial = partials();
             a.ngroups = g.ngroups;
             a.groups_per_wg = g.groups_per_wg;
+            if (k == P - 1) form_bias_sums_in(a, p, g.nwg, bg);
             const bool inc = (p->increasing_stride != 0) != ((k & 1) != 0);
             rc = launch_fast4g(p->dtype == BF_C64, L, inc, true, a, dim3((unsigned)g.nwg, (unsigned)p->nstacks), stream);
             if (rc) return rc;
@@ -1554,6 +1568,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             a.batch = p->batch;
             a.ngroups = g.ngroups;
             a.groups_per_wg = g.groups_per_wg;
+            if (k == P - 1) form_bias_sums_in(a, p, g.nwg, bg);
             const bool inc = (p->increasing_stride != 0) != ((k & 1) != 0);
             rc = launch_fast4(L, inc, true, a, dim3((unsigned)g.nwg, (unsigned)p->nstacks), stream);
             if (rc) return rc;
@@ -1609,7 +1624,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             rc = run_pass4(p, sc, q, true, tw2, tw4, k == 0 ? input : boundary(k), k == 0 ? x_view : dense, nullptr,
                            dense, k == P - 1 ? grad : ws + pl.off_gbuf, k == P - 1 ? g_view : dense,
                            k == 0 ? d_input : ws + pl.off_gbuf, k == 0 ? dn_view : dense, partials(), &nparts,
-                           stream);
+                           stream, k == P - 1 ? bg : nullptr);
             if (rc) return rc;
             rc = reduce(q.t0, q.t1, nparts);
             if (rc) return rc;
@@ -1671,12 +1686,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 a.g_real = k == P - 1 && (real & kRealOut);
                 // (a launch of its own read the gradient once more for rows below 1024: Butterfly(512, 512) at
                 // 32768 rows 87 us a step against 76, Butterfly(256, 1000), two blocks, at 30001 rows 247 against 224)
-                if (k == P - 1 && bg && p->dtype == BF_F32 && g.nwg <= num_cu()) {
-                    a.bias_partial = bg->area;
-                    a.bias_stride = bias_stride(p);
-                    bg->nparts = g.nwg;
-                    bg->formed = true;
-                }
+                if (k == P - 1) form_bias_sums_in(a, p, g.nwg, bg);
                 const dim3 grid((unsigned)g.nwg, (unsigned)p->nstacks, (unsigned)pass_lanes(p, q));
                 // two row groups in flight once a workgroup has enough of them to fill the pipeline
                 if (q.span) {

@@ -134,6 +134,8 @@ struct Fast4Args {
     int64_t batch;
     int64_t ngroups;
     int64_t groups_per_wg;
+    float *bias_partial;       // backward: as in Fast4GArgs
+    int64_t bias_stride;
 };
 
 template <int L, bool INC, bool WITH_COLUMN>
@@ -279,6 +281,7 @@ __global__ __launch_bounds__(kFastThreads) void fast4_bw_kernel(Fast4Args a)
 #pragma unroll
         for (int m = 0; m < 4; ++m) acc[S][m] = 0.0f;
     });
+    float bias_sum = 0.0f;   // column sum of the output gradient (always formed: one add a row)
 
     const int64_t g0 = (int64_t)blockIdx.x * a.groups_per_wg;
     const int64_t g1 = g0 + a.groups_per_wg < a.ngroups ? g0 + a.groups_per_wg : a.ngroups;
@@ -327,6 +330,7 @@ __global__ __launch_bounds__(kFastThreads) void fast4_bw_kernel(Fast4Args a)
         for (int r = 0; r < R; ++r) {
             v[r] = nx[r];
             gv[r] = ngr[r];
+            bias_sum += gv[r];
         }
         load_rows(grel + R, nx, ngr, full);
         float act[NS][R];
@@ -394,6 +398,20 @@ __global__ __launch_bounds__(kFastThreads) void fast4_bw_kernel(Fast4Args a)
     const FastCoords c2 = fast_coords<L>(t2);
     float *part = a.partial + ((int64_t)blockIdx.x * gridDim.y + stack) * NS * (4 * n);
     __shared__ float red[SLOTS > 1 ? 4 * 1024 : 1];
+    if (a.bias_partial) {
+        float *dst = a.bias_partial + ((int64_t)blockIdx.x * gridDim.y + stack) * a.bias_stride;
+        if constexpr (SLOTS == 1) {
+            if (c2.eA < a.g_view.width) dst[c2.eA] = bias_sum;
+        } else {
+            red[c2.slot * n + c2.eA] = bias_sum;
+            __syncthreads();
+            if (t2 < n && t2 < a.g_view.width) {
+                float sum = red[t2];
+                for (int sl = 1; sl < SLOTS; ++sl) sum += red[sl * n + t2];
+                dst[t2] = sum;
+            }
+        }
+    }
     static_for<0, NS>([&](auto S) {
         constexpr int s = S;
         constexpr int b = P::bit(s);

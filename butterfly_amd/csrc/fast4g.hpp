@@ -68,6 +68,10 @@ struct Fast4GArgs {
     int64_t batch;
     int64_t ngroups;
     int64_t groups_per_wg;
+    // backward, float: when set, the column sums of g_out over this workgroup's rows (a layer's bias
+    // gradient) go to (gridDim.x, S, bias_stride)
+    void *bias_partial;
+    int64_t bias_stride;
 };
 
 template <typename T, int L, bool INC, bool WITH_COLUMN>
@@ -235,6 +239,9 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_bw_kernel(Fast4GArgs a)
         for (int m = 0; m < 4; ++m) acc[S][m] = zero_of(T());
     });
     T self2 = zero_of(T()), cross2 = zero_of(T());   // 2x2 stage: dT[r][r], dT[1 - r][r]
+    // Column sum of the output gradient.  Always formed: one add a row against a choice in the row loop.
+    constexpr bool BIAS_SUM = EB == 4;
+    float bias_sum = 0.0f;
 
     const int64_t g0 = (int64_t)blockIdx.x * a.groups_per_wg;
     const int64_t g1 = g0 + a.groups_per_wg < a.ngroups ? g0 + a.groups_per_wg : a.ngroups;
@@ -287,6 +294,7 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_bw_kernel(Fast4GArgs a)
         for (int r = 0; r < R; ++r) {
             v[r] = nx[r];
             gv[r] = ngr[r];
+            if constexpr (BIAS_SUM) bias_sum += gv[r];
         }
         load_rows(grel + R, nx, ngr, full);
         T act[NS][R];
@@ -346,6 +354,26 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_bw_kernel(Fast4GArgs a)
     int t2 = t;
     asm volatile("" : "+v"(t2));   // (recompute the coordinates instead of keeping them alive)
     const FastCoords c2 = fast_coords<L>(t2);
+    if constexpr (BIAS_SUM) {
+        if (a.bias_partial) {
+            float *dst = reinterpret_cast<float *>(a.bias_partial) +
+                         ((int64_t)blockIdx.x * gridDim.y + stack) * a.bias_stride + (chunk << L);
+            const int64_t width = a.g_view.width - (chunk << L);
+            if constexpr (SLOTS == 1) {
+                if (c2.eA < width) dst[c2.eA] = bias_sum;
+            } else {
+                __syncthreads();
+                lds[c2.slot * n + c2.eA] = bias_sum;
+                __syncthreads();
+                if (t2 < n && t2 < width) {
+                    float sum = lds[t2];
+#pragma unroll 4
+                    for (int sl = 1; sl < SLOTS; ++sl) sum += lds[sl * n + t2];
+                    dst[t2] = sum;
+                }
+            }
+        }
+    }
     const int64_t slot = 4 * a.n_full;   // scalars per stage in a partial slice
     T *part = reinterpret_cast<T *>(a.partial) + ((int64_t)blockIdx.x * gridDim.y + stack) * NS * slot;
     static_for<0, NS>([&](auto S) {

@@ -346,3 +346,23 @@ def test_whole_stacks_fill_a_contiguous_tensor(n, out_size, contiguous):
     host = butterfly_amd.Butterfly(n, out_size)
     host.load_state_dict(layer.state_dict())
     assert rel_err(y.detach().cpu().numpy(), host(x.cpu()).detach().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("in_size, out_size, batch, nblocks, increasing", [
+    # even numbers of stages: several rows a workgroup, one; odd ones; rows cut into chunks (the chunk
+    # pass or a single stage last); columns missing from the last stack
+    (4, 3, 1, 1, True), (16, 45, 1030, 2, False), (256, 256, 517, 1, True), (256, 1000, 301, 2, False),
+    (1000, 1001, 37, 1, True), (8, 8, 2050, 1, True), (500, 300, 1027, 2, True), (512, 1025, 5, 1, False),
+    (2000, 2048, 33, 2, True), (2048, 2000, 67, 1, False), (2048, 2048, 9, 1, True), (4096, 4090, 19, 2, True)])
+def test_base4_bias_gradient_formed_in_the_backward_kernels(in_size, out_size, batch, nblocks, increasing):
+    """d_bias of base-4 layers against the column sums in double precision; twice the same bits."""
+    import butterfly_amd
+    say("base-4 bias gradient", in_size, out_size, batch, nblocks, increasing)
+    torch.manual_seed(in_size + out_size)
+    layer = butterfly_amd.ButterflyBase4(in_size, out_size, nblocks=nblocks, increasing_stride=increasing).cuda()
+    x, g = torch.randn(batch, in_size, device="cuda"), torch.randn(batch, out_size, device="cuda")
+    db, again = (torch.autograd.grad(layer(x), layer.bias, g)[0] for _ in range(2))
+    ref = g.double().sum(0)
+    # (sums of `batch` unit normals: a few roundings of their partial sums, at most 33 deep per level)
+    assert (db - ref).abs().max().item() < 1e-6 * max(1.0, batch ** 0.5) * 4
+    assert torch.equal(db, again)
