@@ -12,6 +12,9 @@ namespace bf {
 
 __device__ __forceinline__ float zero_of(float) { return 0.0f; }
 __device__ __forceinline__ float2 zero_of(float2) { return make_float2(0.0f, 0.0f); }
+// (what can be added to any value, zeros of either sign included, without changing it)
+__device__ __forceinline__ float neg_zero_of(float) { return -0.0f; }
+__device__ __forceinline__ float2 neg_zero_of(float2) { return make_float2(-0.0f, -0.0f); }
 
 __device__ __forceinline__ float conj_of(float a) { return a; }
 __device__ __forceinline__ float2 conj_of(float2 a) { return make_float2(a.x, -a.y); }

@@ -68,6 +68,7 @@ struct Fast4GArgs {
     int64_t batch;
     int64_t ngroups;
     int64_t groups_per_wg;
+    const void *bias;          // forward: NULL, or (S, xo_view.width) dense, added to every output row
     // backward, float: when set, the column sums of g_out over this workgroup's rows (a layer's bias
     // gradient) go to (gridDim.x, S, bias_stride)
     void *bias_partial;
@@ -150,7 +151,10 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_fw_kernel(Fast4GArgs a)
         make_rsrc(reinterpret_cast<T *>(a.x_out) + g0 * SLOTS * a.xo_view.sb + stack * a.xo_view.ss);
     const int in_row = (int)(a.x_view.sb * EB), out_row = (int)(a.xo_view.sb * EB);
     const int64_t in_col = view_col(a.x_view, col);
-    const int64_t out_col = view_col(stack_view(a.xo_view, stack), col);
+    const View xo_view = stack_view(a.xo_view, stack);
+    const int64_t out_col = view_col(xo_view, col);
+    const T bias = (a.bias && col < xo_view.width) ? reinterpret_cast<const T *>(a.bias)[stack * a.xo_view.width + col]
+                                                   : neg_zero_of(T());
     const int in_thr = in_col >= 0 ? c.slot * in_row + (int)(in_col * a.x_view.se * EB) : kOob;
     const int out_thr = out_col >= 0 ? c.slot * out_row + (int)(out_col * a.xo_view.se * EB) : kOob;
 
@@ -208,7 +212,7 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_fw_kernel(Fast4GArgs a)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const bool ok = (grel + r) * SLOTS + c.slot < rows_valid;
-            buf_store(out_rs, ok ? out_thr : kOob, (grel + r) * SLOTS * out_row, v[r]);
+            buf_store(out_rs, ok ? out_thr : kOob, (grel + r) * SLOTS * out_row, add(v[r], bias));
         }
     }
 }
@@ -239,7 +243,8 @@ __global__ __launch_bounds__(kFastThreads) void fast4g_bw_kernel(Fast4GArgs a)
         for (int m = 0; m < 4; ++m) acc[S][m] = zero_of(T());
     });
     T self2 = zero_of(T()), cross2 = zero_of(T());   // 2x2 stage: dT[r][r], dT[1 - r][r]
-    // Column sum of the output gradient.  Always formed: one add a row against a choice in the row loop.
+    // Column sum of the output gradient.  Always formed: one add a row against a choice in the row loop
+    // (and see fast4_bw_kernel; 32768 rows of 512, no bias: 98.4 us a step without it, 94.7 with).
     constexpr bool BIAS_SUM = EB == 4;
     float bias_sum = 0.0f;
 

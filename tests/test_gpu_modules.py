@@ -366,3 +366,25 @@ def test_base4_bias_gradient_formed_in_the_backward_kernels(in_size, out_size, b
     # (sums of `batch` unit normals: a few roundings of their partial sums, at most 33 deep per level)
     assert (db - ref).abs().max().item() < 1e-6 * max(1.0, batch ** 0.5) * 4
     assert torch.equal(db, again)
+
+
+@pytest.mark.parametrize("complex_", [False, True], ids=["f32", "c64"])
+@pytest.mark.parametrize("in_size, out_size, batch, nblocks, increasing", [
+    (4, 3, 1, 1, True), (16, 45, 1030, 2, False), (256, 1000, 301, 2, False), (1000, 1001, 37, 1, True),
+    (8, 8, 2050, 3, True), (500, 300, 1027, 2, True), (512, 1025, 5, 1, False), (2048, 2000, 67, 1, False)])
+def test_base4_bias_added_by_the_forward_kernels(in_size, out_size, batch, nblocks, increasing, complex_):
+    """One rounding of output + bias, as adding it afterwards gives, while recording and not."""
+    import butterfly_amd
+    say("base-4 bias", in_size, out_size, batch, nblocks, increasing, complex_)
+    torch.manual_seed(in_size + out_size)
+    layer = butterfly_amd.ButterflyBase4(in_size, out_size, nblocks=nblocks, increasing_stride=increasing,
+                                         complex=complex_).cuda()
+    x = torch.randn(batch, in_size, device="cuda", dtype=layer.bias.dtype)
+    bias = layer.bias
+    for record in (False, True):
+        with torch.set_grad_enabled(record):
+            y = layer(x)
+            layer.bias = None
+            plain = layer(x)
+            layer.bias = bias
+            assert torch.equal(y, plain + bias)
