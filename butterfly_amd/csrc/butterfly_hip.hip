@@ -619,7 +619,8 @@ int fast4_kind(const bf_problem *p, bool base4, bool backward)
     const int64_t n = (int64_t)1 << p->log_n;
     const size_t e = elem_bytes(p->dtype);
     const FastGrid g = fast_grid(p->batch, (int)p->log_n, p->nstacks, backward ? 1 : fast4_fw_rows(p), 1);
-    const int64_t rows = (g.groups_per_wg + kFast4FwRows + 2) * g.slots;
+    // (the row groups that the last iteration requests ahead, backward too)
+    const int64_t rows = (g.groups_per_wg + 2 * kFast4FwRows) * g.slots;
     const int64_t dense[3] = {p->nstacks * n, n, 1};
     if (!span_ok(p->input_stride, rows, n, e) || !span_ok(p->output_stride, rows, n, e) || !span_ok(dense, rows, n, e))
         return 0;

@@ -94,7 +94,8 @@ bool launch_span_t(bool cplx, bool backward, bool two_rows, const FastFwArgs *fw
 template <int L, bool INC>
 void launch_fast4_t(bool backward, const Fast4Args &a, dim3 grid, hipStream_t stream)
 {
-    // row groups per backward iteration: as many as the registers next to the factors allow
+    // row groups per backward iteration, which share its barriers: four fit the registers at any
+    // length, but two are faster at 1024 (16384 rows, two blocks: 179.5 us a step against 194.8)
     constexpr int RB = L <= 8 ? 4 : 2;
     if (backward) hipLaunchKernelGGL((fast4_bw_kernel<L, INC, RB>), grid, dim3(kFastThreads), 0, stream, a);
     else hipLaunchKernelGGL((fast4_fw_kernel<L, INC, kFast4FwRows>), grid, dim3(kFastThreads), 0, stream, a);
@@ -104,8 +105,9 @@ template <typename T, int L, bool INC>
 void launch_fast4g_t(bool backward, const Fast4GArgs &a, dim3 grid, hipStream_t stream)
 {
     constexpr int R = sizeof(T) == 4 ? kFast4FwRows : kFast4GFwRowsComplex;
-    // row groups per backward iteration: what the registers next to the factors allow
-    constexpr int RB = sizeof(T) == 4 ? (L <= 7 ? 4 : 2) : (L <= 6 ? 2 : 1);
+    // row groups per backward iteration: complex64 what the registers next to the factors allow, float
+    // what is faster (32768 rows of 512: 94.7 us a step with two, 88.0 with four)
+    constexpr int RB = sizeof(T) == 4 ? (L <= 9 ? 4 : 2) : (L <= 6 ? 2 : 1);
     if (backward) hipLaunchKernelGGL((fast4g_bw_kernel<T, L, INC, RB>), grid, dim3(kFastThreads), 0, stream, a);
     else hipLaunchKernelGGL((fast4g_fw_kernel<T, L, INC, R>), grid, dim3(kFastThreads), 0, stream, a);
 }
