@@ -12,7 +12,8 @@
 // stage (a "level") is one v_mfma_f32_4x4x1_16b per column of its 4x4 factors: operand A is the factor
 // (lane = 4 * block + output), B the rows (lane = 4 * block + row), and the result comes back in the
 // layout of B, so levels chain without moving data.  The closing 2x2 stage of an odd number of bits
-// runs as a 4x4 matrix that leaves the other bit of its register pair alone.
+// runs pair by pair on the vector units: as a 4x4 matrix with zeros for the other bit of its register
+// pair, an infinity would reach the other pair's outputs as 0 * Inf.
 //
 // The factors are not kept from tile to tile: they stream from L2 while the previous level computes,
 // 4 * RB << (NBITS - log_n) rows sharing each read.  Register-resident factors (fast4g.hpp) reach 1024
@@ -22,6 +23,8 @@
 // it: one workgroup a compute unit at 4096 elements (128 KiB of LDS), whose loads, levels and stores
 // follow one another.
 #pragma once
+
+#include <type_traits>
 
 #include "fast.hpp"
 
@@ -139,6 +142,53 @@ __device__ __forceinline__ void stream_apply(const StreamRows<float2> &m, float2
     }
 }
 
+// The same for a 2x2 stage.  OWN, OTHER: register steps of the stage's bit and of the other bit of
+// the pair.  Lane i of a block holds the factor's row of output i & 1 at the value i >> 1 of the other
+// bit; the block's four lanes read them from each other as DPP operands, two instructions an output
+// (16384 rows of 2048, one block: 76.9 us against 82.2 for a 4x4 matrix on the matrix units).
+template <int QS, int OTHER, int OWN>
+__device__ __forceinline__ void stream_apply2(const StreamRows<float> &m, float (&v)[16])
+{
+    auto pair = [&](int q, auto other) {
+        constexpr int o = decltype(other)::value;
+        float &x0 = v[q * QS + o * OTHER], &x1 = v[q * QS + o * OTHER + OWN];
+        float y0 = mul(dpp_move<(2 * o) * 0x55>(m.a[q][0]), x0), y1 = mul(dpp_move<(2 * o + 1) * 0x55>(m.a[q][0]), x0);
+        y0 = mac(y0, dpp_move<(2 * o) * 0x55>(m.a[q][1]), x1);
+        y1 = mac(y1, dpp_move<(2 * o + 1) * 0x55>(m.a[q][1]), x1);
+        x0 = y0;
+        x1 = y1;
+    };
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        pair(q, std::integral_constant<int, 0>());
+        pair(q, std::integral_constant<int, 1>());
+    }
+}
+template <int QS, int OTHER, int OWN>
+__device__ __forceinline__ void stream_apply2(const StreamRows<float2> &m, float2 (&v)[16])
+{
+    auto pair = [&](int q, auto other) {
+        constexpr int o = decltype(other)::value;
+        float2 &x0 = v[q * QS + o * OTHER], &x1 = v[q * QS + o * OTHER + OWN];
+        auto row = [&](int k, auto own) {
+            constexpr int ctrl = (2 * o + decltype(own)::value) * 0x55;
+            return make_float2(dpp_move<ctrl>(m.re[q][k]), dpp_move<ctrl>(m.im[q][k]));
+        };
+        constexpr std::integral_constant<int, 0> first = {};
+        constexpr std::integral_constant<int, 1> second = {};
+        const float2 zero = zero_of(float2());
+        const float2 y0 = mac(mac(zero, row(0, first), x0), row(1, first), x1);
+        const float2 y1 = mac(mac(zero, row(0, second), x0), row(1, second), x1);
+        x0 = y0;
+        x1 = y1;
+    };
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        pair(q, std::integral_constant<int, 0>());
+        pair(q, std::integral_constant<int, 1>());
+    }
+}
+
 // Two scalars that are next to each other in memory: the row of a 2x2 factor.
 template <typename T> struct StreamPair { T x, y; };
 
@@ -183,8 +233,8 @@ __device__ __forceinline__ void stream_store4(__amdgpu_buffer_rsrc_t r, int voff
 }
 
 // The lane's row of the level's factors, as loaded: a row of the 4x4 factor, or (s1 alone) of the
-// 2x2 factor at the lane's own value of the other bit.  One for each setting q of the register bits
-// outside the level's pair.
+// 2x2 factor at a value of the other bit (stream_apply2).  One for each setting q of the register
+// bits outside the level's pair.
 template <typename T>
 struct StreamRaw { StreamPair<T> s1[4], s2[4]; };
 
@@ -196,26 +246,17 @@ __device__ __forceinline__ int stream_quad(int e, int p) { return ((e >> (p + 2)
 __device__ __forceinline__ void stream_put(StreamRows<float> &m, int q, int k, float v) { m.a[q][k] = v; }
 __device__ __forceinline__ void stream_put(StreamRows<float2> &m, int q, int k, float2 v) { m.re[q][k] = v.x; m.im[q][k] = v.y; }
 
-// KIND 0: a 4x4 factor; 1, 2: a 2x2 factor on the lower / upper bit of the pair, block-diagonal over
-// the other bit.
-template <typename T, int KIND>
-__device__ __forceinline__ void stream_rows(StreamRows<T> &m, const StreamRaw<T> &raw, int i)
+// The lane's row as loaded: of four entries, or (a 2x2 stage) of two.
+template <typename T, bool RADIX4>
+__device__ __forceinline__ void stream_rows(StreamRows<T> &m, const StreamRaw<T> &raw)
 {
-    const bool other = KIND == 1 ? (i >> 1) : (i & 1);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        if constexpr (KIND == 0) {
-            stream_put(m, q, 0, raw.s1[q].x);
-            stream_put(m, q, 1, raw.s1[q].y);
+        stream_put(m, q, 0, raw.s1[q].x);
+        stream_put(m, q, 1, raw.s1[q].y);
+        if constexpr (RADIX4) {
             stream_put(m, q, 2, raw.s2[q].x);
             stream_put(m, q, 3, raw.s2[q].y);
-        } else {
-            const T z = zero_of(T());
-            constexpr int own = KIND == 1 ? 1 : 2, oth = KIND == 1 ? 2 : 1;   // steps of the column number
-            stream_put(m, q, 0, other ? z : raw.s1[q].x);
-            stream_put(m, q, own, other ? z : raw.s1[q].y);
-            stream_put(m, q, oth, other ? raw.s1[q].x : z);
-            stream_put(m, q, 3, other ? raw.s1[q].y : z);
         }
     }
 }
@@ -271,9 +312,8 @@ __global__ __launch_bounds__(W * 64, W == 16 ? 4 : 2) void stream_fw_kernel(Stre
                 raw.s2[q] = stream_load2(tw4_rs, voff + 2 * EB, soff, T());
             }
         } else {
-            const int own = l.upper() ? i >> 1 : i & 1;
-            const int rest = l.upper() ? (i & 1) << (p - 1) : (i >> 1) << (p + 1);
-            const int voff = (stream_pair((e | rest) & emask, p) * 4 + own * 2) * EB;
+            const int rest = (i >> 1) << (l.upper() ? p - 1 : p + 1);
+            const int voff = (stream_pair((e | rest) & emask, p) * 4 + (i & 1) * 2) * EB;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 raw.s1[q] = stream_load2(tw2_rs, voff, (int)l.off + stream_pair((q << other) & emask, p) * 4 * EB, T());
@@ -338,18 +378,31 @@ __global__ __launch_bounds__(W * 64, W == 16 ? 4 : 2) void stream_fw_kernel(Stre
     for (int lv = 0; lv < a.nlevels; ++lv) {
         const StreamLevel l = a.level[lv];
         StreamRows<T> m;
-        if (l.radix4()) stream_rows<T, 0>(m, raw, lane & 3);
-        else if (!l.upper()) stream_rows<T, 1>(m, raw, lane & 3);
-        else stream_rows<T, 2>(m, raw, lane & 3);
+        if (l.radix4()) stream_rows<T, true>(m, raw);
+        else stream_rows<T, false>(m, raw);
         const int cur_base = idx_base, cur_lo = reg_lo;
         if (l.ends()) enter(l.ends() - 1);
         if (lv + 1 < a.nlevels) load_level(lv + 1);
-        if (l.pair()) {
+        if (l.radix4()) {
+            if (l.pair()) {
 #pragma unroll
-            for (int rb = 0; rb < RB; ++rb) stream_apply<1, 4>(m, v[rb]);
+                for (int rb = 0; rb < RB; ++rb) stream_apply<1, 4>(m, v[rb]);
+            } else {
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) stream_apply<4, 1>(m, v[rb]);
+            }
+        } else if (l.pair()) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                if (l.upper()) stream_apply2<1, 4, 8>(m, v[rb]);
+                else stream_apply2<1, 8, 4>(m, v[rb]);
+            }
         } else {
 #pragma unroll
-            for (int rb = 0; rb < RB; ++rb) stream_apply<4, 1>(m, v[rb]);
+            for (int rb = 0; rb < RB; ++rb) {
+                if (l.upper()) stream_apply2<4, 1, 2>(m, v[rb]);
+                else stream_apply2<4, 2, 1>(m, v[rb]);
+            }
         }
         if (l.save()) {
             // straight out of the registers: the plan saves where the lanes or the registers run over
