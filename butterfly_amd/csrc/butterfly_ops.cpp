@@ -547,10 +547,9 @@ using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
 struct MultiplyNode : public torch::autograd::Node {
-    SavedVariable twiddle, twiddle2, input, kept, in_scale, out_scale, scaled;
-    Tensor in_perm, out_index;
+    SavedVariable twiddle, twiddle2, input, kept, in_scale, out_scale, scaled, in_perm, out_index;
     bool base4 = false, increasing_stride = true, with_bias = false, layer = false, has_kept = false;
-    bool real_input = false, real_output = false, has_scaled = false;
+    bool real_input = false, real_output = false, has_scaled = false, has_in_perm = false, has_out_index = false;
     const char *who = nullptr;
 
     // edges: twiddle, twiddle2, input, bias, in_scale, out_scale (those that the call does not have lead nowhere)
@@ -564,8 +563,8 @@ struct MultiplyNode : public torch::autograd::Node {
         Operands o;
         o.twiddle = twiddle.unpack(self);
         if (base4) o.twiddle2 = twiddle2.unpack(self);
-        o.in_perm = in_perm;
-        o.out_index = out_index;
+        if (has_in_perm) o.in_perm = in_perm.unpack(self);
+        if (has_out_index) o.out_index = out_index.unpack(self);
         o.base4 = base4;
         o.increasing_stride = increasing_stride;
         o.real_input = real_input;
@@ -599,6 +598,8 @@ struct MultiplyNode : public torch::autograd::Node {
         in_scale.reset_data();
         out_scale.reset_data();
         scaled.reset_data();
+        in_perm.reset_data();
+        out_index.reset_data();
     }
 
     std::string name() const override { return base4 ? "ButterflyMultiplyBase4Backward" : "ButterflyMultiplyBackward"; }
@@ -645,8 +646,15 @@ Tensor differentiable(const Operands &o, const Tensor &input, bool layer, const 
     }
     node->real_input = o.real_input;
     node->real_output = o.real_output;
-    node->in_perm = o.in_perm;
-    node->out_index = o.out_index;
+    // (saved like the other operands: changed in place before the backward they raise)
+    if (o.in_perm.defined()) {
+        node->in_perm = SavedVariable(o.in_perm, false);
+        node->has_in_perm = true;
+    }
+    if (o.out_index.defined()) {
+        node->out_index = SavedVariable(o.out_index, false);
+        node->has_out_index = true;
+    }
     node->base4 = o.base4;
     node->increasing_stride = o.increasing_stride;
     node->with_bias = o.bias.defined();
