@@ -52,6 +52,22 @@ class Problem(ctypes.Structure):
     ]
 
 
+class Layer(ctypes.Structure):
+    _fields_ = [
+        ("problem", Problem),
+        ("base4", ctypes.c_int32),
+        ("shared_input", ctypes.c_int32),
+        ("real_input", ctypes.c_int32),
+        ("real_output", ctypes.c_int32),
+        ("total_output", ctypes.c_int64),
+        ("twiddle", ctypes.c_void_p),
+        ("twiddle2", ctypes.c_void_p),
+        ("bias", ctypes.c_void_p),
+        ("in_perm", ctypes.c_void_p),
+        ("out_index", ctypes.c_void_p),
+    ]
+
+
 _lib = None
 
 
@@ -104,6 +120,16 @@ def lib():
         L.bf_butterfly_multiply_base4_bw_saved_workspace_bytes.argtypes = [pp]
         L.bf_butterfly_multiply_base4_bw_saved_workspace_bytes.restype = sz
         L.bf_butterfly_multiply_base4_bw_saved.argtypes = [pp, vp, vp, vp, vp, vp, sz, vp, vp, vp, vp, sz, vp]
+        pl = ctypes.POINTER(Layer)
+        L.bf_layer_takes_real.argtypes = [pl]
+        L.bf_layer_kept_bytes.argtypes = [pl]
+        L.bf_layer_kept_bytes.restype = sz
+        L.bf_layer_fw_workspace_bytes.argtypes = [pl]
+        L.bf_layer_fw_workspace_bytes.restype = sz
+        L.bf_layer_fw.argtypes = [pl, vp, vp, vp, sz, vp, sz, vp]
+        L.bf_layer_bw_workspace_bytes.argtypes = [pl, ctypes.c_int, sz]
+        L.bf_layer_bw_workspace_bytes.restype = sz
+        L.bf_layer_bw.argtypes = [pl, vp, vp, vp, sz, vp, vp, vp, vp, vp, sz, vp]
         _lib = L
     return _lib
 

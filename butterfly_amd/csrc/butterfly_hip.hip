@@ -2336,6 +2336,7 @@ int bf_layer_bw(const bf_layer *l, const void *input, const void *grad, const vo
         return fail(BF_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", b.total, workspace_bytes);
     char *ws = static_cast<char *>(workspace);
     const bool sum = l->shared_input && p->nstacks > 1;
+    if (!d_input && !sum && p->batch > 0 && p->nstacks > 0 && p->input_size > 0) return fail(BF_ERR_INVALID, "d_input is NULL");
     bf_problem stacked = *p;
     void *d_stacks = d_input;
     if (sum) {
@@ -2350,7 +2351,7 @@ int bf_layer_bw(const bf_layer *l, const void *input, const void *grad, const vo
     rc = backward(&stacked, l->base4 != 0, l->base4 ? l->twiddle2 : l->twiddle, l->base4 ? l->twiddle : nullptr, input, grad,
                   l->base4 ? d_twiddle2 : d_twiddle, l->base4 ? d_twiddle : nullptr, d_stacks, workspace, b.off_bias, stream_,
                   d_bias ? &bg : nullptr, l->in_perm, l->out_index, b.kept ? kept : nullptr, layer_tail(l), layer_real(l));
-    if (rc || !sum || p->batch == 0 || p->input_size == 0) return rc;
+    if (rc || !sum || !d_input || p->batch == 0 || p->input_size == 0) return rc;
     SumStacksArgs a = {};
     a.in = d_stacks;
     a.out = d_input;

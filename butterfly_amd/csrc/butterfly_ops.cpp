@@ -330,7 +330,8 @@ void backward_call(Call &c, const Tensor &x, const Tensor &g, const Tensor &kept
     Tensor ws;
     if (ws_bytes > 0) ws = bytes_like(x, ws_bytes);
     check_rc(bf_layer_bw(&c.desc, x.data_ptr(), g.data_ptr(), kept_bytes > 0 ? kept.data_ptr() : nullptr, kept_bytes,
-                         d.twiddle.data_ptr(), c.desc.base4 ? d.twiddle2.data_ptr() : nullptr, d.input.data_ptr(),
+                         d.twiddle.data_ptr(), c.desc.base4 ? d.twiddle2.data_ptr() : nullptr,
+                         d.input.defined() ? d.input.data_ptr() : nullptr,
                          with_bias ? d.bias.data_ptr() : nullptr, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
                          current_stream()),
              who);
@@ -498,8 +499,10 @@ Tensor layer_fw(const Operands &o_, const Tensor &input, int64_t out_size, Tenso
     return real_output ? at::real(output).contiguous() : output;
 }
 
+// with_input: whether the input's gradient is wanted.  Where it is not, the sum over the stacks is left
+// out; the kernels of a single stack write it all the same.
 Gradients layer_bw(const Operands &o_, const Tensor &input, const Tensor &grad, const Tensor &kept, const Tensor &scaled,
-                   bool with_bias, const char *who)
+                   bool with_bias, bool with_input, const char *who)
 {
     Operands o = o_;
     TORCH_CHECK(o.real_output ? grad.scalar_type() == at::kFloat : grad.scalar_type() == o.twiddle.scalar_type(), who,
@@ -516,7 +519,7 @@ Gradients layer_bw(const Operands &o_, const Tensor &input, const Tensor &grad, 
         p.output_stride[2] = g.size(1) > 1 ? g.stride(1) : 0;
         p.output_stride[1] = p.output_size * p.output_stride[2];
         if (!takes_real(c, o) || (with_bias && o.real_output)) return false;
-        d.input = at::empty(input.sizes(), x.options());
+        if (with_input || p.nstacks == 1) d.input = at::empty(input.sizes(), x.options());
         backward_call(c, x, g, kept, with_bias, d, who);
         return true;
     };
@@ -526,7 +529,7 @@ Gradients layer_bw(const Operands &o_, const Tensor &input, const Tensor &grad, 
         if (o.real_output) g = as_complex(g);
         o.real_input = o.real_output = false;
         run();
-        if (real_input) d.input = at::real(d.input).contiguous();
+        if (real_input && d.input.defined()) d.input = at::real(d.input).contiguous();
     }
     if (scaled.defined()) {
         const Tensor d_scaled = d.twiddle;
@@ -576,9 +579,11 @@ struct MultiplyNode : public torch::autograd::Node {
             o.out_scale = out_scale.unpack(self);
             with = scaled.unpack(self);
         }
+        // (an input without gradient: every first layer; a frozen bias)
+        const bool want_input = task_should_compute_output(2), want_bias = with_bias && task_should_compute_output(3);
         at::AutoDispatchBelowADInplaceOrView below;
-        Gradients d = layer ? layer_bw(o, x, grads[0], planes, with, with_bias, who)
-                            : multiply_bw(o, x, grads[0], planes, with_bias, who);
+        Gradients d = layer ? layer_bw(o, x, grads[0], planes, with, want_bias, want_input, who)
+                            : multiply_bw(o, x, grads[0], planes, want_bias, who);
         out[0] = std::move(d.twiddle);
         out[1] = std::move(d.twiddle2);
         out[2] = std::move(d.input);

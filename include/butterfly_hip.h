@@ -277,7 +277,8 @@ int bf_layer_fw(const bf_layer *l, const void *input, void *output, void *kept, 
                 void *workspace, size_t workspace_bytes, void *stream);
 /* problem.output_stride are the strides of grad.  kept_bytes: size of the area behind `kept` (0 and
  * NULL: none); where the backward's plan does not fit what was kept, it is recomputed.  d_bias
- * (total_output entries) may be NULL.                                                            */
+ * (total_output entries) may be NULL, and so may d_input where several stacks share the input: their
+ * gradients are not added up then.                                                               */
 size_t bf_layer_bw_workspace_bytes(const bf_layer *l, int with_bias, size_t kept_bytes);
 int bf_layer_bw(const bf_layer *l, const void *input, const void *grad, const void *kept,
                 size_t kept_bytes, void *d_twiddle, void *d_twiddle2, void *d_input, void *d_bias,
