@@ -67,6 +67,12 @@ class FixedPermutation(nn.Module):
         return table
 
 
+def _observed(*modules):
+    """Whether a hook on one of these modules, or one on all modules, expects to see its calls."""
+    return nn.modules.module._has_any_global_hook() or any(
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+
+
 class FusedSequential(nn.Sequential):
     """nn.Sequential (same children, indexing and state) whose forward folds what stands
     directly around a Butterfly into that layer's own call: a FixedPermutation in front of or
@@ -76,7 +82,9 @@ class FusedSequential(nn.Sequential):
     reads / writes its rows, so none costs a pass of its own over the activations.  The accepted
     patterns are [FixedPermutation] [Real2Complex] [Diagonal] Butterfly [Diagonal]
     [FixedPermutation] [Complex2Real], with a permutation and a conversion in either order; any
-    other sequence of children runs one after the other as usual."""
+    other sequence of children runs one after the other as usual.  A conversion runs as a module where
+    a hook on it, on the layer (which would be handed real numbers) or on all modules is there to see
+    it; hooks on permutations and diagonals do not keep them from being folded."""
 
     def forward(self, input):
         from .butterfly import Butterfly, ButterflyBmm  # (butterfly.py does not import this module)
@@ -118,7 +126,8 @@ class FusedSequential(nn.Sequential):
                 if (isinstance(m, FixedPermutation) and back is None and layer.nstacks == 1
                         and self._permutes(m, layer.out_size)):
                     back = m
-                elif isinstance(m, Complex2Real) and to_real is None and layer.complex and plain:
+                elif (isinstance(m, Complex2Real) and to_real is None and layer.complex and plain
+                      and not _observed(m, layer)):
                     to_real = m
                 else:
                     break
@@ -144,7 +153,7 @@ class FusedSequential(nn.Sequential):
         """Whether the modules found in front of the layer can be folded into its call on `input`."""
         if to_complex is not None:
             # (the layer's float32 rows are read as they are; other real types are converted first)
-            if not layer.complex or input.dtype != torch.float32:
+            if not layer.complex or input.dtype != torch.float32 or _observed(to_complex, layer):
                 return False
         elif input.is_complex() != layer.complex:
             return False

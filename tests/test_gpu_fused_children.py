@@ -1,0 +1,61 @@
+"""What a FusedSequential must not fold away."""
+import pytest
+import torch
+from torch import nn
+
+from test_gpu_multiply import say
+
+pytestmark = pytest.mark.gpu
+
+
+def close(a, b):
+    return a.shape == b.shape and a.dtype == b.dtype and (a - b).norm().item() <= 1e-5 * b.norm().item()
+
+
+def chain(n=64):
+    """Real rows through a permutation, a diagonal and a complex layer and back."""
+    from butterfly_amd import Butterfly
+    from butterfly_amd.complex_utils import Complex2Real, Real2Complex
+    from butterfly_amd.diagonal import Diagonal
+    from butterfly_amd.permutation import FixedPermutation, FusedSequential
+    torch.manual_seed(n)
+    return FusedSequential(FixedPermutation(torch.randperm(n)), Real2Complex(), Diagonal(n, complex=True),
+                           Butterfly(n, n, bias=False, complex=True), Complex2Real(), FixedPermutation(torch.randperm(n))).cuda()
+
+
+@pytest.mark.parametrize("kind", ["forward", "forward_pre", "full_backward", "full_backward_pre", "global_forward",
+                                  "global_forward_pre"])
+@pytest.mark.parametrize("child", [1, 4], ids=["Real2Complex", "Complex2Real"])
+def test_hooks_of_conversions_fire(child, kind):
+    say("hooks", child, kind)
+    seq = chain()
+    x = torch.randn(7, 64, device="cuda")
+    y0 = seq(x)
+    calls = []
+    hook = lambda module, *args: calls.append(module) or None
+    if kind.startswith("global"):
+        handle = getattr(nn.modules.module, "register_module_" + kind[len("global_"):] + "_hook")(hook)
+    else:
+        handle = getattr(seq[child], f"register_{kind}_hook")(hook)
+    try:
+        a = x.clone().requires_grad_()
+        y = seq(a)
+        y.sum().backward()
+    finally:
+        handle.remove()
+    assert calls.count(seq[child]) == 1
+    assert close(y.detach(), y0.detach())
+    calls.clear()
+    assert torch.equal(seq(x), y0) and not calls
+
+
+def test_hooks_of_a_layer_see_complex_numbers():
+    """A hook on the layer between two conversions is handed what the layer takes and returns."""
+    seq = chain()
+    seen = []
+    handle = seq[3].register_forward_hook(lambda module, args, out: seen.append((args[0].dtype, out.dtype)) or 2 * out)
+    x = torch.randn(7, 64, device="cuda")
+    y = seq(x)
+    handle.remove()
+    assert seen == [(torch.complex64, torch.complex64)]
+    assert close(y, 2 * seq(x))
