@@ -73,6 +73,11 @@ def _observed(*modules):
         m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
 
 
+def _runs(m, kind):
+    """Whether module m computes what `kind` does (a subclass may have a forward of its own)."""
+    return isinstance(m, kind) and type(m).forward is kind.forward
+
+
 class FusedSequential(nn.Sequential):
     """nn.Sequential (same children, indexing and state) whose forward folds what stands
     directly around a Butterfly into that layer's own call: a FixedPermutation in front of or
@@ -87,7 +92,7 @@ class FusedSequential(nn.Sequential):
     it; hooks on permutations and diagonals do not keep them from being folded."""
 
     def forward(self, input):
-        from .butterfly import Butterfly, ButterflyBmm  # (butterfly.py does not import this module)
+        from .butterfly import Butterfly  # (butterfly.py does not import this module)
         mods = list(self._modules.values())
         if not input.is_cuda:
             for m in mods:
@@ -100,33 +105,32 @@ class FusedSequential(nn.Sequential):
             j = i
             while j < count and scale_in is None:
                 m = mods[j]
-                if isinstance(m, FixedPermutation) and front is None:
+                if _runs(m, FixedPermutation) and front is None:
                     front = m
-                elif isinstance(m, Real2Complex) and to_complex is None:
+                elif _runs(m, Real2Complex) and to_complex is None:
                     to_complex = m
-                elif isinstance(m, Diagonal):
+                elif _runs(m, Diagonal):
                     scale_in = m
                 else:
                     break
                 j += 1
             layer = mods[j] if j < count else None
-            if not (isinstance(layer, Butterfly) and not isinstance(layer, ButterflyBmm)
-                    and self._fits(layer, input, front, to_complex, scale_in)):
+            if not (_runs(layer, Butterfly) and self._fits(layer, input, front, to_complex, scale_in)):
                 input = mods[i](input)
                 i += 1
                 continue
             i = j + 1
             back = scale_out = to_real = None
             plain = layer.bias is None
-            if i < count and plain and isinstance(mods[i], Diagonal) and self._scales(mods[i], layer.out_size, layer):
+            if i < count and plain and _runs(mods[i], Diagonal) and self._scales(mods[i], layer.out_size, layer):
                 scale_out = mods[i]
                 i += 1
             while i < count:
                 m = mods[i]
-                if (isinstance(m, FixedPermutation) and back is None and layer.nstacks == 1
+                if (_runs(m, FixedPermutation) and back is None and layer.nstacks == 1
                         and self._permutes(m, layer.out_size)):
                     back = m
-                elif (isinstance(m, Complex2Real) and to_real is None and layer.complex and plain
+                elif (_runs(m, Complex2Real) and to_real is None and layer.complex and plain
                       and not _observed(m, layer)):
                     to_real = m
                 else:

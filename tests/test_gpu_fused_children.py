@@ -23,6 +23,18 @@ def chain(n=64):
                            Butterfly(n, n, bias=False, complex=True), Complex2Real(), FixedPermutation(torch.randperm(n))).cuda()
 
 
+def compare(fused, x):
+    """Outputs and every gradient against the children one after the other."""
+    plain = nn.Sequential(*fused)
+    a, b = (x.clone().requires_grad_() for _ in range(2))
+    y, z = fused(a), plain(b)
+    assert close(y, z)
+    g = torch.randn_like(z)
+    params = [p for p in fused.parameters()]
+    for u, v in zip(torch.autograd.grad(y, [a] + params, g), torch.autograd.grad(z, [b] + params, g)):
+        assert close(u, v)
+
+
 @pytest.mark.parametrize("kind", ["forward", "forward_pre", "full_backward", "full_backward_pre", "global_forward",
                                   "global_forward_pre"])
 @pytest.mark.parametrize("child", [1, 4], ids=["Real2Complex", "Complex2Real"])
@@ -59,3 +71,31 @@ def test_hooks_of_a_layer_see_complex_numbers():
     handle.remove()
     assert seen == [(torch.complex64, torch.complex64)]
     assert close(y, 2 * seq(x))
+
+
+@pytest.mark.parametrize("child", range(6))
+def test_children_with_a_forward_of_their_own(child):
+    """A subclass that overrides forward is run, whatever it derives from."""
+    say("override", child)
+    seq = chain()
+    base = type(seq[child])
+
+    class Doubled(base):
+        def forward(self, input):
+            return 2 * base.forward(self, input)
+
+    x = torch.randn(7, 64, device="cuda")
+    y = seq(x)
+    seq[child].__class__ = Doubled
+    assert close(seq(x), 2 * y)
+    compare(seq, x)
+
+
+def test_base4_layers_among_the_children():
+    """ButterflyBase4 folds nothing: its neighbours run as modules."""
+    from butterfly_amd import ButterflyBase4
+    from butterfly_amd.diagonal import Diagonal
+    from butterfly_amd.permutation import FixedPermutation, FusedSequential
+    torch.manual_seed(3)
+    seq = FusedSequential(FixedPermutation(torch.randperm(64)), ButterflyBase4(64, 100, bias=False), Diagonal(100)).cuda()
+    compare(seq, torch.randn(9, 64, device="cuda"))
