@@ -94,12 +94,12 @@ class FusedSequential(nn.Sequential):
     def forward(self, input):
         from .butterfly import Butterfly  # (butterfly.py does not import this module)
         mods = list(self._modules.values())
-        if not input.is_cuda:
-            for m in mods:
-                input = m(input)
-            return input
         i, count = 0, len(mods)
         while i < count:
+            if not input.is_cuda:   # (a child may move the rows)
+                input = mods[i](input)
+                i += 1
+                continue
             # the layer that a permutation, a conversion and a diagonal at position i would lead to
             front = scale_in = to_complex = None
             j = i

@@ -99,3 +99,31 @@ def test_base4_layers_among_the_children():
     torch.manual_seed(3)
     seq = FusedSequential(FixedPermutation(torch.randperm(64)), ButterflyBase4(64, 100, bias=False), Diagonal(100)).cuda()
     compare(seq, torch.randn(9, 64, device="cuda"))
+
+
+def test_a_child_that_moves_the_rows():
+    """Rows that leave the GPU between two layers, and rows that arrive there."""
+    from butterfly_amd.permutation import FusedSequential
+
+    class To(nn.Module):
+        def __init__(self, device):
+            super().__init__()
+            self.device = device
+
+        def forward(self, input):
+            return input.to(self.device)
+
+    there, here = chain(), chain().cpu()
+    x = torch.randn(7, 64)
+    want = here(here(x))
+    calls = []
+    handles = [m.register_forward_hook(lambda m, a, o: calls.append(type(m).__name__)) for m in (here[2], there[2])]
+    down = FusedSequential(*there, To("cpu"), *here)(x.cuda())
+    assert close(down, want)
+    assert calls == ["Diagonal"]      # folded on the GPU, run on the host
+    calls.clear()
+    up = FusedSequential(*here, To("cuda"), *there)(x)
+    assert up.is_cuda and close(up.cpu(), want)
+    assert calls == ["Diagonal"]
+    for handle in handles:
+        handle.remove()
