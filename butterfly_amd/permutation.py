@@ -155,6 +155,8 @@ class FusedSequential(nn.Sequential):
 
     def _fits(self, layer, input, front, to_complex, scale_in):
         """Whether the modules found in front of the layer can be folded into its call on `input`."""
+        if (front is not None or scale_in is not None) and input.size(-1) != layer.in_size:
+            return False   # (the layer pads and trims rows of any width, they do not)
         if to_complex is not None:
             # (the layer's float32 rows are read as they are; other real types are converted first)
             if not layer.complex or input.dtype != torch.float32 or _observed(to_complex, layer):

@@ -101,6 +101,28 @@ def test_base4_layers_among_the_children():
     compare(seq, torch.randn(9, 64, device="cuda"))
 
 
+@pytest.mark.parametrize("width", [50, 90])
+def test_rows_of_another_width(width):
+    """A permutation or diagonal in front of a layer refuses (or trims) rows that are not as wide as it
+    is; the layer alone takes rows of any width."""
+    from butterfly_amd import Butterfly
+    from butterfly_amd.diagonal import Diagonal
+    from butterfly_amd.permutation import FixedPermutation, FusedSequential
+    torch.manual_seed(width)
+    x = torch.randn(5, width, device="cuda")
+    layer = Butterfly(64, 64).cuda()
+    for front in (FixedPermutation(torch.randperm(64)).cuda(), Diagonal(64).cuda()):
+        fused, plain = FusedSequential(front, layer), nn.Sequential(front, layer)
+        if isinstance(front, Diagonal):
+            with pytest.raises(RuntimeError):
+                plain(x)
+            with pytest.raises(RuntimeError):
+                fused(x)
+        elif width > 64:
+            assert close(fused(x), plain(x))
+    assert close(FusedSequential(layer)(x), layer(x))
+
+
 def test_a_child_that_moves_the_rows():
     """Rows that leave the GPU between two layers, and rows that arrive there."""
     from butterfly_amd.permutation import FusedSequential
