@@ -91,8 +91,6 @@ class Butterfly(nn.Module):
         nblocks: number of alternating B / B^T blocks.
     """
 
-    _shares_input = True   # all stacks read the same rows
-
     def __init__(self, in_size, out_size, bias=True, complex=False, increasing_stride=True,
                  init="randn", nblocks=1):
         super().__init__()
@@ -196,8 +194,8 @@ class Butterfly(nn.Module):
             output_size = None
         if conjugate and self.complex:
             twiddle = twiddle.conj()
-        # (out_size of a finished layer may have been lowered: not below its last stack here)
-        native = self._shares_input and input.is_cuda and not subtwiddle and self.out_size > (self.nstacks - 1) * self.n
+        native = (not subtwiddle and self._runs_as_one_call(input)
+                  and getattr(self.bias_rows, "__func__", None) is Butterfly.bias_rows)
         if in_scale is not None or out_scale is not None:
             if native and twiddle.dtype in (torch.float32, torch.complex64):
                 for v in (in_scale, out_scale):
@@ -233,6 +231,14 @@ class Butterfly(nn.Module):
             x = butterfly_multiply_bias(twiddle, x, self.bias_rows(cols, subtwiddle), inc, output_size)
         x = self.post_process(input, x, out_size=x.size(-1) if subtwiddle else None, add_bias=False)
         return x.real if real_output else x
+
+    def _runs_as_one_call(self, input):
+        """Whether the layer operator does what forward does step by step: on device rows, as long as
+        neither a subclass nor the object prepares or finishes them in a way of its own.  (out_size of a
+        finished layer may have been lowered: not below its last stack there.)"""
+        return (input.is_cuda and self.out_size > (self.nstacks - 1) * self.n
+                and getattr(self.pre_process, "__func__", None) is Butterfly.pre_process
+                and getattr(self.post_process, "__func__", None) is Butterfly.post_process)
 
     def effective_twiddle(self):
         """(stacks, nblocks, log_n, n/2, 2, 2) factors the multiply runs with."""
@@ -368,8 +374,6 @@ class ButterflyBmm(Butterfly):
     input: (batch, *, matrix_batch, in_size) -> (batch, *, matrix_batch, out_size).  The
     matrices ride on the stack dimension of one multiply (reference:
     torch_butterfly/butterfly.py:308-397)."""
-
-    _shares_input = False
 
     def __init__(self, in_size, out_size, matrix_batch=1, bias=True, complex=False, increasing_stride=True,
                  init="randn", nblocks=1):

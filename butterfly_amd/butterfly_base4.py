@@ -33,7 +33,7 @@ class ButterflyBase4(Butterfly):
         self.twiddle2._is_structured = True
 
     def forward(self, input):
-        if input.is_cuda and self.out_size > (self.nstacks - 1) * self.n:
+        if self._runs_as_one_call(input):
             return torch.ops.torch_butterfly.butterfly_layer_base4(self.twiddle4, self.twiddle2, input, self.layer_bias(),
                                                                    self.increasing_stride, self.out_size)
         x = self.pre_process(input)

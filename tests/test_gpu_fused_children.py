@@ -1,4 +1,4 @@
-"""What a FusedSequential must not fold away."""
+"""What a FusedSequential must not fold away, and layers whose methods a subclass overrides."""
 import pytest
 import torch
 from torch import nn
@@ -149,3 +149,35 @@ def test_a_child_that_moves_the_rows():
     assert calls == ["Diagonal"]
     for handle in handles:
         handle.remove()
+
+
+@pytest.mark.parametrize("kind", ["Butterfly", "ButterflyUnitary", "ButterflyBase4"])
+@pytest.mark.parametrize("method", ["pre_process", "post_process", "bias_rows"])
+@pytest.mark.parametrize("of_the_class", [True, False])
+def test_overridden_steps_of_a_layer(kind, method, of_the_class):
+    """A layer whose rows are prepared or finished differently, by a subclass or on the object."""
+    import butterfly_amd
+    if method == "bias_rows" and kind == "ButterflyBase4":
+        pytest.skip("its bias is added by post_process")
+    say("steps", kind, method, of_the_class)
+    torch.manual_seed(5)
+    base = getattr(butterfly_amd, kind)
+    layer = base(50, 100, nblocks=2).cuda()
+    x = torch.randn(6, 50, dtype=torch.complex64 if kind == "ButterflyUnitary" else torch.float32, device="cuda")
+    with torch.no_grad():
+        plain = layer(x)
+        no_bias = plain - layer.bias
+        if method == "pre_process":
+            change = lambda self, input: base.pre_process(self, 3 * input)
+            want = 3 * no_bias + layer.bias
+        elif method == "post_process":
+            change = lambda self, *args, **kw: 3 * base.post_process(self, *args, **kw)
+            want = 3 * plain
+        else:
+            change = lambda self, *args, **kw: 3 * base.bias_rows(self, *args, **kw)
+            want = no_bias + 3 * layer.bias
+        if of_the_class:
+            layer.__class__ = type("Changed", (base,), {method: change})
+        else:
+            setattr(layer, method, change.__get__(layer))
+        assert close(layer(x), want)
