@@ -879,10 +879,10 @@ void form_bias_sums_in(Args &a, const bf_problem *p, int64_t nwg, BiasGrad *bg)
 }
 
 // One pass forward (backward == false: x_in -> x_out) or backward (x_in, g_out -> g_in and the
-// pass's partial slices; *nparts receives their number per stage).
+// pass's partial slices, pass4_slices of them).
 int run_pass4(const bf_problem *p, const Schedule &sc, const Pass4 &q, bool backward, const void *tw2, const void *tw4,
               const void *x_in, const StackView &x_view, void *x_out, const StackView &xo_view, const void *g_out,
-              const StackView &g_view, void *g_in, const StackView &gi_view, void *partial, int64_t *nparts, hipStream_t stream,
+              const StackView &g_view, void *g_in, const StackView &gi_view, void *partial, hipStream_t stream,
               BiasGrad *bg = nullptr)
 {
     const int64_t n = (int64_t)1 << p->log_n;
@@ -910,7 +910,6 @@ int run_pass4(const bf_problem *p, const Schedule &sc, const Pass4 &q, bool back
         a.batch = p->batch;
         a.ngroups = g.ngroups;
         a.groups_per_wg = g.groups_per_wg;
-        if (nparts) *nparts = g.nwg;
         form_bias_sums_in(a, p, g.nwg, bg);
         return launch_fast4g(cplx, q.LC, q.inc, backward, a,
                              dim3((unsigned)g.nwg, (unsigned)p->nstacks, (unsigned)(n >> q.LC)), stream);
@@ -935,7 +934,6 @@ int run_pass4(const bf_problem *p, const Schedule &sc, const Pass4 &q, bool back
     a.slot = 4 * n;
     a.batch = p->batch;
     a.rows_per_wg = g.rows_per_wg;
-    if (nparts) *nparts = g.nparts;
     const dim3 grid((unsigned)g.nparts, (unsigned)p->nstacks, (unsigned)g.tiles), block(kStageThreads);
     if (!backward) {
         if (cplx && si.radix4) hipLaunchKernelGGL((stage_fw_kernel<float2, 4>), grid, block, 0, stream, a);
@@ -962,8 +960,7 @@ int long4_forward(const bf_problem *p, const Schedule &sc, const Plan4Long &pl, 
     for (int k = first; k < last; ++k) {
         const int rc = run_pass4(p, sc, pl.pass[k], false, tw2, tw4, k == first ? input : scratch,
                                  k == first ? in_view : dense, k == last - 1 ? output : scratch,
-                                 k == last - 1 ? out_view : dense, nullptr, dense, nullptr, dense, nullptr, nullptr,
-                                 stream);
+                                 k == last - 1 ? out_view : dense, nullptr, dense, nullptr, dense, nullptr, stream);
         if (rc) return rc;
     }
     return BF_OK;
@@ -1267,13 +1264,22 @@ struct BwPlan {
     int64_t slot;       // scalars per stage in the partial buffer
     size_t boundary_bytes;  // one (B, S, n) activation plane
     size_t off_boundaries, off_gbuf, off_partials;
-    size_t total;       // with room for the partial slices of every pass: one reduce for the call
-    size_t least;       // with room for those of one pass at a time: one reduce per pass
+    size_t total;       // what the size queries ask for: partial slices of several passes side by side
+    size_t least;       // what a call needs: those of one pass at a time
     bool fits;
     bool fast;          // register-resident pass plan
     bool fast4;         // base-4 register-resident kernels, one launch per block
     bool long4;         // base-4 rows longer than that: chunk and stage passes
 };
+
+// Room for partial slices that the size queries ask for: those of all passes, for one reduce at the
+// end of the call, up to this size (or what one pass needs).  A schedule may have 96 passes of 40 MiB
+// each; and beyond about half of the 256 MB last-level cache the slices are no longer there when the
+// reduce reads them: sixteen blocks of 1024, 2048 rows: 377 us a call with room for 320 MiB, 359 for 256,
+// 329 for 136, 347 for one pass (40 MiB); 16384 rows: 1043, 1044, 1029, 1021; of 256, 300 rows: 151 with room
+// for all 21 MiB, 180 for one pass.
+constexpr size_t kPartialRoom = (size_t)128 << 20;
+size_t partial_room(size_t most, size_t all) { return std::min(all, std::max(most, kPartialRoom)); }
 
 // saved_boundaries: the activations entering every pass after the first come from the caller
 // (left behind by the forward call that saves them) instead of being recomputed into the workspace.
@@ -1305,7 +1311,7 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, i
         pl.off_partials = off;
         const size_t slices = align256((size_t)pl.nparts * p->nstacks * sc.per * pl.slot * e);
         pl.least = off + slices;
-        pl.total = off + slices * (size_t)p->nblocks;
+        pl.total = off + partial_room(slices, slices * (size_t)p->nblocks);
         return pl;
     }
     const Plan4Long lp = plan4_long(p, base4);
@@ -1328,7 +1334,7 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, i
         off += lp.npass > 1 ? pl.boundary_bytes : 0;
         pl.off_partials = off;
         pl.least = off + most;
-        pl.total = off + all;
+        pl.total = off + partial_room(most, all);
         return pl;
     }
     const PassPlan mp = build_passes(p, base4, false, tables);
@@ -1358,7 +1364,7 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, i
         off += mp.npass > 1 ? pl.boundary_bytes : 0;
         pl.off_partials = off;
         pl.least = off + most;
-        pl.total = off + all;
+        pl.total = off + partial_room(most, all);
         return pl;
     }
     pl.fits = 2 * row_bytes <= kGenericBwLds;
@@ -1489,14 +1495,13 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     if (real && (!pl.fast || p->input_size > n || (bg && (real & kRealOut))))
         return fail(BF_ERR_UNSUPPORTED, "rows of real numbers: register-resident kernels and inputs up to n only");
 
-    // Partial slices: every pass leaves its own behind the previous one's, for one reduce at the end
-    // of the call; where the workspace has no room for that, each pass is reduced before the next.
-    // A reduce also finishes the bias gradient, whose sums the first pass has formed by then.
-    const bool one_reduce = workspace_bytes >= pl.total && pl.total > pl.least;
+    // Partial slices: every pass leaves its own behind the previous one's, and a reduce adds up what
+    // has gathered when the room (or the kernel's list of segments) is full and at the end of the call.
+    // It also finishes the bias gradient, whose sums the first pass has formed by then.
+    const size_t room = workspace_bytes > pl.off_partials ? workspace_bytes - pl.off_partials : 0;
     ReduceSegment segs[kReduceSegments];
     int nsegs = 0;
-    size_t used = 0;   // bytes of the partial area
-    auto partials = [&] { return ws + pl.off_partials + used; };
+    size_t used = 0;   // bytes of the room
     auto finish = [&] {
         if (bg && !bg->formed) {
             const int rc_bias = form_bias_sums(p, grad, g_view, *bg, stream);
@@ -1506,17 +1511,25 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
         bg = nullptr;
         const int n_now = nsegs;
         nsegs = 0;
+        used = 0;
         return launch_reduce(p, sc, segs, n_now, ws + pl.off_partials, pl.slot, d_tw2, d_tw4, stream, now, &g_view);
     };
-    auto reduce = [&](int t0, int t1, int64_t nparts) {
+    // Where the pass over stages [t0, t1) leaves its nparts slices.
+    auto partials = [&](int t0, int t1, int64_t nparts, char **at) {
+        const size_t bytes = align256((size_t)nparts * p->nstacks * (t1 - t0) * pl.slot * e_bytes);
+        if (nsegs > 0 && (used + bytes > room || nsegs == kReduceSegments)) {
+            const int rc_reduce = finish();
+            if (rc_reduce) return rc_reduce;
+        }
+        *at = ws + pl.off_partials + used;
         segs[nsegs++] = ReduceSegment{t0, t1, (int)nparts, (int64_t)(used / 4)};
-        if (!one_reduce) return finish();
-        used += align256((size_t)nparts * p->nstacks * (t1 - t0) * pl.slot * e_bytes);
-        return nsegs == kReduceSegments ? finish() : BF_OK;
+        used += bytes;
+        return BF_OK;
     };
+    char *slices = nullptr;
 
     if (pl.nstages == 0) {
-        if (bg && (rc = reduce(0, 0, 0))) return rc;
+        if (bg && (rc = finish())) return rc;
         return launch_copy_pad(p, grad, g_view, d_input, di_view, stream);
     }
 
@@ -1545,14 +1558,13 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             a.g_view = k == P - 1 ? g_view : dense;
             a.g_in = k == 0 ? d_input : ws + pl.off_gbuf;
             a.gi_view = k == 0 ? dn_view : dense;
-            a.partial = partials();
+            if ((rc = partials(k * per, (k + 1) * per, g.nwg, &slices))) return rc;
+            a.partial = slices;
             a.ngroups = g.ngroups;
             a.groups_per_wg = g.groups_per_wg;
             if (k == P - 1) form_bias_sums_in(a, p, g.nwg, bg);
             const bool inc = (p->increasing_stride != 0) != ((k & 1) != 0);
             rc = launch_fast4g(p->dtype == BF_C64, L, inc, true, a, dim3((unsigned)g.nwg, (unsigned)p->nstacks), stream);
-            if (rc) return rc;
-            rc = reduce(k * per, (k + 1) * per, g.nwg);
             if (rc) return rc;
         }
         if (!general && (reinterpret_cast<uintptr_t>(tw4) & 15) != 0)
@@ -1567,15 +1579,14 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             a.g_view = k == P - 1 ? g_view : dense;
             a.g_in = static_cast<float *>(k == 0 ? d_input : ws + pl.off_gbuf);
             a.gi_view = k == 0 ? dn_view : dense;
-            a.partial = reinterpret_cast<float *>(partials());
+            if ((rc = partials(k * per, (k + 1) * per, g.nwg, &slices))) return rc;
+            a.partial = reinterpret_cast<float *>(slices);
             a.batch = p->batch;
             a.ngroups = g.ngroups;
             a.groups_per_wg = g.groups_per_wg;
             if (k == P - 1) form_bias_sums_in(a, p, g.nwg, bg);
             const bool inc = (p->increasing_stride != 0) != ((k & 1) != 0);
             rc = launch_fast4(L, inc, true, a, dim3((unsigned)g.nwg, (unsigned)p->nstacks), stream);
-            if (rc) return rc;
-            rc = reduce(k * per, (k + 1) * per, g.nwg);
             if (rc) return rc;
         }
         if (nsegs > 0 && (rc = finish())) return rc;
@@ -1623,13 +1634,12 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
         const StackView dn_view = make_view(p->d_input_stride, std::min(p->input_size, n), in_perm);
         for (int k = P - 1; k >= 0; --k) {
             const Pass4 &q = lp.pass[k];
-            int64_t nparts = 0;
+            const int64_t nparts = pass4_slices(p, q) / (q.t1 - q.t0);
+            if ((rc = partials(q.t0, q.t1, nparts, &slices))) return rc;
             rc = run_pass4(p, sc, q, true, tw2, tw4, k == 0 ? input : boundary(k), k == 0 ? x_view : dense, nullptr,
                            dense, k == P - 1 ? grad : ws + pl.off_gbuf, k == P - 1 ? g_view : dense,
-                           k == 0 ? d_input : ws + pl.off_gbuf, k == 0 ? dn_view : dense, partials(), &nparts,
-                           stream, k == P - 1 ? bg : nullptr);
-            if (rc) return rc;
-            rc = reduce(q.t0, q.t1, nparts);
+                           k == 0 ? d_input : ws + pl.off_gbuf, k == 0 ? dn_view : dense, slices, stream,
+                           k == P - 1 ? bg : nullptr);
             if (rc) return rc;
         }
         if (nsegs > 0 && (rc = finish())) return rc;
@@ -1665,9 +1675,9 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             const StackView gv = k == P - 1 ? g_view : dense;
             void *gin = k == 0 ? d_input : ws + pl.off_gbuf;
             const StackView giv = k == 0 ? dn_view : dense;
-            int64_t nparts = 0;
             {
                 const FastGrid g = fast_grid(p->batch, q.L, p->nstacks * pass_lanes(p, q), 1, 1, row_cap(p, true), true);
+                if ((rc = partials(q.t0, q.t1, g.nwg, &slices))) return rc;
                 FastBwArgs a = {};
                 a.tw = tw2;
                 a.tw_stack_stride = sc.tw2_stack_stride;
@@ -1680,11 +1690,10 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 a.g_view = gv;
                 a.g_in = gin;
                 a.gi_view = giv;
-                a.partial = partials();
+                a.partial = slices;
                 a.batch = p->batch;
                 a.ngroups = g.ngroups;
                 a.groups_per_wg = g.groups_per_wg;
-                nparts = g.nwg;
                 a.x_real = k == 0 && (real & kRealIn);
                 a.g_real = k == P - 1 && (real & kRealOut);
                 // (a launch of its own read the gradient once more for rows below 1024: Butterfly(512, 512) at
@@ -1704,8 +1713,6 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 }
                 BF_HIP_CHECK(hipGetLastError());
             }
-            rc = reduce(q.t0, q.t1, nparts);
-            if (rc) return rc;
         }
         if (nsegs > 0 && (rc = finish())) return rc;
         if (p->input_size > n) {
@@ -1734,6 +1741,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
     for (int c = pl.nchunks - 1; c >= 0; --c) {
         const int t0 = c * pl.chunk;
         const int t1 = std::min(pl.nstages, t0 + pl.chunk);
+        if ((rc = partials(t0, t1, have_rows ? pl.nparts : 0, &slices))) return rc;
         if (have_rows) {
             GenericBwArgs a;
             a.sc = sc;
@@ -1748,7 +1756,7 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
             a.g_view = c == pl.nchunks - 1 ? g_view : dense;
             a.g_in = c == 0 ? d_input : ws + pl.off_gbuf;
             a.gi_view = c == 0 ? di_view : dense;
-            a.partial = ws + pl.off_partials;
+            a.partial = slices;
             a.slot = pl.slot;
             const dim3 grid((unsigned)pl.nparts, (unsigned)p->nstacks);
             const size_t lds = (size_t)(t1 - t0 + 1) * n * e;
@@ -1758,10 +1766,8 @@ int backward(const bf_problem *p, bool base4, const void *tw2, const void *tw4, 
                 hipLaunchKernelGGL(generic_bw_kernel<float2>, grid, dim3(kGenericThreads), lds, stream, a);
             BF_HIP_CHECK(hipGetLastError());
         }
-        rc = reduce(t0, t1, have_rows ? pl.nparts : 0);
-        if (rc) return rc;
     }
-    return BF_OK;
+    return nsegs > 0 ? finish() : BF_OK;
 }
 
 // ---- built-in scratch for callers that cannot allocate ----------------------------------------
