@@ -280,6 +280,46 @@ struct ReduceArgs {
     int64_t bias_stride, bias_width, bias_tail;   // scalars
 };
 
+// What the workgroups (x, k, s) of the reduce add up.
+struct ReduceSlice {
+    bool is_bias;       // the bias's column sums, otherwise stage `si` of the factors
+    StageInfo si;
+    int64_t count;      // floats that exist
+    int64_t start;      // floats from the start of the area to the first of the slices
+    int64_t between;    // floats from one slice to the next
+    int nparts;
+};
+
+__host__ __device__ __forceinline__ ReduceSlice reduce_slice(const ReduceArgs &a, int k, int s)
+{
+    const int64_t ef = a.elem_floats;
+    ReduceSlice r = {};
+    r.is_bias = k == a.nstages;
+    if (r.is_bias) {
+        r.count = (s == a.nstacks - 1 ? a.bias_tail : a.bias_width) * ef;
+        r.start = s * a.bias_stride * ef;
+        r.between = a.nstacks * a.bias_stride * ef;
+        r.nparts = a.bias_nparts;
+        return r;
+    }
+    ReduceSegment seg = a.seg[0];
+    int first = 0;   // stages of the segments in front
+    for (int i = 1; i < a.nsegs; ++i) {
+        const int here = first + (a.seg[i - 1].t1 - a.seg[i - 1].t0);
+        if (k < here) break;
+        first = here;
+        seg = a.seg[i];
+    }
+    const int ks = k - first;   // stage within its segment
+    const int64_t nst = seg.t1 - seg.t0, slot = a.slot * ef;
+    r.si = stage_info(a.sc, seg.t0 + ks);
+    r.count = (r.si.radix4 ? 4 : 2) * ((int64_t)1 << a.sc.log_n) * ef;
+    r.start = seg.offset + (s * nst + ks) * slot;
+    r.between = a.nstacks * nst * slot;
+    r.nparts = seg.nparts;
+    return r;
+}
+
 // d_twiddle[s][stage][j] = sum over partial slices.  Works on raw floats (a complex sum is
 // two float sums).  A workgroup covers 64 consecutive floats: thread (q, j4) adds the slices
 // of group q (a contiguous sixteenth of them, ascending) for the float4 at j4; the sixteen
@@ -292,60 +332,43 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(ReduceArgs a)
 {
     __shared__ float4 sm[16][16];
     const int j4 = threadIdx.x & 15, q = threadIdx.x >> 4;
-    const int k = blockIdx.y;
     const int s = blockIdx.z;
-    const bool is_bias = k == a.nstages;
-    ReduceSegment seg = a.seg[0];
-    int first = 0;   // stages of the segments in front
-    for (int i = 1; i < a.nsegs; ++i) {
-        const int here = first + (a.seg[i - 1].t1 - a.seg[i - 1].t0);
-        if (k < here) break;
-        first = here;
-        seg = a.seg[i];
-    }
-    const int ks = is_bias ? 0 : k - first;   // stage within its segment
-    const int nst = seg.t1 - seg.t0;
-    const StageInfo si = stage_info(a.sc, seg.t0 + ks);
-    const int64_t n = (int64_t)1 << a.sc.log_n;
-    const int64_t ef = a.elem_floats;
+    const ReduceSlice r = reduce_slice(a, blockIdx.y, s);
     const int64_t f = (int64_t)blockIdx.x * 64 + j4 * 4;
-    const int64_t slot_f = a.slot * ef;
-    // floats that exist here, floats between the slices, slices
-    const int64_t count = is_bias ? (s == a.nstacks - 1 ? a.bias_tail : a.bias_width) * ef : (si.radix4 ? 4 * n : 2 * n) * ef;
-    const int64_t wg_stride = a.nstacks * (is_bias ? a.bias_stride * ef : nst * slot_f);
-    const int nparts = is_bias ? a.bias_nparts : seg.nparts;
+    const int nparts = r.nparts;
     const int chunk = (nparts + 15) / 16;
     const int w0 = q * chunk;
     const int w1 = w0 + chunk < nparts ? w0 + chunk : nparts;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (f < count) {
-        const float *src = is_bias ? a.bias_partial + s * a.bias_stride * ef + f : a.partial + seg.offset + ((int64_t)s * nst + ks) * slot_f + f;
+    if (f < r.count) {
+        const float *src = (r.is_bias ? a.bias_partial : a.partial) + r.start + f;
 #pragma unroll 8
         for (int w = w0; w < w1; ++w) {
-            const float4 v = *reinterpret_cast<const float4 *>(src + (int64_t)w * wg_stride);
+            const float4 v = *reinterpret_cast<const float4 *>(src + (int64_t)w * r.between);
             acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
         }
     }
     sm[q][j4] = acc;
     __syncthreads();
-    if (q == 0 && f < count) {
+    if (q == 0 && f < r.count) {
         float4 t = sm[0][j4];
 #pragma unroll
         for (int qq = 1; qq < 16; ++qq) {
             const float4 v = sm[qq][j4];
             t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
         }
-        if (is_bias) {
+        const int64_t ef = a.elem_floats;
+        if (r.is_bias) {
             // (any width: neither the columns nor the stacks need start at a multiple of four)
             float *dst = a.d_bias + s * a.bias_width * ef + f;
             const float v[4] = {t.x, t.y, t.z, t.w};
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (f + i < count) dst[i] = v[i];
+                if (f + i < r.count) dst[i] = v[i];
             return;
         }
-        float *dst = si.radix4 ? a.d_tw4 + (s * a.sc.tw4_stack_stride + si.tw_off) * ef
-                               : a.d_tw2 + (s * a.sc.tw2_stack_stride + si.tw_off) * ef;
+        float *dst = r.si.radix4 ? a.d_tw4 + (s * a.sc.tw4_stack_stride + r.si.tw_off) * ef
+                                 : a.d_tw2 + (s * a.sc.tw2_stack_stride + r.si.tw_off) * ef;
         *reinterpret_cast<float4 *>(dst + f) = t;
     }
 }
