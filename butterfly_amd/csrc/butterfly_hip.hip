@@ -975,10 +975,20 @@ int64_t stream_rows_per_wg(const bf_problem *p, int waves, int planes)
     return (int64_t)(4 * planes) << (nbits - p->log_n);
 }
 
-// Tiles of one plane up to which the passes of plan4_long are kept: a workgroup reads the factors of
-// the whole schedule by itself (786 KB at 4096 elements and two blocks, 20.9 us on 12 rows), where
-// the chunk pass spreads that over many (19.2 us).
-constexpr int64_t kStreamMinTiles = 16;
+// Tiles of one plane up to which the passes of plan4_long are kept.  A workgroup reads the factors of
+// the whole schedule by itself, so the launch lasts as long with one tile as with 256; the passes share those
+// reads and their time follows the rows.  One block is few passes, and its line lies later, but for rows of
+// 2048 floats, the cheapest to stream.  It is one line for calls with and without a bias (one more pass) or
+// activations to keep (more stores for the streaming launch): their results agree bit by bit.
+// Passes / streaming at 32, 64 and 96 tiles, us: one block of 4096 floats 10.2 / 13.9, 12.1 / 14.2, 15.1 / 14.5
+// (keeping 10.3 / 15.8, 12.1 / 16.4, 15.4 / 16.9; keeping, with a bias 14.0 / 16.6, 17.1 / 17.2, 21.1 / 17.4); one
+// block of 512 complex64 11.0 / 14.1, 12.6 / 14.5, 15.6 / 14.8 (keeping 10.9 / 17.3, 12.6 / 17.9, 15.6 / 18.1); one
+// block of 2048 floats 9.0 / 10.1, 9.8 / 10.3, 11.0 / 10.5 (with a bias 12.6 / 11.1, 14.2 / 11.3, 15.8 / 11.4); two
+// blocks of 4096 floats 21.1 / 20.9, 24.8 / 21.3, 31.2 / 21.6 (keeping 21.1 / 26.7, 25.5 / 27.6, 29.7 / 28.2).
+int64_t stream_min_tiles(const bf_problem *p)
+{
+    return p->nblocks == 1 && !(p->dtype == BF_F32 && p->log_n == 11) ? 64 : 16;
+}
 
 struct StreamPick {
     int waves = 0, planes = 0;   // 0: another path
@@ -999,7 +1009,7 @@ StreamPick pick_stream(const bf_problem *p, bool base4)
     k.waves = p->log_n == 12 ? 16 : 8;
     const int64_t rows = stream_rows_per_wg(p, k.waves, 1);
     const int64_t tiles = (p->batch + rows - 1) / rows * p->nstacks;
-    if (tiles <= kStreamMinTiles) k.waves = 0;
+    if (tiles <= stream_min_tiles(p)) k.waves = 0;
     k.planes = p->dtype == BF_C64 || tiles <= num_cu() ? 1 : 2;
     return k;
 }
