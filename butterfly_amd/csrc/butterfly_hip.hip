@@ -290,7 +290,8 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
     // complex64 needs twice the registers per stage: one block per LOW pass
     const int max_nb = p->dtype == BF_C64 ? 1 : 2;
     // complex64 rows of 2048 and 4096 with tables: each where a pass over bits 0..5 reads (ascending)
-    // or writes (descending) the rows, so that it can run on the tiles made for that
+    // or writes (descending) the rows, so that it can run on the tiles made for that.  (Not where a
+    // forward call takes whole blocks: 8192 rows of 2048 through a bit reversal 68 us against 102.)
     const bool last_inc = (p->increasing_stride != 0) != (((p->nblocks - 1) & 1) != 0);
     const bool edges = (tables & (kTableIn | kTableOut)) && p->dtype == BF_C64 && (L == 11 || L == 12) &&
                        (!(tables & kTableIn) || p->increasing_stride != 0) && (!(tables & kTableOut) || !last_inc);
@@ -305,7 +306,7 @@ PassPlan build_passes(const bf_problem *p, bool base4, bool forward_only = false
             q.L = L;
             q.inc = (p->increasing_stride != 0) != ((k & 1) != 0);
         }
-    } else if (L <= 12 && forward_only && !edges && !(tables & (kRealIn | kRealOut)) && (p->dtype == BF_F32 || L == 11) &&
+    } else if (L <= 12 && forward_only && !(tables & (kRealIn | kRealOut)) && (p->dtype == BF_F32 || L == 11) &&
                p->batch * p->nstacks >= wide_min_rows(p)) {
         for (int k = 0; k < p->nblocks; ++k) {
             if (pl.npass == kMaxPasses) return pl;

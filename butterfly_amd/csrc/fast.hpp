@@ -154,8 +154,11 @@ struct SpanPlan : PlanOps<SpanPlan<H, MODE>> {
 // the bits 0..5 and all 16 of the top four bits, highest first: behind a bit reversal those are runs
 // of 16 adjacent elements.  Layout A puts the top bits on the lanes and serves the table's side,
 // layout B the bits 0..5 (64 adjacent elements a wavefront) and serves the stages and the other side.
-// For other tables this tile is as good as any.  (lb: log2 of the row length.)
-// special.fft(4096) at 8192 rows: the pass took 206 us forward and 446 backward on chunks of 1024.
+// The host does not read the table and takes this tile for any; against chunks of 1024 adjacent
+// columns it gains on tables that scatter them and loses on those that keep neighbours together.
+// A forward / backward call of 8192 rows of 4096, chunks -> these tiles, us: bit reversal 306 / 820 -> 214 /
+// 500, random 294 / 770 -> 282 / 744, evens before odds 218 / 620 -> 229 / 660, identity 216 / 610 -> 228 / 673;
+// backward of 2048: 364 -> 253, 348 -> 347, 304 -> 336, 305 -> 343.  (lb: log2 of the row length.)
 template <bool INC>
 struct EdgePlan : PlanOps<EdgePlan<INC>> {
     static constexpr int LOG = 10;
