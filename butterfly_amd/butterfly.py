@@ -194,8 +194,7 @@ class Butterfly(nn.Module):
             output_size = None
         if conjugate and self.complex:
             twiddle = twiddle.conj()
-        native = (not subtwiddle and self._runs_as_one_call(input)
-                  and getattr(self.bias_rows, "__func__", None) is Butterfly.bias_rows)
+        native = not subtwiddle and self._runs_as_one_call(input)
         if in_scale is not None or out_scale is not None:
             if native and twiddle.dtype in (torch.float32, torch.complex64):
                 for v in (in_scale, out_scale):
@@ -236,9 +235,10 @@ class Butterfly(nn.Module):
         """Whether the layer operator does what forward does step by step: on device rows, as long as
         neither a subclass nor the object prepares or finishes them in a way of its own.  (out_size of a
         finished layer may have been lowered: not below its last stack there.)"""
+        cls, own = type(self), self.__dict__
         return (input.is_cuda and self.out_size > (self.nstacks - 1) * self.n
-                and getattr(self.pre_process, "__func__", None) is Butterfly.pre_process
-                and getattr(self.post_process, "__func__", None) is Butterfly.post_process)
+                and cls.pre_process is _PRE_PROCESS and cls.post_process is _POST_PROCESS and cls.bias_rows is _BIAS_ROWS
+                and "pre_process" not in own and "post_process" not in own and "bias_rows" not in own)
 
     def effective_twiddle(self):
         """(stacks, nblocks, log_n, n/2, 2, 2) factors the multiply runs with."""
@@ -309,6 +309,9 @@ class Butterfly(nn.Module):
         return (f"in_size={self.in_size}, out_size={self.out_size}, bias={self.bias is not None}, "
                 f"complex={self.complex}, increasing_stride={self.increasing_stride}, "
                 f"init={self.init}, nblocks={self.nblocks}")
+
+
+_PRE_PROCESS, _POST_PROCESS, _BIAS_ROWS = Butterfly.pre_process, Butterfly.post_process, Butterfly.bias_rows
 
 
 class ButterflyUnitary(Butterfly):

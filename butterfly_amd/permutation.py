@@ -5,6 +5,7 @@ import numpy as np
 import torch
 from torch import nn
 
+from .butterfly import Butterfly
 from .complex_utils import Complex2Real, Real2Complex, index_last_dim
 from .diagonal import Diagonal
 
@@ -75,7 +76,7 @@ def _observed(*modules):
 
 def _runs(m, kind):
     """Whether module m computes what `kind` does (a subclass may have a forward of its own)."""
-    return isinstance(m, kind) and type(m).forward is kind.forward
+    return type(m) is kind or (isinstance(m, kind) and type(m).forward is kind.forward)
 
 
 class FusedSequential(nn.Sequential):
@@ -92,7 +93,6 @@ class FusedSequential(nn.Sequential):
     it; hooks on permutations and diagonals do not keep them from being folded."""
 
     def forward(self, input):
-        from .butterfly import Butterfly  # (butterfly.py does not import this module)
         mods = list(self._modules.values())
         i, count = 0, len(mods)
         while i < count:
@@ -348,7 +348,6 @@ def modular_balanced_to_butterfly_factor(L):
 def _butterfly_from_gathers(block0, block1, n, size, complex):
     """Two-block Butterfly (decreasing stride first) from its factors given as gathers
     (x -> x[f]): block0 with block sizes n, n/2, ..., 2 and block1 with 2, 4, ..., n."""
-    from .butterfly import Butterfly  # (butterfly.py does not import this module)
     log_n = n.bit_length() - 1
     planes = []
     for factors, sizes in ((block0, range(log_n, 0, -1)), (block1, range(1, log_n + 1))):
@@ -380,7 +379,6 @@ def _padded_permutation(v):
 def _to_increasing_stride(b, size):
     """The decreasing-stride Butterfly of br[v[br]] read with increasing stride and its pairs
     in bit-reversed order is a Butterfly of v (torch_butterfly/permutation.py:322-330)."""
-    from .butterfly import Butterfly
     n = b.twiddle.shape[3] * 2
     pairs = bitreversal_permutation(n // 2, pytorch_format=True)
     out = Butterfly(n, n, bias=False, complex=b.twiddle.is_complex(), increasing_stride=True,
@@ -498,7 +496,6 @@ def perm2butterfly(v, complex=False, increasing_stride=False):
     """A two-block Butterfly whose matrix is the permutation v: ``b(x) == x[..., v]``.
     v is padded with fixed points to the next power of 2
     (reference: torch_butterfly/permutation.py:395-433)."""
-    from .butterfly import Butterfly  # (butterfly.py does not import this module)
     if isinstance(v, torch.Tensor):
         v = v.detach().cpu().numpy()
     v = np.asarray(v, dtype=np.int64)
