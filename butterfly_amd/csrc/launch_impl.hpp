@@ -106,8 +106,15 @@ void launch_fast4g_t(bool backward, const Fast4GArgs &a, dim3 grid, hipStream_t 
 {
     constexpr int R = sizeof(T) == 4 ? kFast4FwRows : kFast4GFwRowsComplex;
     // row groups per backward iteration: complex64 what the registers next to the factors allow, float
-    // what is faster (32768 rows of 512: 94.7 us a step with two, 88.0 with four)
+    // what is faster.  At 512 four, where a workgroup has as many (32768 rows: 94.7 us a step with two, 88.0
+    // with four; backward call of 2048 rows 21.2, 21.0), two below that (1024 rows 19.2, 20.5; two blocks 43.8, 46.7)
     constexpr int RB = sizeof(T) == 4 ? (L <= 9 ? 4 : 2) : (L <= 6 ? 2 : 1);
+    if constexpr (sizeof(T) == 4 && L == 9) {
+        if (backward && a.groups_per_wg < RB) {
+            hipLaunchKernelGGL((fast4g_bw_kernel<T, L, INC, 2>), grid, dim3(kFastThreads), 0, stream, a);
+            return;
+        }
+    }
     if (backward) hipLaunchKernelGGL((fast4g_bw_kernel<T, L, INC, RB>), grid, dim3(kFastThreads), 0, stream, a);
     else hipLaunchKernelGGL((fast4g_fw_kernel<T, L, INC, R>), grid, dim3(kFastThreads), 0, stream, a);
 }
