@@ -1351,7 +1351,7 @@ BwPlan plan_bw(const bf_problem *p, bool base4, bool saved_boundaries = false, i
     const PassPlan mp = build_passes(p, base4, false, tables);
     if (mp.ok && passes_addressable(p, mp, true)) {
         // boundaries: the activation entering every pass after the first; one gradient plane
-        // that the passes update in place; partial slices sized for the widest pass.
+        // that the passes update in place; room for partial slices.
         pl.fits = true;
         pl.fast = true;
         pl.nchunks = mp.npass;

@@ -18,8 +18,9 @@
 // The factors are not kept from tile to tile: they stream from L2 while the previous level computes,
 // 4 * RB << (NBITS - log_n) rows sharing each read.  Register-resident factors (fast4g.hpp) reach 1024
 // elements; beyond that they need a chunk pass and one pass over memory per remaining stage.
-// Measured against those (float): 1500 rows of 2048, two blocks: 24.6 against 42.9 us; 16384 rows of
-// 2048, two blocks: 131 against 211 us; 16384 rows of 4096, one block: 208 against 661 us.  What bounds
+// Measured against those (float): 1500 rows of 2048, two blocks: 23.5 against 43 us; 16384 rows of 2048,
+// two blocks: 121 against 208 us; 8192 rows of 4096, one block: 99 against 123 us, two blocks 139 against 213;
+// 16384 rows of 4096, one block, which those leave to the LDS fallback: 209 against 658 us.  What bounds
 // it: one workgroup a compute unit at 4096 elements (128 KiB of LDS), whose loads, levels and stores
 // follow one another.
 #pragma once

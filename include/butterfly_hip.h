@@ -74,7 +74,9 @@ int bf_butterfly_multiply_fw(const bf_problem *p, const void *twiddle, const voi
  * launch (n <= 1024 with at most two blocks), one (B, S, n) activation otherwise.          */
 size_t bf_butterfly_multiply_fw_workspace_bytes(const bf_problem *p);
 
-/* Workspace the backward call needs for this problem, in bytes. */
+/* Workspace the backward call asks for, in bytes: one gradient and the activations between passes, (B, S, n)
+ * each, for schedules of several passes, and the partial sums of d_twiddle, those of several passes side
+ * by side up to 128 MiB.                                                                     */
 size_t bf_butterfly_multiply_bw_workspace_bytes(const bf_problem *p);
 
 /* Backward multiply: d_twiddle (dense, twiddle shape, fully overwritten) and d_input
@@ -289,9 +291,9 @@ int bf_layer_bw(const bf_layer *l, const void *input, const void *grad, const vo
  * but the partial sums and intermediate activations live in a fixed area of
  * BF_NOALLOC_SCRATCH_BYTES that is part of the library's device image (one copy per GPU, held
  * until the process ends) instead of a workspace argument.  No counterpart in the reference.
- * The call allocates and frees nothing.  A problem whose backward workspace
- * (bf_butterfly_multiply_bw_workspace_bytes) exceeds the area is refused with
- * BF_ERR_WORKSPACE.  The device that is current must be the one `stream` belongs to.  All
+ * The call allocates and frees nothing.  A problem whose backward does not fit the area with the
+ * partial sums of one pass at a time (bf_butterfly_multiply_bw_workspace_bytes may ask for those of
+ * several) is refused with BF_ERR_WORKSPACE.  The device that is current must be the one `stream` belongs to.  All
  * calls on one GPU share that GPU's area: calls that overlap in time on one GPU (different
  * streams or threads) race; calls ordered on one stream are fine.  The first call on a device
  * looks the area's address up (a host-side query, no allocation); make that call outside a
