@@ -68,10 +68,12 @@ class FixedPermutation(nn.Module):
         return table
 
 
-def _observed(*modules):
-    """Whether a hook on one of these modules, or one on all modules, expects to see its calls."""
-    return nn.modules.module._has_any_global_hook() or any(
-        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+_any_global_hook = nn.modules.module._has_any_global_hook
+
+
+def _hooked(m):
+    """Whether module m has a hook that expects to see its calls."""
+    return m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
 
 
 def _runs(m, kind):
@@ -131,7 +133,7 @@ class FusedSequential(nn.Sequential):
                         and self._permutes(m, layer.out_size)):
                     back = m
                 elif (_runs(m, Complex2Real) and to_real is None and layer.complex and plain
-                      and not _observed(m, layer)):
+                      and not (_hooked(m) or _hooked(layer) or _any_global_hook())):
                     to_real = m
                 else:
                     break
@@ -159,7 +161,8 @@ class FusedSequential(nn.Sequential):
             return False   # (the layer pads and trims rows of any width, they do not)
         if to_complex is not None:
             # (the layer's float32 rows are read as they are; other real types are converted first)
-            if not layer.complex or input.dtype != torch.float32 or _observed(to_complex, layer):
+            if (not layer.complex or input.dtype != torch.float32
+                    or _hooked(to_complex) or _hooked(layer) or _any_global_hook()):
                 return False
         elif input.is_complex() != layer.complex:
             return False
