@@ -76,9 +76,18 @@ def _hooked(m):
     return m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
 
 
-def _runs(m, kind):
-    """Whether module m computes what `kind` does (a subclass may have a forward of its own)."""
-    return type(m) is kind or (isinstance(m, kind) and type(m).forward is kind.forward)
+_KINDS = (FixedPermutation, Real2Complex, Complex2Real, Diagonal, Butterfly)
+
+
+def _kind(m):
+    """Which of _KINDS module m computes, None for any other (a subclass may have a forward of its own)."""
+    t = type(m)
+    if t in _KINDS:
+        return t
+    for kind in _KINDS:
+        if isinstance(m, kind):
+            return kind if t.forward is kind.forward else None
+    return None
 
 
 class FusedSequential(nn.Sequential):
@@ -107,32 +116,34 @@ class FusedSequential(nn.Sequential):
             j = i
             while j < count and scale_in is None:
                 m = mods[j]
-                if _runs(m, FixedPermutation) and front is None:
+                kind = _kind(m)
+                if kind is FixedPermutation and front is None:
                     front = m
-                elif _runs(m, Real2Complex) and to_complex is None:
+                elif kind is Real2Complex and to_complex is None:
                     to_complex = m
-                elif _runs(m, Diagonal):
+                elif kind is Diagonal:
                     scale_in = m
                 else:
                     break
                 j += 1
             layer = mods[j] if j < count else None
-            if not (_runs(layer, Butterfly) and self._fits(layer, input, front, to_complex, scale_in)):
+            if not (_kind(layer) is Butterfly and self._fits(layer, input, front, to_complex, scale_in)):
                 input = mods[i](input)
                 i += 1
                 continue
             i = j + 1
             back = scale_out = to_real = None
             plain = layer.bias is None
-            if i < count and plain and _runs(mods[i], Diagonal) and self._scales(mods[i], layer.out_size, layer):
+            if i < count and plain and _kind(mods[i]) is Diagonal and self._scales(mods[i], layer.out_size, layer):
                 scale_out = mods[i]
                 i += 1
             while i < count:
                 m = mods[i]
-                if (_runs(m, FixedPermutation) and back is None and layer.nstacks == 1
+                kind = _kind(m)
+                if (kind is FixedPermutation and back is None and layer.nstacks == 1
                         and self._permutes(m, layer.out_size)):
                     back = m
-                elif (_runs(m, Complex2Real) and to_real is None and layer.complex and plain
+                elif (kind is Complex2Real and to_real is None and layer.complex and plain
                       and not (_hooked(m) or _hooked(layer) or _any_global_hook())):
                     to_real = m
                 else:
