@@ -151,14 +151,14 @@ def test_a_child_that_moves_the_rows():
         handle.remove()
 
 
-@pytest.mark.parametrize("kind", ["Butterfly", "ButterflyUnitary", "ButterflyBase4"])
-@pytest.mark.parametrize("method", ["pre_process", "post_process", "bias_rows"])
+# (the bias of ButterflyBase4 is added by post_process)
+@pytest.mark.parametrize("kind, method", [(kind, method) for kind in ("Butterfly", "ButterflyUnitary", "ButterflyBase4")
+                                          for method in ("pre_process", "post_process", "bias_rows")
+                                          if (kind, method) != ("ButterflyBase4", "bias_rows")])
 @pytest.mark.parametrize("of_the_class", [True, False])
 def test_overridden_steps_of_a_layer(kind, method, of_the_class):
     """A layer whose rows are prepared or finished differently, by a subclass or on the object."""
     import butterfly_amd
-    if method == "bias_rows" and kind == "ButterflyBase4":
-        pytest.skip("its bias is added by post_process")
     say("steps", kind, method, of_the_class)
     torch.manual_seed(5)
     base = getattr(butterfly_amd, kind)
